@@ -155,6 +155,18 @@ struct LuArgs {
     int* status;      // [0] pivot check failed (needs interchanges), [1] spin timeout
     int n;
 };
+constexpr int kLuThreads = 512;   // of lu_step_kernel: waves 0 .. 3 factor, waves 4 .. 7 own the block's strips
+// Workgroups of lu_step_kernel for one system of a batch of `count`: the panel's 1 + 2 nrb (nrb blocks of 64
+// below the panel's) and those that share panel p-1's nrb^2 trailing tiles.  One workgroup fits a CU and the
+// panel's hold theirs for the whole launch, so beyond kLuTrailing workgroups the tiles are shared out: a
+// workgroup that takes several overlaps the loads of the next with the products of the last (N = 2048, 961
+// tiles: one each takes five rounds of the free CUs, longer than the panel's chain).
+constexpr int kLuTrailing = 192;
+inline int lu_step_grid(int nrb, int k0, int count) {
+    const int tiles = k0 > 0 ? nrb * nrb : 0;
+    const int share = (kLuTrailing + count - 1) / count;
+    return 1 + 2 * nrb + (tiles < share ? tiles : share);
+}
 __global__ void lu_step_kernel(LuArgs a, int k0);
 __global__ void lu_backsolve_kernel(LuArgs a);
 __global__ void gepp_fallback_kernel(const SurfDesc* sd, double* M, const double* b, double* x,

@@ -490,9 +490,9 @@ bool Solver::enqueue_solve(const double2* Z, int stage, bool g1) {
             const double pf = 4.0 * kb * kb * rem + 2.0 * kb * kb * kb;
             const double uf = k0 > 0 ? 2.0 * (n - k0) * (double)(n - k0) * kNB : 0.0;
             const double ub = k0 > 0 ? 8.0 * (2.0 * (n - k0) * (double)(n - k0) + 2.0 * (n - k0) * kNB) : 0.0;
-            const int grid = 1 + 2 * nrb + (k0 > 0 ? nrb * nrb : 0);
+            const int grid = lu_step_grid(nrb, k0, count);
             launch("lu_step", (double)count * (pf + uf), 8.0 * count * (2.0 * kb * rem + kb * kb) + count * ub, [&] {
-                go(lu_step_kernel, dim3(grid, 1, count), dim3(256), 0, a, k0);
+                go(lu_step_kernel, dim3(grid, 1, count), dim3(kLuThreads), 0, a, k0);
             });
         }
         const int P = (n + kNB - 1) / kNB;
@@ -1190,8 +1190,20 @@ namespace sfh {
 // Solves A x = b (n x n, row-major, host arrays) with the device LU path used by the stepper:
 // interchange-free blocked LU, and the GEPP kernel when a multiplier exceeds 1.  Returns 1 in
 // *interchanged when the GEPP kernel ran.  Used to test the solver on arbitrary matrices.
-void debug_lu_solve(int n, const double* A, const double* b, double* x, int* interchanged) {
-    if (n < 1) throw ArgError("n must be positive");
+void debug_lu_solve(int n_in, const double* A_in, const double* b_in, double* x_out, int* interchanged) {
+    if (n_in < 1) throw ArgError("n must be positive");
+    // systems of several panels: rows of the last block row in multiples of 16 (the strips of lu.hip), so
+    // other sizes, which the stepper does not have, are extended by identity rows
+    const int n = n_in > kNB ? (n_in + 15) / 16 * 16 : n_in;
+    std::vector<double> A((size_t)n * n, 0.0), b(n, 0.0), x(n);
+    for (int i = 0; i < n; ++i) {
+        if (i < n_in) {
+            std::memcpy(&A[(size_t)i * n], A_in + (size_t)i * n_in, n_in * sizeof(double));
+            b[i] = b_in[i];
+        } else {
+            A[(size_t)i * n + i] = 1.0;
+        }
+    }
     hipStream_t st;
     SFH_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
     const int P = (n + kNB - 1) / kNB;
@@ -1213,10 +1225,10 @@ void debug_lu_solve(int n, const double* A, const double* b, double* x, int* int
     SFH_HIP(hipMalloc(&dcnt, sizeof(int) * 4));
     SFH_HIP(hipMalloc(&ddesc, sizeof(SurfDesc)));
     SFH_HIP(hipMemcpy(ddesc, &desc, sizeof(desc), hipMemcpyHostToDevice));
-    SFH_HIP(hipMemcpy(dA, A, sizeof(double) * n * n, hipMemcpyHostToDevice));
-    SFH_HIP(hipMemcpy(dA0, A, sizeof(double) * n * n, hipMemcpyHostToDevice));
-    SFH_HIP(hipMemcpy(dwork, b, sizeof(double) * n, hipMemcpyHostToDevice));
-    SFH_HIP(hipMemcpy(db, b, sizeof(double) * n, hipMemcpyHostToDevice));
+    SFH_HIP(hipMemcpy(dA, A.data(), sizeof(double) * n * n, hipMemcpyHostToDevice));
+    SFH_HIP(hipMemcpy(dA0, A.data(), sizeof(double) * n * n, hipMemcpyHostToDevice));
+    SFH_HIP(hipMemcpy(dwork, b.data(), sizeof(double) * n, hipMemcpyHostToDevice));
+    SFH_HIP(hipMemcpy(db, b.data(), sizeof(double) * n, hipMemcpyHostToDevice));
     SFH_HIP(hipMemset(dstatus, 0, sizeof(int) * 2));
     SFH_HIP(hipMemset(dcnt, 0, sizeof(int) * 4));
     LuArgs a{dA, dwork, dy, dx, duinv, dflags, dstatus, n};
@@ -1224,7 +1236,7 @@ void debug_lu_solve(int n, const double* A, const double* b, double* x, int* int
         const int kb = std::min(kNB, n - k0);
         const int rem = n - k0 - kb;
         const int nrb = (rem + kNB - 1) / kNB;
-        hipLaunchKernelGGL(lu_step_kernel, dim3(1 + 2 * nrb + (k0 > 0 ? nrb * nrb : 0), 1, 1), dim3(256), 0, st,
+        hipLaunchKernelGGL(lu_step_kernel, dim3(lu_step_grid(nrb, k0, 1), 1, 1), dim3(kLuThreads), 0, st,
                            a, k0);
     }
     hipLaunchKernelGGL(lu_backsolve_kernel, dim3(P, 1, 1), dim3(256), 0, st, a);
@@ -1237,8 +1249,9 @@ void debug_lu_solve(int n, const double* A, const double* b, double* x, int* int
         hipLaunchKernelGGL(gepp_fallback_kernel, dim3(1), dim3(256), 0, st, ddesc, dA, db, dx, dpiv, dstatus, dcnt);
         SFH_HIP(hipGetLastError());
     }
-    SFH_HIP(hipMemcpyAsync(x, dx, sizeof(double) * n, hipMemcpyDeviceToHost, st));
+    SFH_HIP(hipMemcpyAsync(x.data(), dx, sizeof(double) * n, hipMemcpyDeviceToHost, st));
     SFH_HIP(hipStreamSynchronize(st));
+    std::memcpy(x_out, x.data(), n_in * sizeof(double));
     if (interchanged) *interchanged = status[0] ? 1 : 0;
     void* bufs[] = {dA, dA0, dwork, db, dy, dx, duinv, dflags, dstatus, dpiv, dcnt, ddesc};
     for (void* p : bufs) (void)hipFree(p);
