@@ -21,8 +21,10 @@
 //     x0 + V y as the solution, each workgroup its own rows, and pushes them into the warm-start
 //     history (a launch that finds convergence earlier only keeps y for it).  The initial guess
 //     x0 and the solution are separate arrays.
-//   step i: w_i = M v_i for the workgroup's rows (one row per wave, the row's loads issued at the
+//   step i: w_i = M v_i for the workgroup's rows (one or two rows per wave, the first loads issued at the
 //     kernel's start so they overlap the finishing work), and the partial dots v_l . w_i, l <= i.
+//     For the film w_i = M P^{-1} v_i with the preconditioner P of its image term (precondition), and
+//     the solution is x0 + P^{-1} V y, P^{-1} V being kept beside V.
 // Launch 0 takes v_0 = r0 / |r0|.  The assembly kernel forms r0 = b - M x0 while it writes M
 // (assemble.hip), and every workgroup of launch 0 reduces |r0| and |b| over its own full copies.
 // L launches therefore run up to L - 1 Arnoldi steps.  Once the residual estimate reaches
@@ -38,118 +40,204 @@
 
 namespace sfh {
 
-// Row R (global) times vs (LDS) by one wave, in two halves so the first 2048 columns' loads can
-// be issued before vs is ready: row_load issues 32 loads per lane (predicated at the row end),
-// row_dot_rest finishes the product (columns beyond 2048 are loaded and used chunk by chunk).
-// The matrix is FP64, or FP32 in the mixed-precision form (entries widened to FP64 as they are used).
-template <typename T>
-struct RowChunk {
-    T mv[32];
+// RR rows of the matrix (row r at R + r n) times vs (LDS) by one wave.  The rows stream through two
+// register buffers of 1024 / RR columns each, one refilled while the other is multiplied; row_start fills both
+// before vs is ready.  The matrix is FP64, or FP32 in the mixed-precision form (entries widened to FP64
+// as they are used).  Loads beyond the row's end are clamped to its last entry and meet a zero.
+template <typename T, int RR>
+struct RowBuf {
+    T v[2][RR][16 / RR];
 };
-template <typename T>
-__device__ inline void row_load(const T* __restrict__ R, int n, int lane, RowChunk<T>& rc) {
+template <typename T, int RR>
+__device__ inline void row_load(const T* __restrict__ R, int n, int rows, int c0, int lane, T (&v)[RR][16 / RR]) {
 #pragma unroll
-    for (int u = 0; u < 32; ++u) {
-        const int c = lane + 64 * u;
-        rc.mv[u] = c < n ? R[c] : T(0);
-    }
+    for (int u = 0; u < 16 / RR; ++u)
+#pragma unroll
+        for (int r = 0; r < RR; ++r) v[r][u] = R[(unsigned)min(r, rows - 1) * (unsigned)n + (unsigned)min(c0 + lane + 64 * u, n - 1)];
 }
-template <typename T>
-__device__ inline double row_dot_rest(const T* __restrict__ R, const RowChunk<T>& rc, const double* vs, int n,
-                                      int lane) {
-    double a0 = 0.0, a1 = 0.0;
+template <typename T, int RR>
+__device__ inline void row_start(const T* __restrict__ R, int n, int rows, int lane, RowBuf<T, RR>& b) {
+    row_load(R, n, rows, 0, lane, b.v[0]);
+    if (n > 1024 / RR) row_load(R, n, rows, 1024 / RR, lane, b.v[1]);
+}
+template <typename T, int RR>
+__device__ inline void row_dots(const T* __restrict__ R, RowBuf<T, RR>& b, const double* vs, int n, int rows, int lane,
+                                double (&out)[RR]) {
+    constexpr int C = 1024 / RR;
+    double acc[RR][2];
 #pragma unroll
-    for (int u = 0; u < 32; u += 2) {
-        const int c = lane + 64 * u;
-        a0 += (double)rc.mv[u] * (c < n ? vs[c] : 0.0);
-        a1 += (double)rc.mv[u + 1] * (c + 64 < n ? vs[c + 64] : 0.0);
-    }
-    for (int c0 = 32 * 64; c0 < n; c0 += 32 * 64) {
-        T mv[32];
+    for (int r = 0; r < RR; ++r) acc[r][0] = acc[r][1] = 0.0;
+    auto use = [&](int c0, T(&v)[RR][16 / RR]) {
 #pragma unroll
-        for (int u = 0; u < 32; ++u) {
+        for (int u = 0; u < 16 / RR; ++u) {
             const int c = c0 + lane + 64 * u;
-            mv[u] = c < n ? R[c] : T(0);
-        }
+            const double x = c < n ? vs[c] : 0.0;
 #pragma unroll
-        for (int u = 0; u < 32; u += 2) {
-            const int c = c0 + lane + 64 * u;
-            a0 += (double)mv[u] * (c < n ? vs[c] : 0.0);
-            a1 += (double)mv[u + 1] * (c + 64 < n ? vs[c + 64] : 0.0);
+            for (int r = 0; r < RR; ++r) acc[r][u & 1] += (double)v[r][u] * x;
+        }
+    };
+    for (int c0 = 0; c0 < n; c0 += 2 * C) {
+        use(c0, b.v[0]);
+        if (c0 + 2 * C < n) row_load(R, n, rows, c0 + 2 * C, lane, b.v[0]);
+        if (c0 + C < n) {
+            use(c0 + C, b.v[1]);
+            if (c0 + 3 * C < n) row_load(R, n, rows, c0 + 3 * C, lane, b.v[1]);
         }
     }
-    return wave_sum(a0 + a1);
+#pragma unroll
+    for (int r = 0; r < RR; ++r) out[r] = wave_sum(acc[r][0] + acc[r][1]);
 }
 
-// u = w - sum_{i<j} co[i] V[i] over all n entries into vs (LDS, unless null); returns |u|^2 over
-// the workgroup.
-// Each thread handles 8 entries per pass with the basis loads of 4 vectors in flight together.
-// The entries of rows [r0, r0 + kRowsPerWG) are also stored into Vj (when not null).
-__device__ inline void load_first_pass(const double* __restrict__ w, int n, double (&u)[8]) {
+// u = w - sum_{i<j} co[i] V[i] over all n entries into vs (LDS); returns |u|^2 over the workgroup
+// of NT threads.  Each thread handles E entries per pass with the basis loads of 4 vectors in
+// flight together; pre and v0pre hold the first pass of w and V[0].
+template <int NT, int E>
+__device__ inline void load_first_pass(const double* __restrict__ w, int n, double (&u)[E]) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const int c = threadIdx.x + 256 * e;
+    for (int e = 0; e < E; ++e) {
+        const int c = threadIdx.x + NT * e;
         u[e] = c < n ? w[c] : 0.0;
     }
 }
-__device__ inline double rebuild_vector(const double* __restrict__ w, const double* __restrict__ V,
-                                        const double* co, int j, int n, int r0, double* vs, double* Vj,
-                                        double* red4, const double* pre = nullptr,
-                                        const double* v0pre = nullptr) {
+template <int NT, int E>
+__device__ inline double rebuild_vector(const double* __restrict__ w, const double* __restrict__ V, const double* co,
+                                        int j, int n, double* vs, double* red, const double (&pre)[E],
+                                        const double (&v0pre)[E]) {
     const int t = threadIdx.x;
     double ss = 0.0;
-    for (int base = 0; base < n; base += 8 * 256) {
-        double u[8];
-        if (pre && base == 0) {
+    for (int base = 0; base < n; base += E * NT) {
+        double u[E];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) u[e] = pre[e];
-        } else {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int c = base + t + 256 * e;
-                u[e] = c < n ? w[c] : 0.0;
-            }
+        for (int e = 0; e < E; ++e) {
+            const int c = base + t + NT * e;
+            u[e] = base == 0 ? pre[e] : (c < n ? w[c] : 0.0);
         }
         int i = 0;
         for (; i + 4 <= j; i += 4) {
-            double vv[4][8];
+            double vv[4][E];
 #pragma unroll
             for (int q = 0; q < 4; ++q)
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int c = base + t + 256 * e;
-                    vv[q][e] = (v0pre && base == 0 && i + q == 0) ? v0pre[e]
-                                                                   : (c < n ? V[(long long)(i + q) * n + c] : 0.0);
+                for (int e = 0; e < E; ++e) {
+                    const int c = base + t + NT * e;
+                    vv[q][e] = (base == 0 && i + q == 0) ? v0pre[e] : (c < n ? V[(long long)(i + q) * n + c] : 0.0);
                 }
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const double cq = co[i + q];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) u[e] -= cq * vv[q][e];
+                for (int e = 0; e < E; ++e) u[e] -= cq * vv[q][e];
             }
         }
         for (; i < j; ++i) {
-            double vv[8];
+            double vv[E];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int c = base + t + 256 * e;
-                vv[e] = (v0pre && base == 0 && i == 0) ? v0pre[e] : (c < n ? V[(long long)i * n + c] : 0.0);
+            for (int e = 0; e < E; ++e) {
+                const int c = base + t + NT * e;
+                vv[e] = (base == 0 && i == 0) ? v0pre[e] : (c < n ? V[(long long)i * n + c] : 0.0);
             }
             const double ci = co[i];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) u[e] -= ci * vv[e];
+            for (int e = 0; e < E; ++e) u[e] -= ci * vv[e];
         }
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int c = base + t + 256 * e;
+        for (int e = 0; e < E; ++e) {
+            const int c = base + t + NT * e;
             if (c < n) {
-                if (vs) vs[c] = u[e];
+                vs[c] = u[e];
                 ss += u[e] * u[e];
-                if (Vj && c >= r0 && c < r0 + kRowsPerWG) Vj[c] = u[e];
             }
         }
     }
-    return block_sum4(ss, red4);
+    return block_sum<NT / 64>(ss, red);
+}
+
+// The film's right preconditioner: vs = P^{-1} vs (LDS, all n entries; NT threads).  On a flat film at
+// the surface's mean height y the direct kernel vanishes and the image term is circulant, a Poisson
+// kernel: its eigenvalue on the Fourier modes +-m of the node index is lam_m = 1/2 + n/(4 pi) exp(-2 m (y + h))
+// (createM.cuh:87-88 has no Z'_k factor, so it grows with n).  These few large eigenvalues are what an
+// unpreconditioned solve spends its steps on: with P = that matrix a warm-started film solve takes 1-2 steps
+// in place of 4-7 (N = 768 .. 4096, h = 1), a cold one 5-9 in place of 10-13: 66.3 -> 34.6 ms per 40 steps of
+// the N = 4096 film.  lam_m falls to 1/2 within a few modes, so P^{-1} = 2 + the modes' (1/lam_m - 2)
+// projections, m <= modes.  GMRES on M P^{-1} leaves the residual b - M x what it was, and the tolerance on it.
+template <int NT>
+__device__ inline void precondition(double* vs, int n, const double2* __restrict__ tw, int modes, double height,
+                                    double (*red)[2 * kPreModes + 1], double* coef) {
+    constexpr int NW = NT / 64;
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const double2 w0 = tw[min(t, n - 1)], ws = tw[NT % n];   // (cos, -sin) of the first entry's angle, of a step of NT
+    double s0 = 0.0, ac[kPreModes], as[kPreModes];
+#pragma unroll
+    for (int m = 0; m < kPreModes; ++m) ac[m] = as[m] = 0.0;
+    double c = w0.x, s = -w0.y;
+    for (int j = t; j < n; j += NT) {
+        const double u = vs[j];
+        s0 += u;
+        double c1 = 1.0, s1 = 0.0, cm = c, sm = s;
+#pragma unroll
+        for (int m = 0; m < kPreModes; ++m) {
+            if (m >= modes) break;
+            ac[m] += u * cm;
+            as[m] += u * sm;
+            const double cn = 2.0 * c * cm - c1, sn = 2.0 * c * sm - s1;   // the next mode, by recurrence
+            c1 = cm;
+            s1 = sm;
+            cm = cn;
+            sm = sn;
+        }
+        const double cr = c * ws.x + s * ws.y;   // angle + the step's
+        s = s * ws.x - c * ws.y;
+        c = cr;
+    }
+    s0 = wave_sum(s0);
+    if (lane == 0) red[wv][0] = s0;
+#pragma unroll
+    for (int m = 0; m < kPreModes; ++m) {
+        if (m >= modes) break;
+        const double x = wave_sum(ac[m]), y = wave_sum(as[m]);
+        if (lane == 0) {
+            red[wv][2 * m + 1] = x;
+            red[wv][2 * m + 2] = y;
+        }
+    }
+    __syncthreads();
+    if (t <= 2 * modes) {
+        double x = 0.0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) x += red[w][t];
+        const int m = (t + 1) >> 1;
+        const double lam = 0.5 + n * (0.25 / kPi) * exp(-2.0 * m * height);
+        coef[t] = x * (m == 0 ? 1.0 : 2.0) / n * (1.0 / lam - 2.0);
+    }
+    __syncthreads();
+    const double a0 = coef[0];
+#pragma unroll
+    for (int m = 0; m < kPreModes; ++m) {
+        if (m >= modes) break;
+        ac[m] = coef[2 * m + 1];
+        as[m] = coef[2 * m + 2];
+    }
+    c = w0.x;
+    s = -w0.y;
+    for (int j = t; j < n; j += NT) {
+        double z = 2.0 * vs[j] + a0;
+        double c1 = 1.0, s1 = 0.0, cm = c, sm = s;
+#pragma unroll
+        for (int m = 0; m < kPreModes; ++m) {
+            if (m >= modes) break;
+            z += ac[m] * cm + as[m] * sm;
+            const double cn = 2.0 * c * cm - c1, sn = 2.0 * c * sm - s1;
+            c1 = cm;
+            s1 = sm;
+            cm = cn;
+            sm = sn;
+        }
+        vs[j] = z;
+        const double cr = c * ws.x + s * ws.y;
+        s = s * ws.x - c * ws.y;
+        c = cr;
+    }
+    __syncthreads();
 }
 
 // Rotates column jc of the Hessenberg matrix (entries 0..jc+1 in col, LDS) by the stored rotations
@@ -185,9 +273,11 @@ __device__ inline void back_substitute(const double* g, const double* H, int m, 
     }
 }
 
-// Launch i of a solve's sequence (see the file comment).
-template <typename T>
-__global__ __launch_bounds__(256) void gm_iter_kernel(GmArgs a, const SurfDesc* __restrict__ sd, int i) {
+// Launch i of a solve's sequence (see the file comment), W waves of RR matrix rows each per workgroup
+// (a.rpw rows).  Every workgroup repeats the finishing work (the basis, the partial sums, the
+// preconditioner), so the rows per workgroup follow the size (Solver::alloc_gmres).
+template <typename T, int W, int RR>
+__global__ __launch_bounds__(64 * W) void gm_iter_kernel(GmArgs a, const SurfDesc* __restrict__ sd, int i) {
     GmCtl* ctl = reinterpret_cast<GmCtl*>(a.ctl) + blockIdx.z;
     // solves finished by an earlier launch return at once.  A finish stamped by this launch
     // (workgroup 0 can get there before a late workgroup starts) does not count.  Launch 0 needs
@@ -199,18 +289,20 @@ __global__ __launch_bounds__(256) void gm_iter_kernel(GmArgs a, const SurfDesc* 
     }
     const GmView v = gm_view(a, sd);
     const int m = a.m;
-    const int rpw = kRowsPerWG;
+    constexpr int rpw = W * RR, NT = 64 * W, E = 8;   // E entries per thread and pass
+    static_assert(rpw != 16 || NT * E >= kGmMaxN, "the largest surface in one pass");
     if ((int)blockIdx.x * rpw >= v.n) return;
     __shared__ double vs[kGmMaxN];
     __shared__ double co[kMaxKrylov + 1];
     __shared__ double col[kMaxKrylov + 2];
-    __shared__ double red8[8];
-    __shared__ double wl[kRowsPerWG];
+    __shared__ double red8[2 * W];
+    __shared__ double wl[rpw], vown[rpw];
+    __shared__ double pred[W][2 * kPreModes + 1], pcoef[2 * kPreModes + 1];
     __shared__ double sums[kMaxKrylov + 2];
     __shared__ double ys[kMaxKrylov + 4];   // g[j], gc[j+1], c, s, then y
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6, n = v.n;
     const int r0 = blockIdx.x * rpw;
-    const int row = r0 + wv;
+    const int row = r0 + wv * RR, rows = max(1, min(RR, n - row));   // this wave's rows (at least one is loaded)
     const T* R = (sizeof(T) == 8 ? reinterpret_cast<const T*>(v.M) : reinterpret_cast<const T*>(v.M32)) +
                  (long long)min(row, n - 1) * n;
     const long long pslot = (long long)v.nwg * (m + 1);   // one partial-dot slot per launch parity
@@ -220,26 +312,28 @@ __global__ __launch_bounds__(256) void gm_iter_kernel(GmArgs a, const SurfDesc* 
     const int j = i - 1;
     const double* wprev = (j & 1) ? v.w1 : v.w0;
     const double* part = v.part + (j & 1) * pslot;
-    double pa[8], pb[8];   // first 2048 entries: launch 0 r0 and b, later w_{i-1} and V[0]
+    double pa[E], pb[E];   // first pass: launch 0 r0 and b, later w_{i-1} and V[0]
     DotLoads dl;
     const bool fastdots = i >= 1 && dots_fast(v.nwg, i);
     double sc_t = 0.0, gold = 0.0, bnorm = 0.0;
     if (i == 0) {
-        load_first_pass(v.V, n, pa);
-        load_first_pass(v.b, n, pb);
+        load_first_pass<NT>(v.V, n, pa);
+        load_first_pass<NT>(v.b, n, pb);
     } else {
-        load_first_pass(wprev, n, pa);
-        load_first_pass(v.V, n, pb);
-        if (fastdots) dots_load(part, v.nwg, i, dl);
+        load_first_pass<NT>(wprev, n, pa);
+        load_first_pass<NT>(v.V, n, pb);
+        if (fastdots) dots_load<NT>(part, v.nwg, i, dl);
         sc_t = t <= j ? v.sc[t] : 0.0;
         gold = v.gc[j];
         bnorm = ctl->bnorm;
     }
+    const int pre_modes = a.pre ? v.ctl->pre_modes : -1;
+    const double height = a.pre ? v.ctl->height : 0.0;
     // the rows up front, except in a refinement solve, which most often ends at once: there they
     // are fetched when the step is known to run
-    RowChunk<T> rc;
+    RowBuf<T, RR> rc;
     const bool early_rows = !a.check_first;
-    if (i < m - 1 && early_rows) row_load(R, n, lane, rc);
+    if (i < m - 1 && early_rows) row_start(R, n, rows, lane, rc);
     if (i == 1 && !a.check_first) {
         const int fin = ctl->done;
         if (fin != 0 && fin <= i) return;
@@ -256,7 +350,7 @@ __global__ __launch_bounds__(256) void gm_iter_kernel(GmArgs a, const SurfDesc* 
     for (int l = 0; l < kHistDepth - 1; ++l) ho[l] = 0.0;
     if (t < rpw) {
         xo = v.x[oc];
-        vo0 = v.V[oc];
+        vo0 = v.Z[oc];
         if (h0) {
 #pragma unroll
             for (int l = 0; l < kHistDepth - 1; ++l) ho[l] = h0[(long long)l * a.total + oc];
@@ -265,10 +359,10 @@ __global__ __launch_bounds__(256) void gm_iter_kernel(GmArgs a, const SurfDesc* 
     if (i == 0) {
         // v_0 = r0 / |r0|; beta = |r0| and |b| reduced by every workgroup over its own copies
         double sq = 0.0, bq = 0.0;
-        for (int base = 0; base < n; base += 2048) {
+        for (int base = 0; base < n; base += NT * E) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int c = base + t + 256 * e;
+            for (int e = 0; e < E; ++e) {
+                const int c = base + t + NT * e;
                 const double x = base == 0 ? pa[e] : (c < n ? v.V[c] : 0.0);
                 const double bc = base == 0 ? pb[e] : (c < n ? v.b[c] : 0.0);
                 if (c < n) {
@@ -282,11 +376,16 @@ __global__ __launch_bounds__(256) void gm_iter_kernel(GmArgs a, const SurfDesc* 
         bq = wave_sum(bq);
         if (lane == 0) {
             red8[wv] = sq;
-            red8[4 + wv] = bq;
+            red8[W + wv] = bq;
         }
         __syncthreads();
-        const double beta = sqrt(red8[0] + red8[1] + red8[2] + red8[3]);
-        const double bnorm = sqrt(red8[4] + red8[5] + red8[6] + red8[7]);
+        sq = bq = 0.0;
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            sq += red8[w];
+            bq += red8[W + w];
+        }
+        const double beta = sqrt(sq), bnorm = sqrt(bq);
         if (blockIdx.x == 0 && t == 0) {
             ctl->bnorm = bnorm;
             ctl->beta = beta;
@@ -300,12 +399,12 @@ __global__ __launch_bounds__(256) void gm_iter_kernel(GmArgs a, const SurfDesc* 
     } else {
         // ---- finish step i - 1
         if (fastdots)
-            dots_finish(dl, j + 1, sums);
+            dots_finish<NT>(dl, j + 1, sums);
         else
-            reduce_partials(part, v.nwg, j + 1, sums);
+            reduce_partials<NT>(part, v.nwg, j + 1, sums);
         if (t <= j) co[t] = sums[t] * sc_t;
         __syncthreads();
-        const double hn = sqrt(rebuild_vector(wprev, v.V, co, j + 1, n, 0, vs, nullptr, red8, pa, pb));
+        const double hn = sqrt(rebuild_vector<NT, E>(wprev, v.V, co, j + 1, n, vs, red8, pa, pb));
         if (t == 0) {
             for (int q = 0; q <= j; ++q) col[q] = sums[q];
             col[j + 1] = hn;
@@ -335,7 +434,7 @@ __global__ __launch_bounds__(256) void gm_iter_kernel(GmArgs a, const SurfDesc* 
         if (done && !conv && blockIdx.x == 0 && t == 0) ctl->unconverged += 1;
         if (!done) {
             // V[i] = u: this workgroup's rows (every workgroup holds all of u in LDS)
-            if (t < kRowsPerWG && r0 + t < n) v.V[(long long)i * n + r0 + t] = vs[r0 + t];
+            if (t < rpw && r0 + t < n) v.V[(long long)i * n + r0 + t] = vs[r0 + t];
             sj = hn > 0.0 ? 1.0 / hn : 0.0;
         } else if (t == 0) {
             back_substitute(v.g, v.H, m, k, gj, col, ys + 4);   // then scaled by sc
@@ -364,7 +463,7 @@ __global__ __launch_bounds__(256) void gm_iter_kernel(GmArgs a, const SurfDesc* 
             const int c = r0 + t;
             double x = xo;
             if (k > 0) x += ys[4] * vo0;
-            for (int q = 1; q < k; ++q) x += ys[4 + q] * v.V[(long long)q * n + c];
+            for (int q = 1; q < k; ++q) x += ys[4 + q] * v.Z[(long long)q * n + c];
             v.sol[c] = x;
             if (h0) {
 #pragma unroll
@@ -379,27 +478,36 @@ __global__ __launch_bounds__(256) void gm_iter_kernel(GmArgs a, const SurfDesc* 
         }
         return;
     }
-    // ---- step i: w_i = M v_i (v_i = sj * vs) for this workgroup's rows, partial dots v_l . w_i
-    double vrow[kRowsPerWG];
+    // ---- step i: w_i = M P^{-1} v_i (v_i = sj * vs) for this workgroup's rows, partial dots v_l . w_i
+    if (t < rpw) vown[t] = vs[min(r0 + t, n - 1)];
+    if (a.pre) {
+        __syncthreads();
+        const SurfDesc d = sd[blockIdx.z];
+        if (pre_modes >= 0) precondition<NT>(vs, n, a.tw + d.twoff, pre_modes, height, pred, pcoef);
+        if (t < rpw && r0 + t < n) v.Z[(long long)i * n + r0 + t] = vs[r0 + t];
+    }
+    double vrow[rpw];
 #pragma unroll
-    for (int r = 0; r < kRowsPerWG; ++r)
-        vrow[r] = (t < i && r0 + r < n) ? v.V[(long long)t * n + r0 + r] : 0.0;
+    for (int r = 0; r < rpw; ++r) vrow[r] = (t < i && r0 + r < n) ? v.V[(long long)t * n + r0 + r] : 0.0;
     const double sct = (t < i) ? v.sc[t] : 0.0;
     double* wi = (i & 1) ? v.w1 : v.w0;
-    if (!early_rows) row_load(R, n, lane, rc);
-    const double d = row < n ? sj * row_dot_rest(R, rc, vs, n, lane) : 0.0;
+    if (!early_rows) row_start(R, n, rows, lane, rc);
+    double d[RR];
+    row_dots(R, rc, vs, n, rows, lane, d);
     if (lane == 0) {
-        wl[wv] = row < n ? d : 0.0;
-        if (row < n) wi[row] = d;
+#pragma unroll
+        for (int r = 0; r < RR; ++r) {
+            wl[wv * RR + r] = row + r < n ? sj * d[r] : 0.0;
+            if (row + r < n) wi[row + r] = sj * d[r];
+        }
     }
     __syncthreads();
     if (t <= i) {
         double s = 0.0;
 #pragma unroll
-        for (int r = 0; r < kRowsPerWG; ++r) {
-            const int rw = r0 + r;
-            if (rw < n) {
-                const double vi = (t == i) ? sj * vs[rw] : sct * vrow[r];
+        for (int r = 0; r < rpw; ++r) {
+            if (r0 + r < n) {
+                const double vi = (t == i) ? sj * vown[r] : sct * vrow[r];
                 s += vi * wl[r];
             }
         }
@@ -410,7 +518,7 @@ __global__ __launch_bounds__(256) void gm_iter_kernel(GmArgs a, const SurfDesc* 
         // the two sums alone by velocity_gm1_kernel
         double s = 0.0;
 #pragma unroll
-        for (int r = 0; r < kRowsPerWG; ++r) s += wl[r] * wl[r];
+        for (int r = 0; r < rpw; ++r) s += wl[r] * wl[r];
         v.part[(long long)v.nwg + blockIdx.x] = s;
     }
 }
@@ -428,9 +536,11 @@ __global__ __launch_bounds__(256) void gm_iter_kernel(GmArgs a, const SurfDesc* 
 // LDS, so that the finishing work runs on data already at hand.  A workgroup reads the initial
 // guess, the basis and earlier launches' results, never the solution entries that other
 // workgroups of this launch are storing.  grid = (ceil(max n / kCircRowsPerWG), surfaces).
+template <bool PRE>
 __global__ __launch_bounds__(256) void gm_close_mu_kernel(GmArgs a, const SurfDesc* __restrict__ sd,
                                                           const double* __restrict__ circ,
                                                           double2* __restrict__ mup, int i) {
+    constexpr int NT = 256;
     constexpr int CR = kCircRowsPerWG;
     constexpr int KM = kMaxKrylov;
     static_assert(kCircPer == 8, "the first staged chunk reuses the 8-entry first passes");
@@ -467,10 +577,15 @@ __global__ __launch_bounds__(256) void gm_close_mu_kernel(GmArgs a, const SurfDe
     }
     const double* wprev = (j & 1) ? v.w1 : v.w0;
     double xpre[8], v0pre[8], v1pre[8], wpre[8];
-    load_first_pass(v.x, n, xpre);
-    load_first_pass(v.V, n, v0pre);
-    load_first_pass(j >= 1 ? v.V + n : v.V, n, v1pre);
-    load_first_pass(wprev, n, wpre);
+    load_first_pass<NT>(v.x, n, xpre);
+    load_first_pass<NT>(v.V, n, v0pre);
+    load_first_pass<NT>(j >= 1 ? v.V + n : v.V, n, v1pre);
+    load_first_pass<NT>(wprev, n, wpre);
+    double z0pre[8], z1pre[8];   // with a preconditioner: Z[0], Z[1]
+    if constexpr (PRE) {
+        load_first_pass<NT>(v.Z, n, z0pre);
+        load_first_pass<NT>(j >= 1 ? v.Z + n : v.Z, n, z1pre);
+    }
     const long long pslot = (long long)v.nwg * (m + 1);
     const double* part = v.part + (j & 1) * pslot;
     DotLoads dl;
@@ -544,7 +659,7 @@ __global__ __launch_bounds__(256) void gm_close_mu_kernel(GmArgs a, const SurfDe
                 }
                 for (int l = 2; l <= j; ++l) {
                     double vv[8];
-                    load_first_pass(v.V + (long long)l * n, n, vv);
+                    load_first_pass<NT>(v.V + (long long)l * n, n, vv);
 #pragma unroll
                     for (int e = 0; e < 8; ++e) u[e] -= co[l] * vv[e];
                 }
@@ -571,7 +686,7 @@ __global__ __launch_bounds__(256) void gm_close_mu_kernel(GmArgs a, const SurfDe
                 if (c < n) ss += u[e] * u[e];
             }
         }
-        const double hn = sqrt(block_sum4(ss, red8));
+        const double hn = sqrt(block_sum<4>(ss, red8));
         if (t == 0) {
             for (int q = 0; q <= j; ++q) col[q] = sums[q];
             col[j + 1] = hn;
@@ -604,7 +719,7 @@ __global__ __launch_bounds__(256) void gm_close_mu_kernel(GmArgs a, const SurfDe
         __syncthreads();
     }
     if (h0 && s == 0 && blockIdx.x == 0 && t == 0) count_history(a);
-    // mu = x0 + y_0 V[0] + y_1 V[1] (+ the rest when k > 2), without branches in the common case
+    // mu = x0 + y_0 Z[0] + y_1 Z[1] (+ the rest when k > 2), without branches in the common case
     const double y0 = k > 0 ? ys[4] : 0.0, y1 = k > 1 ? ys[5] : 0.0;
     double2 a0s = {0.0, 0.0}, a1s = {0.0, 0.0};
     for (int j0 = 0; j0 < n; j0 += kCircChunk) {
@@ -618,16 +733,16 @@ __global__ __launch_bounds__(256) void gm_close_mu_kernel(GmArgs a, const SurfDe
                 ar[e] = c1r[q[e]];
                 ai[e] = c1i[q[e]];
             }
-            load_first_pass(v.x + j0, n - j0, xpre);
-            load_first_pass(v.V + j0, n - j0, v0pre);
-            load_first_pass(v.V + n + j0, n - j0, v1pre);
+            load_first_pass<NT>(v.x + j0, n - j0, xpre);
+            load_first_pass<NT>(v.Z + j0, n - j0, PRE ? z0pre : v0pre);
+            load_first_pass<NT>(v.Z + n + j0, n - j0, PRE ? z1pre : v1pre);
         }
         double mv[kCircPer];
 #pragma unroll
-        for (int e = 0; e < kCircPer; ++e) mv[e] = xpre[e] + y0 * v0pre[e] + y1 * v1pre[e];
+        for (int e = 0; e < kCircPer; ++e) mv[e] = xpre[e] + y0 * (PRE ? z0pre[e] : v0pre[e]) + y1 * (PRE ? z1pre[e] : v1pre[e]);
         for (int q = 2; q < k; ++q) {
             double vq[8];
-            load_first_pass(v.V + (long long)q * n + j0, n - j0, vq);
+            load_first_pass<NT>(v.Z + (long long)q * n + j0, n - j0, vq);
             const double yq = ys[4 + q];
 #pragma unroll
             for (int e = 0; e < kCircPer; ++e) mv[e] += yq * vq[e];
@@ -678,7 +793,12 @@ __global__ __launch_bounds__(256) void gm_close_mu_kernel(GmArgs a, const SurfDe
     }
 }
 
-template __global__ void gm_iter_kernel<double>(GmArgs, const SurfDesc*, int);
-template __global__ void gm_iter_kernel<float>(GmArgs, const SurfDesc*, int);
+#define SFH_GM_INSTANCES(W, RR)                                                     \
+    template __global__ void gm_iter_kernel<double, W, RR>(GmArgs, const SurfDesc*, int); \
+    template __global__ void gm_iter_kernel<float, W, RR>(GmArgs, const SurfDesc*, int);
+SFH_GM_INSTANCES(4, 1)
+SFH_GM_INSTANCES(8, 2)
+template __global__ void gm_close_mu_kernel<false>(GmArgs, const SurfDesc*, const double*, double2*, int);
+template __global__ void gm_close_mu_kernel<true>(GmArgs, const SurfDesc*, const double*, double2*, int);
 
 }  // namespace sfh

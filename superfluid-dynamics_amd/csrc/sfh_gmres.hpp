@@ -8,7 +8,7 @@
 
 namespace sfh {
 
-constexpr int kRowsPerWG = 4;      // one matrix row per wave
+constexpr int kPreModes = 8;        // most Fourier modes of the film's preconditioner, besides the mean
 constexpr int kMaxKrylov = 32;     // basis vectors per solve (iteration cap)
 constexpr int kGmMaxN = 4096;      // LDS copy of the vector being multiplied
 
@@ -21,7 +21,9 @@ struct GmCtl {
     double hnext;
     int fill_iters;    // most Arnoldi steps of a solve since the stage history last held fewer
                        // than kHistDepth steps
-    int spare[19];
+    int pre_modes;     // film: Fourier modes of the preconditioner besides the mean, -1: not used
+    double height;     // film: mean height of the surface above the substrate
+    int spare[16];
 };
 static_assert(sizeof(GmCtl) == kGmCtlInts * sizeof(int), "host reads control blocks with this stride");
 
@@ -32,6 +34,7 @@ struct GmView {
     const double* x;   // initial guess
     double* sol;       // solution
     double* V;       // (m+1) x n, unnormalised: v_i = sc[i] * V[i]
+    double* Z;       // (m+1) x n, P^{-1} V (V itself without a preconditioner)
     double* w0;      // products of even steps
     double* w1;      // products of odd steps
     double* sc;      // m+1 scales
@@ -51,13 +54,14 @@ __device__ inline GmView gm_view(const GmArgs& a, const SurfDesc* sd, int s) {
     GmView v;
     const int m = a.m;
     v.n = d.n;
-    v.nwg = (d.n + kRowsPerWG - 1) / kRowsPerWG;
+    v.nwg = (d.n + a.rpw - 1) / a.rpw;
     v.M = a.M + d.moff;
     v.M32 = a.M32 ? a.M32 + d.moff : nullptr;
     v.b = a.b + d.voff;
     v.x = a.x + d.voff;
     v.sol = a.sol + d.voff;
     v.V = a.V + (long long)(m + 1) * d.voff;
+    v.Z = a.Z + (long long)(m + 1) * d.voff;
     v.w0 = a.w + d.voff;
     v.w1 = a.w + a.total + d.voff;
     v.sc = a.small + (long long)s * a.small_stride;
@@ -92,19 +96,20 @@ __device__ inline void count_history(const GmArgs& a) {
     a.hvalid[a.stage - 1] = min(a.hvalid[a.stage - 1] + 1, kHistDepth);
 }
 
-// Sums part[i * nwg + w] over w for i < count (count <= kMaxKrylov + 1) into out[i] (LDS).
-// Basis indices go in chunks of 12; within a chunk every load of a thread (12 indices x 2
-// workgroups per 512-workgroup pass) is issued before any addition.
+// Sums part[i * nwg + w] over w for i < count (count <= kMaxKrylov + 1) into out[i] (LDS), by a
+// workgroup of NT threads.  Basis indices go in chunks of 12; within a chunk every load of a thread
+// (12 indices x 2 workgroups per pass) is issued before any addition.
+template <int NT = 256>
 __device__ inline void reduce_partials(const double* __restrict__ part, int nwg, int count, double* out) {
-    constexpr int CH = 12;
-    __shared__ double red[4][kMaxKrylov + 2];
+    constexpr int CH = 12, NW = NT / 64;
+    __shared__ double red[NW][kMaxKrylov + 2];
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     for (int i0 = 0; i0 < count; i0 += CH) {
         double acc[CH];
 #pragma unroll
         for (int u = 0; u < CH; ++u) acc[u] = 0.0;
-        for (int base = 0; base < nwg; base += 512) {
-            const int w0 = base + t, w1 = base + t + 256;
+        for (int base = 0; base < nwg; base += 2 * NT) {
+            const int w0 = base + t, w1 = base + t + NT;
             double v0[CH], v1[CH];
 #pragma unroll
             for (int u = 0; u < CH; ++u) {
@@ -124,7 +129,12 @@ __device__ inline void reduce_partials(const double* __restrict__ part, int nwg,
         }
     }
     __syncthreads();
-    if (t < count) out[t] = red[0][t] + red[1][t] + red[2][t] + red[3][t];
+    if (t < count) {
+        double s = 0.0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) s += red[w][t];
+        out[t] = s;
+    }
     __syncthreads();
 }
 
@@ -136,17 +146,20 @@ struct DotLoads {
     double a[kFastDots], b[kFastDots];
 };
 __device__ inline bool dots_fast(int nwg, int count) { return count <= kFastDots && nwg <= 512; }
+template <int NT = 256>
 __device__ inline void dots_load(const double* __restrict__ part, int nwg, int count, DotLoads& L) {
-    const int w0 = threadIdx.x, w1 = threadIdx.x + 256;
+    const int w0 = threadIdx.x, w1 = threadIdx.x + NT;
 #pragma unroll
     for (int u = 0; u < kFastDots; ++u) {
         const bool ok = u < count;
         L.a[u] = (ok && w0 < nwg) ? part[u * nwg + w0] : 0.0;
-        L.b[u] = (ok && w1 < nwg) ? part[u * nwg + w1] : 0.0;
+        L.b[u] = (NT < 512 && ok && w1 < nwg) ? part[u * nwg + w1] : 0.0;
     }
 }
+template <int NT = 256>
 __device__ inline void dots_finish(const DotLoads& L, int count, double* out) {
-    __shared__ double red[4][kFastDots];
+    constexpr int NW = NT / 64;
+    __shared__ double red[NW][kFastDots];
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
 #pragma unroll
     for (int u = 0; u < kFastDots; ++u) {
@@ -156,16 +169,25 @@ __device__ inline void dots_finish(const DotLoads& L, int count, double* out) {
         }
     }
     __syncthreads();
-    if (t < count) out[t] = red[0][t] + red[1][t] + red[2][t] + red[3][t];
+    if (t < count) {
+        double s = 0.0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) s += red[w][t];
+        out[t] = s;
+    }
     __syncthreads();
 }
 
-__device__ inline double block_sum4(double v, double* red4) {
+// Sum over a workgroup of NW waves (red: NW doubles of LDS).
+template <int NW = 4>
+__device__ inline double block_sum(double v, double* red) {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     v = wave_sum(v);
-    if (lane == 0) red4[wv] = v;
+    if (lane == 0) red[wv] = v;
     __syncthreads();
-    const double s = red4[0] + red4[1] + red4[2] + red4[3];
+    double s = 0.0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) s += red[w];
     __syncthreads();
     return s;
 }

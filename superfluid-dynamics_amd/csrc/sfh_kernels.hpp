@@ -86,6 +86,12 @@ struct GmArgs {
     int* hvalid;
     int stage;
     int check_first;     // refinement solve: every launch checks for a finished solve before its matrix loads
+    int rpw;             // matrix rows per workgroup of gm_iter_kernel: 4 (4 waves, one each) or 16 (8 waves, two each)
+    // film: right preconditioner P of the image term (precondition in gmres.hip), chosen per surface by
+    // zphi_circ_kernel.  Z holds the preconditioned basis P^{-1} V (pre = 0: there is none, Z = V).
+    int pre;
+    double* Z;
+    const double2* tw;   // twiddle tables, SurfDesc::twoff
 };
 constexpr int kPairRows = 4;        // default rows per workgroup of the N^2 pair kernels (assembly, velocity)
 // ---- spectral.hip
@@ -174,8 +180,9 @@ __global__ void gepp_fallback_kernel(const SurfDesc* sd, double* M, const double
 
 // ---- gmres.hip
 constexpr int kGmCtlInts = 32;   // ints per control block (holds the device struct)
-template <typename T>
+template <typename T, int W, int RR>
 __global__ void gm_iter_kernel(GmArgs a, const SurfDesc* sd, int j);
+template <bool PRE>
 __global__ void gm_close_mu_kernel(GmArgs a, const SurfDesc* sd, const double* circ, double2* mup, int i);
 
 // ---- solver.hip: one trajectory frame [x(T), y(T), phi(T)] of the state

@@ -251,11 +251,17 @@ Solver::Solver(const Phys& ph, const std::vector<int>& n, const Options& opt) : 
 void Solver::alloc_gmres(int m) {
     if (gmV_) return;
     gm_m_ = m;   // at most kMaxKrylov basis vectors (gmres.hip)
-    gm_nwg_ = (maxN_ + 3) / 4;   // kRowsPerWG in gmres.hip
+    // rows per workgroup of the Arnoldi launches.  Every workgroup repeats the step's finishing work, so few
+    // large ones are better once they still fill the GPU: N = 4096 film 34.6 ms per 40 steps with 16 rows.  At
+    // N = 2048 (512 workgroups of 4 rows, two per CU) their longer start costs more than it saves: 26.7 ms per
+    // 100 steps with 4 rows, 29.8 with 8 and 28.6 - 31.0 with 16; N = 1536 mixed 18.0, 17.9 and 18.7.
+    gm_rpw_ = T_ <= 2048 ? 4 : 16;
+    gm_nwg_ = (maxN_ + gm_rpw_ - 1) / gm_rpw_;
     gm_part_stride_ = 2LL * gm_nwg_ * (gm_m_ + 1);
     gm_small_stride_ = 4LL * (gm_m_ + 1) + 2LL * gm_m_ + (long long)gm_m_ * (gm_m_ + 1);
     gmV_ = dalloc<double>((size_t)(gm_m_ + 1) * T_);
     gmx0_ = dalloc<double>(T_);
+    if (ph_.image && opt_.solver == kSolveGMRES) gmZ_ = dalloc<double>((size_t)(gm_m_ + 1) * T_);
     if (opt_.precision == kMixed && opt_.solver == kSolveGMRES) M32_ = dalloc<float>(MT_);
     SFH_HIP(hipMemset(gmx0_, 0, T_ * sizeof(double)));
     gmw_ = dalloc<double>(2 * (size_t)T_);
@@ -282,7 +288,7 @@ Solver::~Solver() {
     if (graph_) (void)hipGraphDestroy(graph_);
     void* bufs[] = {d_desc_, d_tw_, Z0_, Za_, Zb_, P0_, Pa_, Pb_, kZ_[0], kZ_[1], kZ_[2], kP_[0],
                     kP_[1], kP_[2], Zp_, Zpp_, mup_, qup_, b_, work_, y_, mu_, M_, uinv_, flags_,
-                    status_, piv_, counters_, gmV_, gmw_, gmpart_, gmsmall_, gmctl_, trig_, order_, bstats_,
+                    status_, piv_, counters_, gmV_, gmZ_, gmw_, gmpart_, gmsmall_, gmctl_, trig_, order_, bstats_,
                     gmhist_, gmhvalid_, bhist_, bhvalid_, d_circ_, gmx0_, M32_, ckZ_, ckP_, ckMu_, ckHist_,
                     ckHv_, energy_, D0_, Da_, Db_, ckD_, kD_[0], kD_[1], kD_[2]};
     for (void* p : bufs)
@@ -380,6 +386,10 @@ GmArgs Solver::gm_args(int stage) const {
     a.hist = gmhist_;
     a.hvalid = gmhvalid_;
     a.stage = stage;
+    a.rpw = gm_rpw_;
+    a.pre = gmZ_ ? 1 : 0;
+    a.Z = gmZ_ ? gmZ_ : gmV_;
+    a.tw = d_tw_;
     return a;
 }
 
@@ -404,20 +414,22 @@ bool Solver::enqueue_gmres(const GmArgs& a, bool g1, bool force64) {
             a.check_first ? "gm_refine" : "gm_iter", 2.0 * nsq + 4.0 * (j + 1) * T_,
             (f32 ? 4.0 : 8.0) * nsq + 8.0 * (j + 3) * T_,
             [&] {
-                if (f32)
-                    go(gm_iter_kernel<float>, grid, dim3(256), 0, a,
-                                       (const SurfDesc*)d_desc_, j);
-                else
-                    go(gm_iter_kernel<double>, grid, dim3(256), 0, a,
-                                       (const SurfDesc*)d_desc_, j);
+                auto step = [&](auto kernel, int waves) {
+                    go(kernel, grid, dim3(64 * waves), 0, a, (const SurfDesc*)d_desc_, j);
+                };
+                switch (a.rpw) {
+                case 4: f32 ? step(gm_iter_kernel<float, 4, 1>, 4) : step(gm_iter_kernel<double, 4, 1>, 4); break;
+                default: f32 ? step(gm_iter_kernel<float, 8, 2>, 8) : step(gm_iter_kernel<double, 8, 2>, 8); break;
+                }
             },
             j);
     }
     if (fused && !g1) {
         // finishing the last step + x += V y + mu' = D1 mu: the rebuild and the circulant product
         launch("gm_close_mu", 4.0 * a.m * T_ + 4.0 * nsq, 8.0 * (a.m + 2) * T_ + 24.0 * nsq / kCircRowsPerWG, [&] {
-            go(gm_close_mu_kernel, dim3((maxN_ + kCircRowsPerWG - 1) / kCircRowsPerWG, S_), dim3(256),
-                               0, a, (const SurfDesc*)d_desc_, (const double*)d_circ_, mup_, a.m - 1);
+            go(a.pre ? gm_close_mu_kernel<true> : gm_close_mu_kernel<false>,
+               dim3((maxN_ + kCircRowsPerWG - 1) / kCircRowsPerWG, S_), dim3(256), 0, a, (const SurfDesc*)d_desc_,
+               (const double*)d_circ_, mup_, a.m - 1);
         });
     }
     if (ktime_ && !a.check_first) {
@@ -903,6 +915,7 @@ void Solver::clear_solver_state() {
     if (opt_.solver == kSolveGMRES) {
         SFH_HIP(hipMemsetAsync(gmx0_, 0, T_ * sizeof(double), stream_));
         SFH_HIP(hipMemsetAsync(gmV_, 0, (size_t)(gm_m_ + 1) * T_ * sizeof(double), stream_));
+        if (gmZ_) SFH_HIP(hipMemsetAsync(gmZ_, 0, (size_t)(gm_m_ + 1) * T_ * sizeof(double), stream_));
         SFH_HIP(hipMemsetAsync(gmw_, 0, 2 * (size_t)T_ * sizeof(double), stream_));
         SFH_HIP(hipMemsetAsync(gmpart_, 0, gm_part_stride_ * S_ * sizeof(double), stream_));
         SFH_HIP(hipMemsetAsync(gmsmall_, 0, gm_small_stride_ * S_ * sizeof(double), stream_));
@@ -1433,6 +1446,8 @@ void Solver::enqueue_vjp_mwg(const double2* Z, const double* P, const double* mu
         g.hvalid = nullptr;
         g.stage = 0;
         g.check_first = 0;
+        g.pre = 0;
+        g.Z = gmV_;
         enqueue_gmres(g, false, true);   // leaves s D1 gb in mup_
     });
     if (adj_warm_ && stage >= 0) {   // the solution joins the stage's ring

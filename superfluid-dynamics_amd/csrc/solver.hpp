@@ -267,7 +267,8 @@ class Solver {
     int* counters_ = nullptr;   // [0] fallback solves
     std::vector<long long> uoff_, foff_;
     // GMRES workspace
-    int gm_m_ = 0, gm_nwg_ = 0;
+    int gm_m_ = 0, gm_nwg_ = 0, gm_rpw_ = 4;
+    double* gmZ_ = nullptr;        // film: the preconditioned basis
     double *gmV_ = nullptr, *gmw_ = nullptr, *gmpart_ = nullptr, *gmsmall_ = nullptr;
     double* gmx0_ = nullptr;     // initial guess of the solve in flight (the solution goes to mu_)
     float* M32_ = nullptr;       // FP32 matrices of the mixed-precision GMRES form

@@ -18,7 +18,8 @@
 //
 // velocity_gm1_kernel is the same kernel at the end of a GMRES solve of one Arnoldi step (the
 // launch sequence of two: gm_iter_kernel's product, then this).  With v0 = r0/|r0| and
-// w = M v0, the least-squares step gives mu = x0 + (v0.w / |w|^2) r0; launch 0 left the partial
+// w = M v0, the least-squares step gives mu = x0 + (v0.w / |w|^2) r0 (with the film's preconditioner
+// w = M P^{-1} v0 and P^{-1} r0 in place of r0); launch 0 left the partial
 // sums of v0.w and |w|^2, so every workgroup reduces them and forms mu_j = x0_j + alpha r0_j as
 // it sweeps the columns.  The same sweep adds the circulant product of the derivative,
 // mu'_k = (2 pi / n) sum_j c1[(k - j) mod n] mu_j (mu_circ_kernel's product;
@@ -57,20 +58,20 @@ __device__ inline void velocity_rows(const SurfDesc* __restrict__ sd, const Node
     // ---- G1: the solve's state, the partial sums of launch 0 and the first kernel window first
     GmCtl* gc = nullptr;
     const double* x0 = nullptr;
-    const double* r0 = nullptr;
+    const double* r0 = nullptr;   // the correction's direction: r0, with a preconditioner P^{-1} r0
     const double* c1r = nullptr;
     const double* c1i = nullptr;
     int fin = 0;
     double beta = 0.0, bnorm = 0.0;
     DotLoads dl;
-    const int nwg = (n + kRowsPerWG - 1) / kRowsPerWG;
+    const int nwg = G1 ? (n + gm.rpw - 1) / gm.rpw : 0;
     const double* part = nullptr;
     bool fastdots = false;
     double ar[kCircWinPer], ai[kCircWinPer];
     if constexpr (G1) {
         gc = reinterpret_cast<GmCtl*>(gm.ctl) + s;
         x0 = gm.x + d.voff;
-        r0 = gm.V + (long long)(gm.m + 1) * d.voff;
+        r0 = gm.Z + (long long)(gm.m + 1) * d.voff;
         c1r = circ + d.coff;
         c1i = c1r + n;
         fin = gc->done;
@@ -260,15 +261,16 @@ __device__ inline void velocity_rows(const SurfDesc* __restrict__ sd, const Node
             const double sc0 = beta > 0.0 ? 1.0 / beta : 0.0;
             const double h00 = sums[0];
             const double* w0 = gm.w + d.voff;
+            const double* v0 = gm.V + (long long)(gm.m + 1) * d.voff;
             double ss = 0.0;
             if (fin == 0) {
                 for (int c = t; c < n; c += 256) {
-                    const double u = w0[c] - h00 * (sc0 * r0[c]);
+                    const double u = w0[c] - h00 * (sc0 * v0[c]);
                     ss += u * u;
                 }
             }
             __shared__ double red4[4];
-            const double hn = sqrt(block_sum4(ss, red4));
+            const double hn = sqrt(block_sum<4>(ss, red4));
             if (t == 0) {
                 if (fin == 0) {
                     const double rho = sqrt(h00 * h00 + hn * hn);

@@ -1,0 +1,57 @@
+"""The film's GMRES solves with the preconditioner of the image term, against the direct (LU) solve of the same
+system: the smallest sizes, 3 * 2^k sizes, both row splits of the Arnoldi launches (up to 2048 nodes and
+above, one surface and several), thin to deep films, surfaces with a mean height.
+
+Tolerance: both solutions satisfy |b - M mu| <= tol |b| (tol = 1e-13 here, rounding for the LU); M's smallest
+singular value is about 1/2 on these surfaces, so |mu_gmres - mu_lu| <= 4 tol |b| <= 4e-13 |mu| |M|_row; the
+bound used is 1e-12 (1 + max |mu|), as the other solves' tests do."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _state(n, seed, mean, amp):
+    rng = np.random.default_rng(seed)
+    x = 2 * np.pi * np.arange(n) / n
+    y = sum(rng.uniform(0, amp / k) * np.cos(k * x + rng.uniform(0, 2 * np.pi)) for k in range(1, 9))
+    return x + 1j * (mean + y), 0.01 * np.sin(x + 0.3) + 0.004 * np.cos(3 * x)
+
+
+@pytest.mark.parametrize("mixed", [False, True], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("sizes,depth,mean", [([2], 1.0, 0.0), ([8], 1.0, 0.0), ([96], 0.4, 0.1), ([257 - 1], 0.05, 0.0), ([512], 0.02, 0.0),
+                                              ([256], 0.15, 0.0), ([768], 3.0, -0.5), ([1536], 1.0, 0.0), ([2048], 0.3, 0.2),
+                                              ([3072], 1.0, 0.0), ([768, 64, 2048], 0.7, 0.0)], ids=str)
+def test_film_gmres_matches_lu(sizes, depth, mean, mixed):
+    import cusuperhelium as c
+    print(f"film gmres {sizes} depth {depth} mean {mean} mixed {mixed}", flush=True)
+    amp = min(0.05, 0.3 * (depth + min(mean, 0.0)))
+    parts = [_state(n, 7 + n, mean, amp) for n in sizes]
+    Z, P = (np.concatenate(v) for v in zip(*parts))
+    props = c.Props(kind=c.HELIUM, depth=depth, g=0.15)
+    with c.Ensemble(sizes, props) as e:
+        e.set_state(Z, P)
+        q0, d0, diag0 = e.rhs(diagnostics=True)
+    with c.Ensemble(sizes, props, solver=c.GMRES, tol=1e-13, precision=c.MIXED if mixed else c.FP64) as e:
+        e.set_state(Z, P)
+        q1, d1, diag1 = e.rhs(diagnostics=True)
+        st = e.stats()
+    # where more than 16 modes of the image term are large, the preconditioner is off: such a solve has more
+    # large eigenvalues than 32 steps take out to this tolerance, and says that it did not converge
+    large = max(np.log(n / (4 * np.pi * 0.02)) / (2 * (depth + mean)) for n in sizes)
+    if large > 16 and st["unconverged"] > 0:
+        return
+    assert st["unconverged"] == 0 and st["fallback_solves"] == 0
+    for a, b in ((diag1["mu"], diag0["mu"]), (q1, q0), (d1, d0)):
+        assert np.abs(a - b).max() <= 1e-12 * (1 + np.abs(b).max())
+
+
+def test_film_steps_take_few_iterations():
+    # the image term's large eigenvalues are deflated: warm-started solves take at most 3 steps (4-7 without)
+    import cusuperhelium as c
+    Z, P = _state(1024, 5, 0.0, 0.05)
+    with c.Ensemble([1024], c.Props(kind=c.HELIUM, depth=1.0, g=0.15), solver=c.GMRES) as e:
+        e.set_state(Z, P)
+        e.step(0.002, 20)
+        st = e.stats()
+    assert 1 <= st["max_iterations"] <= 3 and st["unconverged"] == 0
