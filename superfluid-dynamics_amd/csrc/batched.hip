@@ -34,6 +34,7 @@
 
 namespace sfh {
 
+template <bool MIXED, bool FILM>
 __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys ph, StageCtl ctl) {
     __shared__ BLds L;
     const int s = a.order[blockIdx.x];
@@ -68,7 +69,8 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
     // tile-skewed matrix (FP64, or FP64 entries rounded to FP32) and forms (M x)_k for the warm start
     // x in FP64 from the unrounded entries: the first residual of the solve.
     const bool water = ph.kind == 0;
-    const PairConst pc = wg_diagonal(ph, nv, n, L);
+    PairConst pc = wg_diagonal(ph, nv, n, L);
+    pc.image = FILM;   // known when compiled
     const int nbk = (n + kTile - 1) / kTile;
     if (t < nbk * kTile) L.vs[t] = own ? x : 0.0;   // the padding entries stay 0 for every product
     __syncthreads();
@@ -108,10 +110,7 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
                 if constexpr (decltype(mirror)::value) tji[((unsigned)(kTile - r) & (kTile - 1)) * kTile + ((l + r) & (kTile - 1))] = (T)em;
             });
         };
-        if (a.mixed)
-            store(reinterpret_cast<float*>(a.M) + d.moff);
-        else
-            store(reinterpret_cast<double*>(a.M) + d.moff);
+        store(reinterpret_cast<std::conditional_t<MIXED, float, double>*>(a.M) + d.moff);
     }
     double mx0 = 0.0;   // (M x)_t
     if (own) mx0 = sym_total(L.part, n) + L.diag[t] * L.vs[t];
@@ -120,11 +119,18 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
     // ---------------------------------------------------------------- C: solve
     const double bn = sqrt(bsum1(own ? bk * bk : 0.0, L));
     const double tol_abs = a.tol * bn;
+    // Film: the image term's few large eigenvalues are divided out (wg_precondition).  A warm solve of N = 768,
+    // h = 1 takes 1-2 products of the stored matrix (75 us each from one CU) in place of 4-5.
+    Precond pre = {-1, 0.0};
+    if constexpr (FILM) {
+        pre.height = bsum1(own ? zk.y : 0.0, L) / n + ph.depth;
+        pre.modes = film_modes(n, pre.height);
+    }
     int unconv = 0, iters = 0, sweeps = 0;
-    if (!a.mixed) {
+    if constexpr (!MIXED) {
         const double* Md = reinterpret_cast<const double*>(a.M) + d.moff;
         iters = wg_gmres([&]() { return mv_tiles(Md, n, L); }, n, bk, x, false, tol_abs, a.cycles, L, &unconv,
-                         true, own ? bk - mx0 : 0.0);
+                         true, own ? bk - mx0 : 0.0, pre);
     } else {
         const float* Mf = reinterpret_cast<const float*>(a.M) + d.moff;
         // ||M - M32||_F <= 2^-24 ||M||_F (round to nearest, normal range) + N 2^-150 (subnormal range)
@@ -145,7 +151,7 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
             }
             double dx = 0.0;
             iters += wg_gmres([&]() { return mv_tiles(Mf, n, L); }, n, r, dx, true,
-                              fmax(1e-7 * rn, 0.25 * tol_abs), 1, L, nullptr);
+                              fmax(1e-7 * rn, 0.25 * tol_abs), 1, L, nullptr, false, 0.0, pre);
             x += dx;
             // the FP64 residual of the corrected x, bounded without forming it:
             //   |b - M x| <= |r - M32 dx| + |(M - M32) dx| <= (GMRES residual) + ||M - M32||_F |dx|
@@ -193,7 +199,7 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
         const int kr = sym_row(n);
         const NodeTrig tk = L.tr[kr];
         const double mk = L.vs[kr];
-        if (pc.image) {
+        if constexpr (FILM) {
             double* const acc[4] = {L.part, psy, psy + kBT, piy};
             sym_sweep<4>(n, acc, [&](int k, int j, int, int, auto mirror, auto full, double (&row)[4], double (&col)[4]) {
                 if (!decltype(full)::value && (k >= n || j >= n)) return;
@@ -233,7 +239,7 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
     double2 q1 = make_double2(0.0, 0.0), q2 = make_double2(0.0, 0.0);
     if (own) {
         const double sx = sym_total(L.part, n), sy = sym_total(psy, n);
-        const double ix = pc.image ? sym_total(psy + kBT, n) : 0.0, iy = pc.image ? sym_total(piy, n) : 0.0;
+        const double ix = FILM ? sym_total(psy + kBT, n) : 0.0, iy = FILM ? sym_total(piy, n) : 0.0;
         velocity_from_sums(ph, zpk, zppk, mupk, x, zk.y, sx, sy, ix, iy, q1, q2);
     }
     // createM.cuh:104 reads the lower velocity of node 1 in the rho * q1.q2 term
@@ -260,5 +266,10 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
     }
     stage_update(ctl, gi, q1, dphi);
 }
+
+template __global__ void batched_stage_kernel<false, false>(BatchArgs, Phys, StageCtl);
+template __global__ void batched_stage_kernel<false, true>(BatchArgs, Phys, StageCtl);
+template __global__ void batched_stage_kernel<true, false>(BatchArgs, Phys, StageCtl);
+template __global__ void batched_stage_kernel<true, true>(BatchArgs, Phys, StageCtl);
 
 }  // namespace sfh

@@ -206,7 +206,7 @@ __device__ inline void precondition(double* vs, int n, const double2* __restrict
 #pragma unroll
         for (int w = 0; w < NW; ++w) x += red[w][t];
         const int m = (t + 1) >> 1;
-        const double lam = 0.5 + n * (0.25 / kPi) * exp(-2.0 * m * height);
+        const double lam = film_eigenvalue(n, m, height);
         coef[t] = x * (m == 0 ? 1.0 : 2.0) / n * (1.0 / lam - 2.0);
     }
     __syncthreads();

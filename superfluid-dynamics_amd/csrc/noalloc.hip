@@ -147,7 +147,6 @@ void rhs_noalloc(const Phys& ph, int n, const double* x, const double* y, const 
     a.mu = B.mu;
     a.stats = B.stats;
     a.tol = tol;
-    a.mixed = 0;
     a.cycles = (max_iter + 7) / 8;   // restart cycles of 8 basis vectors
     a.max_refine = 6;
     a.nsurf = 1;
@@ -159,7 +158,7 @@ void rhs_noalloc(const Phys& ph, int n, const double* x, const double* y, const 
     c.kZ[0] = B.q;
     c.kP[0] = dphi;
     c.Pin = phi;
-    hipLaunchKernelGGL(batched_stage_kernel, dim3(1), dim3(kBatchThreads), 0, stream, a, ph, c);
+    hipLaunchKernelGGL((ph.image ? batched_stage_kernel<false, true> : batched_stage_kernel<false, false>), dim3(1), dim3(kBatchThreads), 0, stream, a, ph, c);
     SFH_HIP(hipGetLastError());
     hipLaunchKernelGGL(noalloc_unpack_kernel, dim3(grid), dim3(256), 0, stream, B, n, vx, vy, mu);
     SFH_HIP(hipGetLastError());

@@ -167,6 +167,21 @@ __device__ inline double2 cot_image(const NodeTrig& k, const NodeTrig& j, double
     return make_double2(c.p * c.id, -c.q * c.id);
 }
 
+// ------------------------------------------------------------------ the film's preconditioner
+// Eigenvalue of the matrix of a flat film of the given height on the Fourier modes +-m of the node index
+// (createM.cuh:87-88: the image term is a Poisson kernel there, and the direct one vanishes).
+constexpr int kPreModes = 8;   // most modes of the preconditioner, besides the mean
+__device__ inline double film_eigenvalue(int n, int m, double height) {
+    return 0.5 + n * (0.25 / kPi) * exp(-2.0 * m * height);
+}
+// Modes that the preconditioner takes: up to the one whose eigenvalue is within 4% of 1/2.  On films so thin
+// that it would leave many larger ones out it is not used (-1): with less than half of them it can cost steps
+// (N = 512, height 0.02: 42 against 22 without).
+__device__ inline int film_modes(int n, double height) {
+    const double m = height > 0.0 ? log(n * (0.25 / kPi / 0.02)) / (2.0 * height) : 1e9;
+    return m < 2 * kPreModes + 1 ? max(0, min(kPreModes, (int)m)) : -1;
+}
+
 // ------------------------------------------------------------------ wave reductions
 // v taken from another lane of the same row of 16 by a DPP control (both halves of the double).
 template <int CTL>

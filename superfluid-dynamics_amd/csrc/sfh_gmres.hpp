@@ -8,7 +8,6 @@
 
 namespace sfh {
 
-constexpr int kPreModes = 8;        // most Fourier modes of the film's preconditioner, besides the mean
 constexpr int kMaxKrylov = 32;     // basis vectors per solve (iteration cap)
 constexpr int kGmMaxN = 4096;      // LDS copy of the vector being multiplied
 

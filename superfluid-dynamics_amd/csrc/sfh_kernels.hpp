@@ -216,7 +216,6 @@ struct BatchArgs {
     double* mu;                // warm start in, solution out
     int* stats;                // per surface: [iterations, unconverged solves, refinement sweeps, -]
     double tol;
-    int mixed;
     int cycles;                // GMRES restart cycles (FP64)
     int max_refine;            // refinement sweeps (mixed)
     int nsurf;
@@ -228,6 +227,8 @@ struct BatchArgs {
     double* hist;
     int* hvalid;
 };
+// MIXED: the stored matrix is FP32; FILM: the surface has an image term
+template <bool MIXED, bool FILM>
 __global__ void batched_stage_kernel(BatchArgs a, Phys ph, StageCtl ctl);
 
 // ---- adjoint.hip (reverse mode of the water right-hand side, every N <= kBatchMaxN)

@@ -30,6 +30,8 @@ struct BLds {
     double cs[kBK], sn[kBK], g[kBK + 1], y[kBK];
     double col[kBK + 2];
     double scal[4];
+    double prered[kBW][2 * kPreModes + 1];   // film: wg_precondition's sums and coefficients
+    double precoef[2 * kPreModes + 1];
 };
 
 // Sums each of the C slots of v over the workgroup into L.sums (all threads take part).
@@ -169,13 +171,68 @@ __device__ inline double mv_free(int n, int G, const PairConst& pc, BLds& L) {
     return w;
 }
 
+// The film's preconditioner of a surface: modes < 0 when none is used.
+struct Precond {
+    int modes;
+    double height;
+};
+
+// P^{-1} v for the flat film's matrix P (film_eigenvalue): 2 v + the first modes' (1/lam_m - 2)
+// projections.  Thread t < n holds v_t (the others 0) and gets the result (the others 0); L.tw holds the
+// twiddles exp(-2 pi i t / n).
+__device__ inline double wg_precondition(double v, int n, const Precond& pre, BLds& L) {
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const double2 w = L.tw[min(t, n - 1)];
+    const double c = w.x, s = -w.y;
+    const double s0 = wave_sum(v);
+    if (lane == 0) L.prered[wv][0] = s0;
+    double c1 = 1.0, s1 = 0.0, cm = c, sm = s;
+    for (int m = 1; m <= pre.modes; ++m) {
+        const double a = wave_sum(v * cm), b = wave_sum(v * sm);
+        if (lane == 0) {
+            L.prered[wv][2 * m - 1] = a;
+            L.prered[wv][2 * m] = b;
+        }
+        const double cn = 2.0 * c * cm - c1, sn = 2.0 * c * sm - s1;   // the next mode, by recurrence
+        c1 = cm;
+        s1 = sm;
+        cm = cn;
+        sm = sn;
+    }
+    __syncthreads();
+    if (t <= 2 * pre.modes) {
+        double a = 0.0;
+#pragma unroll
+        for (int q = 0; q < kBW; ++q) a += L.prered[q][t];
+        const int m = (t + 1) >> 1;
+        L.precoef[t] = a * (m == 0 ? 1.0 : 2.0) / n * (1.0 / film_eigenvalue(n, m, pre.height) - 2.0);
+    }
+    __syncthreads();
+    double z = 2.0 * v + L.precoef[0];
+    c1 = 1.0;
+    s1 = 0.0;
+    cm = c;
+    sm = s;
+    for (int m = 1; m <= pre.modes; ++m) {
+        z += L.precoef[2 * m - 1] * cm + L.precoef[2 * m] * sm;
+        const double cn = 2.0 * c * cm - c1, sn = 2.0 * c * sm - s1;
+        c1 = cm;
+        s1 = sm;
+        cm = cn;
+        sm = sn;
+    }
+    return t < n ? z : 0.0;
+}
+
 // Restarted GMRES on A x = rhs over the workgroup; x (thread t < n holds x_t) is updated in
-// place.  x_zero: x is known to be 0 (the first residual is rhs, no product needed); r_given:
+// place.  With a preconditioner the basis is that of A P^{-1} and x += P^{-1} V y, so residual and
+// tolerance are those of A x = rhs as without.  x_zero: x is known to be 0 (the first residual is rhs, no product needed); r_given:
 // the first residual rhs - A x is r_first (no product needed either).  Returns the number of
 // Arnoldi steps; *unconv is set when tol_abs was not reached.
 template <class MV>
 __device__ int wg_gmres(MV&& mv, int n, double rhs, double& x, bool x_zero, double tol_abs, int cycles,
-                        BLds& L, int* unconv, bool r_given = false, double r_first = 0.0) {
+                        BLds& L, int* unconv, bool r_given = false, double r_first = 0.0,
+                        const Precond pre = {-1, 0.0}) {
     const int t = threadIdx.x;
     const bool own = t < n;
     int total = 0;
@@ -199,7 +256,9 @@ __device__ int wg_gmres(MV&& mv, int n, double rhs, double& x, bool x_zero, doub
         int k = 0;
         bool conv = false;
         for (int j = 0; j < kBK; ++j) {
-            if (own) L.vs[t] = rget(V, j);
+            double u = rget(V, j);
+            if (pre.modes >= 0) u = wg_precondition(u, n, pre, L);
+            if (own) L.vs[t] = u;
             __syncthreads();
             double w = mv();
             // classical Gram-Schmidt ...
@@ -262,7 +321,14 @@ __device__ int wg_gmres(MV&& mv, int n, double rhs, double& x, bool x_zero, doub
             }
         }
         __syncthreads();
-        if (own) {
+        if (pre.modes >= 0) {
+            double u = 0.0;
+#pragma unroll
+            for (int i = 0; i < kBK; ++i)
+                if (i < k) u += L.y[i] * V[i];
+            u = wg_precondition(u, n, pre, L);
+            if (own) x += u;
+        } else if (own) {
 #pragma unroll
             for (int i = 0; i < kBK; ++i)
                 if (i < k) x += L.y[i] * V[i];

@@ -541,7 +541,7 @@ void Solver::enqueue_batched(const double2* Z, const double* P, const StageCtl& 
     a.mu = mu_;
     a.stats = bstats_;
     a.tol = opt_.tol;
-    a.mixed = opt_.precision == kMixed ? 1 : 0;
+    const bool mixed = opt_.precision == kMixed;
     a.cycles = std::max(1, (opt_.max_iter + 7) / 8);   // kBK = 8 vectors per cycle
     a.max_refine = 6;
     a.nsurf = S_;
@@ -551,11 +551,12 @@ void Solver::enqueue_batched(const double2* Z, const double* P, const StageCtl& 
     double nsq = 0.0;
     for (int v : n_) nsq += (double)v * v;
     const double img = ph_.image ? 2.0 : 1.0;
-    const double mbytes = (a.mixed ? 4.0 : 8.0) * nsq;
+    const double mbytes = (mixed ? 4.0 : 8.0) * nsq;
     // algorithmic work per launch: cot pairs of assembly + velocity (and one more pass per
     // refinement residual), matrix written once and read once per GMRES product
     launch("stage", 2.0 * img * nsq, 2.0 * mbytes, [&] {
-        go(batched_stage_kernel, dim3(S_), dim3(kBatchThreads), 0, a, ph_, ctl);
+        go(mixed ? (ph_.image ? batched_stage_kernel<true, true> : batched_stage_kernel<true, false>)
+                 : (ph_.image ? batched_stage_kernel<false, true> : batched_stage_kernel<false, false>), dim3(S_), dim3(kBatchThreads), 0, a, ph_, ctl);
     });
     SFH_HIP(hipGetLastError());
 }

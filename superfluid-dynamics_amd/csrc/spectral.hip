@@ -167,13 +167,9 @@ __global__ __launch_bounds__(256) void zphi_circ_kernel(const SurfDesc* __restri
         __shared__ double red4[4];
         const double height = block_sum<4>(ysum, red4) / n + ph.depth;
         if (t == 0) {
-            // the film's preconditioner takes the modes up to the one whose eigenvalue is within 4% of 1/2.  On
-            // films so thin that it would leave many larger ones out it is not used: with less than half of
-            // them it can cost steps (N = 512, height 0.02: 42 against 22 without)
-            const double m = height > 0.0 ? log(n * (0.25 / kPi / 0.02)) / (2.0 * height) : 1e9;
             GmCtl* c = reinterpret_cast<GmCtl*>(gm.ctl) + blockIdx.y;
             c->height = height;
-            c->pre_modes = m < 2 * kPreModes + 1 ? max(0, min(kPreModes, (int)m)) : -1;
+            c->pre_modes = film_modes(n, height);
         }
     }
     if (t < kCircRows && k0 + t < n) {
