@@ -36,6 +36,7 @@
 // polynomial through them (extrapolate_history; with five steps kept its error is fifth order in
 // dt, against first order for the previous stage's mu), which saves Krylov steps on every solve of
 // a time integration.
+#include "sfh_circ.hpp"
 #include "sfh_gmres.hpp"
 
 namespace sfh {
@@ -523,6 +524,14 @@ __global__ __launch_bounds__(64 * W) void gm_iter_kernel(GmArgs a, const SurfDes
     }
 }
 
+// The closing launch's circulant product: 256 threads, two runs of 4 columns each, 8 rows.
+struct CloseGeo {
+    static constexpr int NT = 256, CHUNK = kCircChunk, ROWS = kCircRowsPerWG;
+    static constexpr int WPER = (CHUNK + ROWS - 1 + NT - 1) / NT;
+    static constexpr int WIN = (CHUNK + ROWS + 31) / 32 * 32;
+    static_assert(ROWS == kCR && CHUNK == 2 * kCC * NT, "one group of rows, two runs of columns");
+};
+
 // The last launch of a sequence (i = m - 1 >= 1) fused with the derivative of the solution,
 // mu' = D1 mu 2 pi / n (mu_circ_kernel's circulant product; BaseBoundaryIntegrator.cuh:201-203).
 // Every workgroup finishes Arnoldi step i - 1 as gm_iter_kernel does, forms y and stages
@@ -553,8 +562,10 @@ __global__ __launch_bounds__(256) void gm_close_mu_kernel(GmArgs a, const SurfDe
     GmCtl* ctl = reinterpret_cast<GmCtl*>(a.ctl) + s;
     const int m = a.m;
     const int j = i - 1;
-    __shared__ double ms[kCircChunk];
-    __shared__ double2 c1[kCircWin];
+    using G = CloseGeo;
+    __shared__ alignas(16) double ms[G::CHUNK];
+    __shared__ alignas(16) double c1re[G::WIN], c1im[G::WIN];
+    __shared__ double cred[NT / 64][2 * kCR];
     __shared__ double Hs[KM * (KM + 1)];
     __shared__ double cs_s[KM], sn_s[KM], g_s[KM + 1];
     __shared__ double co[KM + 1];
@@ -562,15 +573,15 @@ __global__ __launch_bounds__(256) void gm_close_mu_kernel(GmArgs a, const SurfDe
     __shared__ double red8[8];
     __shared__ double sums[KM + 2];
     __shared__ double ys[KM + 4];   // g[j], gc[j+1], c, s, then y
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const int t = threadIdx.x, wv = t >> 6;
     const double* c1r = circ + d.coff;
     const double* c1i = c1r + n;
-    double ar[kCircWinPer], ai[kCircWinPer];
+    double ar[G::WPER], ai[G::WPER];
     {
-        int q[kCircWinPer];
-        circ_window(k0, 0, n, q);
+        int q[G::WPER];
+        circ_entries<G>(k0, 0, n, q);
 #pragma unroll
-        for (int e = 0; e < kCircWinPer; ++e) {
+        for (int e = 0; e < G::WPER; ++e) {
             ar[e] = c1r[q[e]];
             ai[e] = c1i[q[e]];
         }
@@ -721,15 +732,17 @@ __global__ __launch_bounds__(256) void gm_close_mu_kernel(GmArgs a, const SurfDe
     if (h0 && s == 0 && blockIdx.x == 0 && t == 0) count_history(a);
     // mu = x0 + y_0 Z[0] + y_1 Z[1] (+ the rest when k > 2), without branches in the common case
     const double y0 = k > 0 ? ys[4] : 0.0, y1 = k > 1 ? ys[5] : 0.0;
-    double2 a0s = {0.0, 0.0}, a1s = {0.0, 0.0};
+    double re[kCR], im[kCR];
+#pragma unroll
+    for (int r = 0; r < kCR; ++r) re[r] = im[r] = 0.0;
     for (int j0 = 0; j0 < n; j0 += kCircChunk) {
         const int jn = min(kCircChunk, n - j0);
         if (j0 > 0) {
             __syncthreads();   // the previous chunk has been consumed
-            int q[kCircWinPer];
-            circ_window(k0, j0, n, q);
+            int q[G::WPER];
+            circ_entries<G>(k0, j0, n, q);
 #pragma unroll
-            for (int e = 0; e < kCircWinPer; ++e) {
+            for (int e = 0; e < G::WPER; ++e) {
                 ar[e] = c1r[q[e]];
                 ai[e] = c1i[q[e]];
             }
@@ -750,18 +763,21 @@ __global__ __launch_bounds__(256) void gm_close_mu_kernel(GmArgs a, const SurfDe
 #pragma unroll
         for (int e = 0; e < kCircPer; ++e) {
             const int c = t + 256 * e;
-            if (c < jn) ms[c] = mv[e];
+            ms[circ_at(c)] = c < jn ? mv[e] : 0.0;
         }
 #pragma unroll
-        for (int e = 0; e < kCircWinPer; ++e) {
+        for (int e = 0; e < G::WPER; ++e) {
             const int u = t + 256 * e;
-            if (u < kCircWin) c1[u] = make_double2(ar[e], ai[e]);
+            if (u < G::CHUNK + G::ROWS) {
+                c1re[circ_at(u)] = ar[e];
+                c1im[circ_at(u)] = ai[e];
+            }
         }
         __syncthreads();
         if (t < CR) {   // the own rows of the solution, as staged
             const int r = k0 + t;
             if (r < n && r >= j0 && r < j0 + jn) {
-                const double x = ms[r - j0];
+                const double x = ms[circ_at(r - j0)];
                 v.sol[r] = x;
                 if (h0) {
 #pragma unroll
@@ -770,26 +786,31 @@ __global__ __launch_bounds__(256) void gm_close_mu_kernel(GmArgs a, const SurfDe
                 }
             }
         }
-#pragma unroll 4
-        for (int c = lane; c < jn; c += 64) {
-            const double x = ms[c];
-            const int u0 = wv - c + kCircChunk - 1;
-            const double2 p0 = c1[u0], p1 = c1[u0 + 4];
-            a0s.x += p0.x * x;
-            a0s.y += p0.y * x;
-            a1s.x += p1.x * x;
-            a1s.y += p1.y * x;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int c0 = kCC * (t + NT * h);
+            if (c0 < jn) {
+                double x[kCC], w[kCC + kCR];
+                circ_samples(ms, c0, x);
+                circ_kernel(c1re, c0, w);
+                circ_fma(w, x, re);
+                circ_kernel(c1im, c0, w);
+                circ_fma(w, x, im);
+            }
         }
     }
-    a0s.x = wave_sum(a0s.x); a0s.y = wave_sum(a0s.y);
-    a1s.x = wave_sum(a1s.x); a1s.y = wave_sum(a1s.y);
-    if (lane < 2) {   // lane 0: row wv, lane 1: row wv + 4
-        const int r = k0 + wv + 4 * lane;
-        if (r < n) {
-            const double2 acc = lane ? a1s : a0s;
-            const double xs = 2.0 * kPi / n;
-            mup[d.voff + r] = make_double2(acc.x * xs, acc.y * xs);
+    reduce_lanes(re, &cred[wv][0]);
+    reduce_lanes(im, &cred[wv][kCR]);
+    __syncthreads();
+    if (t < CR && k0 + t < n) {
+        double x = 0.0, y = 0.0;
+#pragma unroll
+        for (int w = 0; w < NT / 64; ++w) {
+            x += cred[w][t];
+            y += cred[w][kCR + t];
         }
+        const double xs = 2.0 * kPi / n;
+        mup[d.voff + k0 + t] = make_double2(x * xs, y * xs);
     }
 }
 

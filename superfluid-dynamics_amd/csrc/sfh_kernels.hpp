@@ -95,8 +95,8 @@ struct GmArgs {
 };
 constexpr int kPairRows = 4;        // default rows per workgroup of the N^2 pair kernels (assembly, velocity)
 // ---- spectral.hip
-// circulant derivative products: rows per workgroup (wave w owns rows w and w + 4), columns
-// staged in LDS per round, and the kernel window one round needs
+// circulant products of the launches that finish a GMRES solve (gm_close_mu_kernel, velocity_gm1_kernel): most
+// rows per workgroup, columns staged in LDS per round, and the kernel window one round needs
 constexpr int kCircRowsPerWG = 8;
 constexpr int kCircChunk = 2048;
 constexpr int kCircWin = kCircChunk + kCircRowsPerWG - 1;
@@ -117,9 +117,12 @@ __device__ inline void circ_window(int k0, int j0, int n, int (&q)[kCircWinPer])
         if (r >= n) r -= n;
     }
 }
+// TC threads over the columns, TR row groups of 8 rows (spectral.hip)
+template <int TC, int TR>
 __global__ void zphi_circ_kernel(const SurfDesc* sd, const double* circ, const double2* Z, const double* phi,
                                  double2* Zp, double2* Zpp, double* b, double* work, Phys ph, int* status,
                                  NodeTrig* trig, GmArgs gm, int gm_on);
+template <int TC, int TR>
 __global__ void mu_circ_kernel(const SurfDesc* sd, const double* circ, const double* mu, double2* mup);
 // ---- deriv.hip
 constexpr int kDerivThreads = 1024;

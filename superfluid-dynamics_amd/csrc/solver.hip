@@ -2,7 +2,7 @@
 //
 // One RHS evaluation (BaseBoundaryIntegralCalculator::runTimeStep,
 // CuSuperHelium/BaseBoundaryIntegrator.cuh:137-306) is enqueued as
-//   zphi_circ_kernel      Z', Z'', Re Phi'            (circulant products, 8 rows per workgroup)
+//   zphi_circ_kernel      Z', Z'', Re Phi'            (circulant products, 8 or 32 rows per workgroup)
 //   assemble64_kernel     M                           (8 rows per workgroup)
 //   LU solve              mu                          (panel / MFMA update / back substitution)
 //   GEPP fallback         no-op unless a system needed row interchanges
@@ -35,6 +35,15 @@ namespace sfh {
     case 2: { constexpr int R = 2; __VA_ARGS__; } break; \
     default: { constexpr int R = 4; __VA_ARGS__; } break; \
     }
+
+// Shape of the circulant derivative kernels for surfaces of up to n nodes (spectral.hip).  Up to 256 nodes a chunk
+// of 256 columns is the whole surface and 32 rows share it.  Above, 8 rows per workgroup keep all CUs busy: one
+// chunk of 1024 or 2048 columns that holds the surface (N = 2048 8.1 us, in two chunks of 1024 9.2), and beyond
+// 2048 nodes chunks of 1024, whose LDS lets two workgroups share a CU (N = 4096 15.6 us, in chunks of 2048 20.0).
+#define SFH_WITH_CIRC(n, ...)                                                            \
+    if ((n) <= 256) { constexpr int TC = 64, TR = 4; __VA_ARGS__; }                      \
+    else if ((n) <= 1024 || (n) > 2048) { constexpr int TC = 256, TR = 1; __VA_ARGS__; } \
+    else { constexpr int TC = 512, TR = 1; __VA_ARGS__; }
 
 // Steps that run every solve with the full launch cap: kHistDepth while the warm-start history
 // fills, then one with the full history that sets the trimmed length.
@@ -575,12 +584,11 @@ void Solver::enqueue_rhs(const double2* Z, const double* P, const StageCtl& ctl_
     double nsq = 0.0;
     for (int v : n_) nsq += (double)v * v;
     const double img = ph_.image ? 2.0 : 1.0;
-    const dim3 cgrid((maxN_ + kCircRowsPerWG - 1) / kCircRowsPerWG, S_);
     // circulant derivatives: 7 n^2 multiply-adds; bytes: the samples and kernels each workgroup
     // stages (24 B per node and 24 B per kernel entry)
     launch("deriv", 14.0 * nsq, 48.0 * nsq / kCircRowsPerWG, [&] {
-        go(zphi_circ_kernel, cgrid, dim3(256), 0, d_desc_, (const double*)d_circ_, Z, P,
-                           Zp_, Zpp_, b_, work_, ph_, status_, trig_, ga, gm_on);
+        SFH_WITH_CIRC(maxN_, go(zphi_circ_kernel<TC, TR>, circ_grid(8 * TR), dim3(TC * TR), 0, d_desc_,
+                                (const double*)d_circ_, Z, P, Zp_, Zpp_, b_, work_, ph_, status_, trig_, ga, gm_on));
     });
     // assembly: flops counted as cot evaluations (the transcendental-bound unit), bytes = M written
     if (gm_on && opt_.precision == kMixed) {
@@ -600,8 +608,8 @@ void Solver::enqueue_rhs(const double2* Z, const double* P, const StageCtl& ctl_
     const bool g1 = gm_on && opt_.precision != kMixed && ga.m == 2 && !quirk;
     if (!enqueue_solve(Z, ctl.stage, g1)) {
         launch("mu_deriv", 4.0 * nsq, 24.0 * nsq / kCircRowsPerWG, [&] {
-            go(mu_circ_kernel, cgrid, dim3(256), 0, d_desc_, (const double*)d_circ_,
-                               (const double*)mu_, mup_);
+            SFH_WITH_CIRC(maxN_, go(mu_circ_kernel<TC, TR>, circ_grid(8 * TR), dim3(TC * TR), 0, d_desc_,
+                                    (const double*)d_circ_, (const double*)mu_, mup_));
         });
     }
     if (g1) {
@@ -1369,14 +1377,15 @@ void Solver::enqueue_vjp_mwg(const double2* Z, const double* P, const double* mu
     double nsq = 0.0;
     for (int v : n_) nsq += (double)v * v;
     const double img = ph_.image ? 2.0 : 1.0;
-    const dim3 cgrid((maxN_ + kCircRowsPerWG - 1) / kCircRowsPerWG, S_);
     const dim3 pgrid((maxN_ + kAdjRows - 1) / kAdjRows, S_);
     const dim3 wgrid((maxN_ + 3) / 4, S_);
     const dim3 ngrid((maxN_ + 255) / 256, S_);
     launch("vjp_fwd", 14.0 * nsq, 0.0, [&] {
-        go(zphi_circ_kernel, cgrid, dim3(256), 0, d_desc_, (const double*)d_circ_, Z, P, Zp_, Zpp_, b_, work_, ph_,
-           (int*)nullptr, trig_, GmArgs{}, 0);
-        go(mu_circ_kernel, cgrid, dim3(256), 0, d_desc_, (const double*)d_circ_, mu, mup_);
+        SFH_WITH_CIRC(maxN_, {
+            go(zphi_circ_kernel<TC, TR>, circ_grid(8 * TR), dim3(TC * TR), 0, d_desc_, (const double*)d_circ_, Z, P, Zp_,
+               Zpp_, b_, work_, ph_, (int*)nullptr, trig_, GmArgs{}, 0);
+            go(mu_circ_kernel<TC, TR>, circ_grid(8 * TR), dim3(TC * TR), 0, d_desc_, (const double*)d_circ_, mu, mup_);
+        });
     });
     AdjMArgs a{};
     a.sd = d_desc_;

@@ -223,6 +223,7 @@ class Solver {
     // A kernel launch on stream_.  Inside a timed launch() it records the kernel's own start (the
     // group's first kernel) and end into that launch's event pair (hipExtLaunchKernelGGL), as a
     // profiler times a kernel.
+    dim3 circ_grid(int rows) const { return dim3((maxN_ + rows - 1) / rows, S_); }   // circulant derivative kernels
     template <typename K, typename... Args>
     void go(K kernel, dim3 grid, dim3 block, unsigned shm, Args... args);
     hipEvent_t ev_a_ = nullptr, ev_b_ = nullptr;
