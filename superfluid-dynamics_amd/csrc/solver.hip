@@ -233,6 +233,8 @@ Solver::Solver(const Phys& ph, const std::vector<int>& n, const Options& opt) : 
     status_ = dalloc<int>(2 * S_);
     piv_ = dalloc<int>(T_);
     counters_ = dalloc<int>(4);
+    const size_t words = 2 * (size_t)S_ + 4 + (opt_.solver == kSolveGMRES ? (size_t)kGmCtlInts * S_ : 4 * (size_t)S_);
+    SFH_HIP(hipHostMalloc((void**)&host_, 3 * (size_t)T_ * sizeof(double) + words * sizeof(int), hipHostMallocDefault));
     SFH_HIP(hipMemset(status_, 0, 2 * S_ * sizeof(int)));
     SFH_HIP(hipMemset(counters_, 0, 4 * sizeof(int)));
     SFH_HIP(hipMemset(Z0_, 0, T_ * sizeof(double2)));
@@ -318,6 +320,7 @@ Solver::~Solver() {
     for (hipEvent_t e : rec_copied_) (void)hipEventDestroy(e);
     if (rec_ring_) (void)hipFree(rec_ring_);
     if (rec_host_) (void)hipHostFree(rec_host_);
+    if (host_) (void)hipHostFree(host_);
     if (rec_stream_) (void)hipStreamDestroy(rec_stream_);
     if (stream_) (void)hipStreamDestroy(stream_);
 }
@@ -921,6 +924,10 @@ __global__ __launch_bounds__(256) void state_join_kernel(const double2* __restri
 void Solver::clear_solver_state() {
     SFH_HIP(hipMemsetAsync(counters_ + 1, 0, sizeof(int), stream_));
     SFH_HIP(hipMemsetAsync(mu_, 0, T_ * sizeof(double), stream_));
+    clear_gmres_state();
+}
+
+void Solver::clear_gmres_state() {
     if (opt_.solver == kSolveGMRES) {
         SFH_HIP(hipMemsetAsync(gmx0_, 0, T_ * sizeof(double), stream_));
         SFH_HIP(hipMemsetAsync(gmV_, 0, (size_t)(gm_m_ + 1) * T_ * sizeof(double), stream_));
@@ -973,19 +980,46 @@ void Solver::rhs_device(const double2* state, double2* rhs) {
 // Two nodes of one surface at the same point (x mod 2 pi, y) make cot((z_k - z_j)/2) infinite and
 // the dipole matrix singular.  Rounded in FMA the pair terms come out huge but finite rather than
 // NaN, so the case is caught here, by sorting each surface's nodes.
+// x reduced to [0, 2 pi).
+static double reduced_x(double x) {
+    if (x >= 0.0 && x < 2.0 * kPi) return x;   // fmod returns it unchanged
+    double xr = std::fmod(x, 2.0 * kPi);
+    if (xr < 0.0) xr += 2.0 * kPi;
+    return xr >= 2.0 * kPi ? 0.0 : xr;
+}
+
 static void check_distinct_nodes(const double* x, const double* y, const std::vector<int>& sizes) {
     std::vector<std::pair<double, double>> pts;
     std::vector<int> idx;
     int off = 0;
     for (size_t s = 0; s < sizes.size(); ++s) {
         const int n = sizes[s];
+        const double* xs = x + off;
+        // a surface that is a function of x, listed in order: the reduced x increase strictly, but for one wrap
+        // that stays below the first.  All its points differ and it needs no sort (64 surfaces of 256 nodes:
+        // 0.04 ms in place of 0.21)
+        const double first = reduced_x(xs[0]);
+        double last = first;
+        int wraps = 0;
+        bool ordered = true;
+        for (int i = 1; i < n && ordered; ++i) {
+            const double xr = reduced_x(xs[i]);
+            if (xr < last) {
+                ordered = ++wraps == 1;
+            } else {
+                ordered = xr != last;
+            }
+            ordered = ordered && (wraps == 0 || xr < first);
+            last = xr;
+        }
+        if (ordered) {
+            off += n;
+            continue;
+        }
         pts.resize(n);
         idx.resize(n);
         for (int i = 0; i < n; ++i) {
-            double xr = std::fmod(x[off + i], 2.0 * kPi);
-            if (xr < 0.0) xr += 2.0 * kPi;
-            if (xr >= 2.0 * kPi) xr = 0.0;
-            pts[i] = {xr, y[off + i]};
+            pts[i] = {reduced_x(xs[i]), y[off + i]};
             idx[i] = i;
         }
         std::sort(idx.begin(), idx.end(), [&](int a, int b) { return pts[a] < pts[b]; });
@@ -998,34 +1032,85 @@ static void check_distinct_nodes(const double* x, const double* y, const std::ve
     }
 }
 
+// Host transfers of small states: a copy or clear per array costs 5 to 15 us on the host, a kernel launch 3.  The
+// handle keeps a pinned buffer [x | y | phi | status words], which these kernels read and write directly.
+__global__ __launch_bounds__(256) void state_load_kernel(const double* __restrict__ h, double2* __restrict__ Z,
+                                                         double* __restrict__ P, double* __restrict__ mu,
+                                                         int* __restrict__ nonfinite, int total) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) *nonfinite = 0;
+    if (i >= total) return;
+    Z[i] = make_double2(h[i], h[total + i]);
+    P[i] = h[2 * (size_t)total + i];
+    mu[i] = 0.0;
+}
+
+struct StatusWords {
+    const int* src[4];
+    int count[4];
+};
+
+__global__ __launch_bounds__(256) void state_store_kernel(const double2* __restrict__ Z, const double* __restrict__ P,
+                                                          double* __restrict__ h, int total, StatusWords s,
+                                                          int* __restrict__ words) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (Z && i < total) {
+        const double2 z = Z[i];
+        h[i] = z.x;
+        h[total + i] = z.y;
+        h[2 * (size_t)total + i] = P[i];
+    }
+    int o = 0;
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+        if (i < s.count[a]) words[o + i] = s.src[a][i];
+        o += s.count[a];
+    }
+}
+
+// Z and P (when given) and the status words into the pinned buffer; waits for the stream.
+void Solver::store_host(const double2* Z, const double* P) {
+    StatusWords s{{status_, counters_, opt_.solver == kSolveGMRES ? gmctl_ : nullptr,
+                   opt_.solver == kSolveBatched ? bstats_ : nullptr},
+                  {2 * S_, 4, opt_.solver == kSolveGMRES ? kGmCtlInts * S_ : 0, opt_.solver == kSolveBatched ? 4 * S_ : 0}};
+    int most = Z ? T_ : 0;
+    for (int c : s.count) most = std::max(most, c);
+    hipLaunchKernelGGL(state_store_kernel, dim3((most + 255) / 256), dim3(256), 0, stream_, Z, P, host_, T_, s,
+                       reinterpret_cast<int*>(host_ + 3 * (size_t)T_));
+    SFH_HIP(hipGetLastError());
+    SFH_HIP(hipStreamSynchronize(stream_));
+    host_busy_ = false;
+}
+
 void Solver::set_state(const double* x, const double* y, const double* phi) {
     for (int i = 0; i < T_; ++i)
         if (!std::isfinite(x[i]) || !std::isfinite(y[i]) || !std::isfinite(phi[i]))
             throw ArgError("non-finite state at node " + std::to_string(i));
     check_distinct_nodes(x, y, n_);
-    std::vector<double2> z(T_);
-    for (int i = 0; i < T_; ++i) z[i] = make_double2(x[i], y[i]);
-    clear_solver_state();
-    SFH_HIP(hipMemcpyAsync(Z0_, z.data(), T_ * sizeof(double2), hipMemcpyHostToDevice, stream_));
-    SFH_HIP(hipMemcpyAsync(P0_, phi, T_ * sizeof(double), hipMemcpyHostToDevice, stream_));
+    if (host_busy_) SFH_HIP(hipStreamSynchronize(stream_));   // an earlier state is still being read
+    const size_t bytes = T_ * sizeof(double);
+    std::memcpy(host_, x, bytes);
+    std::memcpy(host_ + T_, y, bytes);
+    std::memcpy(host_ + 2 * (size_t)T_, phi, bytes);
+    hipLaunchKernelGGL(state_load_kernel, dim3((T_ + 255) / 256), dim3(256), 0, stream_, (const double*)host_, Z0_, P0_,
+                       mu_, counters_ + 1, T_);
+    SFH_HIP(hipGetLastError());
+    host_busy_ = true;
+    clear_gmres_state();
     if (gmhvalid_) SFH_HIP(hipMemsetAsync(gmhvalid_, 0, 4 * sizeof(int), stream_));   // a new trajectory
     hist_steps_ = 0;
     time_ = drive_t_ = drive_prev_ = 0.0;
     if (D0_) SFH_HIP(hipMemsetAsync(D0_, 0, T_ * sizeof(double), stream_));
     if (bhvalid_) SFH_HIP(hipMemsetAsync(bhvalid_, 0, 4 * S_ * sizeof(int), stream_));
-    SFH_HIP(hipStreamSynchronize(stream_));
 }
 
 void Solver::get_state(double* x, double* y, double* phi) {
-    std::vector<double2> z(T_);
-    SFH_HIP(hipMemcpyAsync(z.data(), Z0_, T_ * sizeof(double2), hipMemcpyDeviceToHost, stream_));
-    SFH_HIP(hipMemcpyAsync(phi, P0_, T_ * sizeof(double), hipMemcpyDeviceToHost, stream_));
-    SFH_HIP(hipStreamSynchronize(stream_));
-    for (int i = 0; i < T_; ++i) {
-        x[i] = z[i].x;
-        y[i] = z[i].y;
-    }
-    check_status();
+    store_host(Z0_, P0_);
+    const size_t bytes = T_ * sizeof(double);
+    std::memcpy(x, host_, bytes);
+    std::memcpy(y, host_ + T_, bytes);
+    std::memcpy(phi, host_ + 2 * (size_t)T_, bytes);
+    parse_status();
 }
 
 void Solver::rhs(double* vx, double* vy, double* dphi, double* mu, double2* zp, double2* zpp, double2* qup) {
@@ -1038,20 +1123,17 @@ void Solver::rhs(double* vx, double* vy, double* dphi, double* mu, double2* zp, 
     set_delayed_ctl(c, D0_, nullptr);
     timed_coefficients(c, drive_t_, 0);   // timed drive: at the handle's time, nothing saved
     enqueue_rhs(Z0_, P0_, c);
-    std::vector<double2> q(T_);
-    SFH_HIP(hipMemcpyAsync(q.data(), kZ_[0], T_ * sizeof(double2), hipMemcpyDeviceToHost, stream_));
-    SFH_HIP(hipMemcpyAsync(dphi, kP_[0], T_ * sizeof(double), hipMemcpyDeviceToHost, stream_));
     if (mu) SFH_HIP(hipMemcpyAsync(mu, mu_, T_ * sizeof(double), hipMemcpyDeviceToHost, stream_));
     if (zp) SFH_HIP(hipMemcpyAsync(zp, Zp_, T_ * sizeof(double2), hipMemcpyDeviceToHost, stream_));
     if (zpp) SFH_HIP(hipMemcpyAsync(zpp, Zpp_, T_ * sizeof(double2), hipMemcpyDeviceToHost, stream_));
     if (qup) SFH_HIP(hipMemcpyAsync(qup, qup_, T_ * sizeof(double2), hipMemcpyDeviceToHost, stream_));
-    SFH_HIP(hipStreamSynchronize(stream_));
-    for (int i = 0; i < T_; ++i) {
-        vx[i] = q[i].x;
-        vy[i] = q[i].y;
-    }
+    store_host(kZ_[0], kP_[0]);
+    const size_t bytes = T_ * sizeof(double);
+    std::memcpy(vx, host_, bytes);
+    std::memcpy(vy, host_ + T_, bytes);
+    std::memcpy(dphi, host_ + 2 * (size_t)T_, bytes);
     stats_.rhs_evals += 1;
-    check_status();
+    parse_status();
 }
 
 void Solver::set_drive(const Phys& d) {
@@ -1136,27 +1218,27 @@ void Solver::get_mu(double* mu) {
     SFH_HIP(hipStreamSynchronize(stream_));
 }
 
-void Solver::sync() {
-    SFH_HIP(hipStreamSynchronize(stream_));
-    check_status();
-}
+void Solver::sync() { check_status(); }
 
 void Solver::check_status() {
-    std::vector<int> st(2 * S_);
-    int cnt[4];
-    SFH_HIP(hipMemcpy(st.data(), status_, 2 * S_ * sizeof(int), hipMemcpyDeviceToHost));
-    SFH_HIP(hipMemcpy(cnt, counters_, sizeof(cnt), hipMemcpyDeviceToHost));
+    store_host(nullptr, nullptr);
+    parse_status();
+}
+
+// The status words that store_host left in the pinned buffer.
+void Solver::parse_status() {
+    const int* st = reinterpret_cast<const int*>(host_ + 3 * (size_t)T_);
+    const int* cnt = st + 2 * S_;
+    const int* ctl = cnt + 4;   // the GMRES control blocks, or the batched solver's per-surface words
     stats_.fallback_solves = cnt[0];
     int timeouts = 0;
     for (int s = 0; s < S_; ++s) timeouts += st[2 * s + 1] != 0;
     stats_.spin_timeouts = timeouts;
     if (opt_.solver == kSolveGMRES) {
-        std::vector<int> ctl((size_t)kGmCtlInts * S_);
-        SFH_HIP(hipMemcpy(ctl.data(), gmctl_, ctl.size() * sizeof(int), hipMemcpyDeviceToHost));
         int mx = 0, unc = 0, fill = 0;
         for (int s = 0; s < S_; ++s) {
             GmCtl c;
-            std::memcpy(&c, ctl.data() + (size_t)kGmCtlInts * s, sizeof(GmCtl));
+            std::memcpy(&c, ctl + (size_t)kGmCtlInts * s, sizeof(GmCtl));
             mx = std::max(mx, c.iters);
             unc += c.unconverged;
             fill = std::max(fill, c.fill_iters);
@@ -1171,8 +1253,7 @@ void Solver::check_status() {
         stats_.unconverged = unc;
     }
     if (opt_.solver == kSolveBatched) {
-        std::vector<int> bs(4 * (size_t)S_);
-        SFH_HIP(hipMemcpy(bs.data(), bstats_, bs.size() * sizeof(int), hipMemcpyDeviceToHost));
+        const int* bs = ctl;
         int mx = 0, unc = 0;
         for (int s = 0; s < S_; ++s) {
             mx = std::max(mx, bs[4 * s]);

@@ -217,7 +217,10 @@ class Solver {
     void calibrate();               // bookkeeping after a full-length step while the history fills
     void save_checkpoint();         // state, last solution and warm-start history, device to device
     void restore_checkpoint();
-    void check_status();
+    void check_status();           // waits for the stream
+    void parse_status();
+    void store_host(const double2* Z, const double* P);
+    void clear_gmres_state();
     template <class F>
     void launch(const char* tag, double flops, double bytes, F&& f, int iter = -1);
     // A kernel launch on stream_.  Inside a timed launch() it records the kernel's own start (the
@@ -226,6 +229,8 @@ class Solver {
     dim3 circ_grid(int rows) const { return dim3((maxN_ + rows - 1) / rows, S_); }   // circulant derivative kernels
     template <typename K, typename... Args>
     void go(K kernel, dim3 grid, dim3 block, unsigned shm, Args... args);
+    double* host_ = nullptr;       // pinned: [x | y | phi] of a state or a right-hand side, then the status words
+    bool host_busy_ = false;       // set_state's kernel may still be reading it
     hipEvent_t ev_a_ = nullptr, ev_b_ = nullptr;
 
     struct Timed {
