@@ -894,9 +894,11 @@ int sfh_get_energies(sfh_handle h, double* out) {
 
 int sfh_device_state(sfh_handle h, void** Z, void** phi) {
     SFH_NEED(h);
-    if (Z) *Z = h->s->device_Z();
-    if (phi) *phi = h->s->device_phi();
-    return 0;
+    return guarded([&] {
+        h->s->share_state();
+        if (Z) *Z = h->s->device_Z();
+        if (phi) *phi = h->s->device_phi();
+    });
 }
 
 const char* sfh_last_error(void) { return g_last_error.c_str(); }

@@ -1102,6 +1102,12 @@ void Solver::set_state(const double* x, const double* y, const double* phi) {
     time_ = drive_t_ = drive_prev_ = 0.0;
     if (D0_) SFH_HIP(hipMemsetAsync(D0_, 0, T_ * sizeof(double), stream_));
     if (bhvalid_) SFH_HIP(hipMemsetAsync(bhvalid_, 0, 4 * S_ * sizeof(int), stream_));
+    if (shared_) SFH_HIP(hipStreamSynchronize(stream_));
+}
+
+void Solver::share_state() {
+    shared_ = true;
+    SFH_HIP(hipStreamSynchronize(stream_));
 }
 
 void Solver::get_state(double* x, double* y, double* phi) {

@@ -154,7 +154,9 @@ class Solver {
     int precision() const { return opt_.precision; }
     int pair_rows() const { return rows_; }
 
-    // Raw device buffers (state y0) for zero-copy interop.
+    // Raw device buffers (state y0) for zero-copy interop.  Once they are given out, set_state returns only when the
+    // state is in them.
+    void share_state();
     double2* device_Z() { return Z0_; }
     double* device_phi() { return P0_; }
 
@@ -230,6 +232,7 @@ class Solver {
     template <typename K, typename... Args>
     void go(K kernel, dim3 grid, dim3 block, unsigned shm, Args... args);
     double* host_ = nullptr;       // pinned: [x | y | phi] of a state or a right-hand side, then the status words
+    bool shared_ = false;          // share_state was called
     bool host_busy_ = false;       // set_state's kernel may still be reading it
     hipEvent_t ev_a_ = nullptr, ev_b_ = nullptr;
 
