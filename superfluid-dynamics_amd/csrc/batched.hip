@@ -1,16 +1,16 @@
 // batched.hip -- persistent per-surface stage kernel for ensembles of independent surfaces
 // (every N <= 1024): ONE launch per RK4 stage advances all surfaces.
 //
-// Workgroup b owns surface order[b]; the order is by decreasing N, so the in-order dispatch of
+// Workgroup b works on surface order[b]; the order is by decreasing N, so the in-order dispatch of
 // workgroups schedules the largest surfaces first and the small ones fill the machine behind them.
-// A workgroup runs the whole right-hand side of its surface with no inter-workgroup
-// synchronisation (BaseBoundaryIntegralCalculator::runTimeStep,
-// CuSuperHelium/BaseBoundaryIntegrator.cuh:137-314, for one member of the batch):
+// With as many surfaces as CUs a surface has one workgroup, which runs its whole right-hand side with no
+// inter-workgroup synchronisation; with fewer, the largest surfaces have several, which share the pair sweeps and the
+// products (sfh_cluster.hpp; SHARED).  The right-hand side is BaseBoundaryIntegralCalculator::runTimeStep
+// (CuSuperHelium/BaseBoundaryIntegrator.cuh:137-314) for one member of the batch:
 //   A  spectral derivatives in LDS: Z' and Z'' from ONE forward transform of Z - 2 pi j / N,
 //      Phi' from a second (Derivatives.cuh:310-384), plus the per-node half-angle table;
-//   B  the dipole matrix M = I/2 + K (createM.cuh:43-92) into HBM, column-major per surface
-//      (element (k, j) at j N + k, the reference's own layout), FP64 or FP32 (FP64 entries
-//      rounded), and in the same pair loop M x for the warm start x (the first residual);
+//   B  the dipole matrix M = I/2 + K (createM.cuh:43-92) into HBM, in the order in which the sweeps visit it
+//      (sfh_sym.hpp), FP64 or FP32 (FP64 entries rounded), and in the same pair loop M x for the warm start x (the first residual);
 //   C  the solve M mu = b, warm-started from the surface's previous mu:
 //        FP64  : GMRES on the stored FP64 matrix (classical Gram-Schmidt with one
 //                re-orthogonalisation, restarted cycles of kBK vectors);
@@ -25,16 +25,20 @@
 //
 // Thread t owns node t.  The pair loops (assembly, the matrix-free FP64 product, velocity) visit
 // every unordered pair of nodes once in 64 x 64 tiles and give both rows of the pair their
-// contribution (sfh_sym.hpp); the matrix is stored in the tiles' skewed layout, so every store
+// contribution (sfh_sym.hpp); a wave stores the entries it forms in rows of its own, so every store
 // and every load of the stored product is one contiguous 512-byte (FP64) or 256-byte (FP32) row
 // per wave, and node data is read from LDS without bank conflicts.
+//
+// Bounds: N = 1024 mixed water, one workgroup, one Arnoldi step 577 us: derivatives 25, assembly sweep 205, product 155
+// (128 such surfaces read their matrices at 3.6 TB/s), the rest of the solve 39, mu' 7, velocity sweep 140; the sweeps
+// issue FP64 instructions back to back.
 #include <type_traits>
 
 #include "sfh_sym.hpp"
 
 namespace sfh {
 
-template <bool MIXED, bool FILM>
+template <bool MIXED, bool FILM, bool SHARED>
 __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys ph, StageCtl ctl) {
     __shared__ BLds L;
     const int s = a.order[blockIdx.x];
@@ -42,12 +46,36 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
     const int n = d.n, off = d.voff, t = threadIdx.x;
     const bool own = t < n;
     const double twopi_n = 2.0 * kPi / n;
+    Cluster cl{1, 1, 0, 1, 0, false, nullptr, nullptr, nullptr};
+    int ticket = 0;
+    if constexpr (SHARED) cl.parts = a.parts[s];
+    if (cl.parts > 1) {
+        cl.launched = min(cl.parts, a.max_wgs);
+        cl.xb = a.xbuf + a.xoff[s];
+        cl.words = a.words + 16 * s;
+        cl.failed = a.status + 2 * s + 1;
+        if (t == 0) ticket = Cluster::add(cl.words, 1);
+    }
 
     // ---------------------------------------------------------------- A: derivatives
     const NodeVals nv = wg_derivatives(d, a.tw_all, a.Zin, a.Pin, ph, L);
     const double2 zk = nv.z, zpk = nv.zp, zppk = nv.zpp;
     const double bk = nv.b;
-    if (own) {
+    if (cl.parts > 1) {
+        __shared__ int joined[2];
+        if (t == 0) {
+            cl.join(ticket);
+            joined[0] = cl.rank;
+            joined[1] = cl.members;
+            if (cl.members == 0) cl.leave();
+        }
+        __syncthreads();
+        cl.rank = __builtin_amdgcn_readfirstlane(joined[0]);
+        cl.members = __builtin_amdgcn_readfirstlane(joined[1]);
+        if (cl.members == 0) return;
+    }
+    const bool lead = cl.rank == 0;   // the one that stores what the others hold as well
+    if (own && lead) {
         a.Zp[off + t] = zpk;
         a.Zpp[off + t] = zppk;
         a.b[off + t] = bk;
@@ -66,15 +94,18 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
 
     // ---------------------------------------------------------------- B: assembly
     // One sweep over the unordered pairs (sfh_sym.hpp) writes both entries of each pair into the
-    // tile-skewed matrix (FP64, or FP64 entries rounded to FP32) and forms (M x)_k for the warm start
+    // wave's rows of the matrix (FP64, or FP64 entries rounded to FP32) and forms (M x)_k for the warm start
     // x in FP64 from the unrounded entries: the first residual of the solve.
     const bool water = ph.kind == 0;
     PairConst pc = wg_diagonal(ph, nv, n, L);
     pc.image = FILM;   // known when compiled
+    using MT = std::conditional_t<MIXED, float, double>;
+    MT* const Mt = reinterpret_cast<MT*>(a.M) + d.moff;
     const int nbk = (n + kTile - 1) / kTile;
     if (t < nbk * kTile) L.vs[t] = own ? x : 0.0;   // the padding entries stay 0 for every product
     __syncthreads();
     double dsq = 0.0;   // mixed: this thread's share of ||M||_F^2
+    double mx0;         // (M x)_t
     {
         const SymGeo sg = sym_geo(n);
         const int kr = sg.I * kTile + sg.l;
@@ -82,38 +113,27 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
         const double2 zq = L.zp[kr];
         const double2 czk = make_double2(pc.c * zq.x, pc.c * zq.y);
         const double vk = L.vs[kr];
+        MT* const Mi = Mt + (long long)(sg.I * nbk) * kTileElems;   // wave-uniform; the offsets are 32-bit
+        const unsigned l = sg.l;
         double* const acc[1] = {L.part};
-        auto store = [&](auto* Mt) {
-            using T = typename std::remove_pointer<decltype(Mt)>::type;
-            // the diagonal: offset 0 of the diagonal tiles
-            if (t < nbk * kTile) {
-                const double dg = own ? L.diag[t] : 0.0;
-                Mt[(long long)((t >> 6) * nbk + (t >> 6)) * kTileElems + (t & 63)] = (T)dg;
-                dsq += dg * dg;
-            }
-            sym_sweep<1>(n, acc, [&](int k, int j, int J, int r, auto mirror, auto full, double (&row)[1], double (&col)[1]) {
-                // tile bases are wave-uniform; the offsets within a tile are 32-bit
-                T* const tij = Mt + (long long)(sg.I * nbk + J) * kTileElems;
-                T* const tji = Mt + (long long)(J * nbk + sg.I) * kTileElems;
-                const unsigned l = sg.l;
-                double e = 0.0, em = 0.0;
-                if (decltype(full)::value || (k < n && j < n)) {
-                    entry_pair(tk, L.tr[j], czk, L.zp[j], pc, e, em);
-                    row[0] += e * L.vs[j];
-                    dsq += e * e;
-                    if constexpr (decltype(mirror)::value) {
-                        col[0] += em * vk;
-                        dsq += em * em;
-                    }
+        double mx[1];
+        if (MIXED && own && lead) dsq = L.diag[t] * L.diag[t];
+        sym_sums<1>(n, acc, [&](int k, int j, int q, auto mirror, auto full, double (&row)[1], double (&col)[1]) {
+            double e = 0.0, em = 0.0;
+            if (decltype(full)::value || (k < n && j < n)) {
+                entry_pair(tk, L.tr[j], czk, L.zp[j], pc, e, em);
+                row[0] += e * L.vs[j];
+                if constexpr (MIXED) dsq += e * e;
+                if constexpr (decltype(mirror)::value) {
+                    col[0] += em * vk;
+                    if constexpr (MIXED) dsq += em * em;
                 }
-                tij[(unsigned)r * kTile + l] = (T)e;
-                if constexpr (decltype(mirror)::value) tji[((unsigned)(kTile - r) & (kTile - 1)) * kTile + ((l + r) & (kTile - 1))] = (T)em;
-            });
-        };
-        store(reinterpret_cast<std::conditional_t<MIXED, float, double>*>(a.M) + d.moff);
+            }
+            Mi[(unsigned)(2 * q) * kTile + l] = (MT)e;
+            Mi[(unsigned)(2 * q + 1) * kTile + l] = decltype(mirror)::value ? (MT)em : (MT)0;
+        }, cl, mx);
+        mx0 = own ? mx[0] + L.diag[t] * L.vs[t] : 0.0;
     }
-    double mx0 = 0.0;   // (M x)_t
-    if (own) mx0 = sym_total(L.part, n) + L.diag[t] * L.vs[t];
     __syncthreads();
 
     // ---------------------------------------------------------------- C: solve
@@ -128,20 +148,20 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
     }
     int unconv = 0, iters = 0, sweeps = 0;
     if constexpr (!MIXED) {
-        const double* Md = reinterpret_cast<const double*>(a.M) + d.moff;
-        iters = wg_gmres([&]() { return mv_tiles(Md, n, L); }, n, bk, x, false, tol_abs, a.cycles, L, &unconv,
+        iters = wg_gmres([&]() { return mv_pairs(Mt, n, cl, L); }, n, bk, x, false, tol_abs, a.cycles, L, &unconv,
                          true, own ? bk - mx0 : 0.0, pre);
     } else {
-        const float* Mf = reinterpret_cast<const float*>(a.M) + d.moff;
         // ||M - M32||_F <= 2^-24 ||M||_F (round to nearest, normal range) + N 2^-150 (subnormal range)
-        const double dM = 0x1p-24 * sqrt(bsum1(dsq, L)) + n * 0x1p-150;
+        dsq = bsum1(dsq, L);
+        if (cl.parts > 1) dsq = cl.sum_members(n, dsq);
+        const double dM = 0x1p-24 * sqrt(dsq) + n * 0x1p-150;
         bool done = false;
         for (; sweeps < a.max_refine; ++sweeps) {
             double mx = mx0;   // sweep 0: formed by the assembly
             if (sweeps > 0) {
                 if (own) L.vs[t] = x;
                 __syncthreads();
-                mx = mv_free_sym(n, pc, L);   // every thread: it synchronises
+                mx = mv_free_sym(n, pc, cl, L);   // every thread: it synchronises
             }
             const double r = own ? bk - mx : 0.0;
             const double rn = sqrt(bsum1(r * r, L));
@@ -150,7 +170,7 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
                 break;
             }
             double dx = 0.0;
-            iters += wg_gmres([&]() { return mv_tiles(Mf, n, L); }, n, r, dx, true,
+            iters += wg_gmres([&]() { return mv_pairs(Mt, n, cl, L); }, n, r, dx, true,
                               fmax(1e-7 * rn, 0.25 * tol_abs), 1, L, nullptr, false, 0.0, pre);
             x += dx;
             // the FP64 residual of the corrected x, bounded without forming it:
@@ -166,18 +186,18 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
         }
         if (!done) unconv = 1;
     }
-    if (t == 0) {
+    if (t == 0 && lead) {
         int* st = a.stats + 4 * s;
         st[0] = iters;
         st[1] += unconv;
         st[2] = sweeps;
         if (h0) a.hvalid[(ctl.stage - 1) * a.nsurf + s] = min(hv + 1, kHistDepth);
     }
-    if (own && h0) push_history(h0 + t, a.total, x);
+    if (own && lead && h0) push_history(h0 + t, a.total, x);
 
     // ---------------------------------------------------------------- D: mu'
     if (own) {
-        a.mu[off + t] = x;
+        if (lead) a.mu[off + t] = x;
         L.fa[lds_index(d, t)] = make_double2(x, 0.0);
     }
     wg_first_derivative(d, L, false);
@@ -185,7 +205,7 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
     if (own) {
         const double2 v = L.fa[lds_index(d, t)];
         mupk = make_double2(v.x * twopi_n, v.y * twopi_n);   // BaseBoundaryIntegrator.cuh:201-203
-        a.mup[off + t] = mupk;
+        if (lead) a.mup[off + t] = mupk;
         L.vs[t] = x;
     }
     __syncthreads();
@@ -195,13 +215,14 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
     // sums too for the film).
     double* psy = reinterpret_cast<double*>(L.fa);   // 2 kBT doubles: sy | ix
     double* piy = reinterpret_cast<double*>(L.fb);
+    double vsum[FILM ? 4 : 2];   // S_x, S_y and the image sums
     {
         const int kr = sym_row(n);
         const NodeTrig tk = L.tr[kr];
         const double mk = L.vs[kr];
         if constexpr (FILM) {
             double* const acc[4] = {L.part, psy, psy + kBT, piy};
-            sym_sweep<4>(n, acc, [&](int k, int j, int, int, auto mirror, auto full, double (&row)[4], double (&col)[4]) {
+            sym_sums<4>(n, acc, [&](int k, int j, int, auto mirror, auto full, double (&row)[4], double (&col)[4]) {
                 if (!decltype(full)::value && (k >= n || j >= n)) return;
                 const NodeTrig tj = L.tr[j];
                 const double mj = L.vs[j];
@@ -219,10 +240,10 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
                     col[2] -= wki * cq.p;
                     col[3] -= wki * cq.q;
                 }
-            });
+            }, cl, vsum);
         } else {
             double* const acc[2] = {L.part, psy};
-            sym_sweep<2>(n, acc, [&](int k, int j, int, int, auto mirror, auto full, double (&row)[2], double (&col)[2]) {
+            sym_sums<2>(n, acc, [&](int k, int j, int, auto mirror, auto full, double (&row)[2], double (&col)[2]) {
                 if (!decltype(full)::value && (k >= n || j >= n)) return;
                 const CotParts cp = cot_parts(tk, L.tr[j]);
                 const double w = L.vs[j] * cp.id;
@@ -233,14 +254,17 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
                     col[0] -= wk * cp.p;
                     col[1] += wk * cp.q;
                 }
-            });
+            }, cl, vsum);
         }
+    }
+    if (cl.parts > 1) {
+        if (t == 0) cl.leave();
+        if (!lead) return;
     }
     double2 q1 = make_double2(0.0, 0.0), q2 = make_double2(0.0, 0.0);
     if (own) {
-        const double sx = sym_total(L.part, n), sy = sym_total(psy, n);
-        const double ix = FILM ? sym_total(psy + kBT, n) : 0.0, iy = FILM ? sym_total(piy, n) : 0.0;
-        velocity_from_sums(ph, zpk, zppk, mupk, x, zk.y, sx, sy, ix, iy, q1, q2);
+        velocity_from_sums(ph, zpk, zppk, mupk, x, zk.y, vsum[0], vsum[1], FILM ? vsum[FILM ? 2 : 0] : 0.0,
+                           FILM ? vsum[FILM ? 3 : 0] : 0.0, q1, q2);
     }
     // createM.cuh:104 reads the lower velocity of node 1 in the rho * q1.q2 term
     double2 q1q = q1;
@@ -267,9 +291,12 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
     stage_update(ctl, gi, q1, dphi);
 }
 
-template __global__ void batched_stage_kernel<false, false>(BatchArgs, Phys, StageCtl);
-template __global__ void batched_stage_kernel<false, true>(BatchArgs, Phys, StageCtl);
-template __global__ void batched_stage_kernel<true, false>(BatchArgs, Phys, StageCtl);
-template __global__ void batched_stage_kernel<true, true>(BatchArgs, Phys, StageCtl);
+#define SFH_BATCHED_INSTANCES(SHARED)                                                        \
+    template __global__ void batched_stage_kernel<false, false, SHARED>(BatchArgs, Phys, StageCtl); \
+    template __global__ void batched_stage_kernel<false, true, SHARED>(BatchArgs, Phys, StageCtl);  \
+    template __global__ void batched_stage_kernel<true, false, SHARED>(BatchArgs, Phys, StageCtl);  \
+    template __global__ void batched_stage_kernel<true, true, SHARED>(BatchArgs, Phys, StageCtl);
+SFH_BATCHED_INSTANCES(false)
+SFH_BATCHED_INSTANCES(true)
 
 }  // namespace sfh

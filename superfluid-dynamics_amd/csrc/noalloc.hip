@@ -158,7 +158,7 @@ void rhs_noalloc(const Phys& ph, int n, const double* x, const double* y, const 
     c.kZ[0] = B.q;
     c.kP[0] = dphi;
     c.Pin = phi;
-    hipLaunchKernelGGL((ph.image ? batched_stage_kernel<false, true> : batched_stage_kernel<false, false>), dim3(1), dim3(kBatchThreads), 0, stream, a, ph, c);
+    hipLaunchKernelGGL((ph.image ? batched_stage_kernel<false, true, false> : batched_stage_kernel<false, false, false>), dim3(1), dim3(kBatchThreads), 0, stream, a, ph, c);
     SFH_HIP(hipGetLastError());
     hipLaunchKernelGGL(noalloc_unpack_kernel, dim3(grid), dim3(256), 0, stream, B, n, vx, vy, mu);
     SFH_HIP(hipGetLastError());

@@ -207,11 +207,11 @@ __host__ __device__ constexpr inline long long tiled_matrix_elems(int n) {
 }
 struct BatchArgs {
     const SurfDesc* sd;
-    const int* order;          // workgroup -> surface, by decreasing N
+    const int* order;          // workgroup -> surface, by decreasing N (one entry per workgroup)
     const double2* tw_all;
     const double2* Zin;        // stage input state
     const double* Pin;
-    void* M;                   // per-surface column-major matrices (double, or float when mixed)
+    void* M;                   // per-surface matrices in the layout of sfh_sym.hpp (double, or float when mixed)
     double2* Zp;
     double2* Zpp;
     double2* mup;
@@ -223,15 +223,23 @@ struct BatchArgs {
     int max_refine;            // refinement sweeps (mixed)
     int nsurf;
     int total;                 // nodes of all surfaces
-    int pad;
+    int max_wgs;               // workgroups of a surface (at most its parts)
     // warm start by extrapolation over steps: stage s (1..4) keeps each surface's mu of the last
     // kHistDepth steps at hist + ((s - 1) kHistDepth + l) total, l = 0 newest;
     // hvalid[(s - 1) nsurf + i] counts them for surface i
     double* hist;
     int* hvalid;
+    // surfaces with several workgroups (sfh_cluster.hpp; null when every surface has one): parts of surface s, its
+    // 16 words, and its exchange buffers at xbuf + xoff[s]
+    const int* parts;
+    int* words;
+    double* xbuf;
+    const long long* xoff;
+    int* status;               // [2 s + 1]: a wait gave up
 };
-// MIXED: the stored matrix is FP32; FILM: the surface has an image term
-template <bool MIXED, bool FILM>
+constexpr int kMaxParts = 8;
+// MIXED: the stored matrix is FP32; FILM: the surface has an image term; SHARED: some surface has several workgroups
+template <bool MIXED, bool FILM, bool SHARED>
 __global__ void batched_stage_kernel(BatchArgs a, Phys ph, StageCtl ctl);
 
 // ---- adjoint.hip (reverse mode of the water right-hand side, every N <= kBatchMaxN)

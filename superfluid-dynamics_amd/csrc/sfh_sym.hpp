@@ -23,13 +23,18 @@
 // one block row only, so the column sums go into an LDS slot per sub-wave without atomics; a barrier
 // separates the phases, and every sum is formed in a fixed order.
 //
-// Stored matrix (tile-skewed): the nb x nb tiles of a surface follow each other, tile (I, J) at
-// element (I nb + J) * 4096; element (row I*64 + l, column J*64 + (l + r) % 64) sits at r * 64 + l
-// of its tile.  A wave's 64 stores of one offset, direct or mirrored, fall in one contiguous row of
-// 64 elements, and so do the 64 loads of one offset in the product.  Rows and columns beyond N hold 0.
+// Parts.  A surface's sweeps can be split into a few parts, each for a workgroup of its own (sfh_cluster.hpp):
+// part p of P takes its share of every range of offsets, as if the sub-waves of a block row were P times as many.
+//
+// Stored matrix.  A wave keeps the entries it forms for its own products: the offset that is the q-th of
+// block row I (phase 0's offsets, then phase 1's, ...) holds its 64 direct entries M_kj at row 2 q and the
+// mirrored ones M_jk (0 where there are none) at row 2 q + 1 of the block row's 64 nb rows of 64 elements; lane l's are at element l.  The
+// product repeats the sweep with loads in place of evaluations, so a wave reads what it wrote itself, in contiguous
+// rows, and no other workgroup's stores.  Entries of nodes beyond N are 0; the diagonal stays in LDS.
 #pragma once
 #include <type_traits>
 
+#include "sfh_cluster.hpp"
 #include "sfh_wg.hpp"
 
 namespace sfh {
@@ -61,9 +66,37 @@ __device__ inline SymGeo sym_geo(int n) {
     return g;
 }
 
+// This wave's share of phase ph: offsets r0 .. r1 of block column J, of which those below rm have mirrored entries;
+// offset r is number q0 + r of the block row.
+struct SymRange {
+    int J, r0, r1, rm, q0;
+};
+__device__ inline SymRange sym_range(const SymGeo& g, int ph, int part, int parts) {
+    SymRange s;
+    s.J = (g.I + ph) % g.nb;
+    int lo, hi;
+    if (ph == 0) {
+        lo = 1;
+        hi = 33;
+    } else if (2 * ph < g.nb) {
+        lo = 0;
+        hi = kTile;
+    } else {
+        lo = g.I < g.nb / 2 ? 1 : 0;
+        hi = lo + 32;
+    }
+    const int i = part * g.wpb + g.sub, m = parts * g.wpb;
+    s.r0 = lo + ((hi - lo) * i) / m;
+    s.r1 = lo + ((hi - lo) * (i + 1)) / m;
+    // offset 32 of the diagonal tile (no column sums) is the last offset of its range
+    s.rm = (ph == 0 && s.r1 == 33) ? 32 : s.r1;
+    s.q0 = (ph == 0 ? 0 : 32 + kTile * (ph - 1)) - lo;
+    return s;
+}
+
 // sym_sweep for n a multiple of 64 (FULL) or not.
 template <int NA, bool FULL, class F>
-__device__ inline void sym_sweep_impl(int n, double* const (&acc)[NA], F& pair) {
+__device__ inline void sym_sweep_impl(int n, double* const (&acc)[NA], F& pair, int part, int parts) {
     const SymGeo g = sym_geo(n);
     const int t = threadIdx.x;
     const int stride = g.nb * kTile;
@@ -77,39 +110,24 @@ __device__ inline void sym_sweep_impl(int n, double* const (&acc)[NA], F& pair) 
     const int nphase = g.nb / 2 + 1;
     for (int ph = 0; ph < nphase; ++ph) {
         if (g.active) {
-            const int J = (g.I + ph) % g.nb;
-            int lo, hi;
-            if (ph == 0) {
-                lo = 1;
-                hi = 33;
-            } else if (2 * ph < g.nb) {
-                lo = 0;
-                hi = kTile;
-            } else {
-                lo = g.I < g.nb / 2 ? 1 : 0;
-                hi = lo + 32;
-            }
-            const int r0 = lo + ((hi - lo) * g.sub) / g.wpb;
-            const int r1 = lo + ((hi - lo) * (g.sub + 1)) / g.wpb;
+            const SymRange s = sym_range(g, ph, part, parts);
             double col[NA];
 #pragma unroll
             for (int a = 0; a < NA; ++a) col[a] = 0.0;
-            // offset 32 of the diagonal tile (no column sums) is the last offset of its range
-            const int rm = (ph == 0 && r1 == 33) ? 32 : r1;
-            for (int r = r0; r < rm; ++r) {
-                const int j = J * kTile + ((g.l + r) & (kTile - 1));
-                pair(k, j, J, r, std::true_type{}, std::integral_constant<bool, FULL>{}, row, col);
+            for (int r = s.r0; r < s.rm; ++r) {
+                const int j = s.J * kTile + ((g.l + r) & (kTile - 1));
+                pair(k, j, s.q0 + r, std::true_type{}, std::integral_constant<bool, FULL>{}, row, col);
 #pragma unroll
                 for (int a = 0; a < NA; ++a) col[a] = dpp_rol1(col[a]);
             }
-            if (rm < r1) {
-                const int j = J * kTile + ((g.l + 32) & (kTile - 1));
-                pair(k, j, J, 32, std::false_type{}, std::integral_constant<bool, FULL>{}, row, col);
+            if (s.rm < s.r1) {
+                const int j = s.J * kTile + ((g.l + 32) & (kTile - 1));
+                pair(k, j, s.q0 + 32, std::false_type{}, std::integral_constant<bool, FULL>{}, row, col);
 #pragma unroll
                 for (int a = 0; a < NA; ++a) col[a] = dpp_rol1(col[a]);
             }
-            if (r1 > r0) {
-                const int c = J * kTile + ((g.l + r1) & (kTile - 1));
+            if (s.r1 > s.r0) {
+                const int c = s.J * kTile + ((g.l + s.r1) & (kTile - 1));
 #pragma unroll
                 for (int a = 0; a < NA; ++a) acc[a][g.sub * stride + c] += col[a];
             }
@@ -124,18 +142,18 @@ __device__ inline void sym_sweep_impl(int n, double* const (&acc)[NA], F& pair) 
 }
 
 // The sweep.  acc[a] (a < NA) are LDS arrays of kBT doubles: slot s of node i at s * nb * 64 + i.
-// pair(k, j, J, r, mirror, full, row, col) is called by every lane of an active wave for row
-// k = I*64 + l and column j = J*64 + (l + r) % 64; it adds the pair's contribution to row k into
+// pair(k, j, q, mirror, full, row, col) is called by every lane of an active wave for row
+// k = I*64 + l and column j = J*64 + (l + r) % 64, q the offset's number in the block row; it adds the pair's contribution to row k into
 // row[] and, when mirror, to row j into col[].  mirror and full are std::integral_constant<bool>:
 // mirror is false only at offset 32 of the diagonal tile, and full (n a multiple of 64) says that
 // k and j are always < n, so the functor checks them only when it is false.  On return the total
 // of node t is sym_total(acc[a], n); the caller synchronises before reusing acc.
 template <int NA, class F>
-__device__ inline void sym_sweep(int n, double* const (&acc)[NA], F&& pair) {
+__device__ inline void sym_sweep(int n, double* const (&acc)[NA], F& pair, int part, int parts) {
     if ((n & (kTile - 1)) == 0)
-        sym_sweep_impl<NA, true>(n, acc, pair);
+        sym_sweep_impl<NA, true>(n, acc, pair, part, parts);
     else
-        sym_sweep_impl<NA, false>(n, acc, pair);
+        sym_sweep_impl<NA, false>(n, acc, pair, part, parts);
 }
 
 // The total of node t (< n) over the slots of a sweep's accumulator.
@@ -169,9 +187,32 @@ __device__ inline void entry_pair(const NodeTrig& tk, const NodeTrig& tj, double
     }
 }
 
+// The sums of a sweep over all parts of the surface: out[a] is the total of node t on threads t < n.  A workgroup
+// sweeps its own parts; with several workgroups the parts' sums meet in the exchange buffer and every workgroup
+// adds them in the parts' order.
+template <int NA, class F>
+__device__ inline void sym_sums(int n, double* const (&acc)[NA], F&& pair, Cluster& cl, double (&out)[NA]) {
+    const int t = threadIdx.x;
+    if (cl.parts == 1) {
+        sym_sweep<NA>(n, acc, pair, 0, 1);
+#pragma unroll
+        for (int a = 0; a < NA; ++a) out[a] = t < n ? sym_total(acc[a], n) : 0.0;
+        return;
+    }
+    for (int p = cl.rank; p < cl.parts; p += cl.members) {
+        sym_sweep<NA>(n, acc, pair, p, cl.parts);
+        if (t < n) {
+#pragma unroll
+            for (int a = 0; a < NA; ++a) cl.put(n, p * NA + a, sym_total(acc[a], n));
+        }
+        __syncthreads();
+    }
+    cl.exchange<NA>(n, out);
+}
+
 // (M v)_t evaluated matrix-free in FP64 (entry_pair and the diagonal), v in L.vs with the padding
 // entries 0 (the caller has synchronised).  Returns the value on threads t < n, 0 elsewhere.
-__device__ inline double mv_free_sym(int n, const PairConst& pc, BLds& L) {
+__device__ inline double mv_free_sym(int n, const PairConst& pc, Cluster& cl, BLds& L) {
     const int t = threadIdx.x;
     const int kr = sym_row(n);
     const NodeTrig tk = L.tr[kr];
@@ -179,55 +220,77 @@ __device__ inline double mv_free_sym(int n, const PairConst& pc, BLds& L) {
     const double2 czk = make_double2(pc.c * zq.x, pc.c * zq.y);
     const double vk = L.vs[kr];
     double* const acc[1] = {L.part};
-    sym_sweep<1>(n, acc, [&](int k, int j, int, int, auto mirror, auto full, double (&row)[1], double (&col)[1]) {
+    double w[1];
+    sym_sums<1>(n, acc, [&](int k, int j, int, auto mirror, auto full, double (&row)[1], double (&col)[1]) {
         if (!decltype(full)::value && (k >= n || j >= n)) return;
         double e, em;
         entry_pair(tk, L.tr[j], czk, L.zp[j], pc, e, em);
         row[0] += e * L.vs[j];
         if constexpr (decltype(mirror)::value) col[0] += em * vk;
-    });
-    double w = 0.0;
-    if (t < n) w = sym_total(L.part, n) + L.diag[t] * L.vs[t];
+    }, cl, w);
+    if (t < n) w[0] += L.diag[t] * L.vs[t];
     __syncthreads();
-    return w;
+    return w[0];
 }
 
-// (M v)_t for the stored tile-skewed matrix, v in L.vs with L.vs[j] = 0 for n <= j < nb*64 (the
-// caller has synchronised).  Returns the value on threads t < n, 0 elsewhere.  The waves of a block
-// row split its nb * 64 offset rows; partial sums meet in L.part.
+// (M v)_t for the matrix that the waves stored (see above), v in L.vs with L.vs[j] = 0 for n <= j < nb*64
+// (the caller has synchronised).  Returns the value on threads t < n, 0 elsewhere.
 template <typename T>
-__device__ inline double mv_tiles(const T* __restrict__ M, int n, BLds& L) {
+__device__ inline double mv_pairs(const T* __restrict__ M, int n, Cluster& cl, BLds& L) {
     const SymGeo g = sym_geo(n);
-    const int t = threadIdx.x;
-    double acc0 = 0.0, acc1 = 0.0;
-    if (g.active) {
-        const int span = g.nb * kTile;   // offset rows of the block row
-        const int i0 = (span * g.sub) / g.wpb, i1 = (span * (g.sub + 1)) / g.wpb;
-        const T* base = M + (long long)g.I * g.nb * kTileElems + g.l;
-        constexpr int U = sizeof(T) == 8 ? 16 : 32;   // loads in flight per lane
-        int i = i0;
-        for (; i + U <= i1; i += U) {
-            T m[U];
+    const int t = threadIdx.x, stride = g.nb * kTile, k = g.I * kTile + g.l;
+    constexpr int U = sizeof(T) == 8 ? 8 : 16;   // offsets in flight per lane, two loads each
+    const T* base = M + (long long)g.I * g.nb * kTileElems + g.l;
+    double w[1] = {0.0};
+    for (int p = cl.rank; p < cl.parts; p += cl.members) {
+        L.part[t] = 0.0;
+        __syncthreads();
+        const double vk = L.vs[k];
+        double row = 0.0;
+        for (int ph = 0; ph <= g.nb / 2; ++ph) {
+            if (g.active) {
+                const SymRange s = sym_range(g, ph, p, cl.parts);
+                double col = 0.0;
+                auto chunk = [&](int r, auto whole) {
+                    constexpr bool W = decltype(whole)::value;
+                    T m[U], mm[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) m[u] = base[(long long)(i + u) * kTile];
+                    for (int u = 0; u < U; ++u) {   // clamped: no branch between the loads, nor around their uses
+                        const unsigned q = 2 * (s.q0 + (W ? r + u : min(r + u, s.r1 - 1))) * kTile;
+                        m[u] = base[q];
+                        mm[u] = base[q + kTile];
+                    }
 #pragma unroll
-            for (int u = 0; u < U; u += 2) {
-                const int ia = i + u, ib = i + u + 1;
-                acc0 += (double)m[u] * L.vs[(ia & ~(kTile - 1)) + ((g.l + ia) & (kTile - 1))];
-                acc1 += (double)m[u + 1] * L.vs[(ib & ~(kTile - 1)) + ((g.l + ib) & (kTile - 1))];
+                    for (int u = 0; u < U; ++u) {
+                        const double vj = L.vs[s.J * kTile + ((g.l + r + u) & (kTile - 1))];
+                        row += (double)m[u] * (W || r + u < s.r1 ? vj : 0.0);
+                        col += (double)mm[u] * (W || r + u < s.r1 ? vk : 0.0);
+                        col = dpp_rol1(col);
+                    }
+                };
+                int r = s.r0;
+                for (; r + U <= s.r1; r += U) chunk(r, std::true_type{});
+                if (r < s.r1) {
+                    chunk(r, std::false_type{});
+                    r += U;
+                }
+                // the register has moved down once per offset taken
+                if (r > s.r0) L.part[g.sub * stride + s.J * kTile + ((g.l + r) & (kTile - 1))] += col;
             }
+            __syncthreads();
         }
-        for (; i < i1; ++i)
-            acc0 += (double)base[(long long)i * kTile] * L.vs[(i & ~(kTile - 1)) + ((g.l + i) & (kTile - 1))];
+        if (g.active) L.part[g.sub * stride + k] += row;
+        __syncthreads();
+        if (t < n) {
+            w[0] = sym_total(L.part, n);
+            if (cl.parts > 1) cl.put(n, p, w[0]);
+        }
+        __syncthreads();
     }
-    const int stride = g.nb * kTile;
-    if (g.active) L.part[g.sub * stride + g.I * kTile + g.l] = acc0 + acc1;
+    if (cl.parts > 1) cl.exchange<1>(n, w);
+    if (t < n) w[0] += (double)(T)L.diag[t] * L.vs[t];
     __syncthreads();
-    double w = 0.0;
-    if (t < n)
-        for (int q = 0; q < g.wpb; ++q) w += L.part[q * stride + t];
-    __syncthreads();
-    return w;
+    return w[0];
 }
 
 }  // namespace sfh

@@ -22,6 +22,7 @@
 
 #include <hip/hip_ext.h>
 
+#include "sfh_cluster.hpp"
 #include "sfh_gmres.hpp"
 #include "solver.hpp"
 
@@ -246,8 +247,28 @@ Solver::Solver(const Phys& ph, const std::vector<int>& n, const Options& opt) : 
         std::vector<int> ord(S_);
         for (int s = 0; s < S_; ++s) ord[s] = s;
         std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return n_[a] > n_[b]; });
-        order_ = dalloc<int>(S_);
-        SFH_HIP(hipMemcpy(order_, ord.data(), S_ * sizeof(int), hipMemcpyHostToDevice));
+        const std::vector<int> parts = batched_parts();
+        const int cap = opt_.force_trim > 0 ? opt_.force_trim : kMaxParts;
+        std::vector<int> wgs;
+        std::vector<long long> xoff(S_);
+        long long xtot = 0;
+        for (int s : ord) {
+            for (int p = 0; p < std::min(parts[s], cap); ++p) wgs.push_back(s);
+            xoff[s] = xtot;
+            if (parts[s] > 1) xtot += 2LL * parts[s] * Cluster::kMaxSums * n_[s];
+        }
+        bgrid_ = (int)wgs.size();
+        order_ = dalloc<int>(wgs.size());
+        SFH_HIP(hipMemcpy(order_, wgs.data(), wgs.size() * sizeof(int), hipMemcpyHostToDevice));
+        if (xtot > 0) {
+            bparts_ = dalloc<int>(S_);
+            bwords_ = dalloc<int>(16 * (size_t)S_);
+            bxoff_ = dalloc<long long>(S_);
+            bxbuf_ = dalloc<double>(xtot);
+            SFH_HIP(hipMemcpy(bparts_, parts.data(), S_ * sizeof(int), hipMemcpyHostToDevice));
+            SFH_HIP(hipMemcpy(bxoff_, xoff.data(), S_ * sizeof(long long), hipMemcpyHostToDevice));
+            SFH_HIP(hipMemset(bwords_, 0, 16 * (size_t)S_ * sizeof(int)));
+        }
         bstats_ = dalloc<int>(4 * (size_t)S_);
         SFH_HIP(hipMemset(bstats_, 0, 4 * S_ * sizeof(int)));
         bhist_ = dalloc<double>(4 * kHistDepth * (size_t)T_);
@@ -255,6 +276,29 @@ Solver::Solver(const Phys& ph, const std::vector<int>& n, const Options& opt) : 
         SFH_HIP(hipMemset(bhvalid_, 0, 4 * S_ * sizeof(int)));
     }
     SFH_HIP(hipDeviceSynchronize());
+}
+
+// Parts of each surface of the batched stage (sfh_cluster.hpp).  The stage lasts as long as its slowest surface, so
+// while CUs are left, the slowest one gets one more.  A stage takes about 30 us that each workgroup repeats, 5.2e-4 us
+// per squared node count to share out, and 15 us for the meetings.  24 films of 768 nodes among 96 surfaces: 373 us
+// with one workgroup each, 136 with 6 or 7; N = 256 water: 76 us with one, 66 with 8.  With as many surfaces as CUs
+// nothing is split: every CU has work.
+std::vector<int> Solver::batched_parts() const {
+    std::vector<int> parts(S_, 1);
+    int dev = 0, cus = 0;
+    SFH_HIP(hipGetDevice(&dev));
+    SFH_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    const auto cost = [&](int s, int p) { return 30.0 + 5.2e-4 * n_[s] * n_[s] / p + (p > 1 ? 15.0 : 0.0); };
+    for (int left = cus - S_; left > 0; --left) {
+        int worst = 0;
+        for (int s = 1; s < S_; ++s)
+            if (cost(s, parts[s]) > cost(worst, parts[worst])) worst = s;
+        const int p = parts[worst];
+        // the first split has to pay for its meetings with more than one extra workgroup's share
+        if (p == kMaxParts || cost(worst, p == 1 ? std::min(3, 1 + left) : p + 1) >= cost(worst, p)) break;
+        ++parts[worst];
+    }
+    return parts;
 }
 
 // GMRES buffers for a Krylov dimension of m (the GMRES solver, and the transposed solves of the
@@ -299,7 +343,7 @@ Solver::~Solver() {
     if (graph_) (void)hipGraphDestroy(graph_);
     void* bufs[] = {d_desc_, d_tw_, Z0_, Za_, Zb_, P0_, Pa_, Pb_, kZ_[0], kZ_[1], kZ_[2], kP_[0],
                     kP_[1], kP_[2], Zp_, Zpp_, mup_, qup_, b_, work_, y_, mu_, M_, uinv_, flags_,
-                    status_, piv_, counters_, gmV_, gmZ_, gmw_, gmpart_, gmsmall_, gmctl_, trig_, order_, bstats_,
+                    status_, piv_, counters_, gmV_, gmZ_, gmw_, gmpart_, gmsmall_, gmctl_, trig_, order_, bstats_, bparts_, bwords_, bxoff_, bxbuf_,
                     gmhist_, gmhvalid_, bhist_, bhvalid_, d_circ_, gmx0_, M32_, ckZ_, ckP_, ckMu_, ckHist_,
                     ckHv_, energy_, D0_, Da_, Db_, ckD_, kD_[0], kD_[1], kD_[2]};
     for (void* p : bufs)
@@ -560,6 +604,12 @@ void Solver::enqueue_batched(const double2* Z, const double* P, const StageCtl& 
     a.total = T_;
     a.hist = bhist_;
     a.hvalid = bhvalid_;
+    a.parts = bparts_;
+    a.words = bwords_;
+    a.xbuf = bxbuf_;
+    a.xoff = bxoff_;
+    a.status = status_;
+    a.max_wgs = opt_.force_trim > 0 ? opt_.force_trim : kMaxParts;
     double nsq = 0.0;
     for (int v : n_) nsq += (double)v * v;
     const double img = ph_.image ? 2.0 : 1.0;
@@ -567,8 +617,16 @@ void Solver::enqueue_batched(const double2* Z, const double* P, const StageCtl& 
     // algorithmic work per launch: cot pairs of assembly + velocity (and one more pass per
     // refinement residual), matrix written once and read once per GMRES product
     launch("stage", 2.0 * img * nsq, 2.0 * mbytes, [&] {
-        go(mixed ? (ph_.image ? batched_stage_kernel<true, true> : batched_stage_kernel<true, false>)
-                 : (ph_.image ? batched_stage_kernel<false, true> : batched_stage_kernel<false, false>), dim3(S_), dim3(kBatchThreads), 0, a, ph_, ctl);
+        const auto stage = [&](auto shared) {
+            constexpr bool S = decltype(shared)::value;
+            go(mixed ? (ph_.image ? batched_stage_kernel<true, true, S> : batched_stage_kernel<true, false, S>)
+                     : (ph_.image ? batched_stage_kernel<false, true, S> : batched_stage_kernel<false, false, S>),
+               dim3(bgrid_), dim3(kBatchThreads), 0, a, ph_, ctl);
+        };
+        if (bparts_)
+            stage(std::true_type{});
+        else
+            stage(std::false_type{});
     });
     SFH_HIP(hipGetLastError());
 }

@@ -223,6 +223,7 @@ class Solver {
     void parse_status();
     void store_host(const double2* Z, const double* P);
     void clear_gmres_state();
+    std::vector<int> batched_parts() const;
     template <class F>
     void launch(const char* tag, double flops, double bytes, F&& f, int iter = -1);
     // A kernel launch on stream_.  Inside a timed launch() it records the kernel's own start (the
@@ -290,6 +291,11 @@ class Solver {
     int* gmhvalid_ = nullptr;
     // persistent per-surface stage kernel (kSolveBatched)
     int* order_ = nullptr;    // workgroup -> surface, by decreasing N
+    int bgrid_ = 0;           // workgroups of the batched stage
+    int* bparts_ = nullptr;   // with several workgroups on a surface: parts, words and exchange buffers
+    int* bwords_ = nullptr;
+    long long* bxoff_ = nullptr;
+    double* bxbuf_ = nullptr;
     int* bstats_ = nullptr;   // 4 ints per surface
     double* bhist_ = nullptr;  // per RK stage, each surface's mu of the last kHistDepth steps
     int* bhvalid_ = nullptr;
