@@ -137,19 +137,23 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
     __syncthreads();
 
     // ---------------------------------------------------------------- C: solve
-    const double bn = sqrt(bsum1(own ? bk * bk : 0.0, L));
+    const double r0 = own ? bk - mx0 : 0.0;
+    const double norms[3] = {own ? bk * bk : 0.0, r0 * r0, own ? zk.y : 0.0};
+    bsum(norms, L);
+    const double bn = sqrt(L.sums[0]), rr0 = L.sums[1];
     const double tol_abs = a.tol * bn;
     // Film: the image term's few large eigenvalues are divided out (wg_precondition).  A warm solve of N = 768,
     // h = 1 takes 1-2 products of the stored matrix (75 us each from one CU) in place of 4-5.
     Precond pre = {-1, 0.0};
     if constexpr (FILM) {
-        pre.height = bsum1(own ? zk.y : 0.0, L) / n + ph.depth;
+        pre.height = L.sums[2] / n + ph.depth;
         pre.modes = film_modes(n, pre.height);
     }
+    __syncthreads();   // the sums are read before they are formed again
     int unconv = 0, iters = 0, sweeps = 0;
     if constexpr (!MIXED) {
         iters = wg_gmres([&]() { return mv_pairs(Mt, n, cl, L); }, n, bk, x, false, tol_abs, a.cycles, L, &unconv,
-                         true, own ? bk - mx0 : 0.0, pre);
+                         {true, r0, rr0}, pre);
     } else {
         // ||M - M32||_F <= 2^-24 ||M||_F (round to nearest, normal range) + N 2^-150 (subnormal range)
         dsq = bsum1(dsq, L);
@@ -163,15 +167,16 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
                 __syncthreads();
                 mx = mv_free_sym(n, pc, cl, L);   // every thread: it synchronises
             }
-            const double r = own ? bk - mx : 0.0;
-            const double rn = sqrt(bsum1(r * r, L));
+            const double r = sweeps > 0 ? (own ? bk - mx : 0.0) : r0;
+            const double rr = sweeps > 0 ? bsum1(r * r, L) : rr0;
+            const double rn = sqrt(rr);
             if (!(rn > tol_abs)) {
                 done = true;
                 break;
             }
             double dx = 0.0;
             iters += wg_gmres([&]() { return mv_pairs(Mt, n, cl, L); }, n, r, dx, true,
-                              fmax(1e-7 * rn, 0.25 * tol_abs), 1, L, nullptr, false, 0.0, pre);
+                              fmax(1e-7 * rn, 0.25 * tol_abs), 1, L, nullptr, {true, r, rr}, pre);
             x += dx;
             // the FP64 residual of the corrected x, bounded without forming it:
             //   |b - M x| <= |r - M32 dx| + |(M - M32) dx| <= (GMRES residual) + ||M - M32||_F |dx|

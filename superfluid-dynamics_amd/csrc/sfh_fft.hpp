@@ -41,14 +41,57 @@ __device__ inline int pass_group(int t, int lm, int R, int lh, int& pos) {
     return (q << lm) + (grp << (lh + R)) + pos;
 }
 
+// The work items of a pass over K fields: ng per field, in whole waves so that the fields' items run side by side
+// (a transform of 256 points has 32 groups of 8 per pass, one wave: five transforms one after the other cost 15
+// passes and barriers where two sets of them cost 6).  Derivatives of N = 1024 27 -> 18 us, N = 512 21 -> 14, N = 128
+// 15 -> 11.  The fields are a fixed distance apart: with a pointer chosen among several the compiler no longer knows
+// that it is LDS (flat loads, 15 us for the inverse transforms in place of 6).
+template <int K>
+struct FieldGroups {
+    int i, t, field;
+    const int ng, pad;
+    __device__ FieldGroups(int n) : i(threadIdx.x), ng(n), pad((n + 63) & ~63) { split(); }
+    __device__ void split() {
+        if constexpr (K == 1) {
+            t = i;
+            field = 0;
+        } else {
+            field = 0;   // by comparisons: a division would cost as much as the pass
+            t = i;
+#pragma unroll
+            for (int k = 1; k < K; ++k) {
+                if (i >= k * pad) {
+                    field = k;
+                    t = i - k * pad;
+                }
+            }
+        }
+    }
+    // skips the padding items, which only follow the groups of a field in its last wave
+    __device__ bool more() {
+        if constexpr (K > 1) {
+            while (i < K * pad && t >= ng) next();
+            return i < K * pad;
+        } else {
+            return t < ng;
+        }
+    }
+    __device__ void next() {
+        i += blockDim.x;
+        split();
+    }
+};
+
 // Decimation-in-time pass: radix-2 stages of half widths h, ..., 2^{R-1} h applied to each
 // group in registers (stage st pairs e and e + 2^st, twiddle W_n^{(pos + (e mod 2^st) h) n / 2^{lh+st+1}}).
-template <int R>
-__device__ inline void dit_pass(double2* s, int n, int lm, int sub, int lh, int sign,
+template <int R, int K>
+__device__ inline void dit_pass(double2* f, int fs, int n, int lm, int sub, int lh, int sign,
                                 const double2* __restrict__ tw) {
     constexpr int G = 1 << R;
     const int h = 1 << lh, ng = sub << (lm - R);
-    for (int t = threadIdx.x; t < ng; t += blockDim.x) {
+    for (FieldGroups<K> it(ng); it.more(); it.next()) {
+        const int t = it.t;
+        double2* const s = f + it.field * fs;
         int pos;
         const int i0 = pass_group(t, lm, R, lh, pos);
         double2 x[G];
@@ -76,12 +119,14 @@ __device__ inline void dit_pass(double2* s, int n, int lm, int sub, int lh, int 
 
 // Decimation-in-frequency pass: the mirror image, stages of half widths 2^{R-1} h, ..., h with
 // the twiddle applied to the difference.
-template <int R>
-__device__ inline void dif_pass(double2* s, int n, int lm, int sub, int lh, int sign,
+template <int R, int K>
+__device__ inline void dif_pass(double2* f, int fs, int n, int lm, int sub, int lh, int sign,
                                 const double2* __restrict__ tw) {
     constexpr int G = 1 << R;
     const int h = 1 << lh, ng = sub << (lm - R);
-    for (int t = threadIdx.x; t < ng; t += blockDim.x) {
+    for (FieldGroups<K> it(ng); it.more(); it.next()) {
+        const int t = it.t;
+        double2* const s = f + it.field * fs;
         int pos;
         const int i0 = pass_group(t, lm, R, lh, pos);
         double2 x[G];
@@ -107,25 +152,28 @@ __device__ inline void dif_pass(double2* s, int n, int lm, int sub, int lh, int 
     __syncthreads();
 }
 
-// Decimation in time: input in lds_index order, output in natural order.
+// Decimation in time, of K fields fs elements apart: input in lds_index order, output in natural order.
 // tw[t] = exp(-2 pi i t / n), t < n (LDS or global); sign -1 forward, +1 inverse (unnormalised).
 // The power-of-two sub-transforms run as radix-2^R passes from half width 1 upwards, then the
 // radix-3 combination when n = 3 * 2^m.
-__device__ inline void fft_dit(double2* s, const SurfDesc& d, int sign, const double2* __restrict__ tw) {
+template <int K>
+__device__ inline void fft_dit(double2* f, int fs, const SurfDesc& d, int sign, const double2* __restrict__ tw) {
     const int n = d.n, lm = d.log2m, m = 1 << lm, sub = d.r3 ? 3 : 1;
     for (int lh = 0; lh < lm;) {
         const int R = min(kFftMaxLogRadix, lm - lh);
         switch (R) {
-            case 4: dit_pass<4>(s, n, lm, sub, lh, sign, tw); break;
-            case 3: dit_pass<3>(s, n, lm, sub, lh, sign, tw); break;
-            case 2: dit_pass<2>(s, n, lm, sub, lh, sign, tw); break;
-            default: dit_pass<1>(s, n, lm, sub, lh, sign, tw); break;
+            case 4: dit_pass<4, K>(f, fs, n, lm, sub, lh, sign, tw); break;
+            case 3: dit_pass<3, K>(f, fs, n, lm, sub, lh, sign, tw); break;
+            case 2: dit_pass<2, K>(f, fs, n, lm, sub, lh, sign, tw); break;
+            default: dit_pass<1, K>(f, fs, n, lm, sub, lh, sign, tw); break;
         }
         lh += R;
     }
     if (d.r3) {   // X[k + q m] = sum_r W_n^{r k} W_3^{r q} F_r[k]
         const double c = -0.5, s3 = 0.86602540378443864676372317075293618 * sign;
-        for (int k = threadIdx.x; k < m; k += blockDim.x) {
+        for (FieldGroups<K> it(m); it.more(); it.next()) {
+            const int k = it.t;
+            double2* const s = f + it.field * fs;
             const double2 f0 = s[k];
             const double2 f1 = cmul(s[m + k], twid(tw, k, sign));
             const double2 f2 = cmul(s[2 * m + k], twid(tw, 2 * k, sign));
@@ -142,11 +190,14 @@ __device__ inline void fft_dit(double2* s, const SurfDesc& d, int sign, const do
 
 // Decimation in frequency: input in natural order, output in lds_index order.  Mirror image of
 // fft_dit: the radix-3 split first, then radix-2^R passes from the widest half width down to 1.
-__device__ inline void fft_dif(double2* s, const SurfDesc& d, int sign, const double2* __restrict__ tw) {
+template <int K>
+__device__ inline void fft_dif(double2* f, int fs, const SurfDesc& d, int sign, const double2* __restrict__ tw) {
     const int n = d.n, lm = d.log2m, m = 1 << lm, sub = d.r3 ? 3 : 1;
     if (d.r3) {   // y_q[j] = W_n^{j q} sum_r x[j + r m] W_3^{r q}
         const double c = -0.5, s3 = 0.86602540378443864676372317075293618 * sign;
-        for (int j = threadIdx.x; j < m; j += blockDim.x) {
+        for (FieldGroups<K> it(m); it.more(); it.next()) {
+            const int j = it.t;
+            double2* const s = f + it.field * fs;
             const double2 x0 = s[j], x1 = s[m + j], x2 = s[2 * m + j];
             const double2 t = cadd(x1, x2), dd = csub(x1, x2);
             const double2 base = make_double2(x0.x + c * t.x, x0.y + c * t.y);
@@ -160,13 +211,20 @@ __device__ inline void fft_dif(double2* s, const SurfDesc& d, int sign, const do
     for (int top = lm; top > 0;) {
         const int R = min(kFftMaxLogRadix, top), lh = top - R;
         switch (R) {
-            case 4: dif_pass<4>(s, n, lm, sub, lh, sign, tw); break;
-            case 3: dif_pass<3>(s, n, lm, sub, lh, sign, tw); break;
-            case 2: dif_pass<2>(s, n, lm, sub, lh, sign, tw); break;
-            default: dif_pass<1>(s, n, lm, sub, lh, sign, tw); break;
+            case 4: dif_pass<4, K>(f, fs, n, lm, sub, lh, sign, tw); break;
+            case 3: dif_pass<3, K>(f, fs, n, lm, sub, lh, sign, tw); break;
+            case 2: dif_pass<2, K>(f, fs, n, lm, sub, lh, sign, tw); break;
+            default: dif_pass<1, K>(f, fs, n, lm, sub, lh, sign, tw); break;
         }
         top = lh;
     }
+}
+
+__device__ inline void fft_dit(double2* s, const SurfDesc& d, int sign, const double2* __restrict__ tw) {
+    fft_dit<1>(s, 0, d, sign, tw);
+}
+__device__ inline void fft_dif(double2* s, const SurfDesc& d, int sign, const double2* __restrict__ tw) {
+    fft_dif<1>(s, 0, d, sign, tw);
 }
 
 // Twiddle source: the LDS copy (staged after the data, when it fits) or the global table.

@@ -7,6 +7,7 @@
 #include "sfh_kernels.hpp"
 #include "sfh_fft.hpp"
 #include "sfh_physics.hpp"
+#include "sfh_circ.hpp"
 
 namespace sfh {
 
@@ -16,11 +17,15 @@ constexpr int kBK = 8;                // Krylov vectors per GMRES cycle
 constexpr int kBR = kBK + 2;          // reduction slots: kBK + 1 dots and one norm
 
 struct BLds {
+    // three transform fields, one after the other
     double2 fa[kBatchMaxN];
     double2 fb[kBatchMaxN];
+    union {
+        double2 zp[kBatchMaxN];
+        double2 fc[kBatchMaxN];   // wg_derivatives' third field, before Z' is there
+    };
     double2 tw[kBatchMaxN];
     NodeTrig tr[kBatchMaxN];
-    double2 zp[kBatchMaxN];
     double diag[kBatchMaxN];
     double vs[kBatchMaxN];
     double part[kBT];
@@ -59,22 +64,26 @@ __device__ inline double bsum1(double v, BLds& L) {
     return L.sums[0];
 }
 
-// L.sums[i] = sum over the workgroup of V[i] * w for i <= j (0 above), L.sums[K] = |w|^2 when
-// with_norm.  The products are formed inside the reduction, no array of them is kept.
-template <int K>
-__device__ inline void bsum_dots(const double (&V)[K], double w, int j, bool with_norm, BLds& L) {
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+// L.sums[i] = sum over the workgroup of V[i] * w for i <= j < kBK, and L.sums[j + 1] = |w|^2 with_norm.  Four values
+// share a wave's lane swaps (reduce_lanes), and only the groups that hold something run: with the rotation by one
+// rsqrt and the first norms formed together, a solve of one step of N = 128 takes 17 us in place of 23.
+__device__ inline void bsum_dots(const double (&V)[kBK + 1], double w, int j, bool with_norm, BLds& L) {
+    static_assert(kBK == 8, "two groups of four, and the norm of the last step");
+    const int t = threadIdx.x, wv = t >> 6, last = j + (with_norm ? 1 : 0);
+    const auto value = [&](int i) { return i <= j ? V[i] * w : (i == last ? w * w : 0.0); };
 #pragma unroll
-    for (int i = 0; i < K; ++i) {
-        const double s = wave_sum((i <= j) ? V[i] * w : 0.0);
-        if (lane == 0) L.red[wv][i] = s;
+    for (int g = 0; g < 2; ++g) {
+        if (4 * g <= last) {
+            const double v[4] = {value(4 * g), value(4 * g + 1), value(4 * g + 2), value(4 * g + 3)};
+            reduce_lanes(v, &L.red[wv][4 * g]);
+        }
     }
-    if (with_norm) {
+    if (last == kBK) {
         const double s = wave_sum(w * w);
-        if (lane == 0) L.red[wv][K] = s;
+        if ((t & 63) == 0) L.red[wv][kBK] = s;
     }
     __syncthreads();
-    if (t <= K) {
+    if (t <= last) {
         double acc = 0.0;
 #pragma unroll
         for (int q = 0; q < kBW; ++q) acc += L.red[q][t];
@@ -224,29 +233,35 @@ __device__ inline double wg_precondition(double v, int n, const Precond& pre, BL
     return t < n ? z : 0.0;
 }
 
+// The first residual rhs - A x and its squared norm, when the caller has formed them.
+struct FirstResidual {
+    bool given;
+    double r, rr;
+};
+
 // Restarted GMRES on A x = rhs over the workgroup; x (thread t < n holds x_t) is updated in
 // place.  With a preconditioner the basis is that of A P^{-1} and x += P^{-1} V y, so residual and
-// tolerance are those of A x = rhs as without.  x_zero: x is known to be 0 (the first residual is rhs, no product needed); r_given:
-// the first residual rhs - A x is r_first (no product needed either).  Returns the number of
+// tolerance are those of A x = rhs as without.  x_zero: x is known to be 0 (the first residual is rhs, no product needed); with a
+// given first residual none is needed either.  Returns the number of
 // Arnoldi steps; *unconv is set when tol_abs was not reached.
 template <class MV>
 __device__ int wg_gmres(MV&& mv, int n, double rhs, double& x, bool x_zero, double tol_abs, int cycles,
-                        BLds& L, int* unconv, bool r_given = false, double r_first = 0.0,
-                        const Precond pre = {-1, 0.0}) {
+                        BLds& L, int* unconv, const FirstResidual first = {}, const Precond pre = {-1, 0.0}) {
     const int t = threadIdx.x;
     const bool own = t < n;
     int total = 0;
     for (int cyc = 0; cyc < cycles; ++cyc) {
-        double r = own ? rhs : 0.0;
-        if (cyc == 0 && r_given) {
-            r = own ? r_first : 0.0;   // the caller formed rhs - M x already
+        double r = own ? rhs : 0.0, rr = first.rr;
+        if (cyc == 0 && first.given) {
+            r = own ? first.r : 0.0;   // the caller formed rhs - M x already
         } else if (!(x_zero && cyc == 0)) {
             if (own) L.vs[t] = x;
             __syncthreads();
             const double w = mv();
             r = own ? rhs - w : 0.0;
         }
-        const double beta = sqrt(bsum1(r * r, L));
+        if (cyc > 0 || !first.given) rr = bsum1(r * r, L);
+        const double beta = sqrt(rr);
         if (!(beta > tol_abs)) return total;
         double V[kBK + 1];
 #pragma unroll
@@ -272,7 +287,7 @@ __device__ int wg_gmres(MV&& mv, int n, double rhs, double& x, bool x_zero, doub
             // coefficients are O(eps |w|), so the subtraction does not cancel)
             __syncthreads();
             bsum_dots(V, w, j, true, L);
-            double hh = L.sums[kBK + 1];
+            double hh = L.sums[j + 1];
 #pragma unroll
             for (int i = 0; i <= kBK; ++i) {
                 if (i <= j) {
@@ -293,12 +308,13 @@ __device__ int wg_gmres(MV&& mv, int n, double rhs, double& x, bool x_zero, doub
                     col[i] = a0;
                     col[i + 1] = a1;
                 }
-                const double den = hypot(col[j], col[j + 1]);
-                const double cj = den > 0.0 ? col[j] / den : 1.0;
-                const double sj = den > 0.0 ? col[j + 1] / den : 0.0;
+                // the entries are of the order of |M| or underflow together with the residual: no scaling
+                const double sq = col[j] * col[j] + col[j + 1] * col[j + 1], inv = sq > 0.0 ? rsqrt(sq) : 0.0;
+                const double cj = sq > 0.0 ? col[j] * inv : 1.0;
+                const double sj = col[j + 1] * inv;
                 L.cs[j] = cj;
                 L.sn[j] = sj;
-                col[j] = den;
+                col[j] = sq * inv;
                 for (int i = 0; i <= j; ++i) L.H[i][j] = col[i];
                 L.g[j + 1] = -sj * L.g[j];
                 L.g[j] = cj * L.g[j];
@@ -360,7 +376,7 @@ struct NodeVals {
 };
 
 // Spectral derivatives of one surface in LDS (Derivatives.cuh:310-384): Z' and Z'' from ONE
-// forward transform of Z - 2 pi j / N, Re Phi' from a second; also fills L.tw (twiddles),
+// forward transform of Z - 2 pi j / N, Re Phi' from a second, both at once, then the three inverse ones at once; also fills L.tw (twiddles),
 // L.tr (half-angle table) and L.zp.
 __device__ inline NodeVals wg_derivatives(const SurfDesc& d, const double2* __restrict__ tw_all,
                                           const double2* __restrict__ Zin, const double* __restrict__ Pin,
@@ -369,6 +385,8 @@ __device__ inline NodeVals wg_derivatives(const SurfDesc& d, const double2* __re
     const bool own = t < n;
     const double twopi_n = 2.0 * kPi / n;
     for (int i = t; i < n; i += kBT) L.tw[i] = tw_all[d.twoff + i];
+    const double plin = -(1 + ph.rho) * kPi * ph.U / n;   // Derivatives.cuh:286
+    double2* const fc = L.fc;   // Phi, then its derivative
     NodeVals v;
     v.z = make_double2(0.0, 0.0);
     v.phi = 0.0;
@@ -376,44 +394,36 @@ __device__ inline NodeVals wg_derivatives(const SurfDesc& d, const double2* __re
         v.z = Zin[off + t];
         v.phi = Pin[off + t];
         L.tr[t] = node_trig(v.z);
-        L.fa[lds_index(d, t)] = make_double2(v.z.x - twopi_n * (double)t, v.z.y);   // :285,317
+        const int i = lds_index(d, t);
+        L.fa[i] = make_double2(v.z.x - twopi_n * (double)t, v.z.y);   // :285,317
+        fc[i] = make_double2(v.phi - plin * (double)t, 0.0);
     }
     __syncthreads();
-    fft_dit(L.fa, d, -1, L.tw);
+    fft_dit<2>(L.fa, 2 * kBatchMaxN, d, -1, L.tw);   // fa and fc
     __syncthreads();
     for (int i = t; i < n; i += kBT) {
         const double2 c = L.fa[i];
         L.fb[i] = second_mult(c, i, n);
         L.fa[i] = first_mult(c, i, n);
+        fc[i] = first_mult(fc[i], i, n);
     }
     __syncthreads();
-    fft_dif(L.fa, d, +1, L.tw);
-    fft_dif(L.fb, d, +1, L.tw);
+    fft_dif<3>(L.fa, kBatchMaxN, d, +1, L.tw);   // fa, fb and fc
     __syncthreads();
     v.zp = make_double2(1.0, 0.0);
     v.zpp = make_double2(0.0, 0.0);
+    v.b = 0.0;
     if (own) {
-        const double2 a = L.fa[lds_index(d, t)], c = L.fb[lds_index(d, t)];
+        const int i = lds_index(d, t);
+        const double2 a = L.fa[i], c = L.fb[i];
         const double sc2 = 4.0 * kPi * kPi / ((double)n * n);
         v.zp = make_double2(a.x * twopi_n + twopi_n, a.y * twopi_n);   // :323, :374
         v.zpp = make_double2(c.x * sc2, c.y * sc2);                    // :321
-        L.zp[t] = v.zp;
-    }
-    __syncthreads();
-    const double plin = -(1 + ph.rho) * kPi * ph.U / n;   // Derivatives.cuh:286
-    if (own) L.fa[lds_index(d, t)] = make_double2(v.phi - plin * (double)t, 0.0);
-    __syncthreads();
-    fft_dit(L.fa, d, -1, L.tw);
-    __syncthreads();
-    for (int i = t; i < n; i += kBT) L.fa[i] = first_mult(L.fa[i], i, n);
-    __syncthreads();
-    fft_dif(L.fa, d, +1, L.tw);
-    __syncthreads();
-    v.b = 0.0;
-    if (own) {
-        v.b = L.fa[lds_index(d, t)].x * twopi_n;   // :324, BaseBoundaryIntegrator.cuh:299
+        v.b = fc[i].x * twopi_n;   // :324, BaseBoundaryIntegrator.cuh:299
         if (ph.U != 0) v.b += plin;                 // :380-383
     }
+    __syncthreads();
+    if (own) L.zp[t] = v.zp;
     __syncthreads();
     return v;
 }
