@@ -39,32 +39,14 @@
 //   gz += i (d/dy dPhi/dt) gp:  -g u^-4 (van der Waals) or the expansion's derivative; the
 //   surface-tension term kappa (x'y'' - y'x'')/|Z'|^3 adds its Z' and Z'' derivatives to gZ', gZ''.
 // The RK4 step adjoint around it (stage recomputation, cotangent combination) is host code.
-#include "sfh_wg.hpp"
+//
+// The pair sums visit every unordered pair once (sfh_sym.hpp): c_jk = -c_kj, so 1 + c^2 is the same for both orders, and
+// e_jk = -conj(e_kj).  The first sweep also stores M, with the two entries of a pair exchanged, so that the stored
+// product (mv_pairs) is M^T v.  24 surfaces of 64 to 256 nodes: 235 us per reverse stage with all ordered pairs and the
+// product evaluated anew in every Arnoldi step, 169 with this.
+#include "sfh_sym.hpp"
 
 namespace sfh {
-
-// (M^T v)_j = M_jj v_j - c Im(sum_{k != j} v_k Z'_k c_jk), v in L.vs.
-__device__ inline double mv_free_t(int n, int G, const PairConst& pc, BLds& L) {
-    const int t = threadIdx.x;
-    double val = 0.0;
-    if (t < G * n) {
-        const int j = t % n, g = t / n;
-        const NodeTrig tj = L.tr[j];
-        double uy = 0.0, ui = 0.0;   // Im sum v_k Z'_k c_jk, and the symmetric image part Im sum v_k e_jk
-        for (int k = g; k < n; k += G) {
-            if (k == j) continue;
-            const double vk = L.vs[k];
-            const double2 zk = L.zp[k];
-            const double2 ct = cot_pair(tj, L.tr[k]);
-            uy += vk * (zk.x * ct.y + zk.y * ct.x);
-            if (pc.image) ui += vk * cot_image(tj, L.tr[k], pc.eh, pc.ehi).y;
-        }
-        val = -pc.c * uy - pc.ci * ui;
-    }
-    double w = gsum(val, n, G, L);
-    if (t < n) w += L.diag[t] * L.vs[t];
-    return w;
-}
 
 __global__ __launch_bounds__(1024) void rhs_vjp_kernel(VjpArgs a, Phys ph) {
     __shared__ BLds L;
@@ -72,9 +54,9 @@ __global__ __launch_bounds__(1024) void rhs_vjp_kernel(VjpArgs a, Phys ph) {
     const SurfDesc d = a.sd[s];
     const int n = d.n, off = d.voff, t = threadIdx.x;
     const bool own = t < n;
-    const int G = kBT / n > 0 ? kBT / n : 1;
-    const int act = t < G * n;
-    const int kr = act ? t % n : 0, grp = act ? t / n : 0;
+    Cluster cl{1, 1, 0, 1, 0, false, nullptr, nullptr, nullptr};   // one workgroup
+    const SymGeo sg = sym_geo(n);
+    const int kr = sg.I * kTile + sg.l;   // this lane's row of the sweeps
     const double sc = 2.0 * kPi / n, sc2 = sc * sc;
     const double q4 = 0.25 / kPi;
     AdjNode* an = a.scratch + off;
@@ -82,14 +64,21 @@ __global__ __launch_bounds__(1024) void rhs_vjp_kernel(VjpArgs a, Phys ph) {
     // ------------------------------------------------ forward recomputation
     const NodeVals nv = wg_derivatives(d, a.tw_all, a.Zin, a.Pin, ph, L);
     const PairConst pc = wg_diagonal(ph, nv, n, L);
+    Precond pre = {-1, 0.0};   // film: of both solves (the image term's matrix is symmetric)
+    if (pc.image) {
+        pre.height = bsum1(own ? nv.z.y : 0.0, L) / n + ph.depth;
+        pre.modes = film_modes(n, pre.height);
+    }
     double mu = 0.0;
     int its = 0, unconv = 0;
     if (a.mu_in) {
         mu = own ? a.mu_in[off + t] : 0.0;
     } else {
         const double bn = sqrt(bsum1(own ? nv.b * nv.b : 0.0, L));
-        its += wg_gmres([&]() { return mv_free(n, G, pc, L); }, n, nv.b, mu, true, a.tol * bn, a.cycles, L,
-                        &unconv);
+        if (t < sg.nb * kTile) L.vs[t] = 0.0;   // the padding entries stay 0
+        __syncthreads();
+        its += wg_gmres([&]() { return mv_free_sym(n, pc, cl, L); }, n, nv.b, mu, true, a.tol * bn, a.cycles, L,
+                        &unconv, {}, pre);
     }
     if (own) L.fa[lds_index(d, t)] = make_double2(mu, 0.0);
     wg_first_derivative(d, L, false);
@@ -97,41 +86,78 @@ __global__ __launch_bounds__(1024) void rhs_vjp_kernel(VjpArgs a, Phys ph) {
     if (own) {
         const double2 v = L.fa[lds_index(d, t)];
         mup = make_double2(v.x * sc, v.y * sc);
-        L.vs[t] = mu;
     }
+    if (t < sg.nb * kTile) L.vs[t] = own ? mu : 0.0;
     __syncthreads();
     // pass A: S_k = sum mu_j c_kj,  P1_k = sum mu_j (1 + c_kj^2) (j != k); film: SI_k = sum mu_j e_kj,
     // PI1_k = sum mu_j (1 + e_kj^2) over all j
-    double sx = 0.0, sy = 0.0, p1x = 0.0, p1y = 0.0, six = 0.0, siy = 0.0, q1x = 0.0, q1y = 0.0;
-    if (act) {
-        const NodeTrig tk = L.tr[kr];
-        for (int j = grp; j < n; j += G) {
-            const double mj = L.vs[j];
-            if (pc.image) {
-                const double2 e = cot_image(tk, L.tr[j], pc.eh, pc.ehi);
-                six += mj * e.x;
-                siy += mj * e.y;
-                q1x += mj * (1.0 + e.x * e.x - e.y * e.y);
-                q1y += mj * (2.0 * e.x * e.y);
+    double* const Mt = a.M + d.moff;
+    const NodeTrig tk = L.tr[kr];
+    const double2 zq = L.zp[kr];
+    const double2 czk = make_double2(pc.c * zq.x, pc.c * zq.y);
+    const double mk = L.vs[kr];
+    double* const ax = reinterpret_cast<double*>(L.fa);   // 2 kBT doubles each
+    double* const bx = reinterpret_cast<double*>(L.fb);
+    double sp[4];
+    {
+        double* const Mi = Mt + (long long)(sg.I * sg.nb) * kTileElems;
+        const unsigned l = sg.l;
+        double* const acc[4] = {ax, ax + kBT, bx, bx + kBT};
+        sym_sums<4>(n, acc, [&](int k, int j, int q, auto mirror, auto full, double (&row)[4], double (&col)[4]) {
+            double e = 0.0, em = 0.0;
+            if (decltype(full)::value || (k < n && j < n)) {
+                const NodeTrig tj = L.tr[j];
+                const double mj = L.vs[j];
+                entry_pair(tk, tj, czk, L.zp[j], pc, e, em);
+                const CotParts cp = cot_parts(tk, tj);
+                const double cx = cp.p * cp.id, cy = -cp.q * cp.id;
+                const double fx = 1.0 + cx * cx - cy * cy, fy = 2.0 * cx * cy;   // 1 + c_kj^2
+                row[0] += mj * cx;
+                row[1] += mj * cy;
+                row[2] += mj * fx;
+                row[3] += mj * fy;
+                if constexpr (decltype(mirror)::value) {
+                    col[0] -= mk * cx;
+                    col[1] -= mk * cy;
+                    col[2] += mk * fx;
+                    col[3] += mk * fy;
+                }
             }
-            if (j == kr) continue;
-            const double2 c = cot_pair(tk, L.tr[j]);
-            sx += mj * c.x;
-            sy += mj * c.y;
-            p1x += mj * (1.0 + c.x * c.x - c.y * c.y);
-            p1y += mj * (2.0 * c.x * c.y);
+            Mi[(unsigned)(2 * q) * kTile + l] = em;
+            Mi[(unsigned)(2 * q + 1) * kTile + l] = decltype(mirror)::value ? e : 0.0;
+        }, cl, sp);
+    }
+    const double sx = sp[0], sy = sp[1], p1x = sp[2], p1y = sp[3];
+    double six = 0.0, siy = 0.0, q1x = 0.0, q1y = 0.0;
+    if (pc.image) {
+        __syncthreads();
+        double* const acc[4] = {ax, ax + kBT, bx, bx + kBT};
+        sym_sums<4>(n, acc, [&](int k, int j, int, auto mirror, auto full, double (&row)[4], double (&col)[4]) {
+            if (!decltype(full)::value && (k >= n || j >= n)) return;
+            const double mj = L.vs[j];
+            const double2 e = cot_image(tk, L.tr[j], pc.eh, pc.ehi);
+            const double fx = 1.0 + e.x * e.x - e.y * e.y, fy = 2.0 * e.x * e.y;
+            row[0] += mj * e.x;
+            row[1] += mj * e.y;
+            row[2] += mj * fx;
+            row[3] += mj * fy;
+            if constexpr (decltype(mirror)::value) {   // e_jk = -conj(e_kj)
+                col[0] -= mk * e.x;
+                col[1] += mk * e.y;
+                col[2] += mk * fx;
+                col[3] -= mk * fy;
+            }
+        }, cl, sp);
+        if (own) {   // j = k
+            const NodeTrig tt = L.tr[t];
+            const double2 e = cot_image(tt, tt, pc.eh, pc.ehi);
+            six = sp[0] + mu * e.x;
+            siy = sp[1] + mu * e.y;
+            q1x = sp[2] + mu * (1.0 + e.x * e.x - e.y * e.y);
+            q1y = sp[3] + mu * (2.0 * e.x * e.y);
         }
     }
-    sx = gsum(sx, n, G, L);
-    sy = gsum(sy, n, G, L);
-    p1x = gsum(p1x, n, G, L);
-    p1y = gsum(p1y, n, G, L);
-    if (pc.image) {
-        six = gsum(six, n, G, L);
-        siy = gsum(siy, n, G, L);
-        q1x = gsum(q1x, n, G, L);
-        q1y = gsum(q1y, n, G, L);
-    }
+    __syncthreads();
 
     // ------------------------------------------------ node-local adjoint of velocity + Bernoulli
     const bool quirk = ph.kind == 0 && ph.rho != 0.0 && ph.rho_quirk && n > 1;
@@ -191,32 +217,39 @@ __global__ __launch_bounds__(1024) void rhs_vjp_kernel(VjpArgs a, Phys ph) {
     if (own) gmu += sc * L.fa[lds_index(d, t)].x;
     // pass B: P3_j = sum_k conj(gw_k) c_jk ;  gmu_j += Re((i/4pi) P3_j); film: Q_j = sum_k gw_k e_jk
     // over all k, gmu_j += -Im(Q_j) / 4pi
-    double p3x = 0.0, p3y = 0.0, qy = 0.0;
-    if (act) {
-        const NodeTrig tj = L.tr[kr];
-        for (int k = grp; k < n; k += G) {
-            const double2 wk = L.fb[k];   // conj(gw_k)
+    {
+        const double2 wk = L.fb[kr];   // conj(gw) of this lane's row; node j's contribution to row k has conj(gw_j)
+        double* const acc[1] = {L.part};
+        double p3[1];
+        sym_sums<1>(n, acc, [&](int k, int j, int, auto mirror, auto full, double (&row)[1], double (&col)[1]) {
+            if (!decltype(full)::value && (k >= n || j >= n)) return;
+            const NodeTrig tj = L.tr[j];
+            const double2 wj = L.fb[j];
+            const double2 c = cot_pair(tk, tj);
+            row[0] += wj.x * c.y + wj.y * c.x;
+            if constexpr (decltype(mirror)::value) col[0] -= wk.x * c.y + wk.y * c.x;
             if (pc.image) {
-                const double2 e = cot_image(tj, L.tr[k], pc.eh, pc.ehi);
-                qy += wk.x * e.y - wk.y * e.x;   // Im(gw_k e_jk), gw_k = conj(wk)
+                const double2 e = cot_image(tk, tj, pc.eh, pc.ehi);
+                row[0] += wj.x * e.y - wj.y * e.x;   // Im(gw_j e_kj), gw_j = conj(wj)
+                if constexpr (decltype(mirror)::value) col[0] += wk.x * e.y + wk.y * e.x;
             }
-            if (k == kr) continue;
-            const double2 c = cot_pair(tj, L.tr[k]);
-            p3x += wk.x * c.x - wk.y * c.y;
-            p3y += wk.x * c.y + wk.y * c.x;
+        }, cl, p3);
+        if (own) {
+            if (pc.image) {   // k = j
+                const NodeTrig tt = L.tr[t];
+                const double2 e = cot_image(tt, tt, pc.eh, pc.ehi), w = L.fb[t];
+                p3[0] += w.x * e.y - w.y * e.x;
+            }
+            gmu -= q4 * p3[0];
         }
     }
-    p3x = gsum(p3x, n, G, L);
-    p3y = gsum(p3y, n, G, L);
-    if (pc.image) qy = gsum(qy, n, G, L);
-    if (own) gmu += -q4 * p3y - q4 * qy;
 
     // ------------------------------------------------ transpose solve M^T gb = gmu
     double gb = 0.0;
     {
         const double gn = sqrt(bsum1(own ? gmu * gmu : 0.0, L));
-        its += wg_gmres([&]() { return mv_free_t(n, G, pc, L); }, n, gmu, gb, true, a.tol * gn, a.cycles, L,
-                        &unconv);
+        its += wg_gmres([&]() { return mv_pairs(Mt, n, cl, L); }, n, gmu, gb, true, a.tol * gn, a.cycles, L, &unconv,
+                        {true, own ? gmu : 0.0, gn * gn}, pre);
     }
 
     // ------------------------------------------------ matrix terms and pair weights gamma
@@ -241,7 +274,6 @@ __global__ __launch_bounds__(1024) void rhs_vjp_kernel(VjpArgs a, Phys ph) {
         // gz_k += conj(gamma_k P1_k)
         gz = cadd(gz, cconj(cmul(gam, A.p1)));
         L.fb[t] = gam;
-        L.vs[t] = muk;
         if (pc.image) {   // gammaI_k = (i/8pi) gw_k - (i ci/2) gb_k;  gz_k += gammaI_k conj(PI1_k)
             const double2 gI = ctimes_i(csub(cscale(A.gw, 0.5 * q4), make_double2(0.5 * pc.ci * gb, 0.0)));
             gz = cadd(gz, cmul(gI, cconj(A.pi1)));
@@ -251,28 +283,43 @@ __global__ __launch_bounds__(1024) void rhs_vjp_kernel(VjpArgs a, Phys ph) {
     __syncthreads();
     // pass C: P2_j = sum_k gamma_k (1 + c_jk^2);  gz_j -= mu_j conj(P2_j); film: PI2_j = sum_k
     // gammaI_k (1 + e_jk^2) over all k, gz_j -= mu_j conj(PI2_j)
-    double p2x = 0.0, p2y = 0.0;
-    if (act) {
-        const NodeTrig tj = L.tr[kr];
-        for (int k = grp; k < n; k += G) {
-            if (pc.image) {
-                const double2 gk = L.fa[k];
-                const double2 e = cot_image(tj, L.tr[k], pc.eh, pc.ehi);
-                const double ex = 1.0 + e.x * e.x - e.y * e.y, ey = 2.0 * e.x * e.y;
-                p2x += gk.x * ex - gk.y * ey;
-                p2y += gk.x * ey + gk.y * ex;
+    double p2[2];
+    {
+        const double2 gk = L.fb[kr], ik = pc.image ? L.fa[kr] : make_double2(0.0, 0.0);
+        double* const acc[2] = {L.part, L.diag};   // the diagonal is not needed any more
+        sym_sums<2>(n, acc, [&](int k, int j, int, auto mirror, auto full, double (&row)[2], double (&col)[2]) {
+            if (!decltype(full)::value && (k >= n || j >= n)) return;
+            const NodeTrig tj = L.tr[j];
+            const double2 gj = L.fb[j];
+            const double2 c = cot_pair(tk, tj);
+            const double fx = 1.0 + c.x * c.x - c.y * c.y, fy = 2.0 * c.x * c.y;
+            row[0] += gj.x * fx - gj.y * fy;
+            row[1] += gj.x * fy + gj.y * fx;
+            if constexpr (decltype(mirror)::value) {
+                col[0] += gk.x * fx - gk.y * fy;
+                col[1] += gk.x * fy + gk.y * fx;
             }
-            if (k == kr) continue;
-            const double2 gk = L.fb[k];
-            const double2 c = cot_pair(tj, L.tr[k]);
-            const double ex = 1.0 + c.x * c.x - c.y * c.y, ey = 2.0 * c.x * c.y;
-            p2x += gk.x * ex - gk.y * ey;
-            p2y += gk.x * ey + gk.y * ex;
+            if (pc.image) {
+                const double2 ij = L.fa[j];
+                const double2 e = cot_image(tk, tj, pc.eh, pc.ehi);
+                const double ex = 1.0 + e.x * e.x - e.y * e.y, ey = 2.0 * e.x * e.y;
+                row[0] += ij.x * ex - ij.y * ey;
+                row[1] += ij.x * ey + ij.y * ex;
+                if constexpr (decltype(mirror)::value) {   // 1 + e_jk^2 = conj(1 + e_kj^2)
+                    col[0] += ik.x * ex + ik.y * ey;
+                    col[1] += ik.y * ex - ik.x * ey;
+                }
+            }
+        }, cl, p2);
+        if (pc.image && own) {   // k = j
+            const NodeTrig tt = L.tr[t];
+            const double2 e = cot_image(tt, tt, pc.eh, pc.ehi), g = L.fa[t];
+            const double ex = 1.0 + e.x * e.x - e.y * e.y, ey = 2.0 * e.x * e.y;
+            p2[0] += g.x * ex - g.y * ey;
+            p2[1] += g.x * ey + g.y * ex;
         }
     }
-    p2x = gsum(p2x, n, G, L);
-    p2y = gsum(p2y, n, G, L);
-    if (own) gz = csub(gz, cscale(make_double2(p2x, -p2y), muk));
+    if (own) gz = csub(gz, cscale(make_double2(p2[0], -p2[1]), muk));
 
     // ------------------------------------------------ through the derivative operators
     // gPhi = s Re(D1^H gb)
@@ -288,8 +335,7 @@ __global__ __launch_bounds__(1024) void rhs_vjp_kernel(VjpArgs a, Phys ph) {
         L.fb[lds_index(d, t)] = gzpp;
     }
     __syncthreads();
-    fft_dit(L.fa, d, -1, L.tw);
-    fft_dit(L.fb, d, -1, L.tw);
+    fft_dit<2>(L.fa, kBatchMaxN, d, -1, L.tw);   // fa and fb
     __syncthreads();
     for (int i = t; i < n; i += kBT) {
         const double2 c1 = first_mult(L.fa[i], i, n);

@@ -265,6 +265,7 @@ struct VjpArgs {
     double2* acc_Z;            // optional accumulator += out
     double* acc_P;
     AdjNode* scratch;
+    double* M;                 // per-surface matrices (tiled_matrix_elems each at SurfDesc::moff)
     int* stats;                // per surface: [iterations, unconverged, -, -]
     double tol;
     int cycles;

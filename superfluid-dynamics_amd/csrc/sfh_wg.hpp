@@ -1,8 +1,7 @@
 // sfh_wg.hpp -- building blocks of the per-surface workgroup kernels (the batched stage kernel
-// and the adjoint kernel): one workgroup of 1024 threads owns one surface of N <= 1024 nodes,
-// thread t owns node t, and pair loops split the columns over G = 1024 / N groups (thread t takes
-// row t % N and columns j = t / N (mod G)).  Everything a surface needs besides its matrix lives
-// in LDS (BLds); reductions are workgroup-local, so no workgroup ever waits for another.
+// and the adjoint kernel): workgroups of 1024 threads on one surface of N <= 1024 nodes, thread t owns
+// node t, the pair loops are those of sfh_sym.hpp.  Everything a surface needs besides its matrix lives
+// in LDS (BLds); reductions are workgroup-local.
 #pragma once
 #include "sfh_kernels.hpp"
 #include "sfh_fft.hpp"
@@ -106,79 +105,12 @@ __device__ inline void rset(double (&V)[K], int i, double x) {
     for (int u = 0; u < K; ++u) V[u] = (i == u) ? x : V[u];
 }
 
-// (M v)_k for the stored column-major matrix, v in L.vs (the caller has synchronised).  Returns
-// the value on threads t < n, 0 elsewhere.
-template <typename T>
-__device__ inline double mv_stored(const T* __restrict__ M, int n, int G, BLds& L) {
-    const int t = threadIdx.x;
-    double acc0 = 0.0, acc1 = 0.0;
-    if (t < G * n) {
-        const int k = t % n, g = t / n;
-        const T* col = M + k;
-        int j = g;
-        constexpr int U = sizeof(T) == 8 ? 8 : 16;   // loads in flight per thread
-        for (; j + (U - 1) * G < n; j += U * G) {
-            T m[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) m[u] = col[(size_t)(j + u * G) * n];
-#pragma unroll
-            for (int u = 0; u < U; u += 2) {
-                acc0 += (double)m[u] * L.vs[j + u * G];
-                acc1 += (double)m[u + 1] * L.vs[j + (u + 1) * G];
-            }
-        }
-        for (; j < n; j += G) acc0 += (double)col[(size_t)j * n] * L.vs[j];
-    }
-    L.part[t] = acc0 + acc1;
-    __syncthreads();
-    double w = 0.0;
-    if (t < n)
-        for (int q = 0; q < G; ++q) w += L.part[q * n + t];
-    __syncthreads();
-    return w;
-}
-
 struct PairConst {
     double c;     // coefficient of Im(Z'_k cot) (createM.cuh:52, :78)
     double ci;    // coefficient of the image term (:87-88)
     double eh, ehi;
     int image;
 };
-
-// (M v)_k evaluated matrix-free in FP64 with the same entry formula as the FP64 assembly.
-__device__ inline double mv_free(int n, int G, const PairConst& pc, BLds& L) {
-    const int t = threadIdx.x;
-    double val = 0.0;
-    if (t < G * n) {
-        const int k = t % n, g = t / n;
-        const NodeTrig tk = L.tr[k];
-        double sx = 0.0, sy = 0.0, si = 0.0;
-        for (int j = g; j < n; j += G) {
-            if (j == k) continue;
-            const NodeTrig tj = L.tr[j];
-            const double vj = L.vs[j];
-            const CotParts cp = cot_parts(tk, tj);
-            const double w = vj * cp.id;
-            sx += w * cp.p;
-            sy -= w * cp.q;
-            if (pc.image) {
-                const CotParts cq = cot_image_parts(tk, tj, pc.eh, pc.ehi);
-                si -= vj * (cq.q * cq.id);
-            }
-        }
-        const double2 zk = L.zp[k];
-        val = pc.c * (zk.x * sy + zk.y * sx) - pc.ci * si;
-    }
-    L.part[t] = val;
-    __syncthreads();
-    double w = 0.0;
-    if (t < n) {
-        for (int q = 0; q < G; ++q) w += L.part[q * n + t];
-        w += L.diag[t] * L.vs[t];
-    }
-    __syncthreads();
-    return w;
-}
 
 // The film's preconditioner of a surface: modes < 0 when none is used.
 struct Precond {
@@ -355,18 +287,6 @@ __device__ int wg_gmres(MV&& mv, int n, double rhs, double& x, bool x_zero, doub
     }
     if (unconv) *unconv = 1;
     return total;
-}
-
-// Sum of v over the G column groups of row t % n (inactive threads pass 0); valid on t < n.
-__device__ inline double gsum(double v, int n, int G, BLds& L) {
-    const int t = threadIdx.x;
-    L.part[t] = v;
-    __syncthreads();
-    double w = 0.0;
-    if (t < n)
-        for (int q = 0; q < G; ++q) w += L.part[q * n + t];
-    __syncthreads();
-    return w;
 }
 
 // Node values produced by the derivative phase (valid on threads t < n).

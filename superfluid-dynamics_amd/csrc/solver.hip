@@ -1500,6 +1500,7 @@ void Solver::enqueue_vjp(const double2* Z, const double* P, const double* mu, co
     a.acc_Z = accumulate ? gAcc_ : nullptr;
     a.acc_P = accumulate ? gAccP_ : nullptr;
     a.scratch = adj_;
+    a.M = M_;
     a.stats = vstats_;
     a.tol = std::min(opt_.tol, 1e-13);
     a.cycles = 6;
