@@ -248,7 +248,7 @@ __global__ __launch_bounds__(256) void adj_pass_b_kernel(AdjMArgs a, Phys ph) {
 // GMRES start for M^T gb = gmu from a zero guess: V[0] = r0 = gmu, x = 0, the control block re-armed.
 __global__ __launch_bounds__(256) void adj_gm_start_kernel(const SurfDesc* __restrict__ sd,
                                                            const double* __restrict__ b, double* __restrict__ V,
-                                                           double* __restrict__ x, int* __restrict__ ctl, int m) {
+                                                           double* __restrict__ x, int* __restrict__ ctl, int m, int reset) {
     const SurfDesc d = sd[blockIdx.y];
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i < d.n) {
@@ -260,6 +260,7 @@ __global__ __launch_bounds__(256) void adj_gm_start_kernel(const SurfDesc* __res
         c->done = 0;
         c->refine_iters = 0;
         c->iters = 0;
+        if (reset) c->most = 0;
     }
 }
 
@@ -286,7 +287,7 @@ __global__ __launch_bounds__(256) void adj_gm_start_warm_kernel(const SurfDesc* 
                                                                 const double* __restrict__ b,
                                                                 const double* __restrict__ x0,
                                                                 double* __restrict__ V, double* __restrict__ x,
-                                                                int* __restrict__ ctl, int m) {
+                                                                int* __restrict__ ctl, int m, int reset) {
     const SurfDesc d = sd[blockIdx.y];
     const int n = d.n, lane = threadIdx.x & 63;
     const int k = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -295,6 +296,7 @@ __global__ __launch_bounds__(256) void adj_gm_start_warm_kernel(const SurfDesc* 
         c->done = 0;
         c->refine_iters = 0;
         c->iters = 0;
+        if (reset) c->most = 0;
     }
     if (k >= n) return;   // the whole wave
     const double* row = Mt + d.moff + (long long)k * n;

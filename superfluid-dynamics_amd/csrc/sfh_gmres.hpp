@@ -22,7 +22,8 @@ struct GmCtl {
                        // than kHistDepth steps
     int pre_modes;     // film: Fourier modes of the preconditioner besides the mean, -1: not used
     double height;     // film: mean height of the surface above the substrate
-    int spare[16];
+    int most;          // most Arnoldi steps of a solve since an RK step (or a reverse step) began
+    int spare[15];
 };
 static_assert(sizeof(GmCtl) == kGmCtlInts * sizeof(int), "host reads control blocks with this stride");
 
@@ -80,6 +81,7 @@ __device__ inline GmView gm_view(const GmArgs& a, const SurfDesc* sd) { return g
 // Arnoldi steps of the solve, in the field of its kind (a refinement solve keeps the first solve's)
 __device__ inline void set_iters(GmCtl* ctl, const GmArgs& a, int k) {
     ctl->fill_iters = max(ctl->fill_iters, k);
+    ctl->most = max(ctl->most, k);
     if (a.check_first)
         ctl->refine_iters = k;
     else

@@ -234,7 +234,7 @@ Solver::Solver(const Phys& ph, const std::vector<int>& n, const Options& opt) : 
     status_ = dalloc<int>(2 * S_);
     piv_ = dalloc<int>(T_);
     counters_ = dalloc<int>(4);
-    const size_t words = 2 * (size_t)S_ + 4 + (opt_.solver == kSolveGMRES ? (size_t)kGmCtlInts * S_ : 4 * (size_t)S_);
+    const size_t words = 2 * (size_t)S_ + 4 + (opt_.solver == kSolveBatched ? 4 * (size_t)S_ : (size_t)kGmCtlInts * S_);
     SFH_HIP(hipHostMalloc((void**)&host_, 3 * (size_t)T_ * sizeof(double) + words * sizeof(int), hipHostMallocDefault));
     SFH_HIP(hipMemset(status_, 0, 2 * S_ * sizeof(int)));
     SFH_HIP(hipMemset(counters_, 0, 4 * sizeof(int)));
@@ -813,7 +813,6 @@ void Solver::calibrate() {
     // truncation error is smaller), and get no spare launch; slower ones, whose step count varies
     // more from solve to solve, get one spare step.  A chunk in which a solve still runs out of
     // launches is run again with the length doubled.
-    sync();
     const int need = fill_iters_ + 1;
     trim_ = std::max(2, std::min(gm_m_, fill_iters_ >= 3 ? need + 1 : need));
     if (opt_.force_trim > 0) trim_ = std::max(2, std::min(gm_m_, opt_.force_trim));
@@ -857,6 +856,32 @@ void Solver::run_steps(double dt, int len, int count) {
     }
 }
 
+// One step while the warm-start history fills.  The first one runs the full launch sequence; the next ones need no
+// more Arnoldi steps than the one before, as their guesses get better, and get that many launches and two spare
+// ones (a launch after the end of a solve costs 2.5 us: N = 2048 2.1 ms for the six steps' 792 launches).  A step in
+// which a solve ran out of them all the same is run again with the full sequence.  Launched directly: each length
+// would need a graph of its own for one use.
+void Solver::fill_step(double dt) {
+    if (hist_steps_ == 0 || fill_len_.empty()) fill_len_.assign(kCalibSteps, gm_m_);
+    const int len = hist_steps_ == 0 ? gm_m_ : std::min(gm_m_, std::max(4, most_ + 3));
+    const int raw0 = unc_raw_;
+    if (len < gm_m_) save_checkpoint();
+    seq_len_ = len;
+    enqueue_step(dt);
+    sync();
+    fill_len_[hist_steps_] = len;
+    if (len < gm_m_ && unc_raw_ > raw0) {
+        restore_checkpoint();
+        unc_discard_ += unc_raw_ - raw0;
+        stats_.unconverged = unc_raw_ - unc_discard_;
+        stats_.redone_steps += 1;
+        fill_len_[hist_steps_] = gm_m_;
+        seq_len_ = gm_m_;
+        enqueue_step(dt);
+        sync();
+    }
+}
+
 void Solver::step(double dt, int nsteps) {
     if (nsteps < 0) throw ArgError("negative step count");
     int i = 0;
@@ -866,8 +891,7 @@ void Solver::step(double dt, int nsteps) {
             run_steps(dt, gm_m_, nsteps - i);
             i = nsteps;
         } else if (hist_steps_ < kCalibSteps) {
-            // the warm-start history fills: full-length sequences, one step at a time
-            run_steps(dt, gm_m_, 1);
+            fill_step(dt);
             ++i;
             calibrate();
         } else {
@@ -1104,8 +1128,8 @@ __global__ __launch_bounds__(256) void state_load_kernel(const double* __restric
 }
 
 struct StatusWords {
-    const int* src[4];
-    int count[4];
+    const int* src[3];
+    int count[3];
 };
 
 __global__ __launch_bounds__(256) void state_store_kernel(const double2* __restrict__ Z, const double* __restrict__ P,
@@ -1120,7 +1144,7 @@ __global__ __launch_bounds__(256) void state_store_kernel(const double2* __restr
     }
     int o = 0;
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
+    for (int a = 0; a < 3; ++a) {
         if (i < s.count[a]) words[o + i] = s.src[a][i];
         o += s.count[a];
     }
@@ -1128,9 +1152,10 @@ __global__ __launch_bounds__(256) void state_store_kernel(const double2* __restr
 
 // Z and P (when given) and the status words into the pinned buffer; waits for the stream.
 void Solver::store_host(const double2* Z, const double* P) {
-    StatusWords s{{status_, counters_, opt_.solver == kSolveGMRES ? gmctl_ : nullptr,
-                   opt_.solver == kSolveBatched ? bstats_ : nullptr},
-                  {2 * S_, 4, opt_.solver == kSolveGMRES ? kGmCtlInts * S_ : 0, opt_.solver == kSolveBatched ? 4 * S_ : 0}};
+    // the GMRES control blocks also of an LU handle that has run transposed solves
+    const bool batched = opt_.solver == kSolveBatched;
+    StatusWords s{{status_, counters_, batched ? bstats_ : gmctl_},
+                  {2 * S_, 4, batched ? 4 * S_ : gmctl_ ? kGmCtlInts * S_ : 0}};
     int most = Z ? T_ : 0;
     for (int c : s.count) most = std::max(most, c);
     hipLaunchKernelGGL(state_store_kernel, dim3((most + 255) / 256), dim3(256), 0, stream_, Z, P, host_, T_, s,
@@ -1298,23 +1323,27 @@ void Solver::parse_status() {
     int timeouts = 0;
     for (int s = 0; s < S_; ++s) timeouts += st[2 * s + 1] != 0;
     stats_.spin_timeouts = timeouts;
-    if (opt_.solver == kSolveGMRES) {
-        int mx = 0, unc = 0, fill = 0;
+    if (opt_.solver != kSolveBatched && gmctl_) {
+        int mx = 0, unc = 0, fill = 0, most = 0;
         for (int s = 0; s < S_; ++s) {
             GmCtl c;
             std::memcpy(&c, ctl + (size_t)kGmCtlInts * s, sizeof(GmCtl));
             mx = std::max(mx, c.iters);
             unc += c.unconverged;
             fill = std::max(fill, c.fill_iters);
+            most = std::max(most, c.most);
         }
         fill_iters_ = fill;
+        most_ = most;
         unc_raw_ = unc;
         unc -= unc_discard_;
-        stats_.last_iterations = ctl[2];
-        // mixed precision: 1 when surface 0's last refinement solve ran Arnoldi steps
-        if (opt_.precision == kMixed) stats_.refinements = ctl[1] > 0 ? 1 : 0;
-        stats_.max_iterations = mx;
-        stats_.unconverged = unc;
+        if (opt_.solver == kSolveGMRES) {
+            stats_.last_iterations = ctl[2];
+            // mixed precision: 1 when surface 0's last refinement solve ran Arnoldi steps
+            if (opt_.precision == kMixed) stats_.refinements = ctl[1] > 0 ? 1 : 0;
+            stats_.max_iterations = mx;
+            stats_.unconverged = unc;
+        }
     }
     if (opt_.solver == kSolveBatched) {
         const int* bs = ctl;
@@ -1578,17 +1607,19 @@ void Solver::enqueue_vjp_mwg(const double2* Z, const double* P, const double* mu
         go(transpose_kernel, dim3((maxN_ + 31) / 32, (maxN_ + 31) / 32, S_), dim3(256), 0, d_desc_, (const double*)M_,
            Mt_);
         // inside a trajectory sweep: the guess extrapolated from this stage's solutions of the previous
-        // reverse steps, and once calibrated a trimmed sequence; else a zero guess, the full sequence
+        // reverse steps, and the sweep's sequence length; else a zero guess, the full sequence
         const bool warm = adj_warm_ && stage >= 0 && adj_hv_[stage] > 0;
-        const int m = (warm && adj_len_ > 0 && adj_hv_[stage] >= kHistDepth) ? adj_len_ : gm_m_;
+        const int m = adj_warm_ && adj_len_ > 0 ? adj_len_ : gm_m_;
+        const int reset = adj_first_ ? 1 : 0;
+        adj_first_ = false;
         if (warm) {
             go(adj_extrapolate_kernel, dim3((T_ + 255) / 256), dim3(256), 0,
                (const double*)(adjRing_ + (size_t)stage * kHistDepth * T_), adj_head_[stage], adj_hv_[stage], adjX_,
                T_);
             go(adj_gm_start_warm_kernel, dim3((maxN_ + 3) / 4, S_), dim3(256), 0, d_desc_, (const double*)Mt_,
-               (const double*)agmu_, (const double*)adjX_, gmV_, gmx0_, gmctl_, m);
+               (const double*)agmu_, (const double*)adjX_, gmV_, gmx0_, gmctl_, m, reset);
         } else {
-            go(adj_gm_start_kernel, ngrid, dim3(256), 0, d_desc_, (const double*)agmu_, gmV_, gmx0_, gmctl_, m);
+            go(adj_gm_start_kernel, ngrid, dim3(256), 0, d_desc_, (const double*)agmu_, gmV_, gmx0_, gmctl_, m, reset);
         }
         GmArgs g = gm_args(0);
         g.M = Mt_;
@@ -1612,12 +1643,6 @@ void Solver::enqueue_vjp_mwg(const double2* Z, const double* P, const double* mu
                                hipMemcpyDeviceToDevice, stream_));
         adj_head_[stage] = slot;
         adj_hv_[stage] = std::min(adj_hv_[stage] + 1, kHistDepth);
-    }
-    if (adj_calib_) {   // the Arnoldi steps this solve took
-        std::vector<int> ctl((size_t)kGmCtlInts * S_);
-        SFH_HIP(hipStreamSynchronize(stream_));
-        SFH_HIP(hipMemcpy(ctl.data(), gmctl_, ctl.size() * sizeof(int), hipMemcpyDeviceToHost));
-        for (int s = 0; s < S_; ++s) adj_calib_max_ = std::max(adj_calib_max_, ctl[(size_t)kGmCtlInts * s + 2]);
     }
     launch("vjp_pairs", img * nsq, 0.0, [&] {
         go(adj_gamma_kernel, ngrid, dim3(256), 0, a, ph_);
@@ -1816,6 +1841,7 @@ int Solver::traj_forward(double dt, int steps, int every) {
             rr.hist_steps[c] = hist_steps_;
             step(dt, std::min(every, steps - c * every));
         }
+        rr.fill_len = fill_len_;
         check_status();
     } catch (...) {
         traj_release(id);
@@ -1853,36 +1879,40 @@ void Solver::traj_backward(int record, const double* gx_in, const double* gy_in,
     const int nck = (r.steps + r.every - 1) / r.every;
     const size_t zb = T_ * sizeof(double2), pb = T_ * sizeof(double);
     // transposed solves (LU and GMRES handles): warm-started from each stage's solutions of the
-    // previous reverse steps; the first reverse step with five of them for every stage measures the
-    // Arnoldi steps its solves take, and from the next segment on the solves get that many launches
-    // plus a spare.  A segment in which one ran out is swept again with full sequences from its saved
-    // start, and the length doubles.
+    // previous reverse steps.  The first reverse step runs full launch sequences; while the stages' rings
+    // fill, each step's solves get the launches that the step before needed and two spare ones, and the
+    // first step with full rings sets the length of all later ones (its need and a spare).  A segment in
+    // which a solve ran out is swept again with full sequences from its saved start, and the length doubles.
     const bool mwg = opt_.solver != kSolveBatched;
     struct SweepState {   // the warm-start state lives only inside this sweep, whatever ends it
         Solver* s;
         ~SweepState() {
             s->adj_warm_ = false;
-            s->adj_calib_ = false;
+            s->adj_first_ = false;
             s->adj_len_ = 0;
         }
     } sweep_state{this};
     adj_warm_ = mwg;
     adj_len_ = 0;
     for (int st = 0; st < 4; ++st) adj_head_[st] = adj_hv_[st] = 0;
-    bool calibrated = false;
-    int pending_len = 0;
+    int sweep_len = 0;        // launches per solve once the rings are full (0: not known yet)
+    int fill = 0;             // and of the next step while they fill (0: the full sequence)
+    bool adapt = mwg;         // shorter sequences while they fill
     for (int seg = nck - 1; seg >= 0; --seg) {
         const int n = std::min(r.every, r.steps - seg * r.every);
         // y_s, ..., y_{s+n-1}: the checkpoint, then n - 1 steps from it, each step keeping its stage
         // states and stage mu (the last step runs only for them).  The solves are warm-started from
-        // the stage histories as in the forward pass; GMRES solves get the full launch sequence while
-        // the histories fill and the forward pass's trimmed length after that, and a segment in which
-        // a trimmed solve ran out of launches is run again with full sequences.
+        // the stage histories as in the forward pass; GMRES solves get the forward pass's launch
+        // sequences, while the histories fill and after that, and a segment in which
+        // one ran out of launches is run again with full sequences.
         const double2* ckZ = r.Z + (size_t)seg * T_;
         const double* ckP = r.P + (size_t)seg * T_;
-        // the steps from the checkpoint before the stage histories hold kHistDepth solutions get the full
-        // sequence (only in a trajectory's first segment: later checkpoints keep full histories)
-        const int cold = std::max(0, kCalibSteps - r.hist_steps[seg]);
+        const bool gmres = opt_.solver == kSolveGMRES;
+        const auto length = [&](int k) {   // of step k of the segment
+            const int h = r.hist_steps[seg] + k;
+            if (h < kCalibSteps) return h < (int)r.fill_len.size() ? r.fill_len[h] : gm_m_;
+            return trim_ >= 2 ? trim_ : gm_m_;
+        };
         auto rerun = [&](bool trimmed) {
             SFH_HIP(hipMemcpyAsync(segZ_, ckZ, zb, hipMemcpyDeviceToDevice, stream_));
             SFH_HIP(hipMemcpyAsync(segP_, ckP, pb, hipMemcpyDeviceToDevice, stream_));
@@ -1899,7 +1929,7 @@ void Solver::traj_backward(int record, const double* gx_in, const double* gy_in,
             }
             hist_steps_ = r.hist_steps[seg];
             for (int k = 0; k < n; ++k) {
-                seq_len_ = (trimmed && k >= cold) ? trim_ : gm_m_;
+                seq_len_ = gmres && trimmed ? length(k) : gm_m_;
                 const StageCapture cap = seg_capture(k);
                 enqueue_step(r.dt, &cap);
                 if (k + 1 < n) {
@@ -1908,7 +1938,8 @@ void Solver::traj_backward(int record, const double* gx_in, const double* gy_in,
                 }
             }
         };
-        const bool trim = opt_.solver == kSolveGMRES && trim_ >= 2 && trim_ < gm_m_ && n > cold;   // calibrated
+        bool trim = false;
+        for (int k = 0; k < n; ++k) trim = trim || (gmres && length(k) < gm_m_);
         if (trim) {
             sync();
             const int unc0 = unc_raw_;
@@ -1923,28 +1954,31 @@ void Solver::traj_backward(int record, const double* gx_in, const double* gy_in,
         } else {
             rerun(false);
         }
-        auto sweep = [&]() {
+        bool shortened = false;
+        auto sweep = [&](bool full) {
             for (int i = n - 1; i >= 0; --i) {
-                bool calib = mwg && !calibrated;
-                for (int st = 0; st < 4; ++st) calib = calib && adj_hv_[st] >= kHistDepth;
-                if (calib) {
-                    adj_calib_ = true;
-                    adj_calib_max_ = 0;
-                }
+                bool rings = mwg;
+                for (int st = 0; st < 4; ++st) rings = rings && adj_hv_[st] >= kHistDepth;
+                adj_len_ = full ? 0 : rings && sweep_len > 0 ? sweep_len : fill;
+                shortened = shortened || adj_len_ > 0;
+                adj_first_ = mwg;
                 const StageCapture cap = seg_capture(i);
                 enqueue_step_vjp(r.dt, segZ_ + (size_t)i * T_, segP_ + (size_t)i * T_, &cap);
-                if (calib) {
-                    adj_calib_ = false;
-                    calibrated = true;
-                    pending_len = std::min(gm_m_, adj_calib_max_ + 2);
-                    if (opt_.force_trim > 0) pending_len = std::max(2, std::min(gm_m_, opt_.force_trim));
+                if (mwg && sweep_len == 0 && (rings || adapt)) {
+                    sync();   // most_: the Arnoldi steps this step's solves took
+                    if (rings) {
+                        sweep_len = std::min(gm_m_, most_ + 2);
+                        if (opt_.force_trim > 0) sweep_len = std::max(2, std::min(gm_m_, opt_.force_trim));
+                    } else {
+                        fill = std::min(gm_m_, std::max(4, most_ + 3));
+                    }
                 }
                 SFH_HIP(hipMemcpyAsync(gA_, gAcc_, zb, hipMemcpyDeviceToDevice, stream_));
                 SFH_HIP(hipMemcpyAsync(gAP_, gAccP_, pb, hipMemcpyDeviceToDevice, stream_));
             }
+            adj_len_ = 0;
         };
-        const bool trimmed = mwg && adj_len_ > 0;
-        if (trimmed) {
+        if (mwg) {
             const size_t ring = (size_t)4 * kHistDepth * T_ * sizeof(double);
             SFH_HIP(hipMemcpyAsync(adjSaveZ_, gA_, zb, hipMemcpyDeviceToDevice, stream_));
             SFH_HIP(hipMemcpyAsync(adjSaveP_, gAP_, pb, hipMemcpyDeviceToDevice, stream_));
@@ -1954,9 +1988,9 @@ void Solver::traj_backward(int record, const double* gx_in, const double* gy_in,
             std::copy(adj_hv_, adj_hv_ + 4, hv);
             sync();
             const int unc0 = unc_raw_;
-            sweep();
-            sync();
-            if (unc_raw_ > unc0) {
+            sweep(false);
+            if (shortened) sync();
+            if (shortened && unc_raw_ > unc0) {
                 unc_discard_ += unc_raw_ - unc0;
                 stats_.unconverged = unc_raw_ - unc_discard_;
                 stats_.redone_steps += n;
@@ -1965,14 +1999,13 @@ void Solver::traj_backward(int record, const double* gx_in, const double* gy_in,
                 SFH_HIP(hipMemcpyAsync(adjRing_, adjSave_, ring, hipMemcpyDeviceToDevice, stream_));
                 std::copy(head, head + 4, adj_head_);
                 std::copy(hv, hv + 4, adj_hv_);
-                const int len = adj_len_;
-                adj_len_ = 0;
-                sweep();
-                adj_len_ = std::min(gm_m_, 2 * len);
+                const int len = sweep_len;
+                adapt = false;
+                sweep(true);
+                if (len > 0) sweep_len = std::min(gm_m_, 2 * len);
             }
         } else {
-            sweep();
-            if (calibrated && pending_len > 0) adj_len_ = pending_len;   // trimmed from the next segment on
+            sweep(true);
         }
     }
     load_state(r.Z, r.P);   // the record's initial state

@@ -217,6 +217,7 @@ class Solver {
     void capture(double dt, int len);
     void run_steps(double dt, int len, int count);   // count steps with GMRES sequences of len launches
     void calibrate();               // bookkeeping after a full-length step while the history fills
+    void fill_step(double dt);
     void save_checkpoint();         // state, last solution and warm-start history, device to device
     void restore_checkpoint();
     void check_status();           // waits for the stream
@@ -340,9 +341,8 @@ class Solver {
     double* adjSaveP_ = nullptr;
     int adj_head_[4] = {0, 0, 0, 0}, adj_hv_[4] = {0, 0, 0, 0};
     bool adj_warm_ = false;          // inside a trajectory sweep
-    int adj_len_ = 0;                // launches per warm transposed solve (0: the full sequence)
-    bool adj_calib_ = false;         // this reverse step measures the Arnoldi steps of its solves
-    int adj_calib_max_ = 0;
+    int adj_len_ = 0;                // launches per transposed solve of a sweep (0: the full sequence)
+    bool adj_first_ = false;         // the next transposed solve is the first of a reverse step
     // one RK4 step back from the state (Z, P): cotangent gA_/gAP_ of the state after it -> gAcc_/gAccP_.
     // The stage states and mu come from `stored` when given, else they are recomputed (solves from
     // zero guesses with the full launch sequence).
@@ -360,6 +360,7 @@ class Solver {
         double* H = nullptr;    // c * hist_len
         int* HV = nullptr;      // c * hv_len
         size_t hist_len = 0, hv_len = 0;
+        std::vector<int> fill_len;   // of the forward pass
         std::vector<int> hist_steps;   // hist_steps_ at each checkpoint
     };
     void free_record(TrajRecord& r);
@@ -394,6 +395,8 @@ class Solver {
     int chunk_ = 2;         // steps of the next trimmed chunk (doubles up to kCheckSteps)
     int unc_raw_ = 0;       // unconverged count of the control blocks (discarded chunks included)
     int unc_discard_ = 0;   // ... of solves in chunks that were run again
+    int most_ = 0;          // most Arnoldi steps of a solve of the last RK (or reverse) step, any surface
+    std::vector<int> fill_len_;   // launches per solve of each step while the warm-start history filled
     int fill_iters_ = 0;    // most Arnoldi steps of a solve with the full history, any surface
     double2* ckZ_ = nullptr;
     double *ckP_ = nullptr, *ckMu_ = nullptr, *ckHist_ = nullptr;

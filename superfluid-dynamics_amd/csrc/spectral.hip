@@ -54,6 +54,7 @@ __global__ __launch_bounds__(TC * TR) void zphi_circ_kernel(const SurfDesc* __re
             c->iters = 0;
             c->refine_iters = 0;
             if (gm.stage > 0 && gm.hvalid[gm.stage - 1] < kHistDepth) c->fill_iters = 0;
+            if (gm.stage == 1) c->most = 0;
         }
     }
     const double* c1r = circ + d.coff;
