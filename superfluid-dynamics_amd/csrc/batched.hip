@@ -11,12 +11,13 @@
 //      Phi' from a second (Derivatives.cuh:310-384), plus the per-node half-angle table;
 //   B  the dipole matrix M = I/2 + K (createM.cuh:43-92) into HBM, in the order in which the sweeps visit it
 //      (sfh_sym.hpp), FP64 or FP32 (FP64 entries rounded), and in the same pair loop M x for the warm start x (the first residual);
-//   C  the solve M mu = b, warm-started from the surface's previous mu:
-//        FP64  : GMRES on the stored FP64 matrix (classical Gram-Schmidt with one
+//   C  the solve M mu = b, warm-started from the surface's previous mu (STORED says where the matrix is stored
+//      and where its products are evaluated anew in FP64):
+//        FP64  : GMRES on the FP64 matrix (classical Gram-Schmidt with one
 //                re-orthogonalisation, restarted cycles of kBK vectors);
 //        mixed : FP64 iterative refinement  r = b - M mu  with the residual evaluated
 //                matrix-free in FP64 (same pair formula as the assembly), correction solves by
-//                GMRES on the stored FP32 matrix; a correction whose GMRES residual plus
+//                GMRES on the FP32 matrix (or on M itself); a correction whose GMRES residual plus
 //                ||M - M32||_F |d| (bounded by 2^-24 ||M||_F) is within the tolerance ends the
 //                refinement without another FP64 residual pass;
 //   D  mu' (one more transform pair);
@@ -29,9 +30,9 @@
 // and every load of the stored product is one contiguous 512-byte (FP64) or 256-byte (FP32) row
 // per wave, and node data is read from LDS without bank conflicts.
 //
-// Bounds: N = 1024 mixed water, one workgroup, one Arnoldi step 577 us: derivatives 25, assembly sweep 205, product 155
-// (128 such surfaces read their matrices at 3.6 TB/s), the rest of the solve 39, mu' 7, velocity sweep 140; the sweeps
-// issue FP64 instructions back to back.
+// Bounds: N = 1024 mixed water among 512 surfaces, one Arnoldi step 450 us (540 with the stored matrix): derivatives
+// 16, assembly sweep 149, product 135, the rest of the solve 16, mu' 7, velocity sweep 125; the three sweeps issue FP64
+// instructions back to back (148 cycles for 64 pairs).
 #include <type_traits>
 
 #include "sfh_sym.hpp"
@@ -40,6 +41,12 @@ namespace sfh {
 
 template <bool MIXED, bool FILM, bool SHARED>
 __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys ph, StageCtl ctl) {
+    // The solve's products come from the matrix that the assembly stores, or are evaluated anew in FP64.  A pair of a
+    // water surface takes the SIMDs 1.24e-4 us per squared node count, and its entries 6e-5 (FP32) or 1.25e-4 (FP64) to
+    // load on an idle GPU, but 1.5e-4 or more once every CU loads its own surface's (N = 1024, 512 surfaces: product
+    // 155 us stored in FP32, 135 evaluated; and the assembly 181 with the stores, 149 without).  A film's pair has two
+    // cotangents, and its matrix is always stored.
+    constexpr bool STORED = FILM || (MIXED && SHARED);
     __shared__ BLds L;
     const int s = a.order[blockIdx.x];
     const SurfDesc d = a.sd[s];
@@ -123,14 +130,16 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
             if (decltype(full)::value || (k < n && j < n)) {
                 entry_pair(tk, L.tr[j], czk, L.zp[j], pc, e, em);
                 row[0] += e * L.vs[j];
-                if constexpr (MIXED) dsq += e * e;
+                if constexpr (MIXED && STORED) dsq += e * e;
                 if constexpr (decltype(mirror)::value) {
                     col[0] += em * vk;
-                    if constexpr (MIXED) dsq += em * em;
+                    if constexpr (MIXED && STORED) dsq += em * em;
                 }
             }
-            Mi[(unsigned)(2 * q) * kTile + l] = (MT)e;
-            Mi[(unsigned)(2 * q + 1) * kTile + l] = decltype(mirror)::value ? (MT)em : (MT)0;
+            if constexpr (STORED) {
+                Mi[(unsigned)(2 * q) * kTile + l] = (MT)e;
+                Mi[(unsigned)(2 * q + 1) * kTile + l] = decltype(mirror)::value ? (MT)em : (MT)0;
+            }
         }, cl, mx);
         mx0 = own ? mx[0] + L.diag[t] * L.vs[t] : 0.0;
     }
@@ -150,15 +159,24 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
         pre.modes = film_modes(n, pre.height);
     }
     __syncthreads();   // the sums are read before they are formed again
+    const auto product = [&]() {
+        if constexpr (STORED)
+            return mv_pairs(Mt, n, cl, L);
+        else
+            return mv_free_sym(n, pc, cl, L);
+    };
     int unconv = 0, iters = 0, sweeps = 0;
     if constexpr (!MIXED) {
-        iters = wg_gmres([&]() { return mv_pairs(Mt, n, cl, L); }, n, bk, x, false, tol_abs, a.cycles, L, &unconv,
+        iters = wg_gmres(product, n, bk, x, false, tol_abs, a.cycles, L, &unconv,
                          {true, r0, rr0}, pre);
     } else {
         // ||M - M32||_F <= 2^-24 ||M||_F (round to nearest, normal range) + N 2^-150 (subnormal range)
-        dsq = bsum1(dsq, L);
-        if (cl.parts > 1) dsq = cl.sum_members(n, dsq);
-        const double dM = 0x1p-24 * sqrt(dsq) + n * 0x1p-150;
+        double dM = 0.0;   // products that are not stored are those of M itself
+        if constexpr (STORED) {
+            dsq = bsum1(dsq, L);
+            if (cl.parts > 1) dsq = cl.sum_members(n, dsq);
+            dM = 0x1p-24 * sqrt(dsq) + n * 0x1p-150;
+        }
         bool done = false;
         for (; sweeps < a.max_refine; ++sweeps) {
             double mx = mx0;   // sweep 0: formed by the assembly
@@ -175,14 +193,15 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
                 break;
             }
             double dx = 0.0;
-            iters += wg_gmres([&]() { return mv_pairs(Mt, n, cl, L); }, n, r, dx, true,
-                              fmax(1e-7 * rn, 0.25 * tol_abs), 1, L, nullptr, {true, r, rr}, pre);
+            iters += wg_gmres(product, n, r, dx, true,
+                              STORED ? fmax(1e-7 * rn, 0.25 * tol_abs) : 0.25 * tol_abs, 1, L, nullptr, {true, r, rr},
+                              pre);
             x += dx;
             // the FP64 residual of the corrected x, bounded without forming it:
             //   |b - M x| <= |r - M32 dx| + |(M - M32) dx| <= (GMRES residual) + ||M - M32||_F |dx|
             // which at steady state is far below the tolerance (|dx| is the warm start's error)
             const double est = L.scal[0];   // |r - M32 dx|, the last rotated right-hand side entry
-            const double dn = sqrt(bsum1(own ? dx * dx : 0.0, L));
+            const double dn = STORED ? sqrt(bsum1(own ? dx * dx : 0.0, L)) : 0.0;
             if (est + dM * dn <= tol_abs) {
                 ++sweeps;
                 done = true;
