@@ -77,7 +77,7 @@ __global__ __launch_bounds__(1024) void rhs_vjp_kernel(VjpArgs a, Phys ph) {
         const double bn = sqrt(bsum1(own ? nv.b * nv.b : 0.0, L));
         if (t < sg.nb * kTile) L.vs[t] = 0.0;   // the padding entries stay 0
         __syncthreads();
-        its += wg_gmres([&]() { return mv_free_sym(n, pc, cl, L); }, n, nv.b, mu, true, a.tol * bn, a.cycles, L,
+        its += wg_gmres([&]() { return mv_free_sym(n, pc, cl, L); }, NoSums{}, n, nv.b, mu, true, a.tol * bn, a.cycles, L,
                         &unconv, {}, pre);
     }
     if (own) L.fa[lds_index(d, t)] = make_double2(mu, 0.0);
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(1024) void rhs_vjp_kernel(VjpArgs a, Phys ph) {
     double gb = 0.0;
     {
         const double gn = sqrt(bsum1(own ? gmu * gmu : 0.0, L));
-        its += wg_gmres([&]() { return mv_pairs(Mt, n, cl, L); }, n, gmu, gb, true, a.tol * gn, a.cycles, L, &unconv,
+        its += wg_gmres([&]() { return mv_pairs(Mt, n, cl, L); }, NoSums{}, n, gmu, gb, true, a.tol * gn, a.cycles, L, &unconv,
                         {true, own ? gmu : 0.0, gn * gn}, pre);
     }
 

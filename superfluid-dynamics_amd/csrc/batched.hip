@@ -11,8 +11,8 @@
 //      Phi' from a second (Derivatives.cuh:310-384), plus the per-node half-angle table;
 //   B  the dipole matrix M = I/2 + K (createM.cuh:43-92) into HBM, in the order in which the sweeps visit it
 //      (sfh_sym.hpp), FP64 or FP32 (FP64 entries rounded), and in the same pair loop M x for the warm start x (the first residual);
-//   C  the solve M mu = b, warm-started from the surface's previous mu (STORED says where the matrix is stored
-//      and where its products are evaluated anew in FP64):
+//   C  the solve M mu = b, warm-started from the surface's previous mu, with products of the stored matrix or
+//      (as B's, without storing) of sums that the velocity needs anyway:
 //        FP64  : GMRES on the FP64 matrix (classical Gram-Schmidt with one
 //                re-orthogonalisation, restarted cycles of kBK vectors);
 //        mixed : FP64 iterative refinement  r = b - M mu  with the residual evaluated
@@ -30,23 +30,46 @@
 // and every load of the stored product is one contiguous 512-byte (FP64) or 256-byte (FP32) row
 // per wave, and node data is read from LDS without bank conflicts.
 //
-// Bounds: N = 1024 mixed water among 512 surfaces, one Arnoldi step 450 us (540 with the stored matrix): derivatives
-// 16, assembly sweep 149, product 135, the rest of the solve 16, mu' 7, velocity sweep 125; the three sweeps issue FP64
-// instructions back to back (148 cycles for 64 pairs).
+// Bounds: N = 1024 mixed water among 512 surfaces, one Arnoldi step, 293 us: derivatives 16, sweep of the warm start 132,
+// sweep of the step 130, the rest of the solve 7, mu' 6, stage 2; the sweeps issue FP64 instructions back to back (150
+// cycles for 64 pairs).
 #include <type_traits>
 
 #include "sfh_sym.hpp"
 
 namespace sfh {
 
+// The cotangent sums of the vector last multiplied, of the solution so far, and (in the matrix's place) of the basis.
+template <int NA>
+struct CotSums {
+    double* basis;   // NA * n for each basis vector
+    int n;
+    double last[NA], sum[NA];
+    __device__ void keep(int j) {
+        const int t = threadIdx.x;
+        if (t >= n) return;
+#pragma unroll
+        for (int a = 0; a < NA; ++a) basis[(size_t)(j * NA + a) * n + t] = last[a];
+    }
+    __device__ void fresh() {
+#pragma unroll
+        for (int a = 0; a < NA; ++a) sum[a] = last[a];
+    }
+    __device__ void add(int k, const double* y) {
+        const int t = threadIdx.x;
+        if (t >= n) return;
+        for (int i = 0; i < k; ++i) {
+            const double c = y[i];
+#pragma unroll
+            for (int a = 0; a < NA; ++a) sum[a] += c * basis[(size_t)(i * NA + a) * n + t];
+        }
+    }
+};
+
 template <bool MIXED, bool FILM, bool SHARED>
 __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys ph, StageCtl ctl) {
-    // The solve's products come from the matrix that the assembly stores, or are evaluated anew in FP64.  A pair of a
-    // water surface takes the SIMDs 1.24e-4 us per squared node count, and its entries 6e-5 (FP32) or 1.25e-4 (FP64) to
-    // load on an idle GPU, but 1.5e-4 or more once every CU loads its own surface's (N = 1024, 512 surfaces: product
-    // 155 us stored in FP32, 135 evaluated; and the assembly 181 with the stores, 149 without).  A film's pair has two
-    // cotangents, and its matrix is always stored.
-    constexpr bool STORED = FILM || (MIXED && SHARED);
+    constexpr bool stored = FILM;   // the matrix: see the assembly
+    constexpr int NA = FILM ? 4 : 2;
     __shared__ BLds L;
     const int s = a.order[blockIdx.x];
     const SurfDesc d = a.sd[s];
@@ -100,9 +123,15 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
     }
 
     // ---------------------------------------------------------------- B: assembly
-    // One sweep over the unordered pairs (sfh_sym.hpp) writes both entries of each pair into the
-    // wave's rows of the matrix (FP64, or FP64 entries rounded to FP32) and forms (M x)_k for the warm start
-    // x in FP64 from the unrounded entries: the first residual of the solve.
+    // The solve's products come from a stored matrix or from the cotangent sums S(v), of which (M v)_k and the velocity
+    // are local combinations.  With the sums nothing is stored, and as S is linear, the velocity's S(mu) is S of the
+    // warm start plus the solve's coefficients times the S of its basis: no sweep of its own.  With k Arnoldi steps that
+    // makes 1 + k sweeps in place of an assembly, k products and the velocity's sweep.  Microseconds per stage of
+    // N = 1024 water: sweep 130, assembly 181 (149 without its stores), product stored in FP32 155 when every CU loads
+    // its own surface's and 65 on an idle GPU: water takes the sums (512 mixed surfaces 450 -> 297 us per stage).  A film's
+    // pair has two cotangents (N = 768 FP64: sweep 124, assembly 147, stored product 75) and its cold solves take 6 or 7
+    // steps, and the four sums leave the solve too few registers: with sums for the solves of one or two steps 96 films
+    // took 11.1 ms, with the stored matrix 9.8.
     const bool water = ph.kind == 0;
     PairConst pc = wg_diagonal(ph, nv, n, L);
     pc.image = FILM;   // known when compiled
@@ -111,9 +140,37 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
     const int nbk = (n + kTile - 1) / kTile;
     if (t < nbk * kTile) L.vs[t] = own ? x : 0.0;   // the padding entries stay 0 for every product
     __syncthreads();
+    double* const psy = reinterpret_cast<double*>(L.fa);   // 2 kBT doubles each
+    double* const piy = reinterpret_cast<double*>(L.fb);
     double dsq = 0.0;   // mixed: this thread's share of ||M||_F^2
     double mx0;         // (M x)_t
-    {
+    CotSums<NA> S{reinterpret_cast<double*>(Mt) + (long long)cl.rank * kBK * NA * n, n, {}, {}};   // each workgroup's own
+    const auto sums_of_vs = [&]() {
+        if constexpr (FILM) {
+            double* const acc[4] = {L.part, psy, psy + kBT, piy};
+            cot_sums<4>(n, acc, pc, cl, L, S.last);
+        } else {
+            double* const acc[2] = {L.part, psy};
+            cot_sums<2>(n, acc, pc, cl, L, S.last);
+        }
+    };
+    const auto product = [&]() {
+        if constexpr (stored) {
+            return mv_pairs(Mt, n, cl, L);
+        } else {
+            sums_of_vs();
+            const double w = own ? product_of_sums<NA>(S.last, pc, zpk, L.diag[t], L.vs[t]) : 0.0;
+            __syncthreads();   // the sums and L.vs have been read
+            return w;
+        }
+    };
+    if constexpr (!stored) {
+        mx0 = product();
+        S.fresh();
+    } else {
+        // One sweep over the unordered pairs (sfh_sym.hpp) writes both entries of each pair into the
+        // wave's rows of the matrix (FP64, or FP64 entries rounded to FP32) and forms (M x)_k for the warm start
+        // x in FP64 from the unrounded entries: the first residual of the solve.
         const SymGeo sg = sym_geo(n);
         const int kr = sg.I * kTile + sg.l;
         const NodeTrig tk = L.tr[kr];
@@ -130,16 +187,14 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
             if (decltype(full)::value || (k < n && j < n)) {
                 entry_pair(tk, L.tr[j], czk, L.zp[j], pc, e, em);
                 row[0] += e * L.vs[j];
-                if constexpr (MIXED && STORED) dsq += e * e;
+                if constexpr (MIXED) dsq += e * e;
                 if constexpr (decltype(mirror)::value) {
                     col[0] += em * vk;
-                    if constexpr (MIXED && STORED) dsq += em * em;
+                    if constexpr (MIXED) dsq += em * em;
                 }
             }
-            if constexpr (STORED) {
-                Mi[(unsigned)(2 * q) * kTile + l] = (MT)e;
-                Mi[(unsigned)(2 * q + 1) * kTile + l] = decltype(mirror)::value ? (MT)em : (MT)0;
-            }
+            Mi[(unsigned)(2 * q) * kTile + l] = (MT)e;
+            Mi[(unsigned)(2 * q + 1) * kTile + l] = decltype(mirror)::value ? (MT)em : (MT)0;
         }, cl, mx);
         mx0 = own ? mx[0] + L.diag[t] * L.vs[t] : 0.0;
     }
@@ -159,20 +214,21 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
         pre.modes = film_modes(n, pre.height);
     }
     __syncthreads();   // the sums are read before they are formed again
-    const auto product = [&]() {
-        if constexpr (STORED)
-            return mv_pairs(Mt, n, cl, L);
+    NoSums none;
+    auto& sums = [&]() -> auto& {
+        if constexpr (stored)
+            return none;
         else
-            return mv_free_sym(n, pc, cl, L);
-    };
+            return S;
+    }();
     int unconv = 0, iters = 0, sweeps = 0;
     if constexpr (!MIXED) {
-        iters = wg_gmres(product, n, bk, x, false, tol_abs, a.cycles, L, &unconv,
+        iters = wg_gmres(product, sums, n, bk, x, false, tol_abs, a.cycles, L, &unconv,
                          {true, r0, rr0}, pre);
     } else {
         // ||M - M32||_F <= 2^-24 ||M||_F (round to nearest, normal range) + N 2^-150 (subnormal range)
         double dM = 0.0;   // products that are not stored are those of M itself
-        if constexpr (STORED) {
+        if constexpr (stored) {
             dsq = bsum1(dsq, L);
             if (cl.parts > 1) dsq = cl.sum_members(n, dsq);
             dM = 0x1p-24 * sqrt(dsq) + n * 0x1p-150;
@@ -183,7 +239,12 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
             if (sweeps > 0) {
                 if (own) L.vs[t] = x;
                 __syncthreads();
-                mx = mv_free_sym(n, pc, cl, L);   // every thread: it synchronises
+                if constexpr (stored) {
+                    mx = mv_free_sym(n, pc, cl, L);   // every thread: it synchronises
+                } else {
+                    mx = product();
+                    S.fresh();
+                }
             }
             const double r = sweeps > 0 ? (own ? bk - mx : 0.0) : r0;
             const double rr = sweeps > 0 ? bsum1(r * r, L) : rr0;
@@ -193,15 +254,15 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
                 break;
             }
             double dx = 0.0;
-            iters += wg_gmres(product, n, r, dx, true,
-                              STORED ? fmax(1e-7 * rn, 0.25 * tol_abs) : 0.25 * tol_abs, 1, L, nullptr, {true, r, rr},
+            iters += wg_gmres(product, sums, n, r, dx, true,
+                              stored ? fmax(1e-7 * rn, 0.25 * tol_abs) : 0.25 * tol_abs, 1, L, nullptr, {true, r, rr},
                               pre);
             x += dx;
             // the FP64 residual of the corrected x, bounded without forming it:
             //   |b - M x| <= |r - M32 dx| + |(M - M32) dx| <= (GMRES residual) + ||M - M32||_F |dx|
             // which at steady state is far below the tolerance (|dx| is the warm start's error)
             const double est = L.scal[0];   // |r - M32 dx|, the last rotated right-hand side entry
-            const double dn = STORED ? sqrt(bsum1(own ? dx * dx : 0.0, L)) : 0.0;
+            const double dn = stored ? sqrt(bsum1(own ? dx * dx : 0.0, L)) : 0.0;
             if (est + dM * dn <= tol_abs) {
                 ++sweeps;
                 done = true;
@@ -235,52 +296,11 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
     __syncthreads();
 
     // ---------------------------------------------------------------- E: velocity + stage
-    // One sweep over the unordered pairs: the cotangent sums of both rows of each pair (the image
-    // sums too for the film).
-    double* psy = reinterpret_cast<double*>(L.fa);   // 2 kBT doubles: sy | ix
-    double* piy = reinterpret_cast<double*>(L.fb);
-    double vsum[FILM ? 4 : 2];   // S_x, S_y and the image sums
-    {
-        const int kr = sym_row(n);
-        const NodeTrig tk = L.tr[kr];
-        const double mk = L.vs[kr];
-        if constexpr (FILM) {
-            double* const acc[4] = {L.part, psy, psy + kBT, piy};
-            sym_sums<4>(n, acc, [&](int k, int j, int, auto mirror, auto full, double (&row)[4], double (&col)[4]) {
-                if (!decltype(full)::value && (k >= n || j >= n)) return;
-                const NodeTrig tj = L.tr[j];
-                const double mj = L.vs[j];
-                const CotParts cp = cot_parts(tk, tj);
-                const CotParts cq = cot_image_parts(tk, tj, pc.eh, pc.ehi);
-                const double w = mj * cp.id, wi = mj * cq.id;
-                row[0] += w * cp.p;
-                row[1] -= w * cp.q;
-                row[2] += wi * cq.p;
-                row[3] -= wi * cq.q;
-                if constexpr (decltype(mirror)::value) {   // p, p' change sign with the pair's order, q changes, q' not
-                    const double wk = mk * cp.id, wki = mk * cq.id;
-                    col[0] -= wk * cp.p;
-                    col[1] += wk * cp.q;
-                    col[2] -= wki * cq.p;
-                    col[3] -= wki * cq.q;
-                }
-            }, cl, vsum);
-        } else {
-            double* const acc[2] = {L.part, psy};
-            sym_sums<2>(n, acc, [&](int k, int j, int, auto mirror, auto full, double (&row)[2], double (&col)[2]) {
-                if (!decltype(full)::value && (k >= n || j >= n)) return;
-                const CotParts cp = cot_parts(tk, L.tr[j]);
-                const double w = L.vs[j] * cp.id;
-                row[0] += w * cp.p;
-                row[1] -= w * cp.q;
-                if constexpr (decltype(mirror)::value) {
-                    const double wk = mk * cp.id;
-                    col[0] -= wk * cp.p;
-                    col[1] += wk * cp.q;
-                }
-            }, cl, vsum);
-        }
-    }
+    // The cotangent sums of mu (the image sums too for the film): from the solve, or one sweep.
+    if constexpr (stored) sums_of_vs();
+    double vsum[NA];
+#pragma unroll
+    for (int i = 0; i < NA; ++i) vsum[i] = stored ? S.last[i] : S.sum[i];
     if (cl.parts > 1) {
         if (t == 0) cl.leave();
         if (!lead) return;

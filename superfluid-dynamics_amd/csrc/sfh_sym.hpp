@@ -233,6 +233,48 @@ __device__ inline double mv_free_sym(int n, const PairConst& pc, Cluster& cl, BL
     return w[0];
 }
 
+// The cotangent sums of v (L.vs) that (M v)_t and the velocity share: out = sum_j v_j of Re and Im cot((z_t - z_j)/2)
+// over j != t, and for the film (NA = 4) of cot((z_t - conj z_j)/2 + i h).  acc: NA LDS arrays of kBT doubles.
+template <int NA>
+__device__ inline void cot_sums(int n, double* const (&acc)[NA], const PairConst& pc, Cluster& cl, BLds& L, double (&out)[NA]) {
+    static_assert(NA == 2 || NA == 4, "water or film");
+    const int kr = sym_row(n);
+    const NodeTrig tk = L.tr[kr];
+    const double vk = L.vs[kr];
+    sym_sums<NA>(n, acc, [&](int k, int j, int, auto mirror, auto full, double (&row)[NA], double (&col)[NA]) {
+        if (!decltype(full)::value && (k >= n || j >= n)) return;
+        const NodeTrig tj = L.tr[j];
+        const double vj = L.vs[j];
+        const CotParts cp = cot_parts(tk, tj);
+        const double w = vj * cp.id;
+        row[0] += w * cp.p;
+        row[1] -= w * cp.q;
+        if constexpr (decltype(mirror)::value) {   // p, p' change sign with the pair's order, q changes, q' not
+            const double wk = vk * cp.id;
+            col[0] -= wk * cp.p;
+            col[1] += wk * cp.q;
+        }
+        if constexpr (NA == 4) {
+            const CotParts cq = cot_image_parts(tk, tj, pc.eh, pc.ehi);
+            const double wi = vj * cq.id;
+            row[2] += wi * cq.p;
+            row[3] -= wi * cq.q;
+            if constexpr (decltype(mirror)::value) {
+                const double wki = vk * cq.id;
+                col[2] -= wki * cq.p;
+                col[3] -= wki * cq.q;
+            }
+        }
+    }, cl, out);
+}
+// (M v)_t from them; t < n.
+template <int NA>
+__device__ inline double product_of_sums(const double (&s)[NA], const PairConst& pc, double2 zp, double diag, double v) {
+    double w = pc.c * (zp.x * s[1] + zp.y * s[0]) + diag * v;
+    if constexpr (NA == 4) w -= pc.ci * s[3];
+    return w;
+}
+
 // (M v)_t for the matrix that the waves stored (see above), v in L.vs with L.vs[j] = 0 for n <= j < nb*64
 // (the caller has synchronised).  Returns the value on threads t < n, 0 elsewhere.
 template <typename T>

@@ -176,8 +176,16 @@ struct FirstResidual {
 // tolerance are those of A x = rhs as without.  x_zero: x is known to be 0 (the first residual is rhs, no product needed); with a
 // given first residual none is needed either.  Returns the number of
 // Arnoldi steps; *unconv is set when tol_abs was not reached.
-template <class MV>
-__device__ int wg_gmres(MV&& mv, int n, double rhs, double& x, bool x_zero, double tol_abs, int cycles,
+// sums keeps a linear by-product of mv (pair sums that mv forms anyway): keep(j) its value for the product of basis
+// vector j, fresh() replaces the value for x by the last product's, add(k, y) adds that of the correction.
+struct NoSums {
+    __device__ void keep(int) {}
+    __device__ void fresh() {}
+    __device__ void add(int, const double*) {}
+};
+
+template <class MV, class Sums>
+__device__ int wg_gmres(MV&& mv, Sums&& sums, int n, double rhs, double& x, bool x_zero, double tol_abs, int cycles,
                         BLds& L, int* unconv, const FirstResidual first = {}, const Precond pre = {-1, 0.0}) {
     const int t = threadIdx.x;
     const bool own = t < n;
@@ -190,6 +198,7 @@ __device__ int wg_gmres(MV&& mv, int n, double rhs, double& x, bool x_zero, doub
             if (own) L.vs[t] = x;
             __syncthreads();
             const double w = mv();
+            sums.fresh();
             r = own ? rhs - w : 0.0;
         }
         if (cyc > 0 || !first.given) rr = bsum1(r * r, L);
@@ -208,6 +217,7 @@ __device__ int wg_gmres(MV&& mv, int n, double rhs, double& x, bool x_zero, doub
             if (own) L.vs[t] = u;
             __syncthreads();
             double w = mv();
+            sums.keep(j);
             // classical Gram-Schmidt ...
             bsum_dots(V, w, j, false, L);
             if (t == 0)
@@ -269,6 +279,7 @@ __device__ int wg_gmres(MV&& mv, int n, double rhs, double& x, bool x_zero, doub
             }
         }
         __syncthreads();
+        sums.add(k, L.y);
         if (pre.modes >= 0) {
             double u = 0.0;
 #pragma unroll

@@ -295,7 +295,9 @@ std::vector<int> Solver::batched_parts() const {
             if (cost(s, parts[s]) > cost(worst, parts[worst])) worst = s;
         const int p = parts[worst];
         // the first split has to pay for its meetings with more than one extra workgroup's share
-        if (p == kMaxParts || cost(worst, p == 1 ? std::min(3, 1 + left) : p + 1) >= cost(worst, p)) break;
+        // each workgroup keeps the cotangent sums of 8 basis vectors in its share of the matrix's place
+        const long long room = tiled_matrix_elems(n_[worst]) * (opt_.precision == kMixed ? 4 : 8) / (8LL * 8 * 4 * n_[worst]);
+        if (p == kMaxParts || p + 1 > room || cost(worst, p == 1 ? std::min(3, 1 + left) : p + 1) >= cost(worst, p)) break;
         ++parts[worst];
     }
     return parts;
