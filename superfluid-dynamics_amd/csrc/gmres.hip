@@ -1,5 +1,5 @@
-// gmres.hip -- FP64 GMRES for M mu = b over the stored dipole matrix, all workgroups of the GPU on
-// one or a few large surfaces (the iterative alternative to the LU of MatrixSolver::solve,
+// gmres.hip -- FP64 GMRES for the dipole system M mu = b, all workgroups of the GPU on one or a few
+// large surfaces (the iterative alternative to the LU of MatrixSolver::solve,
 // CuSuperHelium/MatrixSolver.cuh:113-172).
 //
 // M = I/2 + K is a second-kind operator: its spectrum clusters at 1/2 (for the helium film one
@@ -8,9 +8,10 @@
 //
 // A solve is a fixed sequence of L launches; launch i first finishes Arnoldi step i - 1 and then,
 // unless the solve is done, runs step i.  No workgroup waits for another: every grid-wide result
-// is read by the next launch.  Launches 0 .. L-2 are gm_iter_kernel; the last one, which only
-// finishes a step, is gm_close_mu_kernel, which goes on to form the derivative mu' of the
-// solution (with L = 1 the single launch is gm_iter_kernel).
+// is read by the next launch.  Launches 0 .. L-2 are gm_sums_kernel (products formed from the cotangent sums
+// that the velocity needs as well, sfh_pairs.hpp) or gm_iter_kernel (products of the stored matrix); the last one,
+// which only finishes a step, is gm_close_mu_kernel, which goes on to form the derivative mu' of the
+// solution and, from the sums, the velocity stage (with L = 1 the single launch is gm_iter_kernel).
 //   finish step i-1 (i >= 1), in every workgroup: sum the partial dots v_l . w_{i-1} of all
 //     workgroups (fixed order, so every workgroup gets the same h_{l,i-1}); rebuild
 //     u = w_{i-1} - sum_l h_{l,i-1} v_l over all N entries into LDS (classical Gram-Schmidt, one
@@ -21,12 +22,11 @@
 //     x0 + V y as the solution, each workgroup its own rows, and pushes them into the warm-start
 //     history (a launch that finds convergence earlier only keeps y for it).  The initial guess
 //     x0 and the solution are separate arrays.
-//   step i: w_i = M v_i for the workgroup's rows (one or two rows per wave, the first loads issued at the
-//     kernel's start so they overlap the finishing work), and the partial dots v_l . w_i, l <= i.
+//   step i: w_i = M v_i for the workgroup's rows, and the partial dots v_l . w_i, l <= i.
 //     For the film w_i = M P^{-1} v_i with the preconditioner P of its image term (precondition), and
 //     the solution is x0 + P^{-1} V y, P^{-1} V being kept beside V.
-// Launch 0 takes v_0 = r0 / |r0|.  The assembly kernel forms r0 = b - M x0 while it writes M
-// (assemble.hip), and every workgroup of launch 0 reduces |r0| and |b| over its own full copies.
+// Launch 0 takes v_0 = r0 / |r0|.  gm_start_kernel (or the assembly, while it writes M) forms
+// r0 = b - M x0, and every workgroup of launch 0 reduces |r0| and |b| over its own full copies.
 // L launches therefore run up to L - 1 Arnoldi steps.  Once the residual estimate reaches
 // tol * |b|, the remaining launches return at once.  Partial dots and the rotated right-hand side
 // live in per-launch (even/odd or per-index) slots, because a slot must not be overwritten while
@@ -36,7 +36,7 @@
 // polynomial through them (extrapolate_history; with five steps kept its error is fifth order in
 // dt, against first order for the previous stage's mu), which saves Krylov steps on every solve of
 // a time integration.
-#include "sfh_circ.hpp"
+#include "sfh_pairs.hpp"
 #include "sfh_gmres.hpp"
 
 namespace sfh {
@@ -274,11 +274,105 @@ __device__ inline void back_substitute(const double* g, const double* H, int m, 
     }
 }
 
-// Launch i of a solve's sequence (see the file comment), W waves of RR matrix rows each per workgroup
-// (a.rpw rows).  Every workgroup repeats the finishing work (the basis, the partial sums, the
-// preconditioner), so the rows per workgroup follow the size (Solver::alloc_gmres).
-template <typename T, int W, int RR>
-__global__ __launch_bounds__(64 * W) void gm_iter_kernel(GmArgs a, const SurfDesc* __restrict__ sd, int i) {
+// Where a launch's products come from: a policy with W waves and ROWS matrix rows per workgroup.  start() requests what
+// the product needs besides the vector; run() forms the rows' products of vs (LDS), w = sj * (M vs), in wl (LDS) and wi
+// (the caller synchronises).
+//
+// The stored matrix, RR rows per wave.
+template <typename T, int WAVES, int RR>
+struct StoredRows {
+    static constexpr int W = WAVES, ROWS = W * RR;
+    const T* R;
+    RowBuf<T, RR> rc;
+    int n, row, rows, lane, wv;
+    __device__ StoredRows(const GmArgs&, const GmView& v, const SurfDesc&, int r0) {
+        lane = threadIdx.x & 63;
+        wv = threadIdx.x >> 6;
+        n = v.n;
+        row = r0 + wv * RR;
+        rows = max(1, min(RR, n - row));   // this wave's rows (at least one is loaded)
+        R = (sizeof(T) == 8 ? reinterpret_cast<const T*>(v.M) : reinterpret_cast<const T*>(v.M32)) + (long long)min(row, n - 1) * n;
+    }
+    __device__ void start() { row_start(R, n, rows, lane, rc); }
+    __device__ void run(const double* vs, double sj, double* wi, double* wl, int) {
+        double d[RR];
+        row_dots(R, rc, vs, n, rows, lane, d);
+        if (lane == 0) {
+#pragma unroll
+            for (int r = 0; r < RR; ++r) {
+                wl[wv * RR + r] = row + r < n ? sj * d[r] : 0.0;
+                if (row + r < n) wi[row + r] = sj * d[r];
+            }
+        }
+    }
+};
+
+// Cotangent sums (sfh_pairs.hpp), H groups of 256 threads with 4 rows each; the sums are kept for the velocity.  The
+// evaluation is bound by FP64 issue (23 instructions per pair for water, 41 for the film): N = 4096 film 40 us per
+// launch, of which 22 are issue, N = 2048 water 8 us, of which 3 are issue and 4 the finishing work and first loads.
+template <int NA, int H>
+struct PairSums {
+    static constexpr int W = 4 * H, ROWS = kSumRows * H;
+    const NodeTrig* tr;
+    double* S;
+    NodeTrig tk[kSumRows];
+    SumConst kc;
+    double2 zp;
+    double diag;
+    long long stride;
+    int n, r0, tg, k0;
+    __device__ PairSums(const GmArgs& a, const GmView& v, const SurfDesc& d, int first) {
+        n = v.n;
+        r0 = first;
+        tg = threadIdx.x & 255;
+        k0 = r0 + kSumRows * (threadIdx.x >> 8);
+        tr = a.trig + d.voff;
+        S = a.S + d.voff;
+        stride = a.total;
+        kc = {a.pc, a.pci, a.eh, a.ehi};
+        const int own = d.voff + min(r0 + (int)threadIdx.x, n - 1);
+        zp = a.Zp[own];
+        diag = a.diag[own];
+    }
+    __device__ void start() {
+#pragma unroll
+        for (int r = 0; r < kSumRows; ++r) tk[r] = tr[min(k0 + r, n - 1)];
+    }
+    __device__ void run(const double* vs, double sj, double* wi, double* wl, int i) {
+        __shared__ double red[W][NA * kSumRows];
+        double acc[NA * kSumRows];
+#pragma unroll
+        for (int q = 0; q < NA * kSumRows; ++q) acc[q] = 0.0;
+        const auto value = [&](int j) { return vs[j]; };
+        for (int j0 = 0; j0 < n; j0 += kSumPass) {
+            NodeTrig tj[kSumCols];
+            sum_columns(tr, n, j0, tg, tj);
+            sum_pass<NA>(tk, tj, n, k0, j0, tg, kc.eh, kc.ehi, value, acc);
+        }
+        sum_store<NA>(acc, red);
+        __syncthreads();
+        const int t = threadIdx.x;
+        if (t < ROWS) {
+            double w = 0.0;
+            if (r0 + t < n) {
+                double s[NA];
+#pragma unroll
+                for (int q = 0; q < NA; ++q) {
+                    s[q] = sum_total<NA>(red, t / kSumRows, t % kSumRows, q);
+                    S[(long long)((1 + i) * NA + q) * stride + r0 + t] = s[q];
+                }
+                w = sj * product_of_sums<NA>(s, kc, zp, diag, vs[r0 + t]);
+                wi[r0 + t] = w;
+            }
+            wl[t] = w;
+        }
+    }
+};
+
+// Launch i of a solve's sequence (see the file comment).  Every workgroup repeats the finishing work (the basis, the
+// partial sums, the preconditioner), so the rows per workgroup follow the size (Solver::alloc_gmres).
+template <class P>
+__device__ __forceinline__ void gm_step(const GmArgs& a, const SurfDesc* __restrict__ sd, int i) {
     GmCtl* ctl = reinterpret_cast<GmCtl*>(a.ctl) + blockIdx.z;
     // solves finished by an earlier launch return at once.  A finish stamped by this launch
     // (workgroup 0 can get there before a late workgroup starts) does not count.  Launch 0 needs
@@ -290,8 +384,7 @@ __global__ __launch_bounds__(64 * W) void gm_iter_kernel(GmArgs a, const SurfDes
     }
     const GmView v = gm_view(a, sd);
     const int m = a.m;
-    constexpr int rpw = W * RR, NT = 64 * W, E = 8;   // E entries per thread and pass
-    static_assert(rpw != 16 || NT * E >= kGmMaxN, "the largest surface in one pass");
+    constexpr int W = P::W, rpw = P::ROWS, NT = 64 * W, E = 8;   // E entries per thread and pass
     if ((int)blockIdx.x * rpw >= v.n) return;
     __shared__ double vs[kGmMaxN];
     __shared__ double co[kMaxKrylov + 1];
@@ -303,9 +396,7 @@ __global__ __launch_bounds__(64 * W) void gm_iter_kernel(GmArgs a, const SurfDes
     __shared__ double ys[kMaxKrylov + 4];   // g[j], gc[j+1], c, s, then y
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6, n = v.n;
     const int r0 = blockIdx.x * rpw;
-    const int row = r0 + wv * RR, rows = max(1, min(RR, n - row));   // this wave's rows (at least one is loaded)
-    const T* R = (sizeof(T) == 8 ? reinterpret_cast<const T*>(v.M) : reinterpret_cast<const T*>(v.M32)) +
-                 (long long)min(row, n - 1) * n;
+    P prod(a, v, sd[blockIdx.z], r0);
     const long long pslot = (long long)v.nwg * (m + 1);   // one partial-dot slot per launch parity
     // Loads go out in the order their results are needed, because a wait for one load waits for
     // all loads issued before it: first the vectors and sums of the step being finished (launch
@@ -332,9 +423,8 @@ __global__ __launch_bounds__(64 * W) void gm_iter_kernel(GmArgs a, const SurfDes
     const double height = a.pre ? v.ctl->height : 0.0;
     // the rows up front, except in a refinement solve, which most often ends at once: there they
     // are fetched when the step is known to run
-    RowBuf<T, RR> rc;
     const bool early_rows = !a.check_first;
-    if (i < m - 1 && early_rows) row_start(R, n, rows, lane, rc);
+    if (i < m - 1 && early_rows) prod.start();
     if (i == 1 && !a.check_first) {
         const int fin = ctl->done;
         if (fin != 0 && fin <= i) return;
@@ -492,16 +582,8 @@ __global__ __launch_bounds__(64 * W) void gm_iter_kernel(GmArgs a, const SurfDes
     for (int r = 0; r < rpw; ++r) vrow[r] = (t < i && r0 + r < n) ? v.V[(long long)t * n + r0 + r] : 0.0;
     const double sct = (t < i) ? v.sc[t] : 0.0;
     double* wi = (i & 1) ? v.w1 : v.w0;
-    if (!early_rows) row_start(R, n, rows, lane, rc);
-    double d[RR];
-    row_dots(R, rc, vs, n, rows, lane, d);
-    if (lane == 0) {
-#pragma unroll
-        for (int r = 0; r < RR; ++r) {
-            wl[wv * RR + r] = row + r < n ? sj * d[r] : 0.0;
-            if (row + r < n) wi[row + r] = sj * d[r];
-        }
-    }
+    if (!early_rows) prod.start();
+    prod.run(vs, sj, wi, wl, i);
     __syncthreads();
     if (t <= i) {
         double s = 0.0;
@@ -514,13 +596,76 @@ __global__ __launch_bounds__(64 * W) void gm_iter_kernel(GmArgs a, const SurfDes
         }
         v.part[(i & 1) * pslot + (long long)t * v.nwg + blockIdx.x] = s;
     }
-    if (i == 0 && t == 1) {
-        // launch 0 also leaves |w_0|^2 (slot 1): a sequence of one Arnoldi step is finished from
-        // the two sums alone by velocity_gm1_kernel
-        double s = 0.0;
+}
+
+template <typename T, int W, int RR>
+__global__ __launch_bounds__(64 * W) void gm_iter_kernel(GmArgs a, const SurfDesc* __restrict__ sd, int i) {
+    gm_step<StoredRows<T, W, RR>>(a, sd, i);
+}
+template <int NA, int H>
+__global__ __launch_bounds__(256 * H) void gm_sums_kernel(GmArgs a, const SurfDesc* __restrict__ sd, int i) {
+    gm_step<PairSums<NA, H>>(a, sd, i);
+}
+
+// The start of a solve with products from cotangent sums: S of the initial guess, M_kk, and r0 = b - M x0 as the first
+// (unnormalised) basis vector.  grid = (ceil(max n / kSumRows), surfaces).
+template <int NA>
+__global__ __launch_bounds__(256) void gm_start_kernel(GmArgs a, const SurfDesc* __restrict__ sd, const double2* __restrict__ Z,
+                                                       const double2* __restrict__ Zpp, Phys ph) {
+    const SurfDesc d = sd[blockIdx.y];
+    const int n = d.n, k0 = blockIdx.x * kSumRows, t = threadIdx.x;
+    if (k0 >= n) return;
+    __shared__ double red[4][NA * kSumRows];
+    const NodeTrig* tr = a.trig + d.voff;
+    const double* x0 = a.x + d.voff;
+    NodeTrig tk[kSumRows], tj[kSumCols];
+    double xj[kSumCols];
+    double acc[NA * kSumRows];
 #pragma unroll
-        for (int r = 0; r < rpw; ++r) s += wl[r] * wl[r];
-        v.part[(long long)v.nwg + blockIdx.x] = s;
+    for (int r = 0; r < kSumRows; ++r) tk[r] = tr[min(k0 + r, n - 1)];
+    sum_columns(tr, n, 0, t, tj);
+#pragma unroll
+    for (int e = 0; e < kSumCols; ++e) xj[e] = x0[min(t + 256 * e, n - 1)];
+    // the own rows' inputs, before the sweep
+    const int g = d.voff + min(k0 + t, n - 1);
+    double2 zp = {1.0, 0.0}, zpp = {0.0, 0.0};
+    double y = 0.0, b = 0.0, x = 0.0;
+    if (t < kSumRows) {
+        zp = a.Zp[g];
+        zpp = Zpp[g];
+        y = Z[g].y;
+        b = a.b[g];
+        x = a.x[g];
+    }
+#pragma unroll
+    for (int q = 0; q < NA * kSumRows; ++q) acc[q] = 0.0;
+    for (int j0 = 0; j0 < n; j0 += kSumPass) {
+        if (j0 > 0) {
+            sum_columns(tr, n, j0, t, tj);
+#pragma unroll
+            for (int e = 0; e < kSumCols; ++e) xj[e] = x0[min(j0 + t + 256 * e, n - 1)];
+        }
+        int e = 0;
+        sum_pass<NA>(tk, tj, n, k0, j0, t, a.eh, a.ehi, [&](int) { return xj[e++]; }, acc);
+    }
+    sum_store<NA>(acc, red);
+    double dg = 0.0;
+    if (t < kSumRows) {
+        const double2 q = cdiv(zpp, zp);
+        dg = (ph.kind == 0 ? 0.5 * (1 + ph.rho) : 0.5) + a.pc * q.y;
+        if constexpr (NA == 4) dg -= a.pci * cot64(0.0, y + ph.depth).y;
+    }
+    __syncthreads();
+    if (t < kSumRows && k0 + t < n) {
+        double s[NA];
+#pragma unroll
+        for (int q = 0; q < NA; ++q) {
+            s[q] = sum_total<NA>(red, 0, t, q);
+            a.S[(long long)q * a.total + g] = s[q];
+        }
+        a.diag[g] = dg;
+        const SumConst kc = {a.pc, a.pci, a.eh, a.ehi};
+        a.V[(long long)(a.m + 1) * d.voff + k0 + t] = b - product_of_sums<NA>(s, kc, zp, dg, x);
     }
 }
 
@@ -545,10 +690,12 @@ struct CloseGeo {
 // LDS, so that the finishing work runs on data already at hand.  A workgroup reads the initial
 // guess, the basis and earlier launches' results, never the solution entries that other
 // workgroups of this launch are storing.  grid = (ceil(max n / kCircRowsPerWG), surfaces).
-template <bool PRE>
-__global__ __launch_bounds__(256) void gm_close_mu_kernel(GmArgs a, const SurfDesc* __restrict__ sd,
+template <bool PRE, int NA>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gm_close_mu_kernel(GmArgs a, const SurfDesc* __restrict__ sd,
                                                           const double* __restrict__ circ,
-                                                          double2* __restrict__ mup, int i) {
+                                                          double2* __restrict__ mup, int i,
+                                                          const double2* __restrict__ Z,
+                                                          const double2* __restrict__ Zpp, Phys ph, StageCtl sc) {
     constexpr int NT = 256;
     constexpr int CR = kCircRowsPerWG;
     constexpr int KM = kMaxKrylov;
@@ -574,6 +721,18 @@ __global__ __launch_bounds__(256) void gm_close_mu_kernel(GmArgs a, const SurfDe
     __shared__ double sums[KM + 2];
     __shared__ double ys[KM + 4];   // g[j], gc[j+1], c, s, then y
     const int t = threadIdx.x, wv = t >> 6;
+    // with the solve's cotangent sums: the own rows' sums of x0 and of the first two basis vectors, Z', Z'' and Z
+    constexpr int F = 3 * NA + 6;
+    __shared__ double own[NA ? CR * F : 1];
+    double own_v = 0.0;
+    if constexpr (NA > 0) {
+        if (t < CR * F) {
+            const int f = t / CR, g = d.voff + min(k0 + t % CR, n - 1);
+            const double2* node[3] = {a.Zp, Zpp, Z};
+            const double2* p = f < 3 * NA + 2 ? node[0] : f < 3 * NA + 4 ? node[1] : node[2];
+            own_v = f < 3 * NA ? a.S[(long long)f * a.total + g] : reinterpret_cast<const double*>(p + g)[(f - 3 * NA) & 1];
+        }
+    }
     const double* c1r = circ + d.coff;
     const double* c1i = c1r + n;
     double ar[G::WPER], ai[G::WPER];
@@ -630,6 +789,8 @@ __global__ __launch_bounds__(256) void gm_close_mu_kernel(GmArgs a, const SurfDe
     const int fin = ctl->done;
     const int iters_before = a.check_first ? ctl->refine_iters : ctl->iters;
     const double bnorm = ctl->bnorm;
+    if constexpr (NA > 0)
+        if (t < CR * F) own[t] = own_v;
     // all loads are out; the small state into LDS and the partial dots summed (used when the
     // solve is open)
     if (t < j) {
@@ -731,6 +892,10 @@ __global__ __launch_bounds__(256) void gm_close_mu_kernel(GmArgs a, const SurfDe
     }
     if (h0 && s == 0 && blockIdx.x == 0 && t == 0) count_history(a);
     // mu = x0 + y_0 Z[0] + y_1 Z[1] (+ the rest when k > 2), without branches in the common case
+    double mu_t = 0.0;   // own row, threads t < CR
+    StageIn st{};
+    if constexpr (NA > 0)
+        if (t < CR) st = stage_load(sc, d.voff + min(k0 + t, n - 1));
     const double y0 = k > 0 ? ys[4] : 0.0, y1 = k > 1 ? ys[5] : 0.0;
     double re[kCR], im[kCR];
 #pragma unroll
@@ -779,6 +944,7 @@ __global__ __launch_bounds__(256) void gm_close_mu_kernel(GmArgs a, const SurfDe
             if (r < n && r >= j0 && r < j0 + jn) {
                 const double x = ms[circ_at(r - j0)];
                 v.sol[r] = x;
+                mu_t = x;
                 if (h0) {
 #pragma unroll
                     for (int l = kHistDepth - 1; l > 0; --l) h0[(long long)l * a.total + r] = ho[l - 1];
@@ -810,7 +976,24 @@ __global__ __launch_bounds__(256) void gm_close_mu_kernel(GmArgs a, const SurfDe
             y += cred[w][kCR + t];
         }
         const double xs = 2.0 * kPi / n;
-        mup[d.voff + k0 + t] = make_double2(x * xs, y * xs);
+        const double2 mp = make_double2(x * xs, y * xs);
+        mup[d.voff + k0 + t] = mp;
+        if constexpr (NA > 0) {
+            const int g = d.voff + k0 + t;
+            double S[NA];
+#pragma unroll
+            for (int c = 0; c < NA; ++c) S[c] = own[c * CR + t] + y0 * own[(NA + c) * CR + t] + y1 * own[(2 * NA + c) * CR + t];
+            for (int q = 2; q < k; ++q)
+#pragma unroll
+                for (int c = 0; c < NA; ++c) S[c] += ys[4 + q] * a.S[(long long)((1 + q) * NA + c) * a.total + g];
+            const double* o = own + 3 * NA * CR + t;
+            const double2 zp = make_double2(o[0], o[CR]), zpp = make_double2(o[2 * CR], o[3 * CR]);
+            const double2 z = make_double2(o[4 * CR], o[5 * CR]);
+            double2 q1, q2;
+            velocity_from_sums(ph, zp, zpp, mp, mu_t, z.y, S[0], S[1], NA == 4 ? S[NA == 4 ? 2 : 0] : 0.0,
+                               NA == 4 ? S[NA == 4 ? 3 : 0] : 0.0, q1, q2);
+            finish_node(ph, sc, g, z, zp, zpp, q1, q2, q1, st);
+        }
     }
 }
 
@@ -819,7 +1002,18 @@ __global__ __launch_bounds__(256) void gm_close_mu_kernel(GmArgs a, const SurfDe
     template __global__ void gm_iter_kernel<float, W, RR>(GmArgs, const SurfDesc*, int);
 SFH_GM_INSTANCES(4, 1)
 SFH_GM_INSTANCES(8, 2)
-template __global__ void gm_close_mu_kernel<false>(GmArgs, const SurfDesc*, const double*, double2*, int);
-template __global__ void gm_close_mu_kernel<true>(GmArgs, const SurfDesc*, const double*, double2*, int);
+#define SFH_SUMS_INSTANCES(NA)                                                                          \
+    template __global__ void gm_start_kernel<NA>(GmArgs, const SurfDesc*, const double2*, const double2*, Phys); \
+    template __global__ void gm_sums_kernel<NA, 1>(GmArgs, const SurfDesc*, int);                            \
+    template __global__ void gm_sums_kernel<NA, 2>(GmArgs, const SurfDesc*, int);
+SFH_SUMS_INSTANCES(2)
+SFH_SUMS_INSTANCES(4)
+// stored matrix; sums for water; sums for the film, whose solves always have the preconditioner
+template __global__ void gm_close_mu_kernel<false, 0>(GmArgs, const SurfDesc*, const double*, double2*, int, const double2*,
+                                                      const double2*, Phys, StageCtl);
+template __global__ void gm_close_mu_kernel<false, 2>(GmArgs, const SurfDesc*, const double*, double2*, int, const double2*,
+                                                      const double2*, Phys, StageCtl);
+template __global__ void gm_close_mu_kernel<true, 4>(GmArgs, const SurfDesc*, const double*, double2*, int, const double2*,
+                                                     const double2*, Phys, StageCtl);
 
 }  // namespace sfh

@@ -92,31 +92,22 @@ struct GmArgs {
     int pre;
     double* Z;
     const double2* tw;   // twiddle tables, SurfDesc::twoff
+    // products from cotangent sums (sfh_pairs.hpp; sums = 0: from the stored matrix): S holds the sums of the initial
+    // guess and then of each (preconditioned, unscaled) basis vector, sums arrays of total nodes each
+    int sums;            // 2 (water), 4 (film)
+    double* S;
+    double* diag;        // M_kk
+    const NodeTrig* trig;
+    const double2* Zp;
+    double pc, pci, eh, ehi;
 };
 constexpr int kPairRows = 4;        // default rows per workgroup of the N^2 pair kernels (assembly, velocity)
 // ---- spectral.hip
-// circulant products of the launches that finish a GMRES solve (gm_close_mu_kernel, velocity_gm1_kernel): most
+// circulant products of the launches that finish a GMRES solve (gm_close_mu_kernel):
 // rows per workgroup, columns staged in LDS per round, and the kernel window one round needs
 constexpr int kCircRowsPerWG = 8;
 constexpr int kCircChunk = 2048;
-constexpr int kCircWin = kCircChunk + kCircRowsPerWG - 1;
 constexpr int kCircPer = kCircChunk / 256;               // staged samples per thread
-constexpr int kCircWinPer = (kCircWin + 255) / 256;      // staged kernel entries per thread
-// Window entry u holds c[(k0 - j0 - (kCircChunk - 1) + u) mod n]; row r, column c of the chunk
-// read entry r - c + kCircChunk - 1.  circ_window gives the kernel indices of the entries
-// u = threadIdx.x + 256 e a thread stages (entries beyond the window get valid indices too): one
-// division, then steps of 256 mod n, each reduced by one conditional subtraction.
-__device__ inline void circ_window(int k0, int j0, int n, int (&q)[kCircWinPer]) {
-    int r = (k0 - j0 - (kCircChunk - 1) + (int)threadIdx.x) % n;
-    if (r < 0) r += n;
-    const int step = 256 % n;
-#pragma unroll
-    for (int e = 0; e < kCircWinPer; ++e) {
-        q[e] = r;
-        r += step;
-        if (r >= n) r -= n;
-    }
-}
 // TC threads over the columns, TR row groups of 8 rows (spectral.hip)
 template <int TC, int TR>
 __global__ void zphi_circ_kernel(const SurfDesc* sd, const double* circ, const double2* Z, const double* phi,
@@ -148,10 +139,6 @@ template <int R>
 __global__ void velocity_stage_kernel(const SurfDesc* sd, const NodeTrig* trig, const double2* Z,
                                       const double2* Zp, const double2* Zpp, const double* mu,
                                       const double2* mup, Phys ph, StageCtl ctl);
-template <int R>
-__global__ void velocity_gm1_kernel(const SurfDesc* sd, const NodeTrig* trig, const double2* Z,
-                                    const double2* Zp, const double2* Zpp, double2* mup, Phys ph,
-                                    StageCtl ctl, GmArgs gm, const double* circ);
 
 // ---- lu.hip
 struct LuArgs {
@@ -185,8 +172,15 @@ __global__ void gepp_fallback_kernel(const SurfDesc* sd, double* M, const double
 constexpr int kGmCtlInts = 32;   // ints per control block (holds the device struct)
 template <typename T, int W, int RR>
 __global__ void gm_iter_kernel(GmArgs a, const SurfDesc* sd, int j);
-template <bool PRE>
-__global__ void gm_close_mu_kernel(GmArgs a, const SurfDesc* sd, const double* circ, double2* mup, int i);
+// products from cotangent sums: NA = 2 (water) or 4 (film) sums, H groups of 256 threads
+template <int NA>
+__global__ void gm_start_kernel(GmArgs a, const SurfDesc* sd, const double2* Z, const double2* Zpp, Phys ph);
+template <int NA, int H>
+__global__ void gm_sums_kernel(GmArgs a, const SurfDesc* sd, int j);
+// PRE: the basis is preconditioned; NA > 0: also the velocity stage, from the solve's sums (else Z, Zpp, ph, sc unused)
+template <bool PRE, int NA>
+__global__ void gm_close_mu_kernel(GmArgs a, const SurfDesc* sd, const double* circ, double2* mup, int i, const double2* Z,
+                                   const double2* Zpp, Phys ph, StageCtl sc);
 
 // ---- solver.hip: one trajectory frame [x(T), y(T), phi(T)] of the state
 __global__ void record_frame_kernel(const double2* Z, const double* P, const double* D, double* dst, int total);

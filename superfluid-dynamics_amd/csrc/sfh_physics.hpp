@@ -279,4 +279,20 @@ __device__ inline void stage_update(const StageCtl& ctl, int g, double2 q1, doub
     stage_store(ctl, g, q1, dphi, stage_load(ctl, g));
 }
 
+// The end of a right-hand side at one node: Bernoulli from the velocities, energy and drive terms on request, and the
+// RK stage.  q1q is the lower velocity in the rho q1.q2 term.
+__device__ inline void finish_node(const Phys& ph, const StageCtl& ctl, int g, double2 z, double2 zp, double2 zpp,
+                                   double2 q1, double2 q2, double2 q1q, const StageIn& st) {
+    if (ctl.qup) ctl.qup[g] = q2;
+    if (!ph.need_upper) q2 = make_double2(0.0, 0.0);
+    double dphi = bernoulli(ph, z.y, q1, q2, q1q, zp, zpp);
+    if (ctl.energy) energy_store(ph, ctl, g, z.x, z.y, ctl.Pin[g], zp, q1);
+    if (ph.drive) {
+        double dD;
+        dphi = drive_terms(ph, ctl, g, z.x, z.y, q1, dphi, dD);
+        if (ph.augmented) stage_store_delayed(ctl, g, dD);
+    }
+    stage_store(ctl, g, q1, dphi, st);
+}
+
 }  // namespace sfh

@@ -3,16 +3,18 @@
 // One RHS evaluation (BaseBoundaryIntegralCalculator::runTimeStep,
 // CuSuperHelium/BaseBoundaryIntegrator.cuh:137-306) is enqueued as
 //   zphi_circ_kernel      Z', Z'', Re Phi'            (circulant products, 8 or 32 rows per workgroup)
-//   assemble64_kernel     M                           (8 rows per workgroup)
+// and then, with LU,
+//   assemble64_kernel     M
 //   LU solve              mu                          (panel / MFMA update / back substitution)
 //   GEPP fallback         no-op unless a system needed row interchanges
-//     or GMRES            mu                          (one kernel per Arnoldi step; the last
-//                                                      launch also forms mu', gm_close_mu_kernel)
-//   mu_circ_kernel        mu'                         (LU, and GMRES with a one-launch sequence)
+//   mu_circ_kernel        mu'
 //   velocity_stage_kernel q, dPhi/dt and the RK4 stage update of every node
-//     or velocity_gm1_kernel                          (FP64 GMRES sequence of two launches: the
-//                                                      product, then this kernel, which finishes
-//                                                      the step and forms mu and mu' as well)
+// or with GMRES
+//   gm_start_kernel       cotangent sums of the initial guess, first residual
+//   gm_sums_kernel        one launch per Arnoldi step: the sums of a basis vector, of which the product is a combination
+//   gm_close_mu_kernel    mu, mu', the velocity from the sums of the solve, dPhi/dt and the stage update
+// (with the rho quirk, and with sequences of one launch, GMRES runs on the stored matrix: assemble64_kernel or
+// assemble32_kernel, gm_iter_kernel, gm_close_mu_kernel or mu_circ_kernel, velocity_stage_kernel)
 // and one RK4 step (AutonomousRungeKuttaStepper.cuh:123-361) is four of them.  The step is
 // captured once into a hipGraph and replayed, so a run of many steps costs one graph launch
 // per step and the state never leaves HBM.
@@ -24,6 +26,7 @@
 
 #include "sfh_cluster.hpp"
 #include "sfh_gmres.hpp"
+#include "sfh_pairs.hpp"
 #include "solver.hpp"
 
 namespace sfh {
@@ -313,13 +316,30 @@ void Solver::alloc_gmres(int m) {
     // N = 2048 (512 workgroups of 4 rows, two per CU) their longer start costs more than it saves: 26.7 ms per
     // 100 steps with 4 rows, 29.8 with 8 and 28.6 - 31.0 with 16; N = 1536 mixed 18.0, 17.9 and 18.7.
     gm_rpw_ = T_ <= 2048 ? 4 : 16;
-    gm_nwg_ = (maxN_ + gm_rpw_ - 1) / gm_rpw_;
-    gm_part_stride_ = 2LL * gm_nwg_ * (gm_m_ + 1);
+    gm_part_stride_ = 2LL * ((maxN_ + 3) / 4) * (gm_m_ + 1);   // 4: the fewest rows of a workgroup
     gm_small_stride_ = 4LL * (gm_m_ + 1) + 2LL * gm_m_ + (long long)gm_m_ * (gm_m_ + 1);
     gmV_ = dalloc<double>((size_t)(gm_m_ + 1) * T_);
     gmx0_ = dalloc<double>(T_);
     if (ph_.image && opt_.solver == kSolveGMRES) gmZ_ = dalloc<double>((size_t)(gm_m_ + 1) * T_);
-    if (opt_.precision == kMixed && opt_.solver == kSolveGMRES) M32_ = dalloc<float>(MT_);
+    // Products from cotangent sums, which the velocity needs anyway (gm_start_kernel, gm_sums_kernel): the solve stores
+    // no matrix and the right-hand side ends in the solve's closing launch.  Per right-hand side with one Arnoldi step,
+    // microseconds: N = 2048 water 7.5 + 8 + 8.5 in place of assembly 14.2, product 8, closing 8.2 and velocity 10.2;
+    // N = 4096 film 34 + 40 + 17 in place of 38 + 26 + 22 + 33; N = 1536 mixed film 9.4 + 12 + 10 in place of 12 + 5 + 8
+    // + 11 and a refinement (10 + 4 + 8).  FP64 throughout, so a mixed-precision handle needs no refinement.
+    // Not with the rho quirk, whose node-1 term needs mu' outside a workgroup's rows, nor for solves of one launch,
+    // which have no closing one.
+    const bool quirk = ph_.kind == 0 && ph_.rho_quirk && ph_.rho != 0.0;
+    gm_sums_ = opt_.solver == kSolveGMRES && gm_m_ >= 2 && !quirk;
+    if (gm_sums_) {
+        const size_t words = (size_t)(gm_m_ + 1) * (ph_.image ? 4 : 2) * T_;
+        // every workgroup repeats the finishing work of a step: beyond 2048 nodes, where the workgroups of 4 rows no
+        // longer run all at once, two groups of 256 threads share it
+        sums_rpw_ = maxN_ <= 2048 ? 4 : 8;
+        gmS_ = dalloc<double>(words);
+        gmdiag_ = dalloc<double>(T_);
+        SFH_HIP(hipMemset(gmS_, 0, words * sizeof(double)));
+    }
+    if (opt_.precision == kMixed && opt_.solver == kSolveGMRES && !gm_sums_) M32_ = dalloc<float>(MT_);
     SFH_HIP(hipMemset(gmx0_, 0, T_ * sizeof(double)));
     gmw_ = dalloc<double>(2 * (size_t)T_);
     gmpart_ = dalloc<double>(gm_part_stride_ * S_);
@@ -345,7 +365,7 @@ Solver::~Solver() {
     if (graph_) (void)hipGraphDestroy(graph_);
     void* bufs[] = {d_desc_, d_tw_, Z0_, Za_, Zb_, P0_, Pa_, Pb_, kZ_[0], kZ_[1], kZ_[2], kP_[0],
                     kP_[1], kP_[2], Zp_, Zpp_, mup_, qup_, b_, work_, y_, mu_, M_, uinv_, flags_,
-                    status_, piv_, counters_, gmV_, gmZ_, gmw_, gmpart_, gmsmall_, gmctl_, trig_, order_, bstats_, bparts_, bwords_, bxoff_, bxbuf_,
+                    status_, piv_, counters_, gmV_, gmZ_, gmS_, gmdiag_, gmw_, gmpart_, gmsmall_, gmctl_, trig_, order_, bstats_, bparts_, bwords_, bxoff_, bxbuf_,
                     gmhist_, gmhvalid_, bhist_, bhvalid_, d_circ_, gmx0_, M32_, ckZ_, ckP_, ckMu_, ckHist_,
                     ckHv_, energy_, D0_, Da_, Db_, ckD_, kD_[0], kD_[1], kD_[2]};
     for (void* p : bufs)
@@ -444,7 +464,16 @@ GmArgs Solver::gm_args(int stage) const {
     a.hist = gmhist_;
     a.hvalid = gmhvalid_;
     a.stage = stage;
-    a.rpw = gm_rpw_;
+    a.rpw = gm_sums_ ? sums_rpw_ : gm_rpw_;
+    a.sums = gm_sums_ ? (ph_.image ? 4 : 2) : 0;
+    a.S = gmS_;
+    a.diag = gmdiag_;
+    a.trig = trig_;
+    a.Zp = Zp_;
+    a.pc = (ph_.kind == 0 ? 0.25 * (1 - ph_.rho) : 0.25) / kPi;
+    a.pci = 0.25 / kPi;
+    a.eh = std::exp(ph_.depth);
+    a.ehi = std::exp(-ph_.depth);
     a.pre = gmZ_ ? 1 : 0;
     a.Z = gmZ_ ? gmZ_ : gmV_;
     a.tw = d_tw_;
@@ -455,13 +484,12 @@ GmArgs Solver::gm_args(int stage) const {
 // residual comes from the assembly kernel and the final step applies the correction x += V y,
 // so only the fixed-length sequence of steps is launched here.  With two launches or more the
 // last one is gm_close_mu_kernel, which also forms mu' (returns true: no mu_circ_kernel).
-// g1 (a sequence of two launches): only the product launch; velocity_gm1_kernel finishes the solve.
 // Mixed precision runs the products over the FP32 matrix (4 bytes per entry).
-bool Solver::enqueue_gmres(const GmArgs& a, bool g1, bool force64) {
+bool Solver::enqueue_gmres(const GmArgs& a, bool force64, const double2* Z, const StageCtl* sc) {
     const bool f32 = opt_.precision == kMixed && !force64;
     double nsq = 0.0;
     for (int v : n_) nsq += (double)v * v;
-    const dim3 grid(gm_nwg_, 1, S_);
+    const dim3 grid((maxN_ + a.rpw - 1) / a.rpw, 1, S_);
     const size_t first = timed_.size();
     const bool fused = a.m >= 2;
     const int nprod = fused ? a.m - 1 : a.m;
@@ -470,24 +498,30 @@ bool Solver::enqueue_gmres(const GmArgs& a, bool g1, bool force64) {
         // the stored matrix + the partial dots
         launch(
             a.check_first ? "gm_refine" : "gm_iter", 2.0 * nsq + 4.0 * (j + 1) * T_,
-            (f32 ? 4.0 : 8.0) * nsq + 8.0 * (j + 3) * T_,
+            (a.sums ? 0.0 : f32 ? 4.0 : 8.0) * nsq + 8.0 * (j + 3) * T_,
             [&] {
                 auto step = [&](auto kernel, int waves) {
                     go(kernel, grid, dim3(64 * waves), 0, a, (const SurfDesc*)d_desc_, j);
                 };
-                switch (a.rpw) {
+                if (a.sums == 2) {
+                    a.rpw == 4 ? step(gm_sums_kernel<2, 1>, 4) : step(gm_sums_kernel<2, 2>, 8);
+                } else if (a.sums == 4) {
+                    a.rpw == 4 ? step(gm_sums_kernel<4, 1>, 4) : step(gm_sums_kernel<4, 2>, 8);
+                } else switch (a.rpw) {
                 case 4: f32 ? step(gm_iter_kernel<float, 4, 1>, 4) : step(gm_iter_kernel<double, 4, 1>, 4); break;
                 default: f32 ? step(gm_iter_kernel<float, 8, 2>, 8) : step(gm_iter_kernel<double, 8, 2>, 8); break;
                 }
             },
             j);
     }
-    if (fused && !g1) {
-        // finishing the last step + x += V y + mu' = D1 mu: the rebuild and the circulant product
-        launch("gm_close_mu", 4.0 * a.m * T_ + 4.0 * nsq, 8.0 * (a.m + 2) * T_ + 24.0 * nsq / kCircRowsPerWG, [&] {
-            go(a.pre ? gm_close_mu_kernel<true> : gm_close_mu_kernel<false>,
+    if (fused) {
+        // finishing the last step + x += V y + mu' = D1 mu: the rebuild and the circulant product; with the solve's
+        // sums also the velocity and the stage (a sequence of two launches, the steady case, is timed as the velocity
+        // that it ends in)
+        launch(a.sums && a.m == 2 ? "velocity" : "gm_close_mu", 4.0 * a.m * T_ + 4.0 * nsq, 8.0 * (a.m + 2) * T_ + 24.0 * nsq / kCircRowsPerWG, [&] {
+            go(a.sums == 2 ? gm_close_mu_kernel<false, 2> : a.sums == 4 ? gm_close_mu_kernel<true, 4> : gm_close_mu_kernel<false, 0>,
                dim3((maxN_ + kCircRowsPerWG - 1) / kCircRowsPerWG, S_), dim3(256), 0, a, (const SurfDesc*)d_desc_,
-               (const double*)d_circ_, mup_, a.m - 1);
+               (const double*)d_circ_, mup_, a.m - 1, Z, (const double2*)Zpp_, ph_, sc ? *sc : StageCtl{});
         });
     }
     if (ktime_ && !a.check_first) {
@@ -499,11 +533,6 @@ bool Solver::enqueue_gmres(const GmArgs& a, bool g1, bool force64) {
         SFH_HIP(hipMemcpy(ctl.data(), gmctl_, ctl.size() * sizeof(int), hipMemcpyDeviceToHost));
         int iters = 0;
         for (int s = 0; s < S_; ++s) iters = std::max(iters, ctl[(size_t)kGmCtlInts * s + 2]);
-        if (g1) {   // the velocity kernel finishes the step: launch 0 ran a product unless it ended the solve
-            iters = 0;
-            for (int s = 0; s < S_; ++s)
-                if (ctl[(size_t)kGmCtlInts * s] == 0) iters = 1;
-        }
         for (size_t k = first; k < timed_.size(); ++k) {
             if (timed_[k].tag != std::string("gm_iter")) continue;
             if (timed_[k].iter == iters) {
@@ -525,9 +554,9 @@ bool Solver::enqueue_gmres(const GmArgs& a, bool g1, bool force64) {
 //   refinement solve over the FP32 matrix starts from it (it ends at launch 0 when the residual is
 //   already within the tolerance, the usual case).  Only the refinement solve stores the stage's
 //   warm-start history.
-bool Solver::enqueue_solve(const double2* Z, int stage, bool g1) {
+bool Solver::enqueue_solve(const double2* Z, int stage) {
     if (opt_.solver == kSolveGMRES) {
-        if (opt_.precision != kMixed) return enqueue_gmres(gm_args(stage), g1);
+        if (opt_.precision != kMixed) return enqueue_gmres(gm_args(stage));
         GmArgs first = gm_args(stage);
         first.stage = 0;   // no history: the refinement solve stores the solution
         enqueue_gmres(first);
@@ -653,6 +682,15 @@ void Solver::enqueue_rhs(const double2* Z, const double* P, const StageCtl& ctl_
         SFH_WITH_CIRC(maxN_, go(zphi_circ_kernel<TC, TR>, circ_grid(8 * TR), dim3(TC * TR), 0, d_desc_,
                                 (const double*)d_circ_, Z, P, Zp_, Zpp_, b_, work_, ph_, status_, trig_, ga, gm_on));
     });
+    if (gm_sums_) {
+        launch("gm_start", img * nsq, 96.0 * T_, [&] {
+            go(ph_.image ? gm_start_kernel<4> : gm_start_kernel<2>, dim3((maxN_ + kSumRows - 1) / kSumRows, S_), dim3(256), 0,
+               ga, (const SurfDesc*)d_desc_, Z, (const double2*)Zpp_, ph_);
+        });
+        enqueue_gmres(ga, false, Z, &ctl);
+        SFH_HIP(hipGetLastError());
+        return;
+    }
     // assembly: flops counted as cot evaluations (the transcendental-bound unit), bytes = M written
     if (gm_on && opt_.precision == kMixed) {
         launch("assemble", img * nsq, 4.0 * nsq, [&] {
@@ -665,27 +703,16 @@ void Solver::enqueue_rhs(const double2* Z, const double* P, const StageCtl& ctl_
                                     (const NodeTrig*)trig_, Z, Zp_, Zpp_, M_, ph_, (const int*)nullptr, ga, gm_on));
         });
     }
-    // an FP64 GMRES sequence of two launches (one Arnoldi step) ends in the velocity kernel; not
-    // with the rho quirk, whose node-1 term needs mu' outside a workgroup's rows
-    const bool quirk = ph_.kind == 0 && ph_.rho_quirk && ph_.rho != 0.0;
-    const bool g1 = gm_on && opt_.precision != kMixed && ga.m == 2 && !quirk;
-    if (!enqueue_solve(Z, ctl.stage, g1)) {
+    if (!enqueue_solve(Z, ctl.stage)) {
         launch("mu_deriv", 4.0 * nsq, 24.0 * nsq / kCircRowsPerWG, [&] {
             SFH_WITH_CIRC(maxN_, go(mu_circ_kernel<TC, TR>, circ_grid(8 * TR), dim3(TC * TR), 0, d_desc_,
                                     (const double*)d_circ_, (const double*)mu_, mup_));
         });
     }
-    if (g1) {
-        launch("velocity", img * nsq, 96.0 * T_, [&] {
-            SFH_WITH_ROWS(rows_, go(velocity_gm1_kernel<R>, dim3((maxN_ + R - 1) / R, S_), dim3(256), 0, d_desc_,
-                                    (const NodeTrig*)trig_, Z, Zp_, Zpp_, mup_, ph_, ctl, ga, (const double*)d_circ_));
-        });
-    } else {
-        launch("velocity", img * nsq, 96.0 * T_, [&] {
-            SFH_WITH_ROWS(rows_, go(velocity_stage_kernel<R>, dim3((maxN_ + R - 1) / R, S_), dim3(256), 0, d_desc_,
-                                    (const NodeTrig*)trig_, Z, Zp_, Zpp_, mu_, mup_, ph_, ctl));
-        });
-    }
+    launch("velocity", img * nsq, 96.0 * T_, [&] {
+        SFH_WITH_ROWS(rows_, go(velocity_stage_kernel<R>, dim3((maxN_ + R - 1) / R, S_), dim3(256), 0, d_desc_,
+                                (const NodeTrig*)trig_, Z, Zp_, Zpp_, mu_, mup_, ph_, ctl));
+    });
     SFH_HIP(hipGetLastError());
 }
 
@@ -819,6 +846,7 @@ void Solver::calibrate() {
     trim_ = std::max(2, std::min(gm_m_, fill_iters_ >= 3 ? need + 1 : need));
     if (opt_.force_trim > 0) trim_ = std::max(2, std::min(gm_m_, opt_.force_trim));
     chunk_ = 2;
+    chunks_kept_ = 0;
 }
 
 void Solver::save_checkpoint() {
@@ -912,7 +940,9 @@ void Solver::step(double dt, int nsteps) {
                 chunk_ = 2;
             } else {
                 i += chunk;
-                chunk_ = std::min(kCheckSteps, 2 * chunk_);
+                // twice the first length: solves near the tolerance's rounding level differ from step to step, and a
+                // chunk that has to be run again soon after the calibration is then a short one
+                if (++chunks_kept_ > 1) chunk_ = std::min(kCheckSteps, 2 * chunk_);
             }
         }
     }
@@ -1013,6 +1043,7 @@ void Solver::clear_solver_state() {
 
 void Solver::clear_gmres_state() {
     if (opt_.solver == kSolveGMRES) {
+        if (gmS_) SFH_HIP(hipMemsetAsync(gmS_, 0, (size_t)(gm_m_ + 1) * (ph_.image ? 4 : 2) * T_ * sizeof(double), stream_));
         SFH_HIP(hipMemsetAsync(gmx0_, 0, T_ * sizeof(double), stream_));
         SFH_HIP(hipMemsetAsync(gmV_, 0, (size_t)(gm_m_ + 1) * T_ * sizeof(double), stream_));
         if (gmZ_) SFH_HIP(hipMemsetAsync(gmZ_, 0, (size_t)(gm_m_ + 1) * T_ * sizeof(double), stream_));
@@ -1637,7 +1668,9 @@ void Solver::enqueue_vjp_mwg(const double2* Z, const double* P, const double* mu
         g.check_first = 0;
         g.pre = 0;
         g.Z = gmV_;
-        enqueue_gmres(g, false, true);   // leaves s D1 gb in mup_
+        g.sums = 0;
+        g.rpw = gm_rpw_;
+        enqueue_gmres(g, true);   // leaves s D1 gb in mup_
     });
     if (adj_warm_ && stage >= 0) {   // the solution joins the stage's ring
         const int slot = (adj_head_[stage] + 1) % kHistDepth;

@@ -206,7 +206,7 @@ class Solver {
 
   private:
     void enqueue_rhs(const double2* Z, const double* P, const StageCtl& ctl);
-    bool enqueue_solve(const double2* Z, int stage, bool g1);
+    bool enqueue_solve(const double2* Z, int stage);
     // the stage states Y2..Y4 and the four stage mu of one RK4 step, copied out as the step runs
     struct StageCapture {
         double2* Y[3];
@@ -278,14 +278,18 @@ class Solver {
     int* counters_ = nullptr;   // [0] fallback solves
     std::vector<long long> uoff_, foff_;
     // GMRES workspace
-    int gm_m_ = 0, gm_nwg_ = 0, gm_rpw_ = 4;
+    int gm_m_ = 0, gm_rpw_ = 4;
     double* gmZ_ = nullptr;        // film: the preconditioned basis
     double *gmV_ = nullptr, *gmw_ = nullptr, *gmpart_ = nullptr, *gmsmall_ = nullptr;
     double* gmx0_ = nullptr;     // initial guess of the solve in flight (the solution goes to mu_)
+    bool gm_sums_ = false;       // GMRES: products from cotangent sums, no matrix (sfh_pairs.hpp)
+    int sums_rpw_ = 0;           // rows per workgroup of those launches
+    double* gmS_ = nullptr;
+    double* gmdiag_ = nullptr;
     float* M32_ = nullptr;       // FP32 matrices of the mixed-precision GMRES form
     int* gmctl_ = nullptr;
     long long gm_part_stride_ = 0, gm_small_stride_ = 0;
-    bool enqueue_gmres(const GmArgs& a, bool g1 = false, bool force64 = false);
+    bool enqueue_gmres(const GmArgs& a, bool force64 = false, const double2* Z = nullptr, const StageCtl* sc = nullptr);
     void alloc_gmres(int m);
     GmArgs gm_args(int stage) const;
     double* gmhist_ = nullptr;   // 4 x kHistDepth x total: per RK stage, mu of the last steps
@@ -393,6 +397,7 @@ class Solver {
     int trim_ = 0;          // 0: not determined yet
     int hist_steps_ = 0;    // steps since set_state (saturates at kCalibSteps)
     int chunk_ = 2;         // steps of the next trimmed chunk (doubles up to kCheckSteps)
+    int chunks_kept_ = 0;   // trimmed chunks kept since the calibration
     int unc_raw_ = 0;       // unconverged count of the control blocks (discarded chunks included)
     int unc_discard_ = 0;   // ... of solves in chunks that were run again
     int most_ = 0;          // most Arnoldi steps of a solve of the last RK (or reverse) step, any surface
