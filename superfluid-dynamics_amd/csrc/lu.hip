@@ -734,77 +734,8 @@ __global__ __launch_bounds__(kLuThreads) void lu_step_kernel(LuArgs a, int k0) {
     }
 }
 
-// x_p = U_pp^{-1} (y_p - sum_{q>p} U_pq x_q).  Workgroup b handles block row p = P-1-b, so a
-// workgroup only waits for workgroups dispatched before it; every wait is bounded.  Each U_pq
-// block is staged into LDS before the wait for x_q, so only the x_q load and an LDS GEMV sit on
-// the dependency chain.
-__global__ __launch_bounds__(256) void lu_backsolve_kernel(LuArgs a) {
-    __shared__ double Ub[kNB * LD], Ui[kNB * LD];
-    __shared__ double xq[kNB], part[4][kNB], sv[kNB];
-    const LuView v = view(a);
-    const int n = a.n, t = threadIdx.x;
-    const int P = (n + kNB - 1) / kNB;
-    const int p = P - 1 - blockIdx.x;
-    const int R0 = p * kNB, rb = min(kNB, n - R0);
-    const int r = t & 63, chunk = t >> 6;
-    const double* U = v.uinv + (long long)p * kNB * kNB;
-    load_block<256>(Ui, U, kNB, kNB, kNB);
-    double acc = 0.0;
-    for (int q = P - 1; q > p; --q) {
-        const int C0 = q * kNB, cb = min(kNB, n - C0);
-        load_block<256>(Ub, v.A + (long long)R0 * n + C0, n, rb, cb);
-        if (t == 0) {
-            // relaxed polling, one acquire once the flag is seen: on gfx950 every agent-scope
-            // acquire invalidates this XCD's L2, which other workgroups are reading through
-            int spins = 0;
-            while (__hip_atomic_load(&v.flags[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) {
-                __builtin_amdgcn_s_sleep(1);
-                if (++spins > (1 << 22)) {
-                    atomicOr(&v.status[1], 1);
-                    break;
-                }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        }
-        __syncthreads();
-        if (t < kNB) {
-            xq[t] = (t < cb) ? v.x[C0 + t] : 0.0;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int c = 0; c < 16; ++c) acc += Ub[r * LD + chunk * 16 + c] * xq[chunk * 16 + c];
-        __syncthreads();
-    }
-    part[chunk][r] = acc;
-    __syncthreads();
-    if (t < kNB) sv[t] = (t < rb) ? v.y[R0 + t] - (part[0][t] + part[1][t] + part[2][t] + part[3][t]) : 0.0;
-    __syncthreads();
-    {   // x_p = U_pp^{-1} sv, 4 threads per row
-        double s = 0.0;
-#pragma unroll
-        for (int c = 0; c < 16; ++c) s += Ui[r * LD + chunk * 16 + c] * sv[chunk * 16 + c];
-        part[chunk][r] = s;
-    }
-    __syncthreads();
-    if (t < rb) v.x[R0 + t] = part[0][t] + part[1][t] + part[2][t] + part[3][t];
-    __syncthreads();
-    if (t == 0) __hip_atomic_store(&v.flags[p], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Unblocked GEPP (first row of maximal |a|) and solve by one workgroup per surface, run only
-// for surfaces whose interchange-free factorisation reported a multiplier above 1
-// (status[2 s] != 0).  M holds the freshly re-assembled matrix of that surface.
-__global__ __launch_bounds__(256) void gepp_fallback_kernel(const SurfDesc* sd, double* M, const double* bvec,
-                                                            double* xvec, int* pivv, int* status,
-                                                            int* counters) {
-    const int s_ = blockIdx.x;
-    if (status[2 * s_] == 0) return;
-    const SurfDesc dsc = sd[s_];
-    const int n = dsc.n;
-    double* A = M + dsc.moff;
-    const double* b = bvec + dsc.voff;
-    double* x = xvec + dsc.voff;
-    int* piv = pivv + dsc.voff;
+// Unblocked GEPP (first row of maximal |a|) and solve of A x = b by one workgroup of 256 threads.
+__device__ void gepp_solve(int n, double* A, const double* b, double* x, int* piv, int* counters) {
     if (threadIdx.x == 0) atomicAdd(&counters[0], 1);
     __shared__ double rv[256];
     __shared__ int ri[256];
@@ -869,5 +800,116 @@ __global__ __launch_bounds__(256) void gepp_fallback_kernel(const SurfDesc* sd, 
         __syncthreads();
     }
 }
+
+// For a system of its own (A holds it as it was): run only when the interchange-free factorisation reported a
+// multiplier above 1 (status[2 s] != 0).
+__global__ __launch_bounds__(256) void gepp_fallback_kernel(const SurfDesc* sd, double* M, const double* bvec,
+                                                            double* xvec, int* pivv, int* status,
+                                                            int* counters) {
+    const int s_ = blockIdx.x;
+    if (status[2 * s_] == 0) return;
+    const SurfDesc dsc = sd[s_];
+    gepp_solve(dsc.n, M + dsc.moff, bvec + dsc.voff, xvec + dsc.voff, pivv + dsc.voff, counters);
+}
+
+// The stepper's fallback, by one workgroup: the matrix of surface s as assemble64_kernel forms it (createM.cuh:43-92),
+// then the elimination with interchanges.
+__device__ void fallback_solve(const LuFallback& f, int s) {
+    const SurfDesc d = f.sd[s];
+    const int n = d.n;
+    const NodeTrig* tr = f.trig + d.voff;
+    double* A = f.M + d.moff;
+    const bool water = f.ph.kind == 0;
+    const double c = water ? 0.25 * (1 - f.ph.rho) / kPi : 0.25 / kPi, ci = 0.25 / kPi;
+    const double h = f.ph.depth, eh = exp(h), ehi = exp(-h);
+    for (int k = 0; k < n; ++k) {
+        const NodeTrig tk = tr[k];
+        const double2 zp = f.Zp[d.voff + k];
+        for (int j = threadIdx.x; j < n; j += 256) {
+            double v;
+            if (j == k) {
+                v = (water ? 0.5 * (1 + f.ph.rho) : 0.5) + c * cdiv(f.Zpp[d.voff + k], zp).y;
+                if (f.ph.image) v -= ci * cot64(0.0, f.Z[d.voff + k].y + h).y;
+            } else {
+                const CotParts cp = cot_parts(tk, tr[j]);
+                v = cp.id * (c * zp.y * cp.p - c * zp.x * cp.q);
+                if (f.ph.image) {
+                    const CotParts cq = cot_image_parts(tk, tr[j], eh, ehi);
+                    v += ci * (cq.q * cq.id);
+                }
+            }
+            A[(long long)k * n + j] = v;
+        }
+    }
+    __syncthreads();
+    gepp_solve(n, A, f.b + d.voff, f.x + d.voff, f.piv + d.voff, f.counters);
+}
+
+// x_p = U_pp^{-1} (y_p - sum_{q>p} U_pq x_q).  Workgroup b handles block row p = P-1-b, so a
+// workgroup only waits for workgroups dispatched before it; every wait is bounded.  Each U_pq
+// block is staged into LDS before the wait for x_q, so only the x_q load and an LDS GEMV sit on
+// the dependency chain.
+// FALLBACK: when the factorisation needed interchanges, the surface's first workgroup solves its system anew instead
+// (fallback_solve); as launches of their own the two kernels of that cost every solve 9 us to find nothing to do.
+template <bool FALLBACK>
+__global__ __launch_bounds__(256) void lu_backsolve_kernel(LuArgs a, LuFallback f) {
+    __shared__ double Ub[kNB * LD], Ui[kNB * LD];
+    __shared__ double xq[kNB], part[4][kNB], sv[kNB];
+    const LuView v = view(a);
+    const int n = a.n, t = threadIdx.x;
+    const int P = (n + kNB - 1) / kNB;
+    const int p = P - 1 - blockIdx.x;
+    const int R0 = p * kNB, rb = min(kNB, n - R0);
+    const int r = t & 63, chunk = t >> 6;
+    const double* U = v.uinv + (long long)p * kNB * kNB;
+    const int bad = FALLBACK ? v.status[0] : 0;
+    load_block<256>(Ui, U, kNB, kNB, kNB);
+    if (FALLBACK && bad) {
+        if (blockIdx.x == 0) fallback_solve(f, f.first + blockIdx.z);
+        return;
+    }
+    double acc = 0.0;
+    for (int q = P - 1; q > p; --q) {
+        const int C0 = q * kNB, cb = min(kNB, n - C0);
+        load_block<256>(Ub, v.A + (long long)R0 * n + C0, n, rb, cb);
+        if (t == 0) {
+            // relaxed polling, one acquire once the flag is seen: on gfx950 every agent-scope
+            // acquire invalidates this XCD's L2, which other workgroups are reading through
+            int spins = 0;
+            while (__hip_atomic_load(&v.flags[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) {
+                __builtin_amdgcn_s_sleep(1);
+                if (++spins > (1 << 22)) {
+                    atomicOr(&v.status[1], 1);
+                    break;
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        }
+        __syncthreads();
+        if (t < kNB) {
+            xq[t] = (t < cb) ? v.x[C0 + t] : 0.0;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < 16; ++c) acc += Ub[r * LD + chunk * 16 + c] * xq[chunk * 16 + c];
+        __syncthreads();
+    }
+    part[chunk][r] = acc;
+    __syncthreads();
+    if (t < kNB) sv[t] = (t < rb) ? v.y[R0 + t] - (part[0][t] + part[1][t] + part[2][t] + part[3][t]) : 0.0;
+    __syncthreads();
+    {   // x_p = U_pp^{-1} sv, 4 threads per row
+        double s = 0.0;
+#pragma unroll
+        for (int c = 0; c < 16; ++c) s += Ui[r * LD + chunk * 16 + c] * sv[chunk * 16 + c];
+        part[chunk][r] = s;
+    }
+    __syncthreads();
+    if (t < rb) v.x[R0 + t] = part[0][t] + part[1][t] + part[2][t] + part[3][t];
+    __syncthreads();
+    if (t == 0) __hip_atomic_store(&v.flags[p], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+}
+template __global__ void lu_backsolve_kernel<false>(LuArgs, LuFallback);
+template __global__ void lu_backsolve_kernel<true>(LuArgs, LuFallback);
 
 }  // namespace sfh

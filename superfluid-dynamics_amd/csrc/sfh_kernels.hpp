@@ -125,7 +125,7 @@ __global__ void plain_deriv_kernel(const SurfDesc* sd, const double2* tw_all, co
 template <int R>
 __global__ void assemble64_kernel(const SurfDesc* sd, const NodeTrig* trig, const double2* Z,
                                   const double2* Zp, const double2* Zpp, double* M, Phys ph,
-                                  const int* only_if, GmArgs gm, int gm_on);
+                                  GmArgs gm, int gm_on);
 template <int R>
 __global__ void assemble32_kernel(const SurfDesc* sd, const NodeTrig* trig, const double2* Z,
                                   const double2* Zp, const double2* Zpp, float* M, Phys ph, GmArgs gm);
@@ -164,7 +164,21 @@ inline int lu_step_grid(int nrb, int k0, int count) {
     return 1 + 2 * nrb + (tiles < share ? tiles : share);
 }
 __global__ void lu_step_kernel(LuArgs a, int k0);
-__global__ void lu_backsolve_kernel(LuArgs a);
+// What the back substitution needs to solve a surface's system anew with interchanges.
+struct LuFallback {
+    const SurfDesc* sd;
+    const NodeTrig* trig;
+    const double2 *Z, *Zp, *Zpp;
+    double* M;
+    const double* b;
+    double* x;
+    int* piv;
+    int* counters;   // [0]: fallback solves
+    int first;       // surface of the batch's first system
+    Phys ph;
+};
+template <bool FALLBACK>
+__global__ void lu_backsolve_kernel(LuArgs a, LuFallback f);
 __global__ void gepp_fallback_kernel(const SurfDesc* sd, double* M, const double* b, double* x,
                                      int* piv, int* status, int* counters);
 

@@ -6,7 +6,7 @@
 // and then, with LU,
 //   assemble64_kernel     M
 //   LU solve              mu                          (panel / MFMA update / back substitution)
-//   GEPP fallback         no-op unless a system needed row interchanges
+//                         (a system that needs row interchanges is solved anew by the back substitution's launch)
 //   mu_circ_kernel        mu'
 //   velocity_stage_kernel q, dPhi/dt and the RK4 stage update of every node
 // or with GMRES
@@ -596,7 +596,8 @@ bool Solver::enqueue_solve(const double2* Z, int stage) {
         }
         const int P = (n + kNB - 1) / kNB;
         launch("lu_backsolve", (double)count * n * n, 8.0 * count * 0.5 * n * n, [&] {
-            go(lu_backsolve_kernel, dim3(P, 1, count), dim3(256), 0, a);
+            LuFallback f{d_desc_, trig_, Z, Zp_, Zpp_, M_, b_, mu_, piv_, counters_, s0, ph_};
+            go(lu_backsolve_kernel<true>, dim3(P, 1, count), dim3(256), 0, a, f);
         });
     };
     if (uniform_) {
@@ -604,11 +605,6 @@ bool Solver::enqueue_solve(const double2* Z, int stage) {
     } else {
         for (int s = 0; s < S_; ++s) run(s, 1, n_[s]);
     }
-    // systems whose interchange-free check failed: re-assemble and solve with GEPP
-    go(assemble64_kernel<kPairRows>, dim3((maxN_ + kPairRows - 1) / kPairRows, S_), dim3(256), 0, d_desc_,
-       (const NodeTrig*)trig_, Z, Zp_, Zpp_, M_, ph_, (const int*)status_, GmArgs{}, 0);
-    go(gepp_fallback_kernel, dim3(S_), dim3(256), 0, d_desc_, M_, b_, mu_, piv_,
-                       status_, counters_);
     return false;
 }
 
@@ -700,7 +696,7 @@ void Solver::enqueue_rhs(const double2* Z, const double* P, const StageCtl& ctl_
     } else {
         launch("assemble", img * nsq, 8.0 * nsq, [&] {
             SFH_WITH_ROWS(rows_, go(assemble64_kernel<R>, dim3((maxN_ + R - 1) / R, S_), dim3(256), 0, d_desc_,
-                                    (const NodeTrig*)trig_, Z, Zp_, Zpp_, M_, ph_, (const int*)nullptr, ga, gm_on));
+                                    (const NodeTrig*)trig_, Z, Zp_, Zpp_, M_, ph_, ga, gm_on));
         });
     }
     if (!enqueue_solve(Z, ctl.stage)) {
@@ -1468,7 +1464,7 @@ void debug_lu_solve(int n_in, const double* A_in, const double* b_in, double* x_
         hipLaunchKernelGGL(lu_step_kernel, dim3(lu_step_grid(nrb, k0, 1), 1, 1), dim3(kLuThreads), 0, st,
                            a, k0);
     }
-    hipLaunchKernelGGL(lu_backsolve_kernel, dim3(P, 1, 1), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(lu_backsolve_kernel<false>, dim3(P, 1, 1), dim3(256), 0, st, a, LuFallback{});
     SFH_HIP(hipGetLastError());
     int status[2];
     SFH_HIP(hipMemcpyAsync(status, dstatus, sizeof(status), hipMemcpyDeviceToHost, st));
@@ -1636,7 +1632,7 @@ void Solver::enqueue_vjp_mwg(const double2* Z, const double* P, const double* mu
     // M^T gb = gmu
     launch("vjp_solve", 2.0 * gm_m_ * nsq, 8.0 * gm_m_ * nsq, [&] {
         go(assemble64_kernel<kPairRows>, dim3((maxN_ + kPairRows - 1) / kPairRows, S_), dim3(256), 0, d_desc_,
-           (const NodeTrig*)trig_, Z, Zp_, Zpp_, M_, ph_, (const int*)nullptr, GmArgs{}, 0);
+           (const NodeTrig*)trig_, Z, Zp_, Zpp_, M_, ph_, GmArgs{}, 0);
         go(transpose_kernel, dim3((maxN_ + 31) / 32, (maxN_ + 31) / 32, S_), dim3(256), 0, d_desc_, (const double*)M_,
            Mt_);
         // inside a trajectory sweep: the guess extrapolated from this stage's solutions of the previous
