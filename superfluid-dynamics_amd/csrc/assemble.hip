@@ -146,6 +146,54 @@ __global__ __launch_bounds__(256) void residual64_kernel(const SurfDesc* __restr
     assemble_rows<double, R>(sd, trig, Z, Zp, Zpp, static_cast<double*>(nullptr), ph, gm, 1, true);
 }
 
+// Surfaces of up to 256 nodes (LU): a wave has 4 rows and all their columns, 16 entries per lane, and only the rows' own
+// lanes form the diagonal.  With 256 threads across the columns a workgroup had 4 entries per thread and was mostly
+// first loads and row constants: 64 surfaces of 256 nodes 34 us with assemble64_kernel<4>, 16 here.
+__global__ __launch_bounds__(256) void assemble_small_kernel(const SurfDesc* __restrict__ sd, const NodeTrig* __restrict__ trig,
+                                                             const double2* __restrict__ Z, const double2* __restrict__ Zp,
+                                                             const double2* __restrict__ Zpp, double* __restrict__ M, Phys ph) {
+    const SurfDesc d = sd[blockIdx.y];
+    const int n = d.n, lane = threadIdx.x & 63;
+    const int k0 = blockIdx.x * kSmallRows + 4 * (threadIdx.x >> 6);
+    if (k0 >= n) return;
+    const NodeTrig* tr = trig + d.voff;
+    double* Mk = M + d.moff + (long long)k0 * n;
+    const double c = ph.kind == 0 ? 0.25 * (1 - ph.rho) / kPi : 0.25 / kPi, ci = 0.25 / kPi;
+    const double h = ph.depth, eh = exp(h), ehi = exp(-h);
+    NodeTrig tk[4], tj[4];
+    double2 zk[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tj[e] = tr[min(lane + 64 * e, n - 1)];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        tk[r] = tr[min(k0 + r, n - 1)];
+        zk[r] = Zp[d.voff + min(k0 + r, n - 1)];
+    }
+    if (lane < 4 && k0 + lane < n) {
+        const int g = d.voff + k0 + lane;
+        double v = (ph.kind == 0 ? 0.5 * (1 + ph.rho) : 0.5) + c * cdiv(Zpp[g], Zp[g]).y;
+        if (ph.image) v -= ci * cot64(0.0, Z[g].y + h).y;
+        Mk[(long long)lane * n + k0 + lane] = v;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int j = lane + 64 * e;
+        if (j >= n) break;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (k0 + r >= n) break;
+            if (j == k0 + r) continue;
+            const CotParts cp = cot_parts(tk[r], tj[e]);
+            double v = cp.id * (c * zk[r].y * cp.p - c * zk[r].x * cp.q);
+            if (ph.image) {
+                const CotParts cq = cot_image_parts(tk[r], tj[e], eh, ehi);
+                v += ci * (cq.q * cq.id);
+            }
+            Mk[(long long)r * n + j] = v;
+        }
+    }
+}
+
 // rows per workgroup the solver may launch with (chosen per surface size by the autotuner)
 #define SFH_ASSEMBLE_INSTANCES(R)                                                                             \
     template __global__ void assemble64_kernel<R>(const SurfDesc*, const NodeTrig*, const double2*, const double2*, \

@@ -120,6 +120,13 @@ constexpr int kDerivThreads = 1024;
 __global__ void plain_deriv_kernel(const SurfDesc* sd, const double2* tw_all, const double2* in,
                                    double2* out, int second, double scale, int lds_tw);
 
+constexpr int kSmallNodes = 256;   // surfaces whose pair kernels give each wave whole rows (LU)
+constexpr int kSmallRows = 16;     // rows per workgroup of those
+__global__ void assemble_small_kernel(const SurfDesc* sd, const NodeTrig* trig, const double2* Z, const double2* Zp,
+                                      const double2* Zpp, double* M, Phys ph);
+template <int NA>
+__global__ void velocity_small_kernel(const SurfDesc* sd, const NodeTrig* trig, const double2* Z, const double2* Zp,
+                                      const double2* Zpp, const double* mu, const double2* mup, Phys ph, StageCtl ctl);
 // ---- assemble.hip
 // R = rows per workgroup: 1, 2 or 4 (instantiated in assemble.hip)
 template <int R>

@@ -688,7 +688,14 @@ void Solver::enqueue_rhs(const double2* Z, const double* P, const StageCtl& ctl_
         return;
     }
     // assembly: flops counted as cot evaluations (the transcendental-bound unit), bytes = M written
-    if (gm_on && opt_.precision == kMixed) {
+    const bool quirk = ph_.kind == 0 && ph_.rho_quirk && ph_.rho != 0.0;
+    const bool small = !gm_on && maxN_ <= kSmallNodes;
+    const dim3 sgrid((maxN_ + kSmallRows - 1) / kSmallRows, S_);
+    if (small) {
+        launch("assemble", img * nsq, 8.0 * nsq, [&] {
+            go(assemble_small_kernel, sgrid, dim3(256), 0, d_desc_, (const NodeTrig*)trig_, Z, Zp_, Zpp_, M_, ph_);
+        });
+    } else if (gm_on && opt_.precision == kMixed) {
         launch("assemble", img * nsq, 4.0 * nsq, [&] {
             SFH_WITH_ROWS(rows_, go(assemble32_kernel<R>, dim3((maxN_ + R - 1) / R, S_), dim3(256), 0, d_desc_,
                                     (const NodeTrig*)trig_, Z, Zp_, Zpp_, M32_, ph_, ga));
@@ -706,7 +713,11 @@ void Solver::enqueue_rhs(const double2* Z, const double* P, const StageCtl& ctl_
         });
     }
     launch("velocity", img * nsq, 96.0 * T_, [&] {
-        SFH_WITH_ROWS(rows_, go(velocity_stage_kernel<R>, dim3((maxN_ + R - 1) / R, S_), dim3(256), 0, d_desc_,
+        if (small && !quirk)
+            go(ph_.image ? velocity_small_kernel<4> : velocity_small_kernel<2>, sgrid, dim3(256), 0, d_desc_,
+               (const NodeTrig*)trig_, Z, Zp_, Zpp_, mu_, mup_, ph_, ctl);
+        else
+            SFH_WITH_ROWS(rows_, go(velocity_stage_kernel<R>, dim3((maxN_ + R - 1) / R, S_), dim3(256), 0, d_desc_,
                                 (const NodeTrig*)trig_, Z, Zp_, Zpp_, mu_, mup_, ph_, ctl));
     });
     SFH_HIP(hipGetLastError());

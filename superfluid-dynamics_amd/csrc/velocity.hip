@@ -18,7 +18,7 @@
 //
 // GMRES solves with products from cotangent sums form S_k themselves and finish in gm_close_mu_kernel; this kernel
 // is for LU, and for GMRES with the stored matrix.
-#include "sfh_kernels.hpp"
+#include "sfh_circ.hpp"
 #include "sfh_physics.hpp"
 
 namespace sfh {
@@ -153,6 +153,79 @@ __global__ __launch_bounds__(256) void velocity_stage_kernel(const SurfDesc* __r
     }
     finish_node(ph, ctl, d.voff + k0 + t, z_t, zp_t, zpp_t, q1, q2, q1q, st);
 }
+
+// Surfaces of up to 256 nodes, not with the rho quirk: a wave has 4 rows and all their columns, 16 pairs per lane, and its
+// own sums.  With 256 threads across the columns a workgroup had 4 pairs per thread and was mostly first loads, reductions
+// and the rows' end: 64 surfaces of 256 nodes 39 us with velocity_stage_kernel<4>, 16 here.
+template <int NA>
+__global__ __launch_bounds__(256) void velocity_small_kernel(const SurfDesc* __restrict__ sd, const NodeTrig* __restrict__ trig,
+                                                             const double2* __restrict__ Z, const double2* __restrict__ Zp,
+                                                             const double2* __restrict__ Zpp, const double* __restrict__ mu,
+                                                             const double2* __restrict__ mup, Phys ph, StageCtl ctl) {
+    __shared__ double red[4][4 * NA];
+    const SurfDesc d = sd[blockIdx.y];
+    const int n = d.n, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int k0 = blockIdx.x * kSmallRows + 4 * w;
+    if (blockIdx.x * kSmallRows >= n) return;   // the whole workgroup: the waves meet below
+    const NodeTrig* tr = trig + d.voff;
+    const double eh = exp(ph.depth), ehi = exp(-ph.depth);
+    NodeTrig tk[4], tj[4];
+    double mj[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int j = min(lane + 64 * e, n - 1);
+        tj[e] = tr[j];
+        mj[e] = mu[d.voff + j];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) tk[r] = tr[min(k0 + r, n - 1)];
+    const int k = k0 + lane, g = d.voff + min(k, n - 1);
+    const bool own = lane < 4 && k < n;
+    double2 zp = {1.0, 0.0}, zpp = {0.0, 0.0}, mp = {0.0, 0.0}, z = {0.0, 0.0};
+    double m = 0.0;
+    StageIn st{};
+    if (own) {
+        zp = Zp[g];
+        zpp = Zpp[g];
+        z = Z[g];
+        st = stage_load(ctl, g);
+        mp = mup[g];
+        m = mu[g];
+    }
+    double acc[4 * NA];
+#pragma unroll
+    for (int q = 0; q < 4 * NA; ++q) acc[q] = 0.0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int j = lane + 64 * e;
+        if (j >= n) break;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (j == k0 + r) continue;
+            const CotParts cp = cot_parts(tk[r], tj[e]);
+            const double v = mj[e] * cp.id;
+            acc[r] += v * cp.p;
+            acc[4 + r] -= v * cp.q;
+            if constexpr (NA == 4) {
+                const CotParts cq = cot_image_parts(tk[r], tj[e], eh, ehi);
+                const double vi = mj[e] * cq.id;
+                acc[8 + r] += vi * cq.p;
+                acc[12 + r] -= vi * cq.q;
+            }
+        }
+    }
+    reduce_lanes(acc, red[w]);
+    __syncthreads();
+    if (!own) return;
+    const double* S = red[w] + lane;
+    double2 q1, q2;
+    velocity_from_sums(ph, zp, zpp, mp, m, z.y, S[0], S[4], NA == 4 ? S[NA == 4 ? 8 : 0] : 0.0, NA == 4 ? S[NA == 4 ? 12 : 0] : 0.0, q1, q2);
+    finish_node(ph, ctl, g, z, zp, zpp, q1, q2, q1, st);
+}
+template __global__ void velocity_small_kernel<2>(const SurfDesc*, const NodeTrig*, const double2*, const double2*, const double2*,
+                                                  const double*, const double2*, Phys, StageCtl);
+template __global__ void velocity_small_kernel<4>(const SurfDesc*, const NodeTrig*, const double2*, const double2*, const double2*,
+                                                  const double*, const double2*, Phys, StageCtl);
 
 // rows per workgroup the solver may launch with (chosen per surface size by the autotuner)
 #define SFH_VELOCITY_INSTANCES(R)                                                                                  \
