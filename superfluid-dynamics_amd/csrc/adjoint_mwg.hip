@@ -7,12 +7,13 @@
 //                       gZ'' and the Bernoulli term's gz)
 //   adj_circ_d1_kernel  D1 of the cotangent of mu' (D1^H = -D1)
 //   adj_pass_b_kernel   per row: P3 (the film's Q) -> gmu, the right-hand side of M^T gb = gmu
-//   transpose_kernel    M^T of the re-assembled M; the GMRES launch sequence of the forward path then
-//                       solves for gb (its closing launch also forms s D1 gb)
+//   gm_tstart_kernel, gm_tsums_kernel   the GMRES launch sequence of the forward path, its products M^T v from sums
+//                       over the pairs, solves for gb (its closing launch also forms s D1 gb)
 //   adj_gamma_kernel    the matrix terms and the pair weights gamma (the film's gammaI)
 //   adj_pass_c_kernel   per row: P2 (the film's PI2) -> gz
 //   adj_final_kernel    gZ += -s D1 gZ' + s^2 D2 gZ'', gPhi = -s Re D1 gb; output, accumulation
-// The pair kernels take R rows per workgroup over all columns, as the forward velocity kernel does.
+// The pair kernels take R rows per workgroup over all columns, kAdjCols columns' loads of a thread in flight together.
+// They and the small kernels between them are bound by first loads and reductions at N = 1024, 3 to 8 us each.
 #include "sfh_gmres.hpp"
 #include "sfh_physics.hpp"
 
@@ -54,48 +55,71 @@ __global__ __launch_bounds__(256) void adj_pass_a_kernel(AdjMArgs a, Phys ph) {
     double acc[NV];
 #pragma unroll
     for (int q = 0; q < NV; ++q) acc[q] = 0.0;
-    for (int j = t; j < n; j += 256) {
-        const NodeTrig tj = a.trig[off + j];
-        const double mj = a.mu[off + j];
+    // the rows' own inputs, before the sweep
+    const int g = off + min(k0 + min(t, R - 1), n - 1);
+    double2 zp = {1.0, 0.0}, zpp = {0.0, 0.0}, mup = zpp, kqz = zpp, z = zpp;
+    double mu = 0.0, kp = 0.0;
+    if (t < R) {
+        zp = a.Zp[g];
+        zpp = a.Zpp[g];
+        mup = a.mup[g];
+        mu = a.mu[g];
+        z = a.Z[g];
+        kqz = cscale(a.gA_Z[g], a.ca);
+        kp = a.ca * a.gA_P[g];
+        if (a.gB_Z) {
+            kqz = cadd(kqz, cscale(a.gB_Z[g], a.cb));
+            kp += a.cb * a.gB_P[g];
+        }
+    }
+    for (int j0 = t; j0 < n; j0 += 256 * kAdjCols) {
+        NodeTrig tc[kAdjCols];
+        double mc[kAdjCols];
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int k = k0 + r;
-            if (k >= n) break;
-            double* v = acc + 8 * r;
-            if (pk.image) {
-                const double2 e = cot_image(tk[r], tj, pk.eh, pk.ehi);
-                v[4] += mj * e.x;
-                v[5] += mj * e.y;
-                v[6] += mj * (1.0 + e.x * e.x - e.y * e.y);
-                v[7] += mj * (2.0 * e.x * e.y);
+        for (int e = 0; e < kAdjCols; ++e) {
+            tc[e] = a.trig[off + min(j0 + 256 * e, n - 1)];
+            mc[e] = a.mu[off + min(j0 + 256 * e, n - 1)];
+        }
+#pragma unroll
+        for (int e = 0; e < kAdjCols; ++e) {
+            const int j = j0 + 256 * e;
+            if (j >= n) break;
+            const NodeTrig tj = tc[e];
+            const double mj = mc[e];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int k = k0 + r;
+                if (k >= n) break;
+                double* v = acc + 8 * r;
+                if (pk.image) {
+                    const double2 e = cot_image(tk[r], tj, pk.eh, pk.ehi);
+                    v[4] += mj * e.x;
+                    v[5] += mj * e.y;
+                    v[6] += mj * (1.0 + e.x * e.x - e.y * e.y);
+                    v[7] += mj * (2.0 * e.x * e.y);
+                }
+                if (j == k) continue;
+                const double2 c = cot_pair(tk[r], tj);
+                v[0] += mj * c.x;
+                v[1] += mj * c.y;
+                v[2] += mj * (1.0 + c.x * c.x - c.y * c.y);
+                v[3] += mj * (2.0 * c.x * c.y);
             }
-            if (j == k) continue;
-            const double2 c = cot_pair(tk[r], tj);
-            v[0] += mj * c.x;
-            v[1] += mj * c.y;
-            v[2] += mj * (1.0 + c.x * c.x - c.y * c.y);
-            v[3] += mj * (2.0 * c.x * c.y);
         }
     }
     rows_reduce<NV>(acc, red, sums);
     if (t >= R || k0 + t >= n) return;
-    const int g = off + k0 + t;
     const double* sv = sums + 8 * t;
     const double q4 = 0.25 / kPi;
-    const double2 zp = a.Zp[g], zpp = a.Zpp[g], mup = a.mup[g];
-    const double mu = a.mu[g];
+    // M_kk (createM.cuh:52-58, :87), for the transposed solve
+    a.diag[g] = (ph.kind == 0 ? 0.5 * (1 + ph.rho) : 0.5) + pk.c * cdiv(zpp, zp).y -
+                (pk.image ? pk.ci * cot64(0.0, z.y + ph.depth).y : 0.0);
     const double2 izp = crecip(zp), izp2 = cmul(izp, izp);
     const double2 V2 = ctimes_i(cscale(izp, 1.0 / (2.0 * kPi)));
     const double2 V1 = cadd(ctimes_i(cscale(cmul(zpp, izp2), -q4)), cscale(izp, 0.5));
     double2 w = cadd(cadd(cmul(V2, mup), cscale(V1, mu)), ctimes_i(make_double2(-q4 * sv[0], -q4 * sv[1])));
     if (pk.image) w = cadd(w, ctimes_i(make_double2(q4 * sv[4], q4 * sv[5])));
     const double2 q1 = cconj(w), q2 = cconj(csub(w, cscale(izp, mu)));   // lower and upper velocities
-    double2 kqz = cscale(a.gA_Z[g], a.ca);
-    double kp = a.ca * a.gA_P[g];
-    if (a.gB_Z) {
-        kqz = cadd(kqz, cscale(a.gB_Z[g], a.cb));
-        kp += a.cb * a.gB_P[g];
-    }
     // under the V1[1] quirk node 1's x velocity is not known here: its terms are added by
     // adj_rho_quirk_kernel from the values kept in a.quirk
     const bool quirk = ph.kind == 0 && ph.rho != 0.0 && ph.rho_quirk && n > 1;
@@ -111,7 +135,7 @@ __global__ __launch_bounds__(256) void adj_pass_a_kernel(AdjMArgs a, Phys ph) {
     A.gzp = vj.gzp;
     A.gzpp = vj.gzpp;
     curvature_vjp(ph, zp, zpp, kp, A.gzp, A.gzpp);
-    A.gz = bernoulli_gz(ph, a.Z[g].x, a.Z[g].y, kp);
+    A.gz = bernoulli_gz(ph, z.x, z.y, kp);
     A.gw = vj.gw;
     A.p1 = make_double2(sv[2], sv[3]);
     A.S = make_double2(sv[0], sv[1]);
@@ -192,6 +216,7 @@ __global__ __launch_bounds__(256) void adj_circ_d1_kernel(const SurfDesc* __rest
     const double* c1r = circ + d.coff;
     const double* c1i = c1r + n;
     double ax = 0.0, ay = 0.0;
+#pragma unroll 8   // the loads of eight columns in flight
     for (int j = lane; j < n; j += 64) {
         int q = k - j;
         if (q < 0) q += n;
@@ -222,20 +247,32 @@ __global__ __launch_bounds__(256) void adj_pass_b_kernel(AdjMArgs a, Phys ph) {
     double acc[NV];
 #pragma unroll
     for (int q = 0; q < NV; ++q) acc[q] = 0.0;
-    for (int k = t; k < n; k += 256) {
-        const NodeTrig tk = a.trig[off + k];
-        const double2 wk = a.gwc[off + k];   // conj(gw_k)
+    for (int c0 = t; c0 < n; c0 += 256 * kAdjCols) {
+        NodeTrig tc[kAdjCols];
+        double2 wc[kAdjCols];
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int j = j0 + r;
-            if (j >= n) break;
-            if (pk.image) {
-                const double2 e = cot_image(tj[r], tk, pk.eh, pk.ehi);
-                acc[2 * r + 1] += wk.x * e.y - wk.y * e.x;   // Im(gw_k e_jk)
+        for (int e = 0; e < kAdjCols; ++e) {
+            tc[e] = a.trig[off + min(c0 + 256 * e, n - 1)];
+            wc[e] = a.gwc[off + min(c0 + 256 * e, n - 1)];
+        }
+#pragma unroll
+        for (int e = 0; e < kAdjCols; ++e) {
+            const int k = c0 + 256 * e;
+            if (k >= n) break;
+            const NodeTrig tk = tc[e];
+            const double2 wk = wc[e];   // conj(gw_k)
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int j = j0 + r;
+                if (j >= n) break;
+                if (pk.image) {
+                    const double2 e = cot_image(tj[r], tk, pk.eh, pk.ehi);
+                    acc[2 * r + 1] += wk.x * e.y - wk.y * e.x;   // Im(gw_k e_jk)
+                }
+                if (k == j) continue;
+                const double2 c = cot_pair(tj[r], tk);
+                acc[2 * r] += wk.x * c.y + wk.y * c.x;           // Im(conj(gw_k) c_jk)
             }
-            if (k == j) continue;
-            const double2 c = cot_pair(tj[r], tk);
-            acc[2 * r] += wk.x * c.y + wk.y * c.x;           // Im(conj(gw_k) c_jk)
         }
     }
     rows_reduce<NV>(acc, red, sums);
@@ -278,58 +315,6 @@ __global__ __launch_bounds__(256) void adj_extrapolate_kernel(const double* __re
         h[l] = l < hv ? ring[(long long)slot * total + i] : 0.0;
     }
     x0[i] = extrapolate_values(h, hv);
-}
-
-// The GMRES launch sequence on M^T from the warm start x0: V[0] = b - M^T x0 (one wave per row of the
-// explicit M^T, 4 rows per workgroup), x = x0, and the control block re-armed.
-__global__ __launch_bounds__(256) void adj_gm_start_warm_kernel(const SurfDesc* __restrict__ sd,
-                                                                const double* __restrict__ Mt,
-                                                                const double* __restrict__ b,
-                                                                const double* __restrict__ x0,
-                                                                double* __restrict__ V, double* __restrict__ x,
-                                                                int* __restrict__ ctl, int m, int reset) {
-    const SurfDesc d = sd[blockIdx.y];
-    const int n = d.n, lane = threadIdx.x & 63;
-    const int k = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        GmCtl* c = reinterpret_cast<GmCtl*>(ctl) + blockIdx.y;
-        c->done = 0;
-        c->refine_iters = 0;
-        c->iters = 0;
-        if (reset) c->most = 0;
-    }
-    if (k >= n) return;   // the whole wave
-    const double* row = Mt + d.moff + (long long)k * n;
-    const double* xs = x0 + d.voff;
-    double acc = 0.0;
-    for (int j = lane; j < n; j += 64) acc += row[j] * xs[j];
-    acc = wave_sum(acc);
-    if (lane == 0) {
-        V[(long long)(m + 1) * d.voff + k] = b[d.voff + k] - acc;
-        x[d.voff + k] = xs[k];
-    }
-}
-
-// Mt = M^T per surface, through 32 x 32 LDS tiles.
-__global__ __launch_bounds__(256) void transpose_kernel(const SurfDesc* __restrict__ sd, const double* __restrict__ M,
-                                                        double* __restrict__ Mt) {
-    __shared__ double tile[32][33];
-    const SurfDesc d = sd[blockIdx.z];
-    const int n = d.n;
-    const int bx = blockIdx.x * 32, by = blockIdx.y * 32;
-    if (bx >= n || by >= n) return;   // the whole workgroup
-    const double* A = M + d.moff;
-    double* B = Mt + d.moff;
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-    for (int r = ty; r < 32; r += 8) {
-        const int row = by + r, col = bx + tx;
-        if (row < n && col < n) tile[r][tx] = A[(long long)row * n + col];
-    }
-    __syncthreads();
-    for (int r = ty; r < 32; r += 8) {
-        const int row = bx + r, col = by + tx;
-        if (row < n && col < n) B[(long long)row * n + col] = tile[tx][r];
-    }
 }
 
 // The matrix terms (off-diagonal gZ'_k -= i c gb_k conj(S_k), the diagonal M_kk's Z' and Z'') and the
@@ -379,25 +364,38 @@ __global__ __launch_bounds__(256) void adj_pass_c_kernel(AdjMArgs a, Phys ph) {
     double acc[NV];
 #pragma unroll
     for (int q = 0; q < NV; ++q) acc[q] = 0.0;
-    for (int k = t; k < n; k += 256) {
-        const NodeTrig tk = a.trig[off + k];
-        const double2 gk = a.gam[off + k];
-        const double2 gi = pk.image ? a.gamI[off + k] : make_double2(0.0, 0.0);
+    for (int c0 = t; c0 < n; c0 += 256 * kAdjCols) {
+        NodeTrig tc[kAdjCols];
+        double2 gc[kAdjCols], ic[kAdjCols];
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int j = j0 + r;
-            if (j >= n) break;
-            if (pk.image) {
-                const double2 e = cot_image(tj[r], tk, pk.eh, pk.ehi);
-                const double ex = 1.0 + e.x * e.x - e.y * e.y, ey = 2.0 * e.x * e.y;
-                acc[2 * r] += gi.x * ex - gi.y * ey;
-                acc[2 * r + 1] += gi.x * ey + gi.y * ex;
+        for (int e = 0; e < kAdjCols; ++e) {
+            const int c = off + min(c0 + 256 * e, n - 1);
+            tc[e] = a.trig[c];
+            gc[e] = a.gam[c];
+            ic[e] = pk.image ? a.gamI[c] : make_double2(0.0, 0.0);
+        }
+#pragma unroll
+        for (int e = 0; e < kAdjCols; ++e) {
+            const int k = c0 + 256 * e;
+            if (k >= n) break;
+            const NodeTrig tk = tc[e];
+            const double2 gk = gc[e], gi = ic[e];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int j = j0 + r;
+                if (j >= n) break;
+                if (pk.image) {
+                    const double2 e = cot_image(tj[r], tk, pk.eh, pk.ehi);
+                    const double ex = 1.0 + e.x * e.x - e.y * e.y, ey = 2.0 * e.x * e.y;
+                    acc[2 * r] += gi.x * ex - gi.y * ey;
+                    acc[2 * r + 1] += gi.x * ey + gi.y * ex;
+                }
+                if (k == j) continue;
+                const double2 c = cot_pair(tj[r], tk);
+                const double ex = 1.0 + c.x * c.x - c.y * c.y, ey = 2.0 * c.x * c.y;
+                acc[2 * r] += gk.x * ex - gk.y * ey;
+                acc[2 * r + 1] += gk.x * ey + gk.y * ex;
             }
-            if (k == j) continue;
-            const double2 c = cot_pair(tj[r], tk);
-            const double ex = 1.0 + c.x * c.x - c.y * c.y, ey = 2.0 * c.x * c.y;
-            acc[2 * r] += gk.x * ex - gk.y * ey;
-            acc[2 * r + 1] += gk.x * ey + gk.y * ex;
         }
     }
     rows_reduce<NV>(acc, red, sums);
@@ -420,6 +418,7 @@ __global__ __launch_bounds__(256) void adj_final_kernel(AdjMArgs a, const double
     const double* c1i = c1r + n;
     const double* c2 = c1i + n;
     double ax = 0.0, ay = 0.0, bx = 0.0, by = 0.0;
+#pragma unroll 8   // the loads of eight columns in flight
     for (int j = lane; j < n; j += 64) {
         int q = k - j;
         if (q < 0) q += n;

@@ -369,6 +369,62 @@ struct PairSums {
     }
 };
 
+// The transposed product (reverse mode), one sum per row, nothing kept.
+template <bool FILM>
+struct TransposeSums {
+    static constexpr int W = 4, ROWS = kSumRows;
+    const NodeTrig* tr;
+    const double2* zp;
+    NodeTrig tk[kSumRows];
+    SumConst kc;
+    double diag;
+    int n, r0;
+    __device__ TransposeSums(const GmArgs& a, const GmView& v, const SurfDesc& d, int first) {
+        n = v.n;
+        r0 = first;
+        tr = a.trig + d.voff;
+        zp = a.Zp + d.voff;
+        kc = {a.pc, a.pci, a.eh, a.ehi};
+        diag = a.diag[d.voff + min(r0 + (int)threadIdx.x, n - 1)];
+    }
+    __device__ void start() {
+#pragma unroll
+        for (int r = 0; r < kSumRows; ++r) tk[r] = tr[min(r0 + r, n - 1)];
+    }
+    // (M^T v) of row r0 + t on threads t < ROWS, 0 beyond the surface
+    template <class F>
+    __device__ double product(F&& value) {
+        __shared__ double red[W][kSumRows];
+        const int t = threadIdx.x;
+        double acc[kSumRows] = {};
+        for (int j0 = 0; j0 < n; j0 += kSumPass) {
+            NodeTrig tj[kSumCols];
+            double2 zj[kSumCols];
+            sum_columns(tr, n, j0, t, tj);
+#pragma unroll
+            for (int e = 0; e < kSumCols; ++e) zj[e] = zp[min(j0 + t + 256 * e, n - 1)];
+            transpose_pass<FILM>(tk, tj, zj, n, r0, j0, t, kc.c, kc.ci, kc.eh, kc.ehi, value, acc);
+        }
+        reduce_lanes(acc, red[t >> 6]);
+        __syncthreads();
+        double w = 0.0;
+        if (t < ROWS && r0 + t < n) {
+#pragma unroll
+            for (int q = 0; q < W; ++q) w += red[q][t];
+            w += diag * value(r0 + t);
+        }
+        return w;
+    }
+    __device__ void run(const double* vs, double sj, double* wi, double* wl, int) {
+        const int t = threadIdx.x;
+        const double w = sj * product([&](int j) { return vs[j]; });
+        if (t < ROWS) {
+            wl[t] = w;
+            if (r0 + t < n) wi[r0 + t] = w;
+        }
+    }
+};
+
 // Launch i of a solve's sequence (see the file comment).  Every workgroup repeats the finishing work (the basis, the
 // partial sums, the preconditioner), so the rows per workgroup follow the size (Solver::alloc_gmres).
 template <class P>
@@ -606,6 +662,37 @@ template <int NA, int H>
 __global__ __launch_bounds__(256 * H) void gm_sums_kernel(GmArgs a, const SurfDesc* __restrict__ sd, int i) {
     gm_step<PairSums<NA, H>>(a, sd, i);
 }
+
+template <bool FILM>
+__global__ __launch_bounds__(256) void gm_tsums_kernel(GmArgs a, const SurfDesc* __restrict__ sd, int i) {
+    gm_step<TransposeSums<FILM>>(a, sd, i);
+}
+
+// The warm start of a transposed solve: r0 = b - M^T x0 as the first basis vector.  grid = (ceil(max n / kSumRows), surfaces).
+template <bool FILM>
+__global__ __launch_bounds__(256) void gm_tstart_kernel(GmArgs a, const SurfDesc* __restrict__ sd, int reset) {
+    const SurfDesc d = sd[blockIdx.y];
+    const int r0 = blockIdx.x * kSumRows, t = threadIdx.x;
+    if (blockIdx.x == 0 && t == 0) {
+        GmCtl* c = reinterpret_cast<GmCtl*>(a.ctl) + blockIdx.y;
+        c->done = 0;
+        c->refine_iters = 0;
+        c->iters = 0;
+        if (reset) c->most = 0;
+    }
+    if (r0 >= d.n) return;
+    const GmView v = gm_view(a, sd, blockIdx.y);
+    const double* x0 = a.x + d.voff;
+    const double b = a.b[d.voff + min(r0 + t, d.n - 1)];
+    TransposeSums<FILM> prod(a, v, d, r0);
+    prod.start();
+    const double w = prod.product([&](int j) { return x0[j]; });
+    if (t < kSumRows && r0 + t < d.n) a.V[(long long)(a.m + 1) * d.voff + r0 + t] = b - w;
+}
+template __global__ void gm_tsums_kernel<false>(GmArgs, const SurfDesc*, int);
+template __global__ void gm_tsums_kernel<true>(GmArgs, const SurfDesc*, int);
+template __global__ void gm_tstart_kernel<false>(GmArgs, const SurfDesc*, int);
+template __global__ void gm_tstart_kernel<true>(GmArgs, const SurfDesc*, int);
 
 // The start of a solve with products from cotangent sums: S of the initial guess, M_kk, and r0 = b - M x0 as the first
 // (unnormalised) basis vector.  grid = (ceil(max n / kSumRows), surfaces).

@@ -94,7 +94,7 @@ struct GmArgs {
     const double2* tw;   // twiddle tables, SurfDesc::twoff
     // products from cotangent sums (sfh_pairs.hpp; sums = 0: from the stored matrix): S holds the sums of the initial
     // guess and then of each (preconditioned, unscaled) basis vector, sums arrays of total nodes each
-    int sums;            // 2 (water), 4 (film)
+    int sums;            // 2 (water), 4 (film); -1: transposed products, S unused
     double* S;
     double* diag;        // M_kk
     const NodeTrig* trig;
@@ -198,6 +198,11 @@ template <int NA>
 __global__ void gm_start_kernel(GmArgs a, const SurfDesc* sd, const double2* Z, const double2* Zpp, Phys ph);
 template <int NA, int H>
 __global__ void gm_sums_kernel(GmArgs a, const SurfDesc* sd, int j);
+// transposed products (reverse mode): the first residual, one launch per Arnoldi step
+template <bool FILM>
+__global__ void gm_tstart_kernel(GmArgs a, const SurfDesc* sd, int reset);
+template <bool FILM>
+__global__ void gm_tsums_kernel(GmArgs a, const SurfDesc* sd, int j);
 // PRE: the basis is preconditioned; NA > 0: also the velocity stage, from the solve's sums (else Z, Zpp, ph, sc unused)
 template <bool PRE, int NA>
 __global__ void gm_close_mu_kernel(GmArgs a, const SurfDesc* sd, const double* circ, double2* mup, int i, const double2* Z,
@@ -313,10 +318,12 @@ struct AdjMArgs {
     double* out_P;
     double2* acc_Z;            // optional accumulator += out
     double* acc_P;
+    double* diag;              // M_kk (written by pass A)
     double* quirk;             // water rho != 0 with the V1[1] quirk: rho gp, q2.x, q1.x per node (3 x total)
     int total;                 // nodes of all surfaces
 };
 constexpr int kAdjRows = 2;   // rows per workgroup of the reverse pair kernels
+constexpr int kAdjCols = 4;   // columns per thread and pass of theirs
 __global__ void adj_rho_quirk_kernel(AdjMArgs a);
 __global__ void aug_vjp_kernel(const double2* Z, const double* gA_P, const double* gB_P, const double* gA_D,
                                const double* gB_D, double ca, double cb, double2* outZ, double2* accZ, double* outD,
@@ -327,9 +334,6 @@ template <int R> __global__ void adj_pass_c_kernel(AdjMArgs a, Phys ph);
 __global__ void adj_circ_d1_kernel(const SurfDesc* sd, const double* circ, const double2* v, double2* out);
 __global__ void adj_gm_start_kernel(const SurfDesc* sd, const double* b, double* V, double* x, int* ctl, int m, int reset);
 __global__ void adj_extrapolate_kernel(const double* ring, int head, int hv, double* x0, int total);
-__global__ void adj_gm_start_warm_kernel(const SurfDesc* sd, const double* Mt, const double* b, const double* x0,
-                                         double* V, double* x, int* ctl, int m, int reset);
-__global__ void transpose_kernel(const SurfDesc* sd, const double* M, double* Mt);
 __global__ void adj_gamma_kernel(AdjMArgs a, Phys ph);
 __global__ void adj_final_kernel(AdjMArgs a, const double* circ, const double2* sd1gb);
 

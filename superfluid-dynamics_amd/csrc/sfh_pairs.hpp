@@ -44,6 +44,32 @@ __device__ __forceinline__ void sum_pass(const NodeTrig (&tk)[kSumRows], const N
     }
 }
 
+// The transposed product's sum of each row (reverse mode): with w_k = v_k Z'_k,
+//   (M^T v)_j = M_jj v_j - c Im sum_{k != j} w_k cot((z_j - z_k)/2) - ci Im sum_{k != j} v_k cot((z_j - conj z_k)/2 + i h),
+// the image part being symmetric; acc[r] is minus the sums' contribution.  value(j) = v_j.
+template <bool FILM, class F>
+__device__ __forceinline__ void transpose_pass(const NodeTrig (&tk)[kSumRows], const NodeTrig (&tj)[kSumCols],
+                                               const double2 (&zj)[kSumCols], int n, int k0, int j0, int tg, double c, double ci,
+                                               double eh, double ehi, F&& value, double (&acc)[kSumRows]) {
+#pragma unroll
+    for (int e = 0; e < kSumCols; ++e) {
+        const int j = j0 + tg + 256 * e;
+        if (j >= n) break;
+        const double v = value(j);
+        const double wx = c * v * zj[e].x, wy = c * v * zj[e].y, vi = ci * v;
+#pragma unroll
+        for (int r = 0; r < kSumRows; ++r) {
+            if (j == k0 + r) continue;
+            const CotParts cp = cot_parts(tk[r], tj[e]);
+            acc[r] += cp.id * (wx * cp.q - wy * cp.p);
+            if constexpr (FILM) {
+                const CotParts cq = cot_image_parts(tk[r], tj[e], eh, ehi);
+                acc[r] += vi * (cq.q * cq.id);
+            }
+        }
+    }
+}
+
 // The group's sums of its rows, in LDS red (one row of NA * kSumRows values per wave; the caller synchronises after
 // sum_store): row r's sum a.
 template <int NA>

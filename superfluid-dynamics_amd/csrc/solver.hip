@@ -372,9 +372,9 @@ Solver::~Solver() {
         if (p) (void)hipFree(p);
     void* vbufs[] = {vY_[0], vY_[1], vY_[2], vK_[0], vK_[1], vK_[2], vYP_[0], vYP_[1], vYP_[2], vKP_[0],
                      vKP_[1], vKP_[2], vMu_[0], vMu_[1], vMu_[2], vMu_[3], gA_, gR_[0], gR_[1], gAcc_,
-                     gAP_, gRP_[0], gRP_[1], gAccP_, adj_, vstats_, Mt_, agwc_, agmup_, ad1_, agam_, agamI_,
+                     gAP_, gRP_[0], gRP_[1], gAccP_, adj_, vstats_, agwc_, agmup_, ad1_, agam_, agamI_,
                      agzp_, agzpp_, agz_, agmu_, agb_, aquirk_, gAD_, gAccD_, gRD_[0], gRD_[1], vYD_[0], vYD_[1],
-                     vYD_[2], adjRing_, adjSave_, adjX_, adjSaveZ_, adjSaveP_};
+                     vYD_[2], adjRing_, adjSave_, adjSaveZ_, adjSaveP_};
     for (void* p : vbufs)
         if (p) (void)hipFree(p);
     for (auto& kv : traj_) free_record(kv.second);
@@ -503,7 +503,9 @@ bool Solver::enqueue_gmres(const GmArgs& a, bool force64, const double2* Z, cons
                 auto step = [&](auto kernel, int waves) {
                     go(kernel, grid, dim3(64 * waves), 0, a, (const SurfDesc*)d_desc_, j);
                 };
-                if (a.sums == 2) {
+                if (a.sums < 0) {
+                    step(ph_.image ? gm_tsums_kernel<true> : gm_tsums_kernel<false>, 4);
+                } else if (a.sums == 2) {
                     a.rpw == 4 ? step(gm_sums_kernel<2, 1>, 4) : step(gm_sums_kernel<2, 2>, 8);
                 } else if (a.sums == 4) {
                     a.rpw == 4 ? step(gm_sums_kernel<4, 1>, 4) : step(gm_sums_kernel<4, 2>, 8);
@@ -1506,7 +1508,7 @@ void Solver::ensure_vjp() {
     if (vjp_ready_) return;
     if (opt_.solver != kSolveBatched) {   // the multi-workgroup reverse pass
         alloc_gmres(kGmMaxIter);
-        Mt_ = dalloc<double>(MT_);
+        if (!gmdiag_) gmdiag_ = dalloc<double>(T_);
         for (double2** b : {&agwc_, &agmup_, &ad1_, &agam_, &agamI_, &agzp_, &agzpp_, &agz_}) *b = dalloc<double2>(T_);
         agmu_ = dalloc<double>(T_);
         agb_ = dalloc<double>(T_);
@@ -1514,7 +1516,6 @@ void Solver::ensure_vjp() {
         SFH_HIP(hipMemset(agamI_, 0, T_ * sizeof(double2)));
         adjRing_ = dalloc<double>((size_t)4 * kHistDepth * T_);
         adjSave_ = dalloc<double>((size_t)4 * kHistDepth * T_);
-        adjX_ = dalloc<double>(T_);
         adjSaveZ_ = dalloc<double2>(T_);
         adjSaveP_ = dalloc<double>(T_);
     }
@@ -1584,8 +1585,7 @@ void Solver::enqueue_vjp(const double2* Z, const double* P, const double* mu, co
 
 // The reverse pass over many workgroups per surface (adjoint_mwg.hip), at the state (Z, P) with its
 // forward mu: the derivatives and mu' of the state, pass A, D1 of the cotangent of mu', pass B, the
-// transposed solve M^T gb = gmu (M re-assembled and transposed, the GMRES launch sequence from a zero
-// guess, FP64), the matrix terms and pair weights, pass C, and the spectral adjoints.
+// transposed solve M^T gb = gmu (the GMRES launch sequence, products from sums over the pairs), the matrix terms and pair weights, pass C, and the spectral adjoints.
 void Solver::enqueue_vjp_mwg(const double2* Z, const double* P, const double* mu, const double2* gAZ,
                              const double* gAP, double ca, const double2* gBZ, const double* gBP, double cb,
                              double2* outZ, double* outP, bool accumulate, int stage) {
@@ -1631,6 +1631,7 @@ void Solver::enqueue_vjp_mwg(const double2* Z, const double* P, const double* mu
     a.out_P = outP;
     a.acc_Z = accumulate ? gAcc_ : nullptr;
     a.acc_P = accumulate ? gAccP_ : nullptr;
+    a.diag = gmdiag_;
     a.quirk = aquirk_;
     a.total = T_;
     const bool quirk = ph_.kind == 0 && ph_.rho != 0.0 && ph_.rho_quirk;
@@ -1642,27 +1643,15 @@ void Solver::enqueue_vjp_mwg(const double2* Z, const double* P, const double* mu
     });
     // M^T gb = gmu
     launch("vjp_solve", 2.0 * gm_m_ * nsq, 8.0 * gm_m_ * nsq, [&] {
-        go(assemble64_kernel<kPairRows>, dim3((maxN_ + kPairRows - 1) / kPairRows, S_), dim3(256), 0, d_desc_,
-           (const NodeTrig*)trig_, Z, Zp_, Zpp_, M_, ph_, GmArgs{}, 0);
-        go(transpose_kernel, dim3((maxN_ + 31) / 32, (maxN_ + 31) / 32, S_), dim3(256), 0, d_desc_, (const double*)M_,
-           Mt_);
         // inside a trajectory sweep: the guess extrapolated from this stage's solutions of the previous
         // reverse steps, and the sweep's sequence length; else a zero guess, the full sequence
         const bool warm = adj_warm_ && stage >= 0 && adj_hv_[stage] > 0;
         const int m = adj_warm_ && adj_len_ > 0 ? adj_len_ : gm_m_;
         const int reset = adj_first_ ? 1 : 0;
         adj_first_ = false;
-        if (warm) {
-            go(adj_extrapolate_kernel, dim3((T_ + 255) / 256), dim3(256), 0,
-               (const double*)(adjRing_ + (size_t)stage * kHistDepth * T_), adj_head_[stage], adj_hv_[stage], adjX_,
-               T_);
-            go(adj_gm_start_warm_kernel, dim3((maxN_ + 3) / 4, S_), dim3(256), 0, d_desc_, (const double*)Mt_,
-               (const double*)agmu_, (const double*)adjX_, gmV_, gmx0_, gmctl_, m, reset);
-        } else {
-            go(adj_gm_start_kernel, ngrid, dim3(256), 0, d_desc_, (const double*)agmu_, gmV_, gmx0_, gmctl_, m, reset);
-        }
         GmArgs g = gm_args(0);
-        g.M = Mt_;
+        g.sums = -1;
+        g.rpw = kSumRows;
         g.M32 = nullptr;
         g.b = agmu_;
         g.x = gmx0_;
@@ -1675,8 +1664,14 @@ void Solver::enqueue_vjp_mwg(const double2* Z, const double* P, const double* mu
         g.check_first = 0;
         g.pre = 0;
         g.Z = gmV_;
-        g.sums = 0;
-        g.rpw = gm_rpw_;
+        if (warm) {
+            go(adj_extrapolate_kernel, dim3((T_ + 255) / 256), dim3(256), 0,
+               (const double*)(adjRing_ + (size_t)stage * kHistDepth * T_), adj_head_[stage], adj_hv_[stage], gmx0_, T_);
+            go(ph_.image ? gm_tstart_kernel<true> : gm_tstart_kernel<false>, dim3((maxN_ + kSumRows - 1) / kSumRows, S_),
+               dim3(256), 0, g, (const SurfDesc*)d_desc_, reset);
+        } else {
+            go(adj_gm_start_kernel, ngrid, dim3(256), 0, d_desc_, (const double*)agmu_, gmV_, gmx0_, gmctl_, m, reset);
+        }
         enqueue_gmres(g, true);   // leaves s D1 gb in mup_
     });
     if (adj_warm_ && stage >= 0) {   // the solution joins the stage's ring

@@ -324,7 +324,6 @@ class Solver {
     AdjNode* adj_ = nullptr;
     int* vstats_ = nullptr;
     // multi-workgroup reverse mode (LU and GMRES handles): M^T and the per-node vectors of adjoint_mwg.hip
-    double* Mt_ = nullptr;
     double2 *agwc_ = nullptr, *agmup_ = nullptr, *ad1_ = nullptr, *agam_ = nullptr, *agamI_ = nullptr;
     double2 *agzp_ = nullptr, *agzpp_ = nullptr, *agz_ = nullptr;
     double *agmu_ = nullptr, *agb_ = nullptr;
@@ -339,7 +338,6 @@ class Solver {
     // warm starts of the transposed solves over a trajectory's reverse steps (LU and GMRES handles):
     // per RK stage a ring of the last kHistDepth solutions, extrapolated like the forward warm start
     double* adjRing_ = nullptr;      // 4 stages x kHistDepth x T
-    double* adjX_ = nullptr;         // the extrapolated guess
     double* adjSave_ = nullptr;      // the rings at the start of a segment (for a redo)
     double2* adjSaveZ_ = nullptr;    // the cotangent at the start of a segment
     double* adjSaveP_ = nullptr;
