@@ -395,6 +395,8 @@ class Solver {
     int trim_ = 0;          // 0: not determined yet
     int hist_steps_ = 0;    // steps since set_state (saturates at kCalibSteps)
     int chunk_ = 2;         // steps of the next trimmed chunk (doubles up to kCheckSteps)
+    int lower_left_ = 0;    // chunks that still have to need fewer launches before the sequence is shortened
+    bool lowered_ = false;
     int chunks_kept_ = 0;   // trimmed chunks kept since the calibration
     int unc_raw_ = 0;       // unconverged count of the control blocks (discarded chunks included)
     int unc_discard_ = 0;   // ... of solves in chunks that were run again
