@@ -323,6 +323,7 @@ __global__ __launch_bounds__(1024) void batched_stage_kernel(BatchArgs a, Phys p
     }
     if (!own) return;
     const int gi = off + t;
+    if (ctl.mu_keep) ctl.mu_keep[gi] = x;
     if (ctl.qup) ctl.qup[gi] = q2;
     if (!ph.need_upper) q2 = make_double2(0.0, 0.0);
     double dphi = bernoulli(ph, zk.y, q1, q2, q1q, zpk, zppk);

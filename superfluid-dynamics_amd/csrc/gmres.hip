@@ -1079,7 +1079,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
             double2 q1, q2;
             velocity_from_sums(ph, zp, zpp, mp, mu_t, z.y, S[0], S[1], NA == 4 ? S[NA == 4 ? 2 : 0] : 0.0,
                                NA == 4 ? S[NA == 4 ? 3 : 0] : 0.0, q1, q2);
-            finish_node(ph, sc, g, z, zp, zpp, q1, q2, q1, st);
+            finish_node(ph, sc, g, z, zp, zpp, mu_t, q1, q2, q1, st);
         }
     }
 }

@@ -29,6 +29,10 @@ struct StageCtl {
     double* D0;
     double* Dout;
     double* kD[3];
+    // optional, for the reverse pass: the stage's mu, and (stage 4) the state it leaves
+    double* mu_keep;
+    double2* Zkeep;
+    double* Pkeep;
     int* nonfinite;    // optional: set to 1 when a stage slope of any node is NaN or infinite
     // timed drive: the stage's delayed intensity is dca * Din + dcb * I; dsave: store it in Dout
     double dca, dcb;

@@ -249,8 +249,14 @@ __device__ inline void stage_store(const StageCtl& ctl, int g, double2 q1, doubl
         const double Kx = s.k1.x + 2.0 * s.k2.x + 2.0 * s.k3.x + q1.x;
         const double Ky = s.k1.y + 2.0 * s.k2.y + 2.0 * s.k3.y + q1.y;
         const double Kp = s.p1 + 2.0 * s.p2 + 2.0 * s.p3 + dphi;
-        const_cast<double2*>(ctl.Z0)[g] = make_double2(s.z0.x + ctl.alpha * Kx, s.z0.y + ctl.alpha * Ky);
-        const_cast<double*>(ctl.P0)[g] = s.p0 + ctl.alpha * Kp;
+        const double2 z = make_double2(s.z0.x + ctl.alpha * Kx, s.z0.y + ctl.alpha * Ky);
+        const double p = s.p0 + ctl.alpha * Kp;
+        const_cast<double2*>(ctl.Z0)[g] = z;
+        const_cast<double*>(ctl.P0)[g] = p;
+        if (ctl.Zkeep) {
+            ctl.Zkeep[g] = z;
+            ctl.Pkeep[g] = p;
+        }
     }
 }
 // Per-node terms of EnergyContainer::CalculateEnergy and VolumeFlux (Energies.cuh:136-204),
@@ -282,7 +288,8 @@ __device__ inline void stage_update(const StageCtl& ctl, int g, double2 q1, doub
 // The end of a right-hand side at one node: Bernoulli from the velocities, energy and drive terms on request, and the
 // RK stage.  q1q is the lower velocity in the rho q1.q2 term.
 __device__ inline void finish_node(const Phys& ph, const StageCtl& ctl, int g, double2 z, double2 zp, double2 zpp,
-                                   double2 q1, double2 q2, double2 q1q, const StageIn& st) {
+                                   double mu, double2 q1, double2 q2, double2 q1q, const StageIn& st) {
+    if (ctl.mu_keep) ctl.mu_keep[g] = mu;
     if (ctl.qup) ctl.qup[g] = q2;
     if (!ph.need_upper) q2 = make_double2(0.0, 0.0);
     double dphi = bernoulli(ph, z.y, q1, q2, q1q, zp, zpp);

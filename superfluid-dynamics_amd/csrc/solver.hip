@@ -735,38 +735,33 @@ void Solver::enqueue_step(double dt, const StageCapture* cap) {
         c.kP[i] = kP_[i];
     }
     c.qup = nullptr;
+    // for the adjoint's re-run the stages' states and mu are formed in the segment's own arrays (never inside a
+    // captured graph), which the next stage reads
+    double2* const Y[3] = {cap ? cap->Y[0] : Za_, cap ? cap->Y[1] : Zb_, cap ? cap->Y[2] : Za_};
+    double* const YP[3] = {cap ? cap->YP[0] : Pa_, cap ? cap->YP[1] : Pb_, cap ? cap->YP[2] : Pa_};
+    double* const mu[4] = {cap ? cap->mu[0] : nullptr, cap ? cap->mu[1] : nullptr, cap ? cap->mu[2] : nullptr,
+                           cap ? cap->mu[3] : nullptr};
     // timed drive: stages at t_n, t_n + h/2, t_n + h/2, t_n + h (RK4_Time_Dependent.cuh:173,237,263,270);
     // the first saves the delayed intensity and moves the saved time to t_n
-    c.stage = 1; c.alpha = half; c.Zout = Za_; c.Pout = Pa_;
+    c.stage = 1; c.alpha = half; c.Zout = Y[0]; c.Pout = YP[0]; c.mu_keep = mu[0];
     set_delayed_ctl(c, D0_, Da_);
     timed_coefficients(c, drive_t_, 1);
     enqueue_rhs(Z0_, P0_, c);
-    // the stage's mu and the state it produced, for the adjoint's re-run (never inside a captured graph)
-    auto keep = [&](int st, const double2* Zs, const double* Ps) {
-        if (!cap) return;
-        SFH_HIP(hipMemcpyAsync(cap->mu[st], mu_, T_ * sizeof(double), hipMemcpyDeviceToDevice, stream_));
-        if (st < 3) {
-            SFH_HIP(hipMemcpyAsync(cap->Y[st], Zs, T_ * sizeof(double2), hipMemcpyDeviceToDevice, stream_));
-            SFH_HIP(hipMemcpyAsync(cap->YP[st], Ps, T_ * sizeof(double), hipMemcpyDeviceToDevice, stream_));
-        }
-    };
-    keep(0, Za_, Pa_);
     if (ph_.timed) drive_prev_ = drive_t_;
-    c.stage = 2; c.alpha = half; c.Zout = Zb_; c.Pout = Pb_;
+    c.stage = 2; c.alpha = half; c.Zout = Y[1]; c.Pout = YP[1]; c.mu_keep = mu[1];
     set_delayed_ctl(c, Da_, Db_);
     timed_coefficients(c, drive_t_ + half, 0);
-    enqueue_rhs(Za_, Pa_, c);
-    keep(1, Zb_, Pb_);
-    c.stage = 3; c.alpha = dt; c.Zout = Za_; c.Pout = Pa_;
+    enqueue_rhs(Y[0], YP[0], c);
+    c.stage = 3; c.alpha = dt; c.Zout = Y[2]; c.Pout = YP[2]; c.mu_keep = mu[2];
     set_delayed_ctl(c, Db_, Da_);
     timed_coefficients(c, drive_t_ + half, 0);
-    enqueue_rhs(Zb_, Pb_, c);
-    keep(2, Za_, Pa_);
-    c.stage = 4; c.alpha = sixth; c.Zout = nullptr; c.Pout = nullptr;
+    enqueue_rhs(Y[1], YP[1], c);
+    c.stage = 4; c.alpha = sixth; c.Zout = nullptr; c.Pout = nullptr; c.mu_keep = mu[3];
+    c.Zkeep = cap ? cap->Z : nullptr;
+    c.Pkeep = cap ? cap->P : nullptr;
     set_delayed_ctl(c, Da_, nullptr);
     timed_coefficients(c, drive_t_ + dt, 0);
-    enqueue_rhs(Za_, Pa_, c);
-    keep(3, nullptr, nullptr);
+    enqueue_rhs(Y[2], YP[2], c);
     if (ph_.timed) drive_t_ += dt;   // currentTime += timeStep (RK4_Time_Dependent.cuh:408)
 }
 
@@ -1635,7 +1630,11 @@ void Solver::enqueue_vjp_mwg(const double2* Z, const double* P, const double* mu
     a.gmup = agmup_;
     a.d1 = ad1_;
     a.gmu = agmu_;
-    a.gb = agb_;
+    // inside a sweep the solution goes straight to its slot of the stage's ring
+    const bool ring = adj_warm_ && stage >= 0;
+    const int slot = ring ? (adj_head_[stage] + 1) % kHistDepth : 0;
+    double* const gb = ring ? adjRing_ + ((size_t)stage * kHistDepth + slot) * T_ : agb_;
+    a.gb = gb;
     a.gam = agam_;
     a.gamI = agamI_;
     a.gzp = agzp_;
@@ -1669,7 +1668,7 @@ void Solver::enqueue_vjp_mwg(const double2* Z, const double* P, const double* mu
         g.M32 = nullptr;
         g.b = agmu_;
         g.x = gmx0_;
-        g.sol = agb_;
+        g.sol = gb;
         g.m = m;
         g.tol = std::min(opt_.tol, 1e-13);
         g.hist = nullptr;
@@ -1688,10 +1687,7 @@ void Solver::enqueue_vjp_mwg(const double2* Z, const double* P, const double* mu
         }
         enqueue_gmres(g, true);   // leaves s D1 gb in mup_
     });
-    if (adj_warm_ && stage >= 0) {   // the solution joins the stage's ring
-        const int slot = (adj_head_[stage] + 1) % kHistDepth;
-        SFH_HIP(hipMemcpyAsync(adjRing_ + ((size_t)stage * kHistDepth + slot) * T_, agb_, T_ * sizeof(double),
-                               hipMemcpyDeviceToDevice, stream_));
+    if (ring) {
         adj_head_[stage] = slot;
         adj_hv_[stage] = std::min(adj_hv_[stage] + 1, kHistDepth);
     }
@@ -1834,6 +1830,8 @@ Solver::StageCapture Solver::seg_capture(int k) const {
         c.YP[i] = segYP_ + (i * cap + k) * T;
     }
     for (int i = 0; i < 4; ++i) c.mu[i] = segMu_ + (i * cap + k) * T;
+    c.Z = k + 1 < seg_cap_ ? segZ_ + (k + 1) * T : nullptr;
+    c.P = k + 1 < seg_cap_ ? segP_ + (k + 1) * T : nullptr;
     return c;
 }
 
@@ -1983,10 +1981,6 @@ void Solver::traj_backward(int record, const double* gx_in, const double* gy_in,
                 seq_len_ = gmres && trimmed ? length(k) : gm_m_;
                 const StageCapture cap = seg_capture(k);
                 enqueue_step(r.dt, &cap);
-                if (k + 1 < n) {
-                    SFH_HIP(hipMemcpyAsync(segZ_ + (size_t)(k + 1) * T_, Z0_, zb, hipMemcpyDeviceToDevice, stream_));
-                    SFH_HIP(hipMemcpyAsync(segP_ + (size_t)(k + 1) * T_, P0_, pb, hipMemcpyDeviceToDevice, stream_));
-                }
             }
         };
         bool trim = false;

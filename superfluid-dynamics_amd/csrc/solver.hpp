@@ -212,6 +212,8 @@ class Solver {
         double2* Y[3];
         double* YP[3];
         double* mu[4];
+        double2* Z;       // the state after the step (may be null)
+        double* P;
     };
     void enqueue_step(double dt, const StageCapture* cap = nullptr);
     void capture(double dt, int len);

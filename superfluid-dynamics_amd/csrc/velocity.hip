@@ -151,7 +151,7 @@ __global__ __launch_bounds__(256) void velocity_stage_kernel(const SurfDesc* __r
         double2 u2;
         velocity_from_sums(ph, zp_1, zpp_1, mup_1, m_1, y_1, qo[0], qo[1], 0.0, 0.0, q1q, u2);
     }
-    finish_node(ph, ctl, d.voff + k0 + t, z_t, zp_t, zpp_t, q1, q2, q1q, st);
+    finish_node(ph, ctl, d.voff + k0 + t, z_t, zp_t, zpp_t, m_t, q1, q2, q1q, st);
 }
 
 // Surfaces of up to 256 nodes, not with the rho quirk: a wave has 4 rows and all their columns, 16 pairs per lane, and its
@@ -220,7 +220,7 @@ __global__ __launch_bounds__(256) void velocity_small_kernel(const SurfDesc* __r
     const double* S = red[w] + lane;
     double2 q1, q2;
     velocity_from_sums(ph, zp, zpp, mp, m, z.y, S[0], S[4], NA == 4 ? S[NA == 4 ? 8 : 0] : 0.0, NA == 4 ? S[NA == 4 ? 12 : 0] : 0.0, q1, q2);
-    finish_node(ph, ctl, g, z, zp, zpp, q1, q2, q1, st);
+    finish_node(ph, ctl, g, z, zp, zpp, m, q1, q2, q1, st);
 }
 template __global__ void velocity_small_kernel<2>(const SurfDesc*, const NodeTrig*, const double2*, const double2*, const double2*,
                                                   const double*, const double2*, Phys, StageCtl);
