@@ -13,7 +13,7 @@
 // y_p = L11^{-1} b_p; the other workgroups of the launch apply panel p-1's update A22 -= L21 U12 to the
 // rest of the trailing matrix.
 // lu_backsolve_kernel then runs x_p = U_pp^{-1} (y_p - sum_{q>p} U_pq x_q), one workgroup per
-// block row, chained by per-block ready flags.
+// block row, chained through the entries of x themselves.
 //
 // Row interchanges.  Partial pivoting (getrf: first row of maximal |a| in the current column)
 // leaves the rows in place exactly when every multiplier satisfies |l_ij| <= 1.  Both the
@@ -38,25 +38,6 @@ __device__ inline v4d mfma_f64(double a, double b, v4d c) {
 // c - a b: the FP64 form takes its last operand field as sign bits (bit 0: A negated)
 __device__ inline v4d mfma_f64_sub(double a, double b, v4d c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 1);
-}
-
-// Loads a rows x cols block of row-major global memory (leading dimension ld) into LDS (64 x 64;
-// beyond the block its last row and column are repeated).  Fixed trip count (NT threads x
-// 4096 / NT) and clamped addresses so that all loads of a thread are in flight together.
-template <int NT>
-__device__ __forceinline__ void load_block(double* dst, const double* src, int ld, int rows, int cols) {
-    constexpr int IT = kNB * kNB / NT;
-    double v[IT];
-#pragma unroll
-    for (int it = 0; it < IT; ++it) {
-        const int e = threadIdx.x + it * NT, r = e >> 6, c = e & 63;
-        v[it] = src[(unsigned)min(r, rows - 1) * (unsigned)ld + (unsigned)min(c, cols - 1)];
-    }
-#pragma unroll
-    for (int it = 0; it < IT; ++it) {
-        const int e = threadIdx.x + it * NT;
-        dst[(e >> 6) * LD + (e & 63)] = v[it];
-    }
 }
 
 // The L21 block of the block row at R0 (rows rows) and the panel at kp, from the strips' layout (below)
@@ -351,10 +332,10 @@ __device__ __forceinline__ void strip_solve(v4d (&acc)[4], const double* inv, in
 }
 
 // Per-surface views for gridDim.z batches of equal size: surface s uses A + s n^2, vectors + s n,
-// uinv + s P 64^2, flags + s P, status + 2 s.
+// uinv + s P 64^2, status + 2 s.
 struct LuView {
     double *A, *work, *y, *x, *uinv;
-    int *flags, *status;
+    int* status;
 };
 __device__ inline LuView view(const LuArgs& a) {
     const int s = blockIdx.z, n = a.n, P = (n + kNB - 1) / kNB;
@@ -364,7 +345,6 @@ __device__ inline LuView view(const LuArgs& a) {
     v.y = a.y + (long long)s * n;
     v.x = a.x + (long long)s * n;
     v.uinv = a.uinv + (long long)s * P * kNB * kNB;
-    v.flags = a.flags + (long long)s * P;
     v.status = a.status + 2 * s;
     return v;
 }
@@ -702,6 +682,9 @@ __device__ __forceinline__ void lu_panel(const LuView& v, int n, int k0, int kb,
     }
 }
 
+// An entry of x that is not there yet: a signalling NaN, which no arithmetic gives.  The first panel's launch fills x with it.
+constexpr unsigned long long kNoValue = 0x7ff0dead00000001ull;
+
 // Panel p (columns k0 .. k0 + kb - 1) together with the previous panel's trailing update
 // (kp = k0 - 64; A22 -= L21 U12 with panel p-1's blocks), one launch per panel:
 //   roles 0 .. 2 nrb (panel p): each applies panel p-1's update to the diagonal block A_pp (kept in
@@ -722,8 +705,8 @@ __global__ __launch_bounds__(kLuThreads) void lu_step_kernel(LuArgs a, int k0) {
     const int nrb = (n - k0 - kb + kNB - 1) / kNB;
     const int role = blockIdx.x;
     if (k0 == 0 && role == 0) {
-        const int PB = (n + kNB - 1) / kNB;
-        for (int i = t; i < PB; i += kLuThreads) v.flags[i] = 0;
+        unsigned long long* x = reinterpret_cast<unsigned long long*>(v.x);
+        for (int i = t; i < n; i += kLuThreads) x[i] = kNoValue;
     }
     if (role > 2 * nrb) {   // trailing tiles of panel p-1's update (only when k0 > 0)
         const int wgs = gridDim.x - 1 - 2 * nrb, i = role - 1 - 2 * nrb, tiles = nrb * nrb;
@@ -845,69 +828,92 @@ __device__ void fallback_solve(const LuFallback& f, int s) {
     gepp_solve(n, A, f.b + d.voff, f.x + d.voff, f.piv + d.voff, f.counters);
 }
 
-// x_p = U_pp^{-1} (y_p - sum_{q>p} U_pq x_q).  Workgroup b handles block row p = P-1-b, so a
-// workgroup only waits for workgroups dispatched before it; every wait is bounded.  Each U_pq
-// block is staged into LDS before the wait for x_q, so only the x_q load and an LDS GEMV sit on
-// the dependency chain.
+// x_p = U_pp^{-1} (y_p - sum_{q>p} U_pq x_q).  Workgroup b handles block row p = P-1-b, so a workgroup only waits for
+// workgroups dispatched before it; every wait is bounded.  The chain from x_{p+1} to x_p bounds the launch, so nothing
+// else is on it: the entries of x are polled themselves (agent scope, past the XCDs' L2 caches; a flag would add a fence
+// and a load behind it), thread (r, chunk) holds its 16 entries of U_pq in registers, loaded while it waits for the block
+// before, and one barrier separates the blocks.  N = 2048 67 -> 52 us,
+// N = 768 25 -> 21, N = 256 8.1 -> 7.5; with 8-byte loads of the rows 75 at N = 2048, as much as through LDS.
 // FALLBACK: when the factorisation needed interchanges, the surface's first workgroup solves its system anew instead
 // (fallback_solve); as launches of their own the two kernels of that cost every solve 9 us to find nothing to do.
 template <bool FALLBACK>
 __global__ __launch_bounds__(256) void lu_backsolve_kernel(LuArgs a, LuFallback f) {
-    __shared__ double Ub[kNB * LD], Ui[kNB * LD];
-    __shared__ double xq[kNB], part[4][kNB], sv[kNB];
+    __shared__ double xq[2][kNB], part[4][kNB], sv[kNB];
     const LuView v = view(a);
     const int n = a.n, t = threadIdx.x;
     const int P = (n + kNB - 1) / kNB;
     const int p = P - 1 - blockIdx.x;
     const int R0 = p * kNB, rb = min(kNB, n - R0);
     const int r = t & 63, chunk = t >> 6;
-    const double* U = v.uinv + (long long)p * kNB * kNB;
     const int bad = FALLBACK ? v.status[0] : 0;
-    load_block<256>(Ui, U, kNB, kNB, kNB);
+    // 16 entries of row r of block U_pq, one 128-byte line of it; a row or column beyond the matrix is read clamped and
+    // meets a zero of x (or is not used).  n is even when there are several blocks: 16-byte loads.
+    const double* Ar = v.A + (long long)(R0 + min(r, rb - 1)) * n;
+    auto load = [&](int q, double (&u)[16]) {
+        const int c0 = q * kNB + chunk * 16;
+        if ((q + 1) * kNB <= n) {
+#pragma unroll
+            for (int c = 0; c < 16; c += 2) {
+                const double2 w = *reinterpret_cast<const double2*>(Ar + c0 + c);
+                u[c] = w.x;
+                u[c + 1] = w.y;
+            }
+        } else {
+#pragma unroll
+            for (int c = 0; c < 16; ++c) u[c] = Ar[min(c0 + c, n - 1)];
+        }
+    };
+    double ui[16], u[16], un[16];
+    const double2* U = reinterpret_cast<const double2*>(v.uinv + (long long)p * kNB * kNB + r * kNB + chunk * 16);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        const double2 w = U[c];
+        ui[2 * c] = w.x;
+        ui[2 * c + 1] = w.y;
+    }
+    const double y = t < rb ? v.y[R0 + t] : 0.0;
+    if (P > 1) load(P - 1, u);
     if (FALLBACK && bad) {
         if (blockIdx.x == 0) fallback_solve(f, f.first + blockIdx.z);
         return;
     }
-    double acc = 0.0;
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
     for (int q = P - 1; q > p; --q) {
-        const int C0 = q * kNB, cb = min(kNB, n - C0);
-        load_block<256>(Ub, v.A + (long long)R0 * n + C0, n, rb, cb);
-        if (t == 0) {
-            // relaxed polling, one acquire once the flag is seen: on gfx950 every agent-scope
-            // acquire invalidates this XCD's L2, which other workgroups are reading through
-            int spins = 0;
-            while (__hip_atomic_load(&v.flags[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) {
-                __builtin_amdgcn_s_sleep(1);
-                if (++spins > (1 << 22)) {
-                    atomicOr(&v.status[1], 1);
-                    break;
+        load(max(q - 1, p), un);
+        if (t < kNB) {
+            unsigned long long bits = 0;   // 0.0 beyond the matrix
+            if (q * kNB + t < n) {
+                const unsigned long long* x = reinterpret_cast<const unsigned long long*>(v.x) + q * kNB + t;
+                int spins = 0;
+                while ((bits = __hip_atomic_load(x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == kNoValue) {
+                    if (++spins > (1 << 22)) {
+                        atomicOr(&v.status[1], 1);
+                        break;
+                    }
                 }
             }
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            xq[q & 1][t] = __longlong_as_double((long long)bits);
         }
-        __syncthreads();
-        if (t < kNB) {
-            xq[t] = (t < cb) ? v.x[C0 + t] : 0.0;
-        }
-        __syncthreads();
+        __syncthreads();   // two buffers: this one is written again only after the next barrier
 #pragma unroll
-        for (int c = 0; c < 16; ++c) acc += Ub[r * LD + chunk * 16 + c] * xq[chunk * 16 + c];
-        __syncthreads();
+        for (int c = 0; c < 16; ++c) acc[c & 3] += u[c] * xq[q & 1][chunk * 16 + c];
+#pragma unroll
+        for (int c = 0; c < 16; ++c) u[c] = un[c];
     }
-    part[chunk][r] = acc;
+    part[chunk][r] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
     __syncthreads();
-    if (t < kNB) sv[t] = (t < rb) ? v.y[R0 + t] - (part[0][t] + part[1][t] + part[2][t] + part[3][t]) : 0.0;
+    if (t < kNB) sv[t] = t < rb ? y - (part[0][t] + part[1][t] + part[2][t] + part[3][t]) : 0.0;
     __syncthreads();
     {   // x_p = U_pp^{-1} sv, 4 threads per row
-        double s = 0.0;
+        double s[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (int c = 0; c < 16; ++c) s += Ui[r * LD + chunk * 16 + c] * sv[chunk * 16 + c];
-        part[chunk][r] = s;
+        for (int c = 0; c < 16; ++c) s[c & 3] += ui[c] * sv[chunk * 16 + c];
+        part[chunk][r] = (s[0] + s[1]) + (s[2] + s[3]);
     }
     __syncthreads();
-    if (t < rb) v.x[R0 + t] = part[0][t] + part[1][t] + part[2][t] + part[3][t];
-    __syncthreads();
-    if (t == 0) __hip_atomic_store(&v.flags[p], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    if (t < rb)
+        __hip_atomic_store(v.x + R0 + t, part[0][t] + part[1][t] + part[2][t] + part[3][t], __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
 }
 template __global__ void lu_backsolve_kernel<false>(LuArgs, LuFallback);
 template __global__ void lu_backsolve_kernel<true>(LuArgs, LuFallback);

@@ -158,7 +158,6 @@ struct LuArgs {
     double* y;        // forward-substituted right-hand side L^{-1} P b
     double* x;        // solution
     double* uinv;     // per panel: U11^{-1} (64 x 64)
-    int* flags;       // per panel ready flags for the back substitution
     int* status;      // [0] pivot check failed (needs interchanges), [1] spin timeout
     int n;
 };

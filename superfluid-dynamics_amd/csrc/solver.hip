@@ -224,16 +224,13 @@ Solver::Solver(const Phys& ph, const std::vector<int>& n, const Options& opt) : 
     mu_ = dalloc<double>(T_);
     M_ = dalloc<double>(MT_);
     trig_ = dalloc<NodeTrig>(T_);
-    long long utot = 0, ftot = 0;
+    long long utot = 0;
     for (int s = 0; s < S_; ++s) {
         const int P = (n[s] + kNB - 1) / kNB;
         uoff_.push_back(utot);
-        foff_.push_back(ftot);
         utot += (long long)P * kNB * kNB;
-        ftot += P;
     }
     uinv_ = dalloc<double>(utot);
-    flags_ = dalloc<int>(ftot);
     status_ = dalloc<int>(2 * S_);
     piv_ = dalloc<int>(T_);
     counters_ = dalloc<int>(4);
@@ -364,7 +361,7 @@ Solver::~Solver() {
     if (exec_) (void)hipGraphExecDestroy(exec_);
     if (graph_) (void)hipGraphDestroy(graph_);
     void* bufs[] = {d_desc_, d_tw_, Z0_, Za_, Zb_, P0_, Pa_, Pb_, kZ_[0], kZ_[1], kZ_[2], kP_[0],
-                    kP_[1], kP_[2], Zp_, Zpp_, mup_, qup_, b_, work_, y_, mu_, M_, uinv_, flags_,
+                    kP_[1], kP_[2], Zp_, Zpp_, mup_, qup_, b_, work_, y_, mu_, M_, uinv_,
                     status_, piv_, counters_, gmV_, gmZ_, gmS_, gmdiag_, gmw_, gmpart_, gmsmall_, gmctl_, trig_, order_, bstats_, bparts_, bwords_, bxoff_, bxbuf_,
                     gmhist_, gmhvalid_, bhist_, bhvalid_, d_circ_, gmx0_, M32_, ckZ_, ckP_, ckMu_, ckHist_,
                     ckHv_, energy_, D0_, Da_, Db_, ckD_, kD_[0], kD_[1], kD_[2]};
@@ -579,7 +576,6 @@ bool Solver::enqueue_solve(const double2* Z, int stage) {
         a.y = y_ + desc_[s0].voff;
         a.x = mu_ + desc_[s0].voff;
         a.uinv = uinv_ + uoff_[s0];
-        a.flags = flags_ + foff_[s0];
         a.status = status_ + 2 * s0;
         a.n = n;
         for (int k0 = 0; k0 < n; k0 += kNB) {
@@ -1455,7 +1451,7 @@ void debug_lu_solve(int n_in, const double* A_in, const double* b_in, double* x_
     SFH_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
     const int P = (n + kNB - 1) / kNB;
     double *dA, *dA0, *dwork, *dy, *dx, *duinv, *db;
-    int *dflags, *dstatus, *dpiv, *dcnt;
+    int *dstatus, *dpiv, *dcnt;
     SurfDesc desc{};
     desc.n = n;
     SurfDesc* ddesc;
@@ -1466,7 +1462,6 @@ void debug_lu_solve(int n_in, const double* A_in, const double* b_in, double* x_
     SFH_HIP(hipMalloc(&dy, sizeof(double) * n));
     SFH_HIP(hipMalloc(&dx, sizeof(double) * n));
     SFH_HIP(hipMalloc(&duinv, sizeof(double) * P * kNB * kNB));
-    SFH_HIP(hipMalloc(&dflags, sizeof(int) * P));
     SFH_HIP(hipMalloc(&dstatus, sizeof(int) * 2));
     SFH_HIP(hipMalloc(&dpiv, sizeof(int) * n));
     SFH_HIP(hipMalloc(&dcnt, sizeof(int) * 4));
@@ -1478,7 +1473,7 @@ void debug_lu_solve(int n_in, const double* A_in, const double* b_in, double* x_
     SFH_HIP(hipMemcpy(db, b.data(), sizeof(double) * n, hipMemcpyHostToDevice));
     SFH_HIP(hipMemset(dstatus, 0, sizeof(int) * 2));
     SFH_HIP(hipMemset(dcnt, 0, sizeof(int) * 4));
-    LuArgs a{dA, dwork, dy, dx, duinv, dflags, dstatus, n};
+    LuArgs a{dA, dwork, dy, dx, duinv, dstatus, n};
     for (int k0 = 0; k0 < n; k0 += kNB) {
         const int kb = std::min(kNB, n - k0);
         const int rem = n - k0 - kb;
@@ -1500,7 +1495,7 @@ void debug_lu_solve(int n_in, const double* A_in, const double* b_in, double* x_
     SFH_HIP(hipStreamSynchronize(st));
     std::memcpy(x_out, x.data(), n_in * sizeof(double));
     if (interchanged) *interchanged = status[0] ? 1 : 0;
-    void* bufs[] = {dA, dA0, dwork, db, dy, dx, duinv, dflags, dstatus, dpiv, dcnt, ddesc};
+    void* bufs[] = {dA, dA0, dwork, db, dy, dx, duinv, dstatus, dpiv, dcnt, ddesc};
     for (void* p : bufs) (void)hipFree(p);
     (void)hipStreamDestroy(st);
     if (status[1]) throw HipError("back-substitution wait timed out");

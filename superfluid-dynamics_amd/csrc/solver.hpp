@@ -274,11 +274,10 @@ class Solver {
     double* M_ = nullptr;
     NodeTrig* trig_ = nullptr;
     double* uinv_ = nullptr;
-    int* flags_ = nullptr;
     int* status_ = nullptr;
     int* piv_ = nullptr;
     int* counters_ = nullptr;   // [0] fallback solves
-    std::vector<long long> uoff_, foff_;
+    std::vector<long long> uoff_;
     // GMRES workspace
     int gm_m_ = 0, gm_rpw_ = 4;
     double* gmZ_ = nullptr;        // film: the preconditioned basis
