@@ -206,11 +206,13 @@ typedef struct sfh_solver* sfh_handle;
 enum { SFH_WATER = 0, SFH_HELIUM = 1 };
 enum { SFH_FP64 = 0, SFH_MIXED = 1 };
 /* LU: blocked FP64 LU (the reference's getrf/getrs semantics), one surface at a time or uniform
- * batches.  GMRES: FP64 GMRES over the stored matrix, all surfaces of the handle at once (every
- * N <= 4096); with SFH_MIXED the matrix is stored in FP32, r0 and a refinement residual are FP64.
- * BATCHED: one persistent launch per RK stage, one workgroup per surface (every N <= 1024), GMRES
- * inside the workgroup; with SFH_MIXED the matrix is FP32 and mu is refined in FP64 against a
- * matrix-free FP64 residual. */
+ * batches.  GMRES: FP64 GMRES, all surfaces of the handle at once (every N <= 4096), its products
+ * evaluated from the pair sums that the velocity needs too.  With max_iter 1 or under
+ * rho_quirk (rho != 0) the matrix is stored instead; only there SFH_MIXED makes a difference (the
+ * matrix in FP32, r0 and a refinement residual in FP64).
+ * BATCHED: one persistent launch per RK stage, one workgroup per surface or, with fewer surfaces than
+ * CUs, several for the large ones (every N <= 1024), GMRES inside; with SFH_MIXED a stored matrix is
+ * FP32 and mu is refined in FP64 against a matrix-free FP64 residual. */
 enum { SFH_SOLVE_LU = 0, SFH_SOLVE_GMRES = 1, SFH_SOLVE_BATCHED = 2, SFH_SOLVE_AUTO = 3 };
 
 /* Nondimensional problem (ProblemProperties.hpp:5-32 plus kind and g).  g scales the restoring
@@ -242,7 +244,8 @@ typedef struct sfh_options {
     int force_trim;   /* test hook (0 = off): length of the trimmed GMRES launch sequence instead of
                          the calibrated one (at least 2), also for the warm-started transposed solves
                          of sfh_traj_backward; a chunk of steps (a segment of the sweep) in which a
-                         solve runs out of launches is still run again with the length doubled */
+                         solve runs out of launches is still run again with the length doubled.
+                         SFH_SOLVE_BATCHED: at most that many workgroups per surface */
     double tol;       /* iterative solver / refinement relative tolerance */
     int pair_rows;    /* rows per workgroup of the pair kernels (assembly, velocity): 1, 2 or 4; 0 = 4 */
     int reserved;

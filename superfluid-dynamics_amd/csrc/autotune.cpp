@@ -3,9 +3,9 @@
 //
 // The reference fixes its launch shapes (16 x 16 threads per matrix block, 256 per vector kernel,
 // BoundaryProblem.cuh:27-34) and always solves with getrf/getrs (MatrixSolver.cuh:113-172).  Here the
-// right choice depends on N: the blocked LU is latency-bound for small N, GMRES is HBM-bound for large
-// N, the persistent batched kernel suits N <= 1024, and a workgroup of 4 rows leaves most CUs idle
-// when N / 4 is well below the CU count.  autotune() times each candidate on a seeded 8-mode surface
+// right choice depends on N: the blocked LU is a serial chain of panels, GMRES a few launches bound by their
+// latency (small N) or by FP64 issue (large N), the persistent batched kernel suits N <= 1024, and a workgroup of
+// 4 rows leaves most CUs idle when N / 4 is well below the CU count.  autotune() times each candidate on a seeded 8-mode surface
 // of the handle's physics (warm-up through the GMRES calibration, then timed steps replayed from the
 // step graph), rejects candidates whose solves do not converge, and keeps the fastest.  Results are
 // cached per (GPU architecture, problem kind, image term, N, mixed allowed) in memory and in a text

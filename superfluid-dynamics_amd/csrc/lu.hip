@@ -833,7 +833,7 @@ __device__ void fallback_solve(const LuFallback& f, int s) {
 // else is on it: the entries of x are polled themselves (agent scope, past the XCDs' L2 caches; a flag would add a fence
 // and a load behind it), thread (r, chunk) holds its 16 entries of U_pq in registers, loaded while it waits for the block
 // before, and one barrier separates the blocks.  N = 2048 67 -> 52 us,
-// N = 768 25 -> 21, N = 256 8.1 -> 7.5; with 8-byte loads of the rows 75 at N = 2048, as much as through LDS.
+// N = 768 25 -> 21, N = 256 9.5 -> 7.7; with 8-byte loads of the rows 75 at N = 2048, as much as through LDS.
 // FALLBACK: when the factorisation needed interchanges, the surface's first workgroup solves its system anew instead
 // (fallback_solve); as launches of their own the two kernels of that cost every solve 9 us to find nothing to do.
 template <bool FALLBACK>

@@ -308,7 +308,7 @@ std::vector<int> Solver::batched_parts() const {
 void Solver::alloc_gmres(int m) {
     if (gmV_) return;
     gm_m_ = m;   // at most kMaxKrylov basis vectors (gmres.hip)
-    // rows per workgroup of the Arnoldi launches.  Every workgroup repeats the step's finishing work, so few
+    // rows per workgroup of the Arnoldi launches over a stored matrix.  Every workgroup repeats the step's finishing work, so few
     // large ones are better once they still fill the GPU: N = 4096 film 34.6 ms per 40 steps with 16 rows.  At
     // N = 2048 (512 workgroups of 4 rows, two per CU) their longer start costs more than it saves: 26.7 ms per
     // 100 steps with 4 rows, 29.8 with 8 and 28.6 - 31.0 with 16; N = 1536 mixed 18.0, 17.9 and 18.7.
