@@ -130,7 +130,7 @@ __global__ void assemble_small_kernel(const SurfDesc* sd, const NodeTrig* trig, 
                                       const double2* Zpp, double* M, Phys ph);
 template <int NA>
 __global__ void velocity_small_kernel(const SurfDesc* sd, const NodeTrig* trig, const double2* Z, const double2* Zp,
-                                      const double2* Zpp, const double* mu, const double2* mup, Phys ph, StageCtl ctl);
+                                      const double2* Zpp, const double* mu, const double* circ, Phys ph, StageCtl ctl);
 // ---- assemble.hip
 // R = rows per workgroup: 1, 2 or 4 (instantiated in assemble.hip)
 template <int R>

@@ -704,16 +704,17 @@ void Solver::enqueue_rhs(const double2* Z, const double* P, const StageCtl& ctl_
                                     (const NodeTrig*)trig_, Z, Zp_, Zpp_, M_, ph_, ga, gm_on));
         });
     }
-    if (!enqueue_solve(Z, ctl.stage)) {
+    const bool fused_mup = small && !quirk;
+    if (!enqueue_solve(Z, ctl.stage) && !fused_mup) {
         launch("mu_deriv", 4.0 * nsq, 24.0 * nsq / kCircRowsPerWG, [&] {
             SFH_WITH_CIRC(maxN_, go(mu_circ_kernel<TC, TR>, circ_grid(8 * TR), dim3(TC * TR), 0, d_desc_,
                                     (const double*)d_circ_, (const double*)mu_, mup_));
         });
     }
     launch("velocity", img * nsq, 96.0 * T_, [&] {
-        if (small && !quirk)
+        if (fused_mup)
             go(ph_.image ? velocity_small_kernel<4> : velocity_small_kernel<2>, sgrid, dim3(256), 0, d_desc_,
-               (const NodeTrig*)trig_, Z, Zp_, Zpp_, mu_, mup_, ph_, ctl);
+               (const NodeTrig*)trig_, Z, Zp_, Zpp_, mu_, (const double*)d_circ_, ph_, ctl);
         else
             SFH_WITH_ROWS(rows_, go(velocity_stage_kernel<R>, dim3((maxN_ + R - 1) / R, S_), dim3(256), 0, d_desc_,
                                 (const NodeTrig*)trig_, Z, Zp_, Zpp_, mu_, mup_, ph_, ctl));

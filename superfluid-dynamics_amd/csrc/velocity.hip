@@ -156,19 +156,33 @@ __global__ __launch_bounds__(256) void velocity_stage_kernel(const SurfDesc* __r
 
 // Surfaces of up to 256 nodes, not with the rho quirk: a wave has 4 rows and all their columns, 16 pairs per lane, and its
 // own sums.  With 256 threads across the columns a workgroup had 4 pairs per thread and was mostly first loads, reductions
-// and the rows' end: 64 surfaces of 256 nodes 39 us with velocity_stage_kernel<4>, 16 here.
+// and the rows' end: 64 surfaces of 256 nodes 39 us with velocity_stage_kernel<4>, 16 here.  mu' of the rows is formed
+// here too, from a window of the derivative's kernel in LDS that the workgroup's 16 rows share: 15.8 -> 16.2 us there and
+// 4.9 -> 5.9 for one surface, for a launch of 4.5 us less.
 template <int NA>
 __global__ __launch_bounds__(256) void velocity_small_kernel(const SurfDesc* __restrict__ sd, const NodeTrig* __restrict__ trig,
                                                              const double2* __restrict__ Z, const double2* __restrict__ Zp,
                                                              const double2* __restrict__ Zpp, const double* __restrict__ mu,
-                                                             const double2* __restrict__ mup, Phys ph, StageCtl ctl) {
-    __shared__ double red[4][4 * NA];
+                                                             const double* __restrict__ circ, Phys ph, StageCtl ctl) {
+    constexpr int WIN = kSmallRows + kSmallNodes;   // entry u of the window is c[(k0 + kSmallRows - 1 - u) mod n], k0 the first row
+    __shared__ double red[4][4 * NA + 8], c1[2][WIN];
     const SurfDesc d = sd[blockIdx.y];
     const int n = d.n, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int k0 = blockIdx.x * kSmallRows + 4 * w;
     if (blockIdx.x * kSmallRows >= n) return;   // the whole workgroup: the waves meet below
     const NodeTrig* tr = trig + d.voff;
     const double eh = exp(ph.depth), ehi = exp(-ph.depth);
+    const double* c1r = circ + d.coff;
+    double cw[2][2];
+    {
+        int q = ((int)blockIdx.x * kSmallRows + kSmallRows - 1 - (int)threadIdx.x) % n;
+        if (q < 0) q += n;
+        const int q2 = (q + n - 256 % n) % n;
+        cw[0][0] = c1r[q];
+        cw[0][1] = c1r[n + q];
+        cw[1][0] = c1r[q2];
+        cw[1][1] = c1r[n + q2];
+    }
     NodeTrig tk[4], tj[4];
     double mj[4];
 #pragma unroll
@@ -181,7 +195,7 @@ __global__ __launch_bounds__(256) void velocity_small_kernel(const SurfDesc* __r
     for (int r = 0; r < 4; ++r) tk[r] = tr[min(k0 + r, n - 1)];
     const int k = k0 + lane, g = d.voff + min(k, n - 1);
     const bool own = lane < 4 && k < n;
-    double2 zp = {1.0, 0.0}, zpp = {0.0, 0.0}, mp = {0.0, 0.0}, z = {0.0, 0.0};
+    double2 zp = {1.0, 0.0}, zpp = {0.0, 0.0}, z = {0.0, 0.0};
     double m = 0.0;
     StageIn st{};
     if (own) {
@@ -189,12 +203,16 @@ __global__ __launch_bounds__(256) void velocity_small_kernel(const SurfDesc* __r
         zpp = Zpp[g];
         z = Z[g];
         st = stage_load(ctl, g);
-        mp = mup[g];
         m = mu[g];
     }
-    double acc[4 * NA];
 #pragma unroll
-    for (int q = 0; q < 4 * NA; ++q) acc[q] = 0.0;
+    for (int h = 0; h < 2; ++h) {
+        c1[h][threadIdx.x] = cw[0][h];
+        if (threadIdx.x < kSmallRows) c1[h][256 + threadIdx.x] = cw[1][h];
+    }
+    double acc[4 * NA + 8];
+#pragma unroll
+    for (int q = 0; q < 4 * NA + 8; ++q) acc[q] = 0.0;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const int j = lane + 64 * e;
@@ -214,18 +232,32 @@ __global__ __launch_bounds__(256) void velocity_small_kernel(const SurfDesc* __r
             }
         }
     }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int j = lane + 64 * e;
+        if (j >= n) break;
+        const int u = kSmallRows - 1 - 4 * w + j;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            acc[4 * NA + r] += c1[0][u - r] * mj[e];
+            acc[4 * NA + 4 + r] += c1[1][u - r] * mj[e];
+        }
+    }
     reduce_lanes(acc, red[w]);
     __syncthreads();
     if (!own) return;
     const double* S = red[w] + lane;
+    const double xs = 2.0 * kPi / n;
+    const double2 mp = {S[4 * NA] * xs, S[4 * NA + 4] * xs};
     double2 q1, q2;
     velocity_from_sums(ph, zp, zpp, mp, m, z.y, S[0], S[4], NA == 4 ? S[NA == 4 ? 8 : 0] : 0.0, NA == 4 ? S[NA == 4 ? 12 : 0] : 0.0, q1, q2);
     finish_node(ph, ctl, g, z, zp, zpp, m, q1, q2, q1, st);
 }
 template __global__ void velocity_small_kernel<2>(const SurfDesc*, const NodeTrig*, const double2*, const double2*, const double2*,
-                                                  const double*, const double2*, Phys, StageCtl);
+                                                  const double*, const double*, Phys, StageCtl);
 template __global__ void velocity_small_kernel<4>(const SurfDesc*, const NodeTrig*, const double2*, const double2*, const double2*,
-                                                  const double*, const double2*, Phys, StageCtl);
+                                                  const double*, const double*, Phys, StageCtl);
 
 // rows per workgroup the solver may launch with (chosen per surface size by the autotuner)
 #define SFH_VELOCITY_INSTANCES(R)                                                                                  \
