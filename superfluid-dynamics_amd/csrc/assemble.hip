@@ -15,7 +15,7 @@
 // With the GMRES solver the kernel also starts the solve: while it writes row k it accumulates
 // (M x0)_k and stores r0_k = b_k - (M x0)_k as the first (unnormalised) basis vector; the first
 // Arnoldi step normalises it.
-#include "sfh_kernels.hpp"
+#include "sfh_circ.hpp"
 
 namespace sfh {
 
@@ -146,47 +146,118 @@ __global__ __launch_bounds__(256) void residual64_kernel(const SurfDesc* __restr
     assemble_rows<double, R>(sd, trig, Z, Zp, Zpp, static_cast<double*>(nullptr), ph, gm, 1, true);
 }
 
-// Surfaces of up to 256 nodes (LU): a wave has 4 rows and all their columns, 16 entries per lane, and only the rows' own
-// lanes form the diagonal.  With 256 threads across the columns a workgroup had 4 entries per thread and was mostly
-// first loads and row constants: 64 surfaces of 256 nodes 34 us with assemble64_kernel<4>, 16 here.
-__global__ __launch_bounds__(256) void assemble_small_kernel(const SurfDesc* __restrict__ sd, const NodeTrig* __restrict__ trig,
-                                                             const double2* __restrict__ Z, const double2* __restrict__ Zp,
-                                                             const double2* __restrict__ Zpp, double* __restrict__ M, Phys ph) {
+// Surfaces of up to 256 nodes (LU): the derivatives, the half-angle table and the matrix rows in one launch.  A wave has 4
+// rows and all their columns, 16 products and 16 entries per lane, and only the rows' own lanes form the diagonal; a
+// workgroup's 16 rows share the samples, the table (formed anew by every workgroup) and the windows of the derivatives'
+// kernels in LDS.  With 256 threads across the columns a workgroup had 4 entries per thread and was mostly first loads and
+// row constants: 64 surfaces of 256 nodes 34 us with assemble64_kernel<4>, 16 with whole rows; that and the
+// derivatives' launch 16.8 + 6.5 us, 19.2 together; one surface of 256 4.9 + 4.8, 6.3 together.
+__global__ __launch_bounds__(256) void form_small_kernel(const SurfDesc* __restrict__ sd, const double* __restrict__ circ,
+                                                         const double2* __restrict__ Z, const double* __restrict__ phi,
+                                                         double2* __restrict__ Zp, double2* __restrict__ Zpp,
+                                                         double* __restrict__ b, double* __restrict__ work,
+                                                         double* __restrict__ M, NodeTrig* __restrict__ trig, Phys ph,
+                                                         int* __restrict__ status) {
+    constexpr int WIN = kSmallRows + kSmallNodes;   // entry u of a window is c[(kb + kSmallRows - 1 - u) mod n], kb the first row
+    __shared__ double zx[kSmallNodes], zy[kSmallNodes], p[kSmallNodes];   // samples minus their linear parts
+    __shared__ double ts[kSmallNodes], tc[kSmallNodes], te[kSmallNodes], ti[kSmallNodes];
+    __shared__ double cw[3][WIN], red[4][20];
     const SurfDesc d = sd[blockIdx.y];
-    const int n = d.n, lane = threadIdx.x & 63;
-    const int k0 = blockIdx.x * kSmallRows + 4 * (threadIdx.x >> 6);
+    const int n = d.n, off = d.voff, t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int kb = blockIdx.x * kSmallRows, k0 = kb + 4 * w;
+    if (kb >= n) return;   // the whole workgroup
+    if (blockIdx.x == 0 && t == 0) status[2 * blockIdx.y] = 0;   // re-armed for the solve that follows
+    const double xs = 2.0 * kPi / n;                       // Derivatives.cuh:285,317
+    const double plin = -(1 + ph.rho) * kPi * ph.U / n;    // Derivatives.cuh:286
+    const double2 zt = Z[off + min(t, n - 1)];
+    const double pt = phi[off + min(t, n - 1)];
+    int q = (kb + kSmallRows - 1 - t) % n;
+    if (q < 0) q += n;
+    const int q2 = (q + n - 256 % n) % n;
+    double c[2][3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        c[0][i] = circ[d.coff + i * n + q];
+        c[1][i] = circ[d.coff + i * n + q2];
+    }
+    const NodeTrig own = node_trig(zt);
+    zx[t] = t < n ? zt.x - 2 * kPi * (double)t / n : 0.0;
+    zy[t] = t < n ? zt.y : 0.0;
+    p[t] = t < n ? pt - plin * (double)t : 0.0;
+    ts[t] = own.s;
+    tc[t] = own.c;
+    te[t] = own.e;
+    ti[t] = own.ei;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        cw[i][t] = c[0][i];
+        if (t < kSmallRows) cw[i][256 + t] = c[1][i];
+    }
+    __syncthreads();
+    double acc[20];   // 4 rows each of Re Z', Im Z', Re Z'', Im Z'', Re Phi'
+#pragma unroll
+    for (int i = 0; i < 20; ++i) acc[i] = 0.0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int j = lane + 64 * e;
+        if (j >= n) break;
+        const double x = zx[j], y = zy[j], f = p[j];
+        const int u = kSmallRows - 1 - 4 * w + j;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const double wr = cw[0][u - r], wi = cw[1][u - r], w2 = cw[2][u - r];
+            acc[r] += wr * x;
+            acc[r] -= wi * y;
+            acc[4 + r] += wr * y;
+            acc[4 + r] += wi * x;
+            acc[8 + r] += w2 * x;
+            acc[12 + r] += w2 * y;
+            acc[16 + r] += wr * f;
+        }
+    }
+    reduce_lanes(acc, red[w]);
+    __syncthreads();
     if (k0 >= n) return;
-    const NodeTrig* tr = trig + d.voff;
+    const double* S = red[w];
     double* Mk = M + d.moff + (long long)k0 * n;
-    const double c = ph.kind == 0 ? 0.25 * (1 - ph.rho) / kPi : 0.25 / kPi, ci = 0.25 / kPi;
+    const double cm = ph.kind == 0 ? 0.25 * (1 - ph.rho) / kPi : 0.25 / kPi, ci = 0.25 / kPi;
     const double h = ph.depth, eh = exp(h), ehi = exp(-h);
-    NodeTrig tk[4], tj[4];
+    if (lane < 4 && k0 + lane < n) {
+        const int k = k0 + lane, g = off + k;
+        const double s2 = 4.0 * kPi * kPi / ((double)n * n);                  // Derivatives.cuh:321
+        const double2 zp = {S[lane] * xs + xs, S[4 + lane] * xs}, zpp = {S[8 + lane] * s2, S[12 + lane] * s2};
+        Zp[g] = zp;                                                           // :323,374
+        Zpp[g] = zpp;
+        double r = S[16 + lane] * xs;                                         // :324, :299
+        if (ph.U != 0) r += -(1 + ph.rho) * kPi * ph.U / n;                   // :380-383
+        b[g] = r;
+        work[g] = r;
+        trig[g] = NodeTrig{ts[k], tc[k], te[k], ti[k]};
+        double v = (ph.kind == 0 ? 0.5 * (1 + ph.rho) : 0.5) + cm * cdiv(zpp, zp).y;
+        if (ph.image) v -= ci * cot64(0.0, zy[k] + h).y;
+        Mk[(long long)lane * n + k] = v;
+    }
+    NodeTrig tk[4];
     double2 zk[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) tj[e] = tr[min(lane + 64 * e, n - 1)];
-#pragma unroll
     for (int r = 0; r < 4; ++r) {
-        tk[r] = tr[min(k0 + r, n - 1)];
-        zk[r] = Zp[d.voff + min(k0 + r, n - 1)];
-    }
-    if (lane < 4 && k0 + lane < n) {
-        const int g = d.voff + k0 + lane;
-        double v = (ph.kind == 0 ? 0.5 * (1 + ph.rho) : 0.5) + c * cdiv(Zpp[g], Zp[g]).y;
-        if (ph.image) v -= ci * cot64(0.0, Z[g].y + h).y;
-        Mk[(long long)lane * n + k0 + lane] = v;
+        const int k = min(k0 + r, n - 1);
+        tk[r] = NodeTrig{ts[k], tc[k], te[k], ti[k]};
+        zk[r] = {S[r] * xs + xs, S[4 + r] * xs};
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const int j = lane + 64 * e;
         if (j >= n) break;
+        const NodeTrig tj = {ts[j], tc[j], te[j], ti[j]};
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             if (k0 + r >= n) break;
             if (j == k0 + r) continue;
-            const CotParts cp = cot_parts(tk[r], tj[e]);
-            double v = cp.id * (c * zk[r].y * cp.p - c * zk[r].x * cp.q);
+            const CotParts cp = cot_parts(tk[r], tj);
+            double v = cp.id * (cm * zk[r].y * cp.p - cm * zk[r].x * cp.q);
             if (ph.image) {
-                const CotParts cq = cot_image_parts(tk[r], tj[e], eh, ehi);
+                const CotParts cq = cot_image_parts(tk[r], tj, eh, ehi);
                 v += ci * (cq.q * cq.id);
             }
             Mk[(long long)r * n + j] = v;

@@ -126,8 +126,8 @@ __global__ void plain_deriv_kernel(const SurfDesc* sd, const double2* tw_all, co
 
 constexpr int kSmallNodes = 256;   // surfaces whose pair kernels give each wave whole rows (LU)
 constexpr int kSmallRows = 16;     // rows per workgroup of those
-__global__ void assemble_small_kernel(const SurfDesc* sd, const NodeTrig* trig, const double2* Z, const double2* Zp,
-                                      const double2* Zpp, double* M, Phys ph);
+__global__ void form_small_kernel(const SurfDesc* sd, const double* circ, const double2* Z, const double* phi, double2* Zp,
+                                  double2* Zpp, double* b, double* work, double* M, NodeTrig* trig, Phys ph, int* status);
 template <int NA>
 __global__ void velocity_small_kernel(const SurfDesc* sd, const NodeTrig* trig, const double2* Z, const double2* Zp,
                                       const double2* Zpp, const double* mu, const double* circ, Phys ph, StageCtl ctl);

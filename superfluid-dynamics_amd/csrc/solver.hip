@@ -670,9 +670,10 @@ void Solver::enqueue_rhs(const double2* Z, const double* P, const StageCtl& ctl_
     double nsq = 0.0;
     for (int v : n_) nsq += (double)v * v;
     const double img = ph_.image ? 2.0 : 1.0;
+    const bool small = !gm_on && maxN_ <= kSmallNodes;
     // circulant derivatives: 7 n^2 multiply-adds; bytes: the samples and kernels each workgroup
     // stages (24 B per node and 24 B per kernel entry)
-    launch("deriv", 14.0 * nsq, 48.0 * nsq / kCircRowsPerWG, [&] {
+    if (!small) launch("deriv", 14.0 * nsq, 48.0 * nsq / kCircRowsPerWG, [&] {
         SFH_WITH_CIRC(maxN_, go(zphi_circ_kernel<TC, TR>, circ_grid(8 * TR), dim3(TC * TR), 0, d_desc_,
                                 (const double*)d_circ_, Z, P, Zp_, Zpp_, b_, work_, ph_, status_, trig_, ga, gm_on));
     });
@@ -687,11 +688,11 @@ void Solver::enqueue_rhs(const double2* Z, const double* P, const StageCtl& ctl_
     }
     // assembly: flops counted as cot evaluations (the transcendental-bound unit), bytes = M written
     const bool quirk = ph_.kind == 0 && ph_.rho_quirk && ph_.rho != 0.0;
-    const bool small = !gm_on && maxN_ <= kSmallNodes;
     const dim3 sgrid((maxN_ + kSmallRows - 1) / kSmallRows, S_);
     if (small) {
-        launch("assemble", img * nsq, 8.0 * nsq, [&] {
-            go(assemble_small_kernel, sgrid, dim3(256), 0, d_desc_, (const NodeTrig*)trig_, Z, Zp_, Zpp_, M_, ph_);
+        launch("assemble", img * nsq, 8.0 * nsq, [&] {   // with the derivatives
+            go(form_small_kernel, sgrid, dim3(256), 0, d_desc_, (const double*)d_circ_, Z, P, Zp_, Zpp_, b_, work_, M_, trig_, ph_,
+               status_);
         });
     } else if (gm_on && opt_.precision == kMixed) {
         launch("assemble", img * nsq, 4.0 * nsq, [&] {
