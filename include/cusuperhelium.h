@@ -247,7 +247,9 @@ typedef struct sfh_options {
                          solve runs out of launches is still run again with the length doubled.
                          SFH_SOLVE_BATCHED: at most that many workgroups per surface */
     double tol;       /* iterative solver / refinement relative tolerance */
-    int pair_rows;    /* rows per workgroup of the pair kernels (assembly, velocity): 1, 2 or 4; 0 = 4 */
+    int pair_rows;    /* rows per workgroup of the pair kernels (assembly, velocity): 1, 2 or 4; 0 = 4.  Without
+                         effect where no such kernel runs: GMRES without a stored matrix, LU of surfaces
+                         of at most 256 nodes each */
     int reserved;
 } sfh_options;
 
