@@ -1733,6 +1733,7 @@ void Solver::rhs_vjp(const double* gvx, const double* gvy, const double* gdphi, 
         c.kP[i] = vKP_[i];
     }
     set_delayed_ctl(c, D0_, nullptr);
+    seq_len_ = gm_m_;           // a standalone solve: no extrapolated guess, the full launch sequence
     enqueue_rhs(Z0_, P0_, c);   // the forward mu at the current state
     SFH_HIP(hipMemcpyAsync(vMu_[0], mu_, T_ * sizeof(double), hipMemcpyDeviceToDevice, stream_));
     enqueue_vjp(Z0_, P0_, vMu_[0], gA_, gAP_, 1.0, nullptr, nullptr, 0.0, gR_[0], gRP_[0], false, -1, gAD_, nullptr,
