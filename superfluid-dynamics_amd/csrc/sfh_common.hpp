@@ -174,12 +174,13 @@ constexpr int kPreModes = 8;   // most modes of the preconditioner, besides the 
 __device__ inline double film_eigenvalue(int n, int m, double height) {
     return 0.5 + n * (0.25 / kPi) * exp(-2.0 * m * height);
 }
-// Modes that the preconditioner takes: up to the one whose eigenvalue is within 4% of 1/2.  On films so thin
-// that it would leave many larger ones out it is not used (-1): with less than half of them it can cost steps
-// (N = 512, height 0.02: 42 against 22 without).
+// Modes that the preconditioner takes: up to the one whose eigenvalue is within 4% of 1/2, and below n/2, where the
+// modes' projections are orthogonal (beyond, mode m is mode n - m again: at n = 3, height 0.107 the sum of the
+// projections is singular).  On films so thin that it would leave many larger ones out it is not used (-1): with less
+// than half of them it can cost steps (N = 512, height 0.02: 42 against 22 without).
 __device__ inline int film_modes(int n, double height) {
     const double m = height > 0.0 ? log(n * (0.25 / kPi / 0.02)) / (2.0 * height) : 1e9;
-    return m < 2 * kPreModes + 1 ? max(0, min(kPreModes, (int)m)) : -1;
+    return m < 2 * kPreModes + 1 ? max(0, min(min(kPreModes, (n - 1) / 2), (int)m)) : -1;
 }
 
 // ------------------------------------------------------------------ wave reductions
