@@ -281,7 +281,7 @@ __device__ inline void back_substitute(const double* g, const double* H, int m, 
 // The stored matrix, RR rows per wave.
 template <typename T, int WAVES, int RR>
 struct StoredRows {
-    static constexpr int W = WAVES, ROWS = W * RR;
+    static constexpr int W = WAVES, ROWS = W * RR, MAXN = kGmMaxN;
     const T* R;
     RowBuf<T, RR> rc;
     int n, row, rows, lane, wv;
@@ -312,7 +312,7 @@ struct StoredRows {
 // launch, of which 22 are issue, N = 2048 water 8 us, of which 3 are issue and 4 the finishing work and first loads.
 template <int NA, int H>
 struct PairSums {
-    static constexpr int W = 4 * H, ROWS = kSumRows * H;
+    static constexpr int W = 4 * H, ROWS = kSumRows * H, MAXN = kGmMaxN;
     const NodeTrig* tr;
     double* S;
     NodeTrig tk[kSumRows];
@@ -369,10 +369,10 @@ struct PairSums {
     }
 };
 
-// The transposed product (reverse mode), one sum per row, nothing kept.
-template <bool FILM>
+// The transposed product (reverse mode), one sum per row, nothing kept.  Surfaces of up to N nodes.
+template <bool FILM, int N>
 struct TransposeSums {
-    static constexpr int W = 4, ROWS = kSumRows;
+    static constexpr int W = 4, ROWS = kSumRows, MAXN = N;
     const NodeTrig* tr;
     const double2* zp;
     NodeTrig tk[kSumRows];
@@ -442,7 +442,7 @@ __device__ __forceinline__ void gm_step(const GmArgs& a, const SurfDesc* __restr
     const int m = a.m;
     constexpr int W = P::W, rpw = P::ROWS, NT = 64 * W, E = 8;   // E entries per thread and pass
     if ((int)blockIdx.x * rpw >= v.n) return;
-    __shared__ double vs[kGmMaxN];
+    __shared__ double vs[P::MAXN];
     __shared__ double co[kMaxKrylov + 1];
     __shared__ double col[kMaxKrylov + 2];
     __shared__ double red8[2 * W];
@@ -663,9 +663,9 @@ __global__ __launch_bounds__(256 * H) void gm_sums_kernel(GmArgs a, const SurfDe
     gm_step<PairSums<NA, H>>(a, sd, i);
 }
 
-template <bool FILM>
+template <bool FILM, int N>
 __global__ __launch_bounds__(256) void gm_tsums_kernel(GmArgs a, const SurfDesc* __restrict__ sd, int i) {
-    gm_step<TransposeSums<FILM>>(a, sd, i);
+    gm_step<TransposeSums<FILM, N>>(a, sd, i);
 }
 
 // The warm start of a transposed solve: r0 = b - M^T x0 as the first basis vector.  grid = (ceil(max n / kSumRows), surfaces).
@@ -684,13 +684,17 @@ __global__ __launch_bounds__(256) void gm_tstart_kernel(GmArgs a, const SurfDesc
     const GmView v = gm_view(a, sd, blockIdx.y);
     const double* x0 = a.x + d.voff;
     const double b = a.b[d.voff + min(r0 + t, d.n - 1)];
-    TransposeSums<FILM> prod(a, v, d, r0);
+    TransposeSums<FILM, kGmMaxNT> prod(a, v, d, r0);   // the product alone keeps nothing of size N
     prod.start();
     const double w = prod.product([&](int j) { return x0[j]; });
     if (t < kSumRows && r0 + t < d.n) a.V[(long long)(a.m + 1) * d.voff + r0 + t] = b - w;
 }
-template __global__ void gm_tsums_kernel<false>(GmArgs, const SurfDesc*, int);
-template __global__ void gm_tsums_kernel<true>(GmArgs, const SurfDesc*, int);
+// the vector of up to 4096 nodes leaves room for four workgroups on a CU; larger surfaces, which only LU handles have,
+// get an instance of their own
+template __global__ void gm_tsums_kernel<false, kGmMaxN>(GmArgs, const SurfDesc*, int);
+template __global__ void gm_tsums_kernel<true, kGmMaxN>(GmArgs, const SurfDesc*, int);
+template __global__ void gm_tsums_kernel<false, kGmMaxNT>(GmArgs, const SurfDesc*, int);
+template __global__ void gm_tsums_kernel<true, kGmMaxNT>(GmArgs, const SurfDesc*, int);
 template __global__ void gm_tstart_kernel<false>(GmArgs, const SurfDesc*, int);
 template __global__ void gm_tstart_kernel<true>(GmArgs, const SurfDesc*, int);
 

@@ -9,7 +9,8 @@
 namespace sfh {
 
 constexpr int kMaxKrylov = 32;     // basis vectors per solve (iteration cap)
-constexpr int kGmMaxN = 4096;      // LDS copy of the vector being multiplied
+constexpr int kGmMaxN = 4096;      // nodes of a surface of the GMRES solver: LDS copy of the vector being multiplied
+constexpr int kGmMaxNT = 8192;     // ... of a transposed solve (LU handles take surfaces of up to 8192 nodes)
 
 struct GmCtl {
     int done;          // 0 while the solve runs, else 1 + the launch that finished it

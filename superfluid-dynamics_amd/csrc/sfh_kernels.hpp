@@ -204,7 +204,7 @@ __global__ void gm_sums_kernel(GmArgs a, const SurfDesc* sd, int j);
 // transposed products (reverse mode): the first residual, one launch per Arnoldi step
 template <bool FILM>
 __global__ void gm_tstart_kernel(GmArgs a, const SurfDesc* sd, int reset);
-template <bool FILM>
+template <bool FILM, int N>   // N: most nodes of a surface
 __global__ void gm_tsums_kernel(GmArgs a, const SurfDesc* sd, int j);
 // PRE: the basis is preconditioned; NA > 0: also the velocity stage, from the solve's sums (else Z, Zpp, ph, sc unused)
 template <bool PRE, int NA>

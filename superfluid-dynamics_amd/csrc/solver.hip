@@ -501,7 +501,10 @@ bool Solver::enqueue_gmres(const GmArgs& a, bool force64, const double2* Z, cons
                     go(kernel, grid, dim3(64 * waves), 0, a, (const SurfDesc*)d_desc_, j);
                 };
                 if (a.sums < 0) {
-                    step(ph_.image ? gm_tsums_kernel<true> : gm_tsums_kernel<false>, 4);
+                    if (maxN_ <= kGmMaxN)
+                        step(ph_.image ? gm_tsums_kernel<true, kGmMaxN> : gm_tsums_kernel<false, kGmMaxN>, 4);
+                    else
+                        step(ph_.image ? gm_tsums_kernel<true, kGmMaxNT> : gm_tsums_kernel<false, kGmMaxNT>, 4);
                 } else if (a.sums == 2) {
                     a.rpw == 4 ? step(gm_sums_kernel<2, 1>, 4) : step(gm_sums_kernel<2, 2>, 8);
                 } else if (a.sums == 4) {
