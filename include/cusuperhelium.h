@@ -282,7 +282,8 @@ typedef struct sfh_stats {
     int spin_timeouts;
     int last_iterations;   /* GMRES: iterations of surface 0 in the last solve */
     int max_iterations;    /* GMRES: most iterations any surface needed in the last solve */
-    int unconverged;       /* GMRES: solves of kept steps that reached the iteration cap (accumulated) */
+    int unconverged;       /* GMRES: solves of kept steps that reached the iteration cap (accumulated); LU: transposed
+                              solves that did */
     int refinements;       /* mixed precision, surface 0, last solve: FP64 refinement sweeps (batched);
                               1 if the refinement solve ran Arnoldi steps, else 0 (GMRES) */
     int redone_steps;      /* SFH_SOLVE_GMRES: steps run again because a solve of their chunk ran out of

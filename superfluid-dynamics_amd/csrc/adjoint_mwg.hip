@@ -302,8 +302,8 @@ __global__ __launch_bounds__(256) void adj_gm_start_kernel(const SurfDesc* __res
 }
 
 // The warm start of a transposed solve: x0 = the extrapolation (quartic once five are kept) of the
-// solutions of the same stage over the previous reverse steps, kept in a ring of kHistDepth vectors
-// (slot (head - l) mod kHistDepth holds the solution l steps back).
+// solutions of the same stage over the previous reverse steps, kept in a ring of kAdjRing vectors
+// (slot (head - l) mod kAdjRing holds the solution l steps back).
 __global__ __launch_bounds__(256) void adj_extrapolate_kernel(const double* __restrict__ ring, int head, int hv,
                                                               double* __restrict__ x0, int total) {
     const int i = blockIdx.x * 256 + threadIdx.x;
@@ -311,7 +311,7 @@ __global__ __launch_bounds__(256) void adj_extrapolate_kernel(const double* __re
     double h[kHistDepth];
 #pragma unroll
     for (int l = 0; l < kHistDepth; ++l) {
-        const int slot = (head - l + kHistDepth) % kHistDepth;
+        const int slot = (head - l + kAdjRing) % kAdjRing;
         h[l] = l < hv ? ring[(long long)slot * total + i] : 0.0;
     }
     x0[i] = extrapolate_values(h, hv);

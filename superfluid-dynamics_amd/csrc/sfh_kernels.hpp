@@ -336,6 +336,9 @@ template <int R> __global__ void adj_pass_b_kernel(AdjMArgs a, Phys ph);
 template <int R> __global__ void adj_pass_c_kernel(AdjMArgs a, Phys ph);
 __global__ void adj_circ_d1_kernel(const SurfDesc* sd, const double* circ, const double2* v, double2* out);
 __global__ void adj_gm_start_kernel(const SurfDesc* sd, const double* b, double* V, double* x, int* ctl, int m, int reset);
+// slots of a stage's ring of transposed solutions: the kHistDepth in use and the one that the next solve writes, so
+// that a reverse step can be run again
+constexpr int kAdjRing = kHistDepth + 1;
 __global__ void adj_extrapolate_kernel(const double* ring, int head, int hv, double* x0, int total);
 __global__ void adj_gamma_kernel(AdjMArgs a, Phys ph);
 __global__ void adj_final_kernel(AdjMArgs a, const double* circ, const double2* sd1gb);

@@ -1389,12 +1389,12 @@ void Solver::parse_status() {
         most_ = most;
         unc_raw_ = unc;
         unc -= unc_discard_;
+        stats_.unconverged = unc;   // of an LU handle: transposed solves
         if (opt_.solver == kSolveGMRES) {
             stats_.last_iterations = ctl[2];
             // mixed precision: 1 when surface 0's last refinement solve ran Arnoldi steps
             if (opt_.precision == kMixed) stats_.refinements = ctl[1] > 0 ? 1 : 0;
             stats_.max_iterations = mx;
-            stats_.unconverged = unc;
         }
     }
     if (opt_.solver == kSolveBatched) {
@@ -1523,8 +1523,8 @@ void Solver::ensure_vjp() {
         agb_ = dalloc<double>(T_);
         aquirk_ = dalloc<double>((size_t)3 * T_);
         SFH_HIP(hipMemset(agamI_, 0, T_ * sizeof(double2)));
-        adjRing_ = dalloc<double>((size_t)4 * kHistDepth * T_);
-        adjSave_ = dalloc<double>((size_t)4 * kHistDepth * T_);
+        adjRing_ = dalloc<double>((size_t)4 * kAdjRing * T_);
+        adjSave_ = dalloc<double>((size_t)4 * kAdjRing * T_);
         adjSaveZ_ = dalloc<double2>(T_);
         adjSaveP_ = dalloc<double>(T_);
     }
@@ -1632,8 +1632,8 @@ void Solver::enqueue_vjp_mwg(const double2* Z, const double* P, const double* mu
     a.gmu = agmu_;
     // inside a sweep the solution goes straight to its slot of the stage's ring
     const bool ring = adj_warm_ && stage >= 0;
-    const int slot = ring ? (adj_head_[stage] + 1) % kHistDepth : 0;
-    double* const gb = ring ? adjRing_ + ((size_t)stage * kHistDepth + slot) * T_ : agb_;
+    const int slot = ring ? (adj_head_[stage] + 1) % kAdjRing : 0;
+    double* const gb = ring ? adjRing_ + ((size_t)stage * kAdjRing + slot) * T_ : agb_;
     a.gb = gb;
     a.gam = agam_;
     a.gamI = agamI_;
@@ -1679,7 +1679,7 @@ void Solver::enqueue_vjp_mwg(const double2* Z, const double* P, const double* mu
         g.Z = gmV_;
         if (warm) {
             go(adj_extrapolate_kernel, dim3((T_ + 255) / 256), dim3(256), 0,
-               (const double*)(adjRing_ + (size_t)stage * kHistDepth * T_), adj_head_[stage], adj_hv_[stage], gmx0_, T_);
+               (const double*)(adjRing_ + (size_t)stage * kAdjRing * T_), adj_head_[stage], adj_hv_[stage], gmx0_, T_);
             go(ph_.image ? gm_tstart_kernel<true> : gm_tstart_kernel<false>, dim3((maxN_ + kSumRows - 1) / kSumRows, S_),
                dim3(256), 0, g, (const SurfDesc*)d_desc_, reset);
         } else {
@@ -1878,6 +1878,8 @@ int Solver::traj_forward(double dt, int steps, int every) {
             rr.HV = dalloc<int>((size_t)nck * rr.hv_len);
         }
         rr.hist_steps.assign(nck, 0);
+        rr.unc.assign(nck, 0);
+        check_status();
         for (int c = 0; c < nck; ++c) {
             SFH_HIP(hipMemcpyAsync(rr.Z + (size_t)c * T_, Z0_, T_ * sizeof(double2), hipMemcpyDeviceToDevice, stream_));
             SFH_HIP(hipMemcpyAsync(rr.P + (size_t)c * T_, P0_, T_ * sizeof(double), hipMemcpyDeviceToDevice, stream_));
@@ -1889,7 +1891,12 @@ int Solver::traj_forward(double dt, int steps, int every) {
                                        stream_));
             }
             rr.hist_steps[c] = hist_steps_;
+            const int unc = stats_.unconverged;
             step(dt, std::min(every, steps - c * every));
+            if (opt_.solver == kSolveGMRES) {
+                check_status();
+                rr.unc[c] = stats_.unconverged - unc;
+            }
         }
         rr.fill_len = fill_len_;
         check_status();
@@ -1931,8 +1938,9 @@ void Solver::traj_backward(int record, const double* gx_in, const double* gy_in,
     // transposed solves (LU and GMRES handles): warm-started from each stage's solutions of the
     // previous reverse steps.  The first reverse step runs full launch sequences; while the stages' rings
     // fill, each step's solves get the launches that the step before needed and two spare ones, and the
-    // first step with full rings sets the length of all later ones (its need and a spare).  A segment in
-    // which a solve ran out is swept again with full sequences from its saved start, and the length doubles.
+    // first step with full rings sets the length of all later ones (its need and a spare).  A step of the former in
+    // which a solve ran out is run again with full sequences, and so is, from its saved start, a segment with such a
+    // step of the latter, and the length doubles.
     const bool mwg = opt_.solver != kSolveBatched;
     struct SweepState {   // the warm-start state lives only inside this sweep, whatever ends it
         Solver* s;
@@ -1947,14 +1955,14 @@ void Solver::traj_backward(int record, const double* gx_in, const double* gy_in,
     for (int st = 0; st < 4; ++st) adj_head_[st] = adj_hv_[st] = 0;
     int sweep_len = 0;        // launches per solve once the rings are full (0: not known yet)
     int fill = 0;             // and of the next step while they fill (0: the full sequence)
-    bool adapt = mwg;         // shorter sequences while they fill
     for (int seg = nck - 1; seg >= 0; --seg) {
         const int n = std::min(r.every, r.steps - seg * r.every);
         // y_s, ..., y_{s+n-1}: the checkpoint, then n - 1 steps from it, each step keeping its stage
         // states and stage mu (the last step runs only for them).  The solves are warm-started from
         // the stage histories as in the forward pass; GMRES solves get the forward pass's launch
         // sequences, while the histories fill and after that, and a segment in which
-        // one ran out of launches is run again with full sequences.
+        // one ran out of launches (beside those that ran out in the forward pass, where the full sequence
+        // did not converge either) is run again with full sequences.
         const double2* ckZ = r.Z + (size_t)seg * T_;
         const double* ckP = r.P + (size_t)seg * T_;
         const bool gmres = opt_.solver == kSolveGMRES;
@@ -1991,27 +1999,47 @@ void Solver::traj_backward(int record, const double* gx_in, const double* gy_in,
             const int unc0 = unc_raw_;
             rerun(true);
             sync();
-            if (unc_raw_ > unc0) {
+            if (unc_raw_ - unc0 > r.unc[seg]) {
                 unc_discard_ += unc_raw_ - unc0;
-                stats_.unconverged = unc_raw_ - unc_discard_;
                 stats_.redone_steps += n;
                 rerun(false);
             }
         } else {
             rerun(false);
         }
-        bool shortened = false;
+        bool shortened = false;   // steps with full rings whose solves got fewer launches
+        int unc0 = 0;             // unc_raw_ before the first of them
         auto sweep = [&](bool full) {
             for (int i = n - 1; i >= 0; --i) {
                 bool rings = mwg;
                 for (int st = 0; st < 4; ++st) rings = rings && adj_hv_[st] >= kHistDepth;
-                adj_len_ = full ? 0 : rings && sweep_len > 0 ? sweep_len : fill;
-                shortened = shortened || adj_len_ > 0;
-                adj_first_ = mwg;
+                const bool filling = mwg && sweep_len == 0;
+                int len = full ? 0 : filling ? fill : sweep_len;
+                if (len >= gm_m_) len = 0;
+                shortened = shortened || (!filling && len > 0);
+                int head[4], hv[4];
+                std::copy(adj_head_, adj_head_ + 4, head);
+                std::copy(adj_hv_, adj_hv_ + 4, hv);
                 const StageCapture cap = seg_capture(i);
-                enqueue_step_vjp(r.dt, segZ_ + (size_t)i * T_, segP_ + (size_t)i * T_, &cap);
-                if (mwg && sweep_len == 0 && (rings || adapt)) {
+                const auto step_back = [&](int launches) {
+                    adj_len_ = launches;
+                    adj_first_ = mwg;
+                    enqueue_step_vjp(r.dt, segZ_ + (size_t)i * T_, segP_ + (size_t)i * T_, &cap);
+                };
+                step_back(len);
+                if (filling) {
                     sync();   // most_: the Arnoldi steps this step's solves took
+                    if (len > 0 && unc_raw_ > unc0) {
+                        // one ran out of launches: this step again (its cotangent is still in gA_, and the slots it
+                        // wrote were not in use) rather than the segment, whose steps before this one are sound
+                        unc_discard_ += unc_raw_ - unc0;
+                        stats_.redone_steps += 1;
+                        std::copy(head, head + 4, adj_head_);
+                        std::copy(hv, hv + 4, adj_hv_);
+                        step_back(0);
+                        sync();
+                    }
+                    unc0 = unc_raw_;
                     if (rings) {
                         sweep_len = std::min(gm_m_, most_ + 2);
                         if (opt_.force_trim > 0) sweep_len = std::max(2, std::min(gm_m_, opt_.force_trim));
@@ -2025,7 +2053,7 @@ void Solver::traj_backward(int record, const double* gx_in, const double* gy_in,
             adj_len_ = 0;
         };
         if (mwg) {
-            const size_t ring = (size_t)4 * kHistDepth * T_ * sizeof(double);
+            const size_t ring = (size_t)4 * kAdjRing * T_ * sizeof(double);
             SFH_HIP(hipMemcpyAsync(adjSaveZ_, gA_, zb, hipMemcpyDeviceToDevice, stream_));
             SFH_HIP(hipMemcpyAsync(adjSaveP_, gAP_, pb, hipMemcpyDeviceToDevice, stream_));
             SFH_HIP(hipMemcpyAsync(adjSave_, adjRing_, ring, hipMemcpyDeviceToDevice, stream_));
@@ -2033,12 +2061,11 @@ void Solver::traj_backward(int record, const double* gx_in, const double* gy_in,
             std::copy(adj_head_, adj_head_ + 4, head);
             std::copy(adj_hv_, adj_hv_ + 4, hv);
             sync();
-            const int unc0 = unc_raw_;
+            const int seg_unc = unc0 = unc_raw_, seg_discard = unc_discard_;
             sweep(false);
             if (shortened) sync();
             if (shortened && unc_raw_ > unc0) {
-                unc_discard_ += unc_raw_ - unc0;
-                stats_.unconverged = unc_raw_ - unc_discard_;
+                unc_discard_ = seg_discard + unc_raw_ - seg_unc;
                 stats_.redone_steps += n;
                 SFH_HIP(hipMemcpyAsync(gA_, adjSaveZ_, zb, hipMemcpyDeviceToDevice, stream_));
                 SFH_HIP(hipMemcpyAsync(gAP_, adjSaveP_, pb, hipMemcpyDeviceToDevice, stream_));
@@ -2046,9 +2073,8 @@ void Solver::traj_backward(int record, const double* gx_in, const double* gy_in,
                 std::copy(head, head + 4, adj_head_);
                 std::copy(hv, hv + 4, adj_hv_);
                 const int len = sweep_len;
-                adapt = false;
                 sweep(true);
-                if (len > 0) sweep_len = std::min(gm_m_, 2 * len);
+                sweep_len = std::min(gm_m_, 2 * len);
             }
         } else {
             sweep(true);

@@ -338,7 +338,7 @@ class Solver {
                          bool accumulate, int stage);
     // warm starts of the transposed solves over a trajectory's reverse steps (LU and GMRES handles):
     // per RK stage a ring of the last kHistDepth solutions, extrapolated like the forward warm start
-    double* adjRing_ = nullptr;      // 4 stages x kHistDepth x T
+    double* adjRing_ = nullptr;      // 4 stages x kAdjRing x T
     double* adjSave_ = nullptr;      // the rings at the start of a segment (for a redo)
     double2* adjSaveZ_ = nullptr;    // the cotangent at the start of a segment
     double* adjSaveP_ = nullptr;
@@ -364,6 +364,7 @@ class Solver {
         int* HV = nullptr;      // c * hv_len
         size_t hist_len = 0, hv_len = 0;
         std::vector<int> fill_len;   // of the forward pass
+        std::vector<int> unc;        // solves of the forward pass that the full sequence left unconverged, per segment
         std::vector<int> hist_steps;   // hist_steps_ at each checkpoint
     };
     void free_record(TrajRecord& r);
