@@ -178,9 +178,11 @@ __device__ inline double film_eigenvalue(int n, int m, double height) {
 // modes' projections are orthogonal (beyond, mode m is mode n - m again: at n = 3, height 0.107 the sum of the
 // projections is singular).  On films so thin that it would leave many larger ones out it is not used (-1): with less
 // than half of them it can cost steps (N = 512, height 0.02: 42 against 22 without).
-__device__ inline int film_modes(int n, double height) {
+__host__ __device__ inline int film_modes(int n, double height) {
     const double m = height > 0.0 ? log(n * (0.25 / kPi / 0.02)) / (2.0 * height) : 1e9;
-    return m < 2 * kPreModes + 1 ? max(0, min(min(kPreModes, (n - 1) / 2), (int)m)) : -1;
+    if (!(m < 2 * kPreModes + 1)) return -1;
+    const int most = (n - 1) / 2 < kPreModes ? (n - 1) / 2 : kPreModes;
+    return m < 0.0 ? 0 : m < most ? (int)m : most;
 }
 
 // ------------------------------------------------------------------ wave reductions

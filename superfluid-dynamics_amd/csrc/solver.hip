@@ -317,16 +317,25 @@ void Solver::alloc_gmres(int m) {
     gm_small_stride_ = 4LL * (gm_m_ + 1) + 2LL * gm_m_ + (long long)gm_m_ * (gm_m_ + 1);
     gmV_ = dalloc<double>((size_t)(gm_m_ + 1) * T_);
     gmx0_ = dalloc<double>(T_);
-    if (ph_.image && opt_.solver == kSolveGMRES) gmZ_ = dalloc<double>((size_t)(gm_m_ + 1) * T_);
+    const bool thin = ph_.image && film_modes(maxN_, ph_.depth) < 0 && maxN_ > 128 && (ph_.depth >= 0.05 || maxN_ > 2048);
+    if (ph_.image && !thin && opt_.solver == kSolveGMRES) gmZ_ = dalloc<double>((size_t)(gm_m_ + 1) * T_);
     // Products from cotangent sums, which the velocity needs anyway (gm_start_kernel, gm_sums_kernel): the solve stores
     // no matrix and the right-hand side ends in the solve's closing launch.  Per right-hand side with one Arnoldi step,
     // microseconds: N = 2048 water 7.5 + 8 + 8.5 in place of assembly 14.2, product 8, closing 8.2 and velocity 10.2;
     // N = 4096 film 34 + 40 + 17 in place of 38 + 26 + 22 + 33; N = 1536 mixed film 9.4 + 12 + 10 in place of 12 + 5 + 8
     // + 11 and a refinement (10 + 4 + 8).  FP64 throughout, so a mixed-precision handle needs no refinement.
     // Not with the rho quirk, whose node-1 term needs mu' outside a workgroup's rows, nor for solves of one launch,
-    // which have no closing one.
+    // which have no closing one, nor for films too thin for the preconditioner (at their depth; the rule of film_modes):
+    // their solves take 10 to 20 steps, and a film's sums cost more per step than a stored row.  16 steps from a fresh
+    // state, sums / stored FP64 matrix, ms: N = 1024 depth 0.2 18.7 / 16.8, N = 1536 depth 0.2 22.7 / 19.3, N = 2048
+    // depth 0.1 25.4 / 22.5, N = 4096 depth 0.2 54.9 / 42.7.  Below a depth of 0.05 the low modes' eigenvalues are nearly
+    // equal and a solve takes a few steps again: N = 1024 depth 0.02 3.8 / 4.5, N = 2048 depth 0.01 8.5 / 9.3, but N = 3072
+    // depth 0.01 2% to 10% for the matrix.  N = 64 3% to 6% for the sums at every depth.  Mixed-precision handles take
+    // the FP64 matrix there too (an FP32 one with its refinement 24 ms in place of 16.8 at N = 1024, 86 in place of 42.5 at
+    // N = 4096, depth 0.2).
     const bool quirk = ph_.kind == 0 && ph_.rho_quirk && ph_.rho != 0.0;
-    gm_sums_ = opt_.solver == kSolveGMRES && gm_m_ >= 2 && !quirk;
+    gm_sums_ = opt_.solver == kSolveGMRES && gm_m_ >= 2 && !quirk && !thin;
+    gm_f32_ = opt_.solver == kSolveGMRES && opt_.precision == kMixed && !gm_sums_ && !thin;
     if (gm_sums_) {
         const size_t words = (size_t)(gm_m_ + 1) * (ph_.image ? 4 : 2) * T_;
         // every workgroup repeats the finishing work of a step: beyond 2048 nodes, where the workgroups of 4 rows no
@@ -336,7 +345,7 @@ void Solver::alloc_gmres(int m) {
         gmdiag_ = dalloc<double>(T_);
         SFH_HIP(hipMemset(gmS_, 0, words * sizeof(double)));
     }
-    if (opt_.precision == kMixed && opt_.solver == kSolveGMRES && !gm_sums_) M32_ = dalloc<float>(MT_);
+    if (gm_f32_) M32_ = dalloc<float>(MT_);
     SFH_HIP(hipMemset(gmx0_, 0, T_ * sizeof(double)));
     gmw_ = dalloc<double>(2 * (size_t)T_);
     gmpart_ = dalloc<double>(gm_part_stride_ * S_);
@@ -483,7 +492,7 @@ GmArgs Solver::gm_args(int stage) const {
 // last one is gm_close_mu_kernel, which also forms mu' (returns true: no mu_circ_kernel).
 // Mixed precision runs the products over the FP32 matrix (4 bytes per entry).
 bool Solver::enqueue_gmres(const GmArgs& a, bool force64, const double2* Z, const StageCtl* sc) {
-    const bool f32 = opt_.precision == kMixed && !force64;
+    const bool f32 = gm_f32_ && !force64;
     double nsq = 0.0;
     for (int v : n_) nsq += (double)v * v;
     const dim3 grid((maxN_ + a.rpw - 1) / a.rpw, 1, S_);
@@ -558,7 +567,7 @@ bool Solver::enqueue_gmres(const GmArgs& a, bool force64, const double2* Z, cons
 //   warm-start history.
 bool Solver::enqueue_solve(const double2* Z, int stage) {
     if (opt_.solver == kSolveGMRES) {
-        if (opt_.precision != kMixed) return enqueue_gmres(gm_args(stage));
+        if (!gm_f32_) return enqueue_gmres(gm_args(stage));
         GmArgs first = gm_args(stage);
         first.stage = 0;   // no history: the refinement solve stores the solution
         enqueue_gmres(first);
@@ -697,7 +706,7 @@ void Solver::enqueue_rhs(const double2* Z, const double* P, const StageCtl& ctl_
             go(form_small_kernel, sgrid, dim3(256), 0, d_desc_, (const double*)d_circ_, Z, P, Zp_, Zpp_, b_, work_, M_, trig_, ph_,
                status_);
         });
-    } else if (gm_on && opt_.precision == kMixed) {
+    } else if (gm_f32_) {
         launch("assemble", img * nsq, 4.0 * nsq, [&] {
             SFH_WITH_ROWS(rows_, go(assemble32_kernel<R>, dim3((maxN_ + R - 1) / R, S_), dim3(256), 0, d_desc_,
                                     (const NodeTrig*)trig_, Z, Zp_, Zpp_, M32_, ph_, ga));
@@ -893,14 +902,15 @@ void Solver::run_steps(double dt, int len, int count) {
     }
 }
 
-// One step while the warm-start history fills.  The first one runs the full launch sequence; the next ones need no
-// more Arnoldi steps than the one before, as their guesses get better, and get that many launches and two spare
-// ones (a launch after the end of a solve costs 2.5 us: N = 2048 2.1 ms for the six steps' 792 launches).  A step in
-// which a solve ran out of them all the same is run again with the full sequence.  Launched directly: each length
-// would need a graph of its own for one use.
+// One step while the warm-start history fills.  The first one runs the full launch sequence; the next ones mostly need
+// no more Arnoldi steps than the one before, as their guesses get better, and get that many launches, two spare
+// ones and a quarter of the steps more (a launch after the end of a solve costs 2.5 us: N = 2048 2.1 ms for the six
+// steps' 792 launches; thin films, whose 10 to 20 steps vary more, ran out in one of the six without the quarter).  A
+// step in which a solve ran out of them all the same is run again with the full sequence.  Launched directly: each
+// length would need a graph of its own for one use.
 void Solver::fill_step(double dt) {
     if (hist_steps_ == 0 || fill_len_.empty()) fill_len_.assign(kCalibSteps, gm_m_);
-    const int len = hist_steps_ == 0 ? gm_m_ : std::min(gm_m_, std::max(4, most_ + 3));
+    const int len = hist_steps_ == 0 ? gm_m_ : std::min(gm_m_, std::max(4, most_ + 3 + most_ / 4));
     const int raw0 = unc_raw_;
     if (len < gm_m_) save_checkpoint();
     seq_len_ = len;

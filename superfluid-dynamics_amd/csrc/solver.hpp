@@ -287,7 +287,8 @@ class Solver {
     int sums_rpw_ = 0;           // rows per workgroup of those launches
     double* gmS_ = nullptr;
     double* gmdiag_ = nullptr;
-    float* M32_ = nullptr;       // FP32 matrices of the mixed-precision GMRES form
+    bool gm_f32_ = false;        // GMRES, mixed precision with a stored matrix: FP32, and a refinement solve
+    float* M32_ = nullptr;       // its matrices
     int* gmctl_ = nullptr;
     long long gm_part_stride_ = 0, gm_small_stride_ = 0;
     bool enqueue_gmres(const GmArgs& a, bool force64 = false, const double2* Z = nullptr, const StageCtl* sc = nullptr);
