@@ -222,7 +222,6 @@ Solver::Solver(const Phys& ph, const std::vector<int>& n, const Options& opt) : 
     work_ = dalloc<double>(T_);
     y_ = dalloc<double>(T_);
     mu_ = dalloc<double>(T_);
-    M_ = dalloc<double>(MT_);
     trig_ = dalloc<NodeTrig>(T_);
     long long utot = 0;
     for (int s = 0; s < S_; ++s) {
@@ -243,6 +242,7 @@ Solver::Solver(const Phys& ph, const std::vector<int>& n, const Options& opt) : 
     SFH_HIP(hipMemset(mu_, 0, T_ * sizeof(double)));
     SFH_HIP(hipMemset(mup_, 0, T_ * sizeof(double2)));
     if (opt_.solver == kSolveGMRES) alloc_gmres(opt_.max_iter);
+    if (!gm_sums_ && !gm_f32_) M_ = dalloc<double>(MT_);
     if (opt_.solver == kSolveBatched) {
         std::vector<int> ord(S_);
         for (int s = 0; s < S_; ++s) ord[s] = s;

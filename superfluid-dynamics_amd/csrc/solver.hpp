@@ -271,7 +271,7 @@ class Solver {
     double* kP_[3] = {nullptr, nullptr, nullptr};
     double2 *Zp_ = nullptr, *Zpp_ = nullptr, *mup_ = nullptr, *qup_ = nullptr;
     double *b_ = nullptr, *work_ = nullptr, *y_ = nullptr, *mu_ = nullptr;
-    double* M_ = nullptr;
+    double* M_ = nullptr;        // FP64 matrices (not of GMRES handles that store none, or FP32 ones)
     NodeTrig* trig_ = nullptr;
     double* uinv_ = nullptr;
     int* status_ = nullptr;
