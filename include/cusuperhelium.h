@@ -266,11 +266,11 @@ typedef struct sfh_tuning {
     int from_cache;       /* 1 when sfh_tuned found the result in the cache */
     double ms_per_step;   /* measured ms per RK4 step of the chosen form */
 } sfh_tuning;
-/* Times every candidate (LU and GMRES with 1, 2 and 4 rows per workgroup, the batched form for
- * n <= 1024; the mixed forms too when allow_mixed) for `steps` RK4 steps of a seeded surface of n nodes
- * after an 8-step warm-up, keeps the fastest whose solves converge, and caches it per (GPU
- * architecture, kind, image term, n, allow_mixed) in $SFH_TUNE_CACHE, $XDG_CACHE_HOME or
- * ~/.cache (cusuperhelium/tuning.txt). */
+/* Times every candidate (LU, GMRES, the batched form for n <= 1024, with 1, 2 and 4 rows per workgroup and, when
+ * allow_mixed, the mixed form where these change what is launched; else with the defaults) for `steps` RK4 steps of a
+ * seeded surface of n nodes after an 8-step warm-up, keeps the fastest whose solves converge, and caches it per (GPU
+ * architecture, kind, image term, whether GMRES stores its matrix, n, allow_mixed) in $SFH_TUNE_CACHE, $XDG_CACHE_HOME
+ * or ~/.cache (cusuperhelium/tuning.txt). */
 int sfh_autotune(const sfh_props* props, int n, int allow_mixed, int steps, sfh_tuning* out);
 /* The cached result, or sfh_autotune(..., 10, ...) on a miss. */
 int sfh_tuned(const sfh_props* props, int n, int allow_mixed, sfh_tuning* out);

@@ -7,8 +7,9 @@
 // latency (small N) or by FP64 issue (large N), the persistent batched kernel suits N <= 1024, and a workgroup of
 // 4 rows leaves most CUs idle when N / 4 is well below the CU count.  autotune() times each candidate on a seeded 8-mode surface
 // of the handle's physics (warm-up through the GMRES calibration, then timed steps replayed from the
-// step graph), rejects candidates whose solves do not converge, and keeps the fastest.  Results are
-// cached per (GPU architecture, problem kind, image term, N, mixed allowed) in memory and in a text
+// step graph), rejects candidates whose solves do not converge, and keeps the fastest.  Options that the launched
+// kernels do not depend on are not tried (candidates()).  Results are
+// cached per (GPU architecture, problem kind, image term and GMRES route, N, mixed allowed) in memory and in a text
 // file: $SFH_TUNE_CACHE, else $XDG_CACHE_HOME/cusuperhelium/tuning.txt, else
 // $HOME/.cache/cusuperhelium/tuning.txt (memory only when none is writable).
 #include <chrono>
@@ -47,10 +48,19 @@ std::string arch_name() {
     return a.empty() ? std::string("unknown") : a;
 }
 
-std::string key_of(const std::string& arch, const Phys& ph, int n, bool mixed) {
+// The first field carries the version of the kernels that were timed: entries of other versions match no key.  The third
+// is the image term (1), plus 2 where GMRES stores its matrix (rho quirk, thin films) and is another candidate.
+constexpr const char* kTuneVersion = "/2";
+
+int route_of(const Phys& ph, int n) { return (ph.image ? 1 : 0) + (gmres_sums(ph, n, kGmMaxIter) ? 0 : 2); }
+
+std::string key_of(const std::string& arch, int kind, int route, int n, bool mixed) {
     std::ostringstream k;
-    k << arch << ' ' << ph.kind << ' ' << ph.image << ' ' << n << ' ' << (mixed ? 1 : 0);
+    k << arch << ' ' << kind << ' ' << route << ' ' << n << ' ' << (mixed ? 1 : 0);
     return k.str();
+}
+std::string key_of(const Phys& ph, int n, bool mixed) {
+    return key_of(arch_name() + kTuneVersion, ph.kind, route_of(ph, n), n, mixed);
 }
 
 std::string cache_path() {
@@ -73,14 +83,10 @@ void load_file() {
         if (line.empty() || line[0] == '#') continue;
         std::istringstream ls(line);
         std::string arch;
-        int kind, image, n, mixed;
+        int kind, route, n, mixed;
         Tuning t;
-        if (ls >> arch >> kind >> image >> n >> mixed >> t.solver >> t.precision >> t.pair_rows >> t.ms_per_step) {
-            Phys ph{};
-            ph.kind = kind;
-            ph.image = image;
-            g_tunings[key_of(arch, ph, n, mixed != 0)] = t;
-        }
+        if (ls >> arch >> kind >> route >> n >> mixed >> t.solver >> t.precision >> t.pair_rows >> t.ms_per_step)
+            g_tunings[key_of(arch, kind, route, n, mixed != 0)] = t;
     }
 }
 
@@ -97,7 +103,7 @@ void save_file() {
     {
         std::ofstream out(tmp);
         if (!out) return;
-        out << "# arch kind image n mixed_allowed solver precision pair_rows ms_per_step\n";
+        out << "# arch/version kind image+2*stored n mixed_allowed solver precision pair_rows ms_per_step\n";
         for (const auto& kv : g_tunings) {
             const Tuning& t = kv.second;
             out << kv.first << ' ' << t.solver << ' ' << t.precision << ' ' << t.pair_rows << ' ' << t.ms_per_step
@@ -147,6 +153,30 @@ double time_candidate(const Phys& ph, int n, const Options& o, int steps, const 
     }
 }
 
+struct Cand {
+    int solver, precision, rows;
+};
+
+// The forms that differ in what they launch.  Rows per workgroup of the pair kernels matter to LU above 256 nodes and
+// with the rho quirk, and to GMRES with a stored matrix; the mixed form of GMRES only where that matrix is FP32 (water).
+std::vector<Cand> candidates(const Phys& ph, int n, bool allow_mixed) {
+    const bool quirk = ph.kind == 0 && ph.rho_quirk && ph.rho != 0.0;
+    const bool stored = !gmres_sums(ph, n, kGmMaxIter);
+    std::vector<Cand> c;
+    for (int rows : {1, 2, 4}) {
+        if (rows == kPairRows || n > kSmallNodes || quirk) c.push_back({kSolveLU, kFP64, rows});
+        if (n <= kGmMaxN && (rows == kPairRows || stored)) {
+            c.push_back({kSolveGMRES, kFP64, rows});
+            if (allow_mixed && stored && !ph.image) c.push_back({kSolveGMRES, kMixed, rows});
+        }
+    }
+    if (n <= kBatchMaxN) {
+        c.push_back({kSolveBatched, kFP64, kPairRows});
+        if (allow_mixed) c.push_back({kSolveBatched, kMixed, kPairRows});
+    }
+    return c;
+}
+
 }  // namespace
 
 Tuning autotune(const Phys& ph_in, int n, bool allow_mixed, int steps) {
@@ -156,22 +186,9 @@ Tuning autotune(const Phys& ph_in, int n, bool allow_mixed, int steps) {
     ph.drive = ph.augmented = 0;   // the drive's per-node epilogue does not change the ranking
     std::vector<double> x, y, p;
     probe_state(n, x, y, p);
-    struct Cand {
-        int solver, precision, rows;
-    };
-    std::vector<Cand> cands;
-    for (int rows : {1, 2, 4}) {
-        cands.push_back({kSolveLU, kFP64, rows});
-        if (n <= kGmMaxN) cands.push_back({kSolveGMRES, kFP64, rows});
-        if (allow_mixed && n <= kGmMaxN) cands.push_back({kSolveGMRES, kMixed, rows});
-    }
-    if (n <= kBatchMaxN) {
-        cands.push_back({kSolveBatched, kFP64, kPairRows});
-        if (allow_mixed) cands.push_back({kSolveBatched, kMixed, kPairRows});
-    }
     Tuning best;
     best.ms_per_step = INFINITY;
-    for (const Cand& c : cands) {
+    for (const Cand& c : candidates(ph, n, allow_mixed)) {
         Options o;
         o.solver = c.solver;
         o.precision = c.precision;
@@ -188,7 +205,7 @@ Tuning autotune(const Phys& ph_in, int n, bool allow_mixed, int steps) {
     if (!std::isfinite(best.ms_per_step)) throw HipError("autotune: no candidate ran");
     std::lock_guard<std::mutex> lk(g_tune_mu);
     load_file();
-    g_tunings[key_of(arch_name(), ph, n, allow_mixed)] = best;
+    g_tunings[key_of(ph, n, allow_mixed)] = best;
     save_file();
     best.from_cache = 0;
     return best;
@@ -198,7 +215,7 @@ Tuning tuned(const Phys& ph, int n, bool allow_mixed) {
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
         load_file();
-        auto it = g_tunings.find(key_of(arch_name(), ph, n, allow_mixed));
+        auto it = g_tunings.find(key_of(ph, n, allow_mixed));
         if (it != g_tunings.end()) {
             Tuning t = it->second;
             t.from_cache = 1;

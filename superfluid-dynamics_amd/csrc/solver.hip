@@ -303,6 +303,26 @@ std::vector<int> Solver::batched_parts() const {
     return parts;
 }
 
+// Products from cotangent sums, which the velocity needs anyway (gm_start_kernel, gm_sums_kernel): the solve stores
+// no matrix and the right-hand side ends in the solve's closing launch.  Per right-hand side with one Arnoldi step,
+// microseconds: N = 2048 water 7.5 + 8 + 8.5 in place of assembly 14.2, product 8, closing 8.2 and velocity 10.2;
+// N = 4096 film 34 + 40 + 17 in place of 38 + 26 + 22 + 33; N = 1536 mixed film 9.4 + 12 + 10 in place of 12 + 5 + 8
+// + 11 and a refinement (10 + 4 + 8).  FP64 throughout, so a mixed-precision handle needs no refinement.
+// Not with the rho quirk, whose node-1 term needs mu' outside a workgroup's rows, nor for solves of one launch,
+// which have no closing one, nor for films too thin for the preconditioner (at their depth; the rule of film_modes):
+// their solves take 10 to 20 steps, and a film's sums cost more per step than a stored row.  16 steps from a fresh
+// state, sums / stored FP64 matrix, ms: N = 1024 depth 0.2 18.7 / 16.8, N = 1536 depth 0.2 22.7 / 19.3, N = 2048
+// depth 0.1 25.4 / 22.5, N = 4096 depth 0.2 54.9 / 42.7.  Below a depth of 0.05 the low modes' eigenvalues are nearly
+// equal and a solve takes a few steps again: N = 1024 depth 0.02 3.8 / 4.5, N = 2048 depth 0.01 8.5 / 9.3; but N = 3072
+// depth 0.01 7% to 10% less with the matrix, N = 4096 1% to 3% more.  N = 64 3% to 6% less with the sums at every depth.
+// Mixed-precision handles take the FP64 matrix there too (an FP32 one with its refinement 24 ms in place of 16.8 at
+// N = 1024, 86 in place of 42.5 at N = 4096, depth 0.2).
+bool gmres_sums(const Phys& ph, int n, int m) {
+    const bool quirk = ph.kind == 0 && ph.rho_quirk && ph.rho != 0.0;
+    const bool thin = ph.image && film_modes(n, ph.depth) < 0 && n > 128 && (ph.depth >= 0.05 || n > 2048);
+    return m >= 2 && !quirk && !thin;
+}
+
 // GMRES buffers for a Krylov dimension of m (the GMRES solver, and the transposed solves of the
 // multi-workgroup adjoint of the other solvers)
 void Solver::alloc_gmres(int m) {
@@ -317,25 +337,10 @@ void Solver::alloc_gmres(int m) {
     gm_small_stride_ = 4LL * (gm_m_ + 1) + 2LL * gm_m_ + (long long)gm_m_ * (gm_m_ + 1);
     gmV_ = dalloc<double>((size_t)(gm_m_ + 1) * T_);
     gmx0_ = dalloc<double>(T_);
-    const bool thin = ph_.image && film_modes(maxN_, ph_.depth) < 0 && maxN_ > 128 && (ph_.depth >= 0.05 || maxN_ > 2048);
-    if (ph_.image && !thin && opt_.solver == kSolveGMRES) gmZ_ = dalloc<double>((size_t)(gm_m_ + 1) * T_);
-    // Products from cotangent sums, which the velocity needs anyway (gm_start_kernel, gm_sums_kernel): the solve stores
-    // no matrix and the right-hand side ends in the solve's closing launch.  Per right-hand side with one Arnoldi step,
-    // microseconds: N = 2048 water 7.5 + 8 + 8.5 in place of assembly 14.2, product 8, closing 8.2 and velocity 10.2;
-    // N = 4096 film 34 + 40 + 17 in place of 38 + 26 + 22 + 33; N = 1536 mixed film 9.4 + 12 + 10 in place of 12 + 5 + 8
-    // + 11 and a refinement (10 + 4 + 8).  FP64 throughout, so a mixed-precision handle needs no refinement.
-    // Not with the rho quirk, whose node-1 term needs mu' outside a workgroup's rows, nor for solves of one launch,
-    // which have no closing one, nor for films too thin for the preconditioner (at their depth; the rule of film_modes):
-    // their solves take 10 to 20 steps, and a film's sums cost more per step than a stored row.  16 steps from a fresh
-    // state, sums / stored FP64 matrix, ms: N = 1024 depth 0.2 18.7 / 16.8, N = 1536 depth 0.2 22.7 / 19.3, N = 2048
-    // depth 0.1 25.4 / 22.5, N = 4096 depth 0.2 54.9 / 42.7.  Below a depth of 0.05 the low modes' eigenvalues are nearly
-    // equal and a solve takes a few steps again: N = 1024 depth 0.02 3.8 / 4.5, N = 2048 depth 0.01 8.5 / 9.3, but N = 3072
-    // depth 0.01 2% to 10% for the matrix.  N = 64 3% to 6% for the sums at every depth.  Mixed-precision handles take
-    // the FP64 matrix there too (an FP32 one with its refinement 24 ms in place of 16.8 at N = 1024, 86 in place of 42.5 at
-    // N = 4096, depth 0.2).
-    const bool quirk = ph_.kind == 0 && ph_.rho_quirk && ph_.rho != 0.0;
-    gm_sums_ = opt_.solver == kSolveGMRES && gm_m_ >= 2 && !quirk && !thin;
-    gm_f32_ = opt_.solver == kSolveGMRES && opt_.precision == kMixed && !gm_sums_ && !thin;
+    gm_sums_ = opt_.solver == kSolveGMRES && gmres_sums(ph_, maxN_, gm_m_);
+    // a mixed-precision handle with a stored matrix: FP32 (not for thin films, see gmres_sums)
+    gm_f32_ = opt_.solver == kSolveGMRES && opt_.precision == kMixed && !gm_sums_ && !ph_.image;
+    if (ph_.image && gm_sums_) gmZ_ = dalloc<double>((size_t)(gm_m_ + 1) * T_);
     if (gm_sums_) {
         const size_t words = (size_t)(gm_m_ + 1) * (ph_.image ? 4 : 2) * T_;
         // every workgroup repeats the finishing work of a step: beyond 2048 nodes, where the workgroups of 4 rows no

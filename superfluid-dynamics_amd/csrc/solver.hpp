@@ -66,6 +66,9 @@ struct Stats {
 };
 
 bool supported_n(int n);
+// Whether GMRES with m Arnoldi steps forms its products from cotangent sums, for surfaces of up to n nodes (else from a
+// stored matrix).
+bool gmres_sums(const Phys& ph, int n, int m);
 void debug_lu_solve(int n, const double* A, const double* b, double* x, int* interchanged);
 
 // Autotuner (autotune.cpp): the fastest (solver, precision, pair-kernel rows) for one surface of n
