@@ -282,6 +282,7 @@ __device__ inline void back_substitute(const double* g, const double* H, int m, 
 template <typename T, int WAVES, int RR>
 struct StoredRows {
     static constexpr int W = WAVES, ROWS = W * RR, MAXN = kGmMaxN;
+    static constexpr bool PRE = false;
     const T* R;
     RowBuf<T, RR> rc;
     int n, row, rows, lane, wv;
@@ -313,6 +314,7 @@ struct StoredRows {
 template <int NA, int H>
 struct PairSums {
     static constexpr int W = 4 * H, ROWS = kSumRows * H, MAXN = kGmMaxN;
+    static constexpr bool PRE = NA == 4;   // the film's preconditioner
     const NodeTrig* tr;
     double* S;
     NodeTrig tk[kSumRows];
@@ -373,6 +375,7 @@ struct PairSums {
 template <bool FILM, int N>
 struct TransposeSums {
     static constexpr int W = 4, ROWS = kSumRows, MAXN = N;
+    static constexpr bool PRE = false;
     const NodeTrig* tr;
     const double2* zp;
     NodeTrig tk[kSumRows];
@@ -447,7 +450,7 @@ __device__ __forceinline__ void gm_step(const GmArgs& a, const SurfDesc* __restr
     __shared__ double col[kMaxKrylov + 2];
     __shared__ double red8[2 * W];
     __shared__ double wl[rpw], vown[rpw];
-    __shared__ double pred[W][2 * kPreModes + 1], pcoef[2 * kPreModes + 1];
+    __shared__ double pred[P::PRE ? W : 1][2 * kPreModes + 1], pcoef[2 * kPreModes + 1];
     __shared__ double sums[kMaxKrylov + 2];
     __shared__ double ys[kMaxKrylov + 4];   // g[j], gc[j+1], c, s, then y
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6, n = v.n;
@@ -475,8 +478,8 @@ __device__ __forceinline__ void gm_step(const GmArgs& a, const SurfDesc* __restr
         gold = v.gc[j];
         bnorm = ctl->bnorm;
     }
-    const int pre_modes = a.pre ? v.ctl->pre_modes : -1;
-    const double height = a.pre ? v.ctl->height : 0.0;
+    const int pre_modes = P::PRE ? v.ctl->pre_modes : -1;
+    const double height = P::PRE ? v.ctl->height : 0.0;
     // the rows up front, except in a refinement solve, which most often ends at once: there they
     // are fetched when the step is known to run
     const bool early_rows = !a.check_first;
@@ -627,7 +630,7 @@ __device__ __forceinline__ void gm_step(const GmArgs& a, const SurfDesc* __restr
     }
     // ---- step i: w_i = M P^{-1} v_i (v_i = sj * vs) for this workgroup's rows, partial dots v_l . w_i
     if (t < rpw) vown[t] = vs[min(r0 + t, n - 1)];
-    if (a.pre) {
+    if constexpr (P::PRE) {
         __syncthreads();
         const SurfDesc d = sd[blockIdx.z];
         if (pre_modes >= 0) precondition<NT>(vs, n, a.tw + d.twoff, pre_modes, height, pred, pcoef);

@@ -328,10 +328,11 @@ bool gmres_sums(const Phys& ph, int n, int m) {
 void Solver::alloc_gmres(int m) {
     if (gmV_) return;
     gm_m_ = m;   // at most kMaxKrylov basis vectors (gmres.hip)
-    // rows per workgroup of the Arnoldi launches over a stored matrix.  Every workgroup repeats the step's finishing work, so few
-    // large ones are better once they still fill the GPU: N = 4096 film 34.6 ms per 40 steps with 16 rows.  At
-    // N = 2048 (512 workgroups of 4 rows, two per CU) their longer start costs more than it saves: 26.7 ms per
-    // 100 steps with 4 rows, 29.8 with 8 and 28.6 - 31.0 with 16; N = 1536 mixed 18.0, 17.9 and 18.7.
+    // rows per workgroup of the Arnoldi launches over a stored matrix.  Every workgroup repeats the step's finishing
+    // work, so few large ones are better once they still fill the GPU; up to 2048 nodes in all (512 workgroups of 4 rows,
+    // two per CU) their longer start costs more than it saves.  4 / 16 rows, ms for 30 steps of water with the rho quirk:
+    // N = 1024 5.3 / 5.8, N = 2048 7.3 / 8.5, N = 3072 12.8 / 11.7, N = 4096 17.0 / 16.2, 12 surfaces of 256 6.5 / 6.2;
+    // 20 steps of thin films: N = 2048 28.1 / 31.1, N = 4096 92.7 / 67.7, 3 of 1024 30.4 / 24.4, 2 of 1024 19.9 / 23.2.
     gm_rpw_ = T_ <= 2048 ? 4 : 16;
     gm_part_stride_ = 2LL * ((maxN_ + 3) / 4) * (gm_m_ + 1);   // 4: the fewest rows of a workgroup
     gm_small_stride_ = 4LL * (gm_m_ + 1) + 2LL * gm_m_ + (long long)gm_m_ * (gm_m_ + 1);
@@ -343,8 +344,9 @@ void Solver::alloc_gmres(int m) {
     if (ph_.image && gm_sums_) gmZ_ = dalloc<double>((size_t)(gm_m_ + 1) * T_);
     if (gm_sums_) {
         const size_t words = (size_t)(gm_m_ + 1) * (ph_.image ? 4 : 2) * T_;
-        // every workgroup repeats the finishing work of a step: beyond 2048 nodes, where the workgroups of 4 rows no
-        // longer run all at once, two groups of 256 threads share it
+        // every workgroup repeats the finishing work of its surface's step, which grows with that surface: beyond 2048
+        // nodes two groups of 256 threads share it.  4 / 8 rows per workgroup, ms for 40 steps: N = 2048 water 6.7 / 6.7,
+        // film 9.7 / 9.5, N = 4096 15.0 / 14.0 and 24.2 / 22.4, but 3 surfaces of 1024 7.3 / 7.6 and 10.5 / 11.1.
         sums_rpw_ = maxN_ <= 2048 ? 4 : 8;
         gmS_ = dalloc<double>(words);
         gmdiag_ = dalloc<double>(T_);
