@@ -434,9 +434,13 @@ int sfh_get_stats(sfh_handle h, sfh_stats* out);
 int sfh_device_state(sfh_handle h, void** Z, void** phi);
 /* Kernel timing.  While enabled, sfh_step / sfh_rhs launch without graph replay and bracket
  * every kernel launch with hipEvents on the solver's stream.  sfh_kernel_report sums, for one
- * kernel tag ("deriv", "assemble", "lu_step", "lu_backsolve", "mu_deriv", "velocity", and the GMRES
- * tags "gm_iter", "gm_close", "gm_close_mu"), the launches, milliseconds, algorithmic flops and algorithmic bytes recorded since
- * timing was enabled.  No counterpart in the reference (it has no timers). */
+ * kernel tag, the launches, milliseconds, algorithmic flops and algorithmic bytes recorded since timing was
+ * enabled.  Tags: "deriv", "assemble", "mu_deriv", "velocity"; LU "lu_step", "lu_backsolve" (up to 256 nodes
+ * "assemble" forms the derivatives too and "velocity" mu'); GMRES "gm_iter" (a launch that runs an Arnoldi step),
+ * "gm_close" (one that finds its solve finished), with a stored matrix "gm_close_mu" (the launch that ends the
+ * solve and forms mu') and for an FP32 one "residual" and "gm_refine", without one "gm_start" and no other closing launch than "velocity", which also ends the
+ * solve; BATCHED "stage"; reverse mode "vjp" or "vjp_fwd", "vjp_pairs", "vjp_solve".  No counterpart in the
+ * reference (it has no timers). */
 int sfh_kernel_timing(sfh_handle h, int enable);
 int sfh_kernel_report(sfh_handle h, const char* tag, int* launches, double* ms, double* flops, double* bytes);
 

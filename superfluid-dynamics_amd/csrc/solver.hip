@@ -534,9 +534,8 @@ bool Solver::enqueue_gmres(const GmArgs& a, bool force64, const double2* Z, cons
     }
     if (fused) {
         // finishing the last step + x += V y + mu' = D1 mu: the rebuild and the circulant product; with the solve's
-        // sums also the velocity and the stage (a sequence of two launches, the steady case, is timed as the velocity
-        // that it ends in)
-        launch(a.sums && a.m == 2 ? "velocity" : "gm_close_mu", 4.0 * a.m * T_ + 4.0 * nsq, 8.0 * (a.m + 2) * T_ + 24.0 * nsq / kCircRowsPerWG, [&] {
+        // sums it is the right-hand side's velocity and stage launch and timed as that
+        launch(a.sums > 0 ? "velocity" : "gm_close_mu", 4.0 * a.m * T_ + 4.0 * nsq, 8.0 * (a.m + 2) * T_ + 24.0 * nsq / kCircRowsPerWG, [&] {
             go(a.sums == 2 ? gm_close_mu_kernel<false, 2> : a.sums == 4 ? gm_close_mu_kernel<true, 4> : gm_close_mu_kernel<false, 0>,
                dim3((maxN_ + kCircRowsPerWG - 1) / kCircRowsPerWG, S_), dim3(256), 0, a, (const SurfDesc*)d_desc_,
                (const double*)d_circ_, mup_, a.m - 1, Z, (const double2*)Zpp_, ph_, sc ? *sc : StageCtl{});
