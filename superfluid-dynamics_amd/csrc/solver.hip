@@ -1474,10 +1474,10 @@ void debug_lu_solve(int n_in, const double* A_in, const double* b_in, double* x_
     double *dA, *dA0, *dwork, *dy, *dx, *duinv, *db;
     int *dstatus, *dpiv, *dcnt;
     SurfDesc desc{};
-    desc.n = n;
+    desc.n = n_in;   // with interchanges: the system as it is
     SurfDesc* ddesc;
     SFH_HIP(hipMalloc(&dA, sizeof(double) * n * n));
-    SFH_HIP(hipMalloc(&dA0, sizeof(double) * n * n));
+    SFH_HIP(hipMalloc(&dA0, sizeof(double) * n_in * n_in));
     SFH_HIP(hipMalloc(&dwork, sizeof(double) * n));
     SFH_HIP(hipMalloc(&db, sizeof(double) * n));
     SFH_HIP(hipMalloc(&dy, sizeof(double) * n));
@@ -1489,7 +1489,7 @@ void debug_lu_solve(int n_in, const double* A_in, const double* b_in, double* x_
     SFH_HIP(hipMalloc(&ddesc, sizeof(SurfDesc)));
     SFH_HIP(hipMemcpy(ddesc, &desc, sizeof(desc), hipMemcpyHostToDevice));
     SFH_HIP(hipMemcpy(dA, A.data(), sizeof(double) * n * n, hipMemcpyHostToDevice));
-    SFH_HIP(hipMemcpy(dA0, A.data(), sizeof(double) * n * n, hipMemcpyHostToDevice));
+    SFH_HIP(hipMemcpy(dA0, A_in, sizeof(double) * n_in * n_in, hipMemcpyHostToDevice));
     SFH_HIP(hipMemcpy(dwork, b.data(), sizeof(double) * n, hipMemcpyHostToDevice));
     SFH_HIP(hipMemcpy(db, b.data(), sizeof(double) * n, hipMemcpyHostToDevice));
     SFH_HIP(hipMemset(dstatus, 0, sizeof(int) * 2));
@@ -1508,8 +1508,7 @@ void debug_lu_solve(int n_in, const double* A_in, const double* b_in, double* x_
     SFH_HIP(hipMemcpyAsync(status, dstatus, sizeof(status), hipMemcpyDeviceToHost, st));
     SFH_HIP(hipStreamSynchronize(st));
     if (status[0]) {
-        SFH_HIP(hipMemcpyAsync(dA, dA0, sizeof(double) * n * n, hipMemcpyDeviceToDevice, st));
-        hipLaunchKernelGGL(gepp_fallback_kernel, dim3(1), dim3(256), 0, st, ddesc, dA, db, dx, dpiv, dstatus, dcnt);
+        hipLaunchKernelGGL(gepp_fallback_kernel, dim3(1), dim3(256), 0, st, ddesc, dA0, db, dx, dpiv, dstatus, dcnt);
         SFH_HIP(hipGetLastError());
     }
     SFH_HIP(hipMemcpyAsync(x.data(), dx, sizeof(double) * n, hipMemcpyDeviceToHost, st));
