@@ -1894,7 +1894,11 @@ int Solver::traj_forward(double dt, int steps, int every) {
         }
         rr.hist_steps.assign(nck, 0);
         rr.unc.assign(nck, 0);
-        check_status();
+        // step() leaves the count of unconverged solves current but where it runs full sequences without a check
+        const auto current = [&] {
+            if (opt_.solver == kSolveGMRES && trim_ >= gm_m_) check_status();
+            return stats_.unconverged;
+        };
         for (int c = 0; c < nck; ++c) {
             SFH_HIP(hipMemcpyAsync(rr.Z + (size_t)c * T_, Z0_, T_ * sizeof(double2), hipMemcpyDeviceToDevice, stream_));
             SFH_HIP(hipMemcpyAsync(rr.P + (size_t)c * T_, P0_, T_ * sizeof(double), hipMemcpyDeviceToDevice, stream_));
@@ -1906,12 +1910,9 @@ int Solver::traj_forward(double dt, int steps, int every) {
                                        stream_));
             }
             rr.hist_steps[c] = hist_steps_;
-            const int unc = stats_.unconverged;
+            const int unc = current();
             step(dt, std::min(every, steps - c * every));
-            if (opt_.solver == kSolveGMRES) {
-                check_status();
-                rr.unc[c] = stats_.unconverged - unc;
-            }
+            rr.unc[c] = current() - unc;
         }
         rr.fill_len = fill_len_;
         check_status();
