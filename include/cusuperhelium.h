@@ -207,9 +207,9 @@ enum { SFH_WATER = 0, SFH_HELIUM = 1 };
 enum { SFH_FP64 = 0, SFH_MIXED = 1 };
 /* LU: blocked FP64 LU (the reference's getrf/getrs semantics), one surface at a time or uniform
  * batches.  GMRES: FP64 GMRES, all surfaces of the handle at once (every N <= 4096), its products
- * evaluated from the pair sums that the velocity needs too.  With max_iter 1 or under
- * rho_quirk (rho != 0) the matrix is stored instead; only there SFH_MIXED makes a difference (the
- * matrix in FP32, r0 and a refinement residual in FP64).
+ * evaluated from the pair sums that the velocity needs too.  With max_iter 1, under rho_quirk
+ * (rho != 0) and on thin films (depth below 0.2 to 0.3, by size) the matrix is stored instead, for water
+ * with SFH_MIXED in FP32 (r0 and a refinement residual in FP64); elsewhere SFH_MIXED makes no difference.
  * BATCHED: one persistent launch per RK stage, one workgroup per surface or, with fewer surfaces than
  * CUs, several for the large ones (every N <= 1024), GMRES inside; with SFH_MIXED a stored matrix is
  * FP32 and mu is refined in FP64 against a matrix-free FP64 residual. */
@@ -236,8 +236,8 @@ typedef struct sfh_options {
     int precision;    /* SFH_FP64 (the drop-in arithmetic) or SFH_MIXED (SFH_SOLVE_BATCHED or _GMRES) */
     int solver;       /* SFH_SOLVE_LU, SFH_SOLVE_GMRES or SFH_SOLVE_BATCHED */
     int use_graph;    /* replay RK4 steps from a captured hipGraph */
-    int max_iter;     /* SFH_SOLVE_GMRES: Arnoldi steps per solve, 1..32 (sfh_create rejects more: the
-                         launch sequence has no restart); SFH_SOLVE_BATCHED: GMRES iteration cap,
+    int max_iter;     /* SFH_SOLVE_GMRES: launches per solve, 1..32, the last of which only ends it: at most
+                         max_iter - 1 Arnoldi steps (sfh_create rejects more: there is no restart); SFH_SOLVE_BATCHED: GMRES iteration cap,
                          rounded up to restart cycles of 8 */
     int restart;      /* unused (0): the GMRES of SFH_SOLVE_GMRES does not restart, the in-workgroup
                          GMRES of SFH_SOLVE_BATCHED restarts every 8 basis vectors */
@@ -289,7 +289,7 @@ typedef struct sfh_stats {
     int redone_steps;      /* SFH_SOLVE_GMRES: steps run again because a solve of their chunk ran out of
                               launches of the trimmed sequence (accumulated) */
     int sequence_length;   /* SFH_SOLVE_GMRES: launches per solve of the trimmed step graph, 0 while the
-                              warm-start history fills (then every solve gets max_iter + 1) */
+                              warm-start history fills (then it follows each step's need) */
     int solver;            /* the form the handle runs (what SFH_SOLVE_AUTO resolved to) */
     int precision;
     int pair_rows;
@@ -438,8 +438,8 @@ int sfh_device_state(sfh_handle h, void** Z, void** phi);
  * enabled.  Tags: "deriv", "assemble", "mu_deriv", "velocity"; LU "lu_step", "lu_backsolve" (up to 256 nodes
  * "assemble" forms the derivatives too and "velocity" mu'); GMRES "gm_iter" (a launch that runs an Arnoldi step),
  * "gm_close" (one that finds its solve finished), with a stored matrix "gm_close_mu" (the launch that ends the
- * solve and forms mu') and for an FP32 one "residual" and "gm_refine", without one "gm_start" and no other closing launch than "velocity", which also ends the
- * solve; BATCHED "stage"; reverse mode "vjp" or "vjp_fwd", "vjp_pairs", "vjp_solve".  No counterpart in the
+ * solve and forms mu') and for an FP32 one "residual" and "gm_refine", without one "gm_start" and no other
+ * closing launch than "velocity", which also ends the solve; BATCHED "stage"; reverse mode "vjp" or "vjp_fwd", "vjp_pairs", "vjp_solve".  No counterpart in the
  * reference (it has no timers). */
 int sfh_kernel_timing(sfh_handle h, int enable);
 int sfh_kernel_report(sfh_handle h, const char* tag, int* launches, double* ms, double* flops, double* bytes);

@@ -13,7 +13,7 @@
 //   gm_start_kernel       cotangent sums of the initial guess, first residual
 //   gm_sums_kernel        one launch per Arnoldi step: the sums of a basis vector, of which the product is a combination
 //   gm_close_mu_kernel    mu, mu', the velocity from the sums of the solve, dPhi/dt and the stage update
-// (with the rho quirk, and with sequences of one launch, GMRES runs on the stored matrix: assemble64_kernel or
+// (with the rho quirk, on thin films and with sequences of one launch GMRES runs on a stored matrix: assemble64_kernel or
 // assemble32_kernel, gm_iter_kernel, gm_close_mu_kernel or mu_circ_kernel, velocity_stage_kernel)
 // and one RK4 step (AutonomousRungeKuttaStepper.cuh:123-361) is four of them.  The step is
 // captured once into a hipGraph and replayed, so a run of many steps costs one graph launch
@@ -49,8 +49,8 @@ namespace sfh {
     else if ((n) <= 1024 || (n) > 2048) { constexpr int TC = 256, TR = 1; __VA_ARGS__; } \
     else { constexpr int TC = 512, TR = 1; __VA_ARGS__; }
 
-// Steps that run every solve with the full launch cap: kHistDepth while the warm-start history
-// fills, then one with the full history that sets the trimmed length.
+// Steps from a fresh state to the trimmed launch sequence: kHistDepth while the warm-start history
+// fills, then one with the full history that sets the length.
 constexpr int kCalibSteps = kHistDepth + 1;
 // Longest chunk of trimmed steps between two checks.
 constexpr int kCheckSteps = 32;
@@ -1425,7 +1425,9 @@ void Solver::parse_status() {
         stats_.unconverged = unc;
         stats_.refinements = bs[2];
     }
-    if (timeouts) throw HipError("back-substitution wait timed out; results are invalid");
+    if (timeouts)
+        throw HipError(opt_.solver == kSolveBatched ? "a wait between the workgroups of a surface timed out; results are invalid"
+                                                    : "back-substitution wait timed out; results are invalid");
     if (cnt[1])
         throw NonFiniteError("non-finite right-hand side (NaN or infinite state, or coincident nodes); set a new state");
 }
@@ -1609,7 +1611,8 @@ void Solver::enqueue_vjp(const double2* Z, const double* P, const double* mu, co
 
 // The reverse pass over many workgroups per surface (adjoint_mwg.hip), at the state (Z, P) with its
 // forward mu: the derivatives and mu' of the state, pass A, D1 of the cotangent of mu', pass B, the
-// transposed solve M^T gb = gmu (the GMRES launch sequence, products from sums over the pairs), the matrix terms and pair weights, pass C, and the spectral adjoints.
+// transposed solve M^T gb = gmu (the GMRES launch sequence, products from sums over the pairs), the matrix
+// terms and pair weights, pass C, and the spectral adjoints.
 void Solver::enqueue_vjp_mwg(const double2* Z, const double* P, const double* mu, const double2* gAZ,
                              const double* gAP, double ca, const double2* gBZ, const double* gBP, double cb,
                              double2* outZ, double* outP, bool accumulate, int stage) {

@@ -41,7 +41,7 @@ struct Options {
     int precision = kFP64;
     int solver = kSolveLU;
     int use_graph = 1;
-    int max_iter = 32;       // GMRES Arnoldi steps per solve (at most kGmMaxIter) / batched GMRES cap
+    int max_iter = 32;       // GMRES launches per solve (at most kGmMaxIter), one more than Arnoldi steps / batched GMRES cap
     int restart = 0;         // unused: the multi-workgroup GMRES does not restart, the batched one
                              // restarts every 8 vectors
     int force_trim = 0;      // test hook: trimmed GMRES sequence length instead of the calibrated one
@@ -66,7 +66,7 @@ struct Stats {
 };
 
 bool supported_n(int n);
-// Whether GMRES with m Arnoldi steps forms its products from cotangent sums, for surfaces of up to n nodes (else from a
+// Whether GMRES with m launches per solve forms its products from cotangent sums, for surfaces of up to n nodes (else from a
 // stored matrix).
 bool gmres_sums(const Phys& ph, int n, int m);
 void debug_lu_solve(int n, const double* A, const double* b, double* x, int* interchanged);
@@ -328,7 +328,7 @@ class Solver {
     double *gAP_ = nullptr, *gRP_[2] = {nullptr, nullptr}, *gAccP_ = nullptr;
     AdjNode* adj_ = nullptr;
     int* vstats_ = nullptr;
-    // multi-workgroup reverse mode (LU and GMRES handles): M^T and the per-node vectors of adjoint_mwg.hip
+    // multi-workgroup reverse mode (LU and GMRES handles): the per-node vectors of adjoint_mwg.hip
     double2 *agwc_ = nullptr, *agmup_ = nullptr, *ad1_ = nullptr, *agam_ = nullptr, *agamI_ = nullptr;
     double2 *agzp_ = nullptr, *agzpp_ = nullptr, *agz_ = nullptr;
     double *agmu_ = nullptr, *agb_ = nullptr;
@@ -387,10 +387,10 @@ class Solver {
     double graph_dt_ = 0.0;
     int graph_len_ = 0;
     // GMRES launch sequence per solve.  The step graph holds a fixed number of Arnoldi launches per
-    // solve (launches after convergence return at once but still cost a dispatch each).  While the
-    // warm-start history fills (the first kHistDepth steps after set_state) and for one step with
-    // the full history, every solve gets the full cap gm_m_; afterwards the sequence is trimmed to
-    // what the solves of that last step needed (one launch per Arnoldi step, one to finish, a spare
+    // solve (launches after convergence return at once but still cost a dispatch each).  The first
+    // step after set_state gets the full cap gm_m_ for every solve; while the warm-start history fills
+    // (kHistDepth steps) and for one step with the full history each step follows the need of the one
+    // before (fill_step); afterwards the sequence is trimmed to what the solves of that last step needed (one launch per Arnoldi step, one to finish, a spare
     // step when they needed 3 or more), and doubled (up to the cap) whenever a check finds a solve
     // that ran out of launches.  seq_len_ is the length the kernels are being enqueued with.
     // A trimmed sequence is run in chunks of steps.  Before a chunk the state, the last solution and

@@ -261,7 +261,7 @@ __global__ __launch_bounds__(TC * TR) void mu_circ_kernel(const SurfDesc* __rest
     }
 }
 
-// (TC, TR) that Solver::circ_shape may choose
+// (TC, TR) that SFH_WITH_CIRC (solver.hip) chooses
 #define SFH_CIRC_INSTANCES(TC, TR)                                                                                 \
     template __global__ void zphi_circ_kernel<TC, TR>(const SurfDesc*, const double*, const double2*, const double*, \
                                                       double2*, double2*, double*, double*, Phys, int*, NodeTrig*,  \
