@@ -909,14 +909,15 @@ void Solver::run_steps(double dt, int len, int count) {
 }
 
 // One step while the warm-start history fills.  The first one runs the full launch sequence; the next ones mostly need
-// no more Arnoldi steps than the one before, as their guesses get better, and get that many launches, two spare
-// ones and a quarter of the steps more (a launch after the end of a solve costs 2.5 us: N = 2048 2.1 ms for the six
-// steps' 792 launches; thin films, whose 10 to 20 steps vary more, ran out in one of the six without the quarter).  A
-// step in which a solve ran out of them all the same is run again with the full sequence.  Launched directly: each
-// length would need a graph of its own for one use.
+// no more Arnoldi steps than the one before, as their guesses get better, and get that many launches and two spare
+// ones (a launch after the end of a solve costs 2.5 us: N = 2048 2.1 ms for the six steps' 792 launches).  Thin films,
+// whose 10 to 20 steps vary more and ran out in one of the six, get a quarter of the steps more (elsewhere that costs a
+// water trajectory of three steps 2% and gains nothing).  A step in which a solve ran out of them all the same is run
+// again with the full sequence.  Launched directly: each length would need a graph of its own for one use.
 void Solver::fill_step(double dt) {
     if (hist_steps_ == 0 || fill_len_.empty()) fill_len_.assign(kCalibSteps, gm_m_);
-    const int len = hist_steps_ == 0 ? gm_m_ : std::min(gm_m_, std::max(4, most_ + 3 + most_ / 4));
+    const int more = ph_.image && !gm_sums_ ? most_ / 4 : 0;
+    const int len = hist_steps_ == 0 ? gm_m_ : std::min(gm_m_, std::max(4, most_ + 3 + more));
     const int raw0 = unc_raw_;
     if (len < gm_m_) save_checkpoint();
     seq_len_ = len;
